@@ -120,6 +120,43 @@ def test_linear(ops, dtype, m, n, k):
     assert rel(acc.cpu(), base.double().cpu() + want) < 1e-5
 
 
+# The tiles of eight wavefronts (256 and 128 rows by 256) at the edges of tiles, with one, two and three steps along k, columns that
+# do and do not allow 16 bytes a store; by the rule of the launcher: large tiles alone, half tiles alone, both in one launch.
+@pytest.mark.parametrize("kind", ["plain", "packed", "rotary"])
+@pytest.mark.parametrize("m,n,k", [(250, 61001, 64), (257, 47104, 128), (130, 61440, 192), (520, 16128, 320), (1100, 16000, 128), (2048, 11008, 64)])
+def test_linear_large_tiles(ops, m, n, k, kind):
+    if kind == "rotary" and n % 256 != 0:
+        pytest.skip("whole heads")
+    a = rand(m, k, dtype=torch.bfloat16, seed=m)
+    w = rand(n, k, dtype=torch.bfloat16, seed=n, scale=0.1)
+    want = (a.double() @ w.double().t()).cpu()
+    w = w if kind == "plain" else ops.pack(w, "tiles") if kind == "packed" else ops.pack(w, "rotary", head_dim=128, rotated_heads=n // 256)
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops.linear(a, w, out)
+    assert rel(out.cpu(), want) < ULP["bfloat16"] * 2           # the rounding of the result
+    base = rand(m, n, seed=5)
+    acc = base.clone()
+    ops.linear(a, w, acc, accumulate=True)
+    assert rel(acc.cpu(), base.double().cpu() + want) < 1e-5    # float32 sums
+    out32 = torch.empty(m, n, device=DEV)
+    ops.linear(a, w, out32)
+    assert rel(out32.cpu(), want) < 1e-5
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("m,n,k", [(250, 30504, 64), (257, 24000, 128), (140, 31000, 192), (520, 8200, 320), (2048, 5504, 64)])
+def test_linear_glu_large_tiles(ops, m, n, k, packed):
+    a = rand(m, k, dtype=torch.bfloat16, seed=m)
+    w = rand(2 * n, k, dtype=torch.bfloat16, seed=n, scale=0.3)
+    both = a.double() @ w.double().t()
+    want = P.swiglu(both[:, :n], both[:, n:]).cpu()
+    w = packed_or_not(ops, w, packed, "gated", gated_n=n)
+    for dtype in (torch.bfloat16, torch.float32):
+        out = torch.empty(m, n, dtype=dtype, device=DEV)
+        ops.linear_glu(a, w, out)
+        assert rel(out.cpu(), want) < (ULP["bfloat16"] * 2 if dtype == torch.bfloat16 else 1e-5)
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16", "bfloat16 packed"])
 @pytest.mark.parametrize("m,n,k", [(1, 176, 64), (9, 100, 96), (64, 520, 200), (200, 1000, 72), (48, 2000, 520),
                                    (3, 8, 32), (16, 24, 160), (30, 1000, 96), (64, 4104, 224), (8, 14336, 4096),

@@ -14,13 +14,13 @@ inline int activation_of(int mode) { return mode >> 8; }
 
 // QUICK: the exponential and the division by the hardware's own instructions (a few units in the last place of a
 // float32), for results that are rounded to bfloat16 anyway: five instructions where the exact ones take some thirty,
-// which a tile of a prefill's gate/up product pays 64 times a lane.
+// which a tile of a prefill's gate/up product pays 64 times a lane. (__frcp_rn would be the exact division again.)
 template <bool QUICK = false>
 __device__ __forceinline__ float gate_activation(float z, int activation) {
     switch (activation) {
         case XRT_ACT_SILU:
         default:                                    // silu(z) = z / (1 + exp(-z)): crates/xrt-kernels/src/cpu/silu.rs:1-3 of the reference
-            if constexpr (QUICK) return z * __frcp_rn(1.0f + __expf(-z));
+            if constexpr (QUICK) return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z));
             else return z / (1.0f + expf(-z));
     }
 }

@@ -1,7 +1,8 @@
 // Matrix product for many rows (prefill), bfloat16 operands, float32 accumulation on the
 // matrix cores: out[m, n] = sum_k a[m, k] * w[n, k]; both operands are contiguous along k.
 //
-// A workgroup computes a BM x BN tile of the output with v_mfma_f32_32x32x16_bf16. Tiles of
+// The large tiles (256 or 128 rows by 256, eight wavefronts; K a multiple of 64) are gemm_large_tile. In the others
+// a workgroup computes a BM x BN tile of the output with v_mfma_f32_32x32x16_bf16. Tiles of
 // a and w travel through LDS, several steps ahead of the matrix cores, with one barrier per
 // step. When K is a multiple of 64 they are loaded from global memory straight into LDS, in a
 // swizzled layout; otherwise they pass through registers into rows padded by 16 bytes (64 wide
@@ -18,6 +19,7 @@
 // them (rows n and n + N of w), arranged so that each wavefront holds both of a pair.
 #include <climits>
 #include <cstdlib>
+#include <type_traits>
 #include "packing.h"
 #include "gemm_skinny.h"
 #include "activation.h"
@@ -26,19 +28,37 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+
+template <typename T> struct alignas(sizeof(T) * 4) Four { T e[4]; };
 
 constexpr int BK = 64;
 constexpr int PITCH = BK + 8;          // bf16 elements per LDS row
 enum { MODE_STORE = 0, MODE_ACCUMULATE = 1, MODE_GATED = 2 };
 
+// Which tile of tiles_m x tiles_n a workgroup takes. Ids are dealt to the XCDs round-robin: each XCD gets a contiguous run of
+// tiles, and a run is walked n-fastest inside panels of 8 n-tiles, so that the tiles that run at one time on an XCD share a
+// and w in its L2. An id beyond the tiles (grids are whole rounds over the XCDs) has none: m is negative.
+struct TilePlace { int m, n; };
+__device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, int tiles_n) {
+    const int total = tiles_m * tiles_n;
+    const int xcds = 8;
+    id = (id % xcds) * ((total + xcds - 1) / xcds) + id / xcds;
+    if (id >= total) return TilePlace{-1, 0};
+    constexpr int PANEL = 8;
+    const int panel = id / (PANEL * tiles_m), in_panel = id % (PANEL * tiles_m);
+    const int panel_width = min(PANEL, tiles_n - panel * PANEL);
+    return TilePlace{in_panel / panel_width, panel * PANEL + in_panel % panel_width};
+}
 
-// One tile of the product, by one workgroup: `id` is the workgroup's number among those that work
-// on the output columns from n_first on, tiles_m x tiles_n of them.
 // The rows of a that come without their RMSNorm's division (see xrt_linear_norm in xrt_hip.h): the sums of
 // squares per tile of 16 columns, from which a tile of up to 64 rows works out 1 / rms of its rows and
 // multiplies its sums by it before the epilogue. squares null: nothing of the kind.
 struct RowScale { const float* squares; int tiles; int width; float eps; int activation; };     // (activation: of a gated epilogue)
 
+// One tile of the product, by one workgroup: `id` is the workgroup's number among those that work
+// on the output columns from n_first on, tiles_m x tiles_n of them.
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO>
 __device__ __forceinline__ void gemm_tile(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
@@ -54,25 +74,11 @@ __device__ __forceinline__ void gemm_tile(
     bf16* lds_a = reinterpret_cast<bf16*>(lds_raw);                    // [2][BM][PITCH]; laid out differently on the direct path
     bf16* lds_b = lds_a + 2 * BM * PITCH;                              // [2][BN][PITCH]
 
-    // ---- which tile: ids are dealt to XCDs round-robin; give each XCD a contiguous run of tiles,
-    // and walk a run m-fastest inside panels of 8 n-tiles so that concurrent tiles share w
-    const int total = tiles_m * tiles_n;
-    {
-        const int xcds = 8;
-        const int per = (total + xcds - 1) / xcds;
-        const int mapped = (id % xcds) * per + id / xcds;
-        id = mapped;
-    }
-    if (id >= total) return;
-    constexpr int PANEL = 8;
-    const int panel = id / (PANEL * tiles_m);
-    const int in_panel = id % (PANEL * tiles_m);
-    const int panel_width = min(PANEL, tiles_n - panel * PANEL);
-    const int tile_n = panel * PANEL + in_panel % panel_width;
-    const int tile_m = in_panel / panel_width;
-    const long m0 = (long)tile_m * BM;
+    const TilePlace place = tile_place(id, tiles_m, tiles_n);
+    if (place.m < 0) return;
+    const long m0 = (long)place.m * BM;
     constexpr int BN_OUT = MODE == MODE_GATED ? BN / 2 : BN;          // output columns of a tile
-    const long n0 = n_first + (long)tile_n * BN_OUT;      // this launch covers output columns from n_first on
+    const long n0 = n_first + (long)place.n * BN_OUT;      // this launch covers output columns from n_first on
 
     const int tid = threadIdx.x, lane = tid % XRT_WAVE, wave = tid / XRT_WAVE;
     const int wave_m = wave / WN, wave_n = wave % WN;
@@ -459,6 +465,380 @@ __device__ __forceinline__ void gemm_tile(
     }
 }
 
+// ---- the large tiles' small pieces
+// The upper 32 lanes of `low` change places with the lower 32 lanes of `high`.
+__device__ __forceinline__ void exchange_halves(float& low, float& high) {
+    const auto both = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, low), __builtin_bit_cast(unsigned, high), false, false);
+    const unsigned first = both[0], second = both[1];          // (a vector's element itself is not what a bit cast takes)
+    low = __builtin_bit_cast(float, first);
+    high = __builtin_bit_cast(float, second);
+}
+// In every row of 16 lanes the upper eight lanes of `low` change places with the lower eight lanes of `high`.
+__device__ __forceinline__ void exchange_eights(unsigned& low, unsigned& high) {
+    const unsigned l = low, h = high;
+    low = __builtin_amdgcn_update_dpp(l, h, 0x128 /* row_ror:8 */, 0xf, 0xc /* lanes 8 to 15 */, false);
+    high = __builtin_amdgcn_update_dpp(h, l, 0x128, 0xf, 0x3 /* lanes 0 to 7 */, false);
+}
+__device__ __forceinline__ void exchange_eights(float& low, float& high) {
+    unsigned l = __builtin_bit_cast(unsigned, low), h = __builtin_bit_cast(unsigned, high);
+    exchange_eights(l, h);
+    low = __builtin_bit_cast(float, l);
+    high = __builtin_bit_cast(float, h);
+}
+template <typename TO>
+__device__ __forceinline__ unsigned two_bf16(float a, float b) {
+    return (unsigned)__builtin_bit_cast(unsigned short, from_float<bf16>(a)) | (unsigned)__builtin_bit_cast(unsigned short, from_float<bf16>(b)) << 16;
+}
+// Four values of each of two blocks, rounded to bfloat16, exchanged between the two rows of 16 lanes of each half of the
+// wavefront: the first row gets the first block's values of both rows (eight neighbours), the second row the second block's.
+template <typename TO>
+__device__ __forceinline__ uint4v join_rows(const float (&first)[4], const float (&second)[4]) {
+    const auto low = __builtin_amdgcn_permlane16_swap(two_bf16<TO>(first[0], first[1]), two_bf16<TO>(second[0], second[1]), false, false);
+    const auto high = __builtin_amdgcn_permlane16_swap(two_bf16<TO>(first[2], first[3]), two_bf16<TO>(second[2], second[3]), false, false);
+    return uint4v{low[0], high[0], low[1], high[1]};
+}
+// Four neighbouring columns of a row of out [M][N], in one piece where `wide` says that rows and columns allow it.
+template <typename TO>
+__device__ __forceinline__ void load_four(const TO* out, long m, long n, int M, int N, float (&v)[4], bool wide) {
+    const TO* row = out + min(m, (long)M - 1) * (long)N;       // (rows and columns beyond the matrix: something inside, not used)
+    if (wide) {
+        const Four<TO> four = *reinterpret_cast<const Four<TO>*>(row + min(n, (long)N - 4));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = to_float(four.e[e]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = to_float(row[min(n + e, (long)N - 1)]);
+    }
+}
+template <typename TO>
+__device__ __forceinline__ void store_four(TO* out, long m, long n, int M, int N, const float (&v)[4], bool wide) {
+    if (m >= M || n >= N) return;
+    TO* row = out + m * (long)N;
+    if (wide) {
+        Four<TO> four;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) four.e[e] = from_float<TO>(v[e]);
+        *reinterpret_cast<Four<TO>*>(row + n) = four;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < N) row[n + e] = from_float<TO>(v[e]);
+    }
+}
+
+constexpr int LARGE_BN = 256;
+
+// The large tiles: eight wavefronts, two to a SIMD, BM x 256, for K that is a multiple of 64; any split of k and all three epilogues.
+//
+// What bounds them is the chip's power: run without a pause on random operands the clock falls to 1.5 GHz, and what counts is
+// the energy of a product, not its cycles. v_mfma_f32_16x16x32_bf16 moves half as many partial sums per product through the
+// registers as the 32x32x16 instruction does: on operands that stay in registers 2060 against 1820 TFLOP/s (zeros, which cost
+// no power: 2430 and 2460). The instruction's A operand is w and its B operand x, so that a lane ends up with four
+// neighbouring columns of one row of the output, and the epilogue moves 16 bytes a lane.
+//
+// The wavefronts take turns: of the two on a SIMD (one of each group of four) one reads the operands of its next products
+// from LDS and asks for tiles to come while the other multiplies; a barrier ends a turn, and the second group runs one barrier
+// behind the first. A wavefront's part (BM/2 x 64) is four quarters of 64 x 64 along k: (half h of its rows of x, half g of its
+// rows of w) in the order (0,0) (0,1) (1,1) (1,0), so that every turn reads one new half: w0, w1, x1, and x0 of the next tile.
+// A half is loaded into the place of the same half two tiles ago as soon as both groups have read that, seven quarters before
+// it is needed, and the waits leave the newer six quarters' loads in flight. So the matrix cores are busy in 98 % of the
+// loop's cycles (2084 a step of 64 for 2048 of products; with one barrier a step and every wavefront doing both at once: 61 %).
+template <int BM, int MODE, typename TO>
+__device__ __forceinline__ void gemm_large_tile(
+    const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
+    const TilePlace place, int n_first, int k_per_split, const Packing packing, const int activation, const int lda = 0, const int ldw = 0) {
+    constexpr int BN = LARGE_BN, DK = 64, WAVES_N = 4;
+    constexpr int WAVE_M = BM / 2, WAVE_N = BN / WAVES_N;      // the wavefront's part of the tile
+    constexpr int TM = WAVE_M / 16, TN = WAVE_N / 16, HM = TM / 2, HN = TN / 2;      // blocks of 16 rows of x and of w: all, and a half
+    constexpr int LOADS_A = BM / 128, LOADS_B = BN / 128;      // load instructions of a wavefront for one half
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    bf16* stage_a = reinterpret_cast<bf16*>(lds_raw);          // [2][BM][64]: rows of eight 16-byte pieces, swizzled
+    bf16* stage_b = stage_a + 2 * BM * DK;                     // [2][256][64]: likewise, or packed tiles as they lie
+
+    const long m0 = (long)place.m * BM;
+    constexpr int BN_OUT = MODE == MODE_GATED ? BN / 2 : BN;   // output columns of a tile
+    const long n0 = n_first + (long)place.n * BN_OUT;
+    const int lane = threadIdx.x % XRT_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / XRT_WAVE);
+    const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
+    const int quad = lane / 16;                                // which four rows of a 16 x 16 block of sums this lane holds
+
+    // Row of w behind row r of the tile (w not packed). Gated: a wavefront's rows are half gate rows and half the up rows of
+    // the same outputs. Rows beyond the operands are clamped to the last one: what they make is not written.
+    auto w_row = [&](int r) -> long {
+        if constexpr (MODE == MODE_GATED) {
+            constexpr int HALF = WAVE_N / 2;
+            const int within = r % WAVE_N;
+            return min(n0 + (r / WAVE_N) * HALF + within % HALF, (long)N - 1) + (long)(within / HALF) * N;
+        } else {
+            return min(n0 + r, (long)N - 1);
+        }
+    };
+    // Piece c (16 bytes) of row r of 64 lies at place c ^ (r % 8) of the row. The sixteen lanes that a 16-byte read serves at
+    // once are not neighbours (0 to 3, 12 to 15, 20 to 23 and 24 to 27, say): in this order they take 16 different groups of
+    // banks (no conflicts counted, 2084 cycles a step; with the order of the smaller tiles 2470).
+    auto swizzle_of = [](int r) { return r % 8; };
+    // The kilobyte of LDS (8 rows of 64, or a packed tile of 16 rows and 32 columns) that load i of half h fills, for a
+    // wavefront; rows: a wavefront's rows of the operand in the tile.
+    auto block_of = [&](int h, int i, int rows) {
+        const int p = i * 8 + wave, per = rows / 16;
+        return (p / per * rows + h * (rows / 2)) / 8 + p % per;
+    };
+    const long row_a = lda > 0 ? lda : K, row_w = ldw > 0 ? ldw : K;
+    const bool packed_b = is_packed(packing);
+    const long first_packed = MODE == MODE_GATED ? 2 * n0 : n0;
+    const long last_group = ((MODE == MODE_GATED ? 2L * N : (long)N) + 15) / 16 - 1;
+    unsigned off_a[2][LOADS_A], off_b[2][LOADS_B];             // bytes
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int i = 0; i < LOADS_A; ++i) {
+            const int r = block_of(h, i, WAVE_M) * 8 + lane / 8;
+            off_a[h][i] = (unsigned)(min(m0 + r, (long)M - 1) * row_a + ((lane % 8) ^ swizzle_of(r)) * 8) * 2u;
+        }
+#pragma unroll
+        for (int i = 0; i < LOADS_B; ++i) {
+            const int block = block_of(h, i, WAVE_N);
+            if (packed_b) {
+                const long group = min(first_packed / 16 + block / 2, last_group);       // groups beyond the matrix: the last one again
+                off_b[h][i] = (unsigned)(((group * (row_w / 32) + block % 2) * 512 + lane * 8) * 2);
+            } else {
+                const int r = block * 8 + lane / 8;
+                off_b[h][i] = (unsigned)(w_row(r) * row_w + ((lane % 8) ^ swizzle_of(r)) * 8) * 2u;
+            }
+        }
+    }
+    const unsigned w_step = packed_b ? 32u : 2u;               // bytes per column of k
+    const unsigned lds_a0 = lds_address(stage_a), lds_b0 = lds_address(stage_b);
+    auto issue_a = [&](int h, int stage, int k0) {
+#pragma unroll
+        for (int i = 0; i < LOADS_A; ++i)
+            load_to_lds(a, off_a[h][i] + (unsigned)k0 * 2u, lds_a0 + (unsigned)(stage * BM * DK * 2 + block_of(h, i, WAVE_M) * 1024));
+    };
+    auto issue_b = [&](int h, int stage, int k0) {
+#pragma unroll
+        for (int i = 0; i < LOADS_B; ++i)
+            load_to_lds(w, off_b[h][i] + (unsigned)k0 * w_step, lds_b0 + (unsigned)(stage * BN * DK * 2 + block_of(h, i, WAVE_N) * 1024));
+    };
+    // where this lane finds its 16 bytes of block 0 of its wavefront, for either 32 columns of the tile
+    const bf16* place_a[2];
+    const bf16* place_b[2];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        const int piece = ((ks * 4 + quad) ^ swizzle_of(lane % 16)) * 8;                 // (rows of further blocks differ by multiples of 16)
+        place_a[ks] = stage_a + (wave_m * WAVE_M + lane % 16) * DK + piece;
+        place_b[ks] = stage_b + wave_n * WAVE_N * DK + (packed_b ? ks * 512 + lane * 8 : lane % 16 * DK + piece);
+    }
+    bf16x8 xa[2][2][HM], wb[2][2][HN];                         // [half][32 columns][block]
+    auto read_a = [&](int h, int stage) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < HM; ++i)
+                xa[h][ks][i] = *reinterpret_cast<const bf16x8*>(place_a[ks] + stage * BM * DK + (h * HM + i) * 16 * DK);
+    };
+    auto read_b = [&](int h, int stage) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int j = 0; j < HN; ++j)
+                wb[h][ks][j] = *reinterpret_cast<const bf16x8*>(place_b[ks] + stage * BN * DK + (h * HN + j) * 16 * DK);
+    };
+    floatx4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](int h, int g) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int i = 0; i < HM; ++i)
+#pragma unroll
+                for (int j = 0; j < HN; ++j)
+                    acc[h * HM + i][g * HN + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[g][ks][j], xa[h][ks][i], acc[h * HM + i][g * HN + j], 0, 0, 0);
+    };
+    // a launch with several grid rows splits k among them: row y takes k_per_split from y * k_per_split on (less at the
+    // end) and writes its sums to the y-th copy of out
+    const int k_begin = blockIdx.y * k_per_split;
+    const int steps = min(k_per_split, K - k_begin) / DK;
+    const int last_k = k_begin + (steps - 1) * DK;
+    out += (long)blockIdx.y * M * N;
+    auto k_of = [&](int t) { return min(k_begin + t * DK, last_k); };    // (tiles beyond the end: the last one again, into a place nobody reads)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        issue_a(0, t, k_of(t));
+        issue_b(0, t, k_of(t));
+        issue_b(1, t, k_of(t));
+        issue_a(1, t, k_of(t));
+    }
+    // Loads that may stay in flight behind a quarter's reads: those of the six quarters after the next one.
+    constexpr int ALL = 2 * (LOADS_A + LOADS_B);
+    wait_loads_and_barrier<ALL + LOADS_A + LOADS_B>();         // x0 and w0 of tile 0 are in LDS
+    read_a(0, 0);
+    wait_loads_and_barrier<ALL + LOADS_A + LOADS_B>();         // and x0 is read by all: the first turn fills its place again
+    auto barrier = [] {
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto turn = [&](auto in_flight, int h, int g) {
+        __builtin_amdgcn_sched_barrier(0);
+        wait_loads_and_barrier<decltype(in_flight)::value>();  // this wavefront's reads are done: what it read may be overwritten
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(h, g);
+        barrier();
+    };
+    if (wave >= 4) barrier();
+    for (int t = 0; t < steps; ++t) {
+        const int now = t % 2, k_next = k_of(t + 2);
+        read_b(0, now);
+        issue_a(0, now, k_next);
+        turn(std::integral_constant<int, ALL + 2 * LOADS_A>{}, 0, 0);           // in flight: x1 x0 w0 w1 x1 x0
+        read_b(1, now);
+        issue_b(0, now, k_next);
+        turn(std::integral_constant<int, ALL + LOADS_A + LOADS_B>{}, 0, 1);     // x0 w0 w1 x1 x0 w0
+        read_a(1, now);
+        issue_b(1, now, k_next);
+        turn(std::integral_constant<int, ALL + 2 * LOADS_B>{}, 1, 1);           // w0 w1 x1 x0 w0 w1
+        read_a(0, now ^ 1);
+        issue_a(1, now, k_next);
+        turn(std::integral_constant<int, ALL + LOADS_A + LOADS_B>{}, 1, 0);     // w1 x1 x0 w0 w1 x1
+    }
+    if (wave < 4) barrier();
+    wait_loads_and_barrier<0>();                               // nothing lands in LDS after this
+
+    // ---- epilogue: element e of acc[i][j] is row i * 16 + lane % 16 of x and row j * 16 + quad * 4 + e of w
+    const long row0 = m0 + wave_m * WAVE_M + lane % 16;
+    if (MODE == MODE_GATED && packed_b) {
+        // A group of 16 packed rows holds the gate rows of 8 outputs, then their up rows: the lane with an output's up sum
+        // is 32 lanes away. One exchange of half a register between the sums of two blocks of x leaves gate and up of
+        // every output of both in one lane (lanes 0 to 31 the first block's outputs, the others the second's); for
+        // bfloat16 another one between two groups of w brings eight neighbouring outputs together: 16 bytes a store.
+        const long n_wave = n0 + wave_n * (WAVE_N / 2);
+        const bool wide = N % 8 == 0 && (uintptr_t)out % 16 == 0;
+#pragma unroll
+        for (int i = 0; i < TM; i += 2) {
+            const long m = row0 + i * 16 + lane / 32 * 16;
+#pragma unroll
+            for (int j = 0; j < TN; j += 2) {
+                float made[2][4];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        float gate = acc[i][j + u][e], up = acc[i + 1][j + u][e];
+                        exchange_halves(gate, up);
+                        made[u][e] = gate_activation<sizeof(TO) == 2>(gate, activation) * up;
+                    }
+                if constexpr (sizeof(TO) == 2) {
+                    if (wide) {
+                        uint4v piece = join_rows<TO>(made[0], made[1]);
+                        const long n = n_wave + (j + quad % 2) * 8;
+                        if (m < M && n < N) *reinterpret_cast<uint4v*>(out + m * (long)N + n) = piece;
+                        continue;
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    store_four<TO>(out, m, n_wave + (j + u) * 8 + quad % 2 * 4, M, N, made[u], wide);
+            }
+        }
+    } else if constexpr (MODE == MODE_GATED) {
+        const bool wide = N % 4 == 0 && (uintptr_t)out % 16 == 0;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < HN; ++j) {
+                float made[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) made[e] = gate_activation<sizeof(TO) == 2>(acc[i][j][e], activation) * acc[i][j + HN][e];
+                store_four<TO>(out, row0 + i * 16, n0 + wave_n * (WAVE_N / 2) + j * 16 + quad * 4, M, N, made, wide);
+            }
+    } else {
+        const bool wide = N % 8 == 0 && (uintptr_t)out % 16 == 0;
+        // The output column behind packed row q of w. Every order of packed rows keeps runs of eight together.
+        auto column_of = [&](long q) -> long { return packed_b && q < N ? logical_row(packing, q) : q; };
+        // Two neighbouring blocks of columns change eight lanes with each other, so that an instruction takes eight rows of
+        // 128 bytes, whole cache lines, instead of sixteen of 64 (adding onto a float32 residual of 8192 x 4096: 54 instead of 17
+        // microseconds a round of tiles without it).
+        const long row8 = m0 + wave_m * WAVE_M + lane % 8;
+        const int upper = lane % 16 / 8;
+        if constexpr (MODE == MODE_STORE && sizeof(TO) == 2) {
+            if (wide) {
+                static_assert(TN == 4, "two pieces of 32 columns");
+                const long q = n0 + wave_n * WAVE_N + (2 * upper + quad % 2) * 16 + quad / 2 * 8, n = column_of(q);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    uint4v piece[2];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const floatx4 x = acc[i][2 * u], y = acc[i][2 * u + 1];
+                        const float first[4] = {x[0], x[1], x[2], x[3]}, second[4] = {y[0], y[1], y[2], y[3]};
+                        piece[u] = join_rows<TO>(first, second);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        unsigned low = piece[0][e], high = piece[1][e];
+                        exchange_eights(low, high);
+                        piece[0][e] = low;
+                        piece[1][e] = high;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        const long m = row8 + i * 16 + u * 8;
+                        if (m < M && q < N) *reinterpret_cast<uint4v*>(out + m * (long)N + n) = piece[u];
+                    }
+                }
+                return;
+            }
+        }
+        constexpr int RUN = 4;                                 // blocks of x whose old values are read in one go, before any is written
+#pragma unroll
+        for (int i0 = 0; i0 < TM; i0 += RUN) {
+            float before[RUN][TN][4];
+            if constexpr (MODE == MODE_ACCUMULATE) {
+#pragma unroll
+                for (int i = 0; i < RUN; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        load_four<TO>(out, row8 + (i0 + i) * 16 + j % 2 * 8, column_of(n0 + wave_n * WAVE_N + (j / 2 * 2 + upper) * 16 + quad * 4),
+                                      M, N, before[i][j], wide);
+            }
+#pragma unroll
+            for (int i = 0; i < RUN; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; j += 2) {
+                    float made[2][4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        made[0][e] = acc[i0 + i][j][e];
+                        made[1][e] = acc[i0 + i][j + 1][e];
+                        exchange_eights(made[0][e], made[1][e]);
+                        if constexpr (MODE == MODE_ACCUMULATE) {
+                            made[0][e] = before[i][j][e] + made[0][e];
+                            made[1][e] = before[i][j + 1][e] + made[1][e];
+                        }
+                    }
+                    const long q = n0 + wave_n * WAVE_N + (j + upper) * 16 + quad * 4;
+                    if (q < N) {
+                        const long n = column_of(q);
+                        store_four<TO>(out, row8 + (i0 + i) * 16, n, M, N, made[0], wide);
+                        store_four<TO>(out, row8 + (i0 + i) * 16 + 8, n, M, N, made[1], wide);
+                    }
+                }
+        }
+    }
+}
+
+template <int BM, int MODE, typename TO>
+__global__ void __launch_bounds__(8 * XRT_WAVE) gemm_large_kernel(
+    const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
+    int tiles_m, int tiles_n, int k_per_split, const Packing packing, int activation) {
+    const TilePlace place = tile_place(blockIdx.x, tiles_m, tiles_n);
+    if (place.m < 0) return;
+    gemm_large_tile<BM, MODE, TO>(a, w, out, M, N, K, place, 0, k_per_split, packing, activation);
+}
+
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO>
 __global__ void __launch_bounds__(WM * WN * XRT_WAVE) gemm_mfma_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
@@ -475,12 +855,14 @@ template <int MODE, typename TO>
 __global__ void __launch_bounds__(8 * XRT_WAVE) gemm_mfma_mixed_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
     int large_blocks, int large_tiles_m, int large_tiles_n, int split, int small_tiles_m, int small_tiles_n,
-    const Packing packing, const RowScale scale) {
-    if ((int)blockIdx.x < large_blocks)
-        gemm_tile<256, 256, 2, 4, MODE, 64, 2, TO>(a, w, out, M, N, K, blockIdx.x, large_tiles_m, large_tiles_n, 0, K, packing, scale);
-    else
-        gemm_tile<128, 256, 2, 4, MODE, 64, 2, TO>(a, w, out, M, N, K, blockIdx.x - large_blocks, small_tiles_m,
-                                                   small_tiles_n, split, K, packing, scale);
+    const Packing packing, int activation) {
+    if ((int)blockIdx.x < large_blocks) {
+        const TilePlace place = tile_place(blockIdx.x, large_tiles_m, large_tiles_n);
+        if (place.m >= 0) gemm_large_tile<256, MODE, TO>(a, w, out, M, N, K, place, 0, K, packing, activation);
+    } else {
+        const TilePlace place = tile_place(blockIdx.x - large_blocks, small_tiles_m, small_tiles_n);
+        if (place.m >= 0) gemm_large_tile<128, MODE, TO>(a, w, out, M, N, K, place, split, K, packing, activation);
+    }
 }
 
 // Products of groups of rows with matrices of their own (experts): the rows of a stand sorted by group, every group's stretch
@@ -490,26 +872,26 @@ __global__ void __launch_bounds__(8 * XRT_WAVE) gemm_mfma_mixed_kernel(
 // some columns of a wider one), K is what is summed over. Grid: x the tiles along n (a whole number of rounds over the XCDs,
 // so that all tiles of one n and one group, which share their w, run on one XCD), y the parts that k is split into (each
 // writes its sums to a copy of the tile's outputs: out is [tiles][parts][BM][N] then), z the tiles of rows.
-constexpr int GROUPED_BN = 256;
 template <int BM, int MODE, typename TO>
 __global__ void __launch_bounds__(8 * XRT_WAVE) gemm_grouped_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, long w_stride, TO* __restrict__ out, int N, int K, int lda, int ldw,
-    int tiles_n, const int* __restrict__ tile_group, const Packing packing, const RowScale scale) {
+    int tiles_n, const int* __restrict__ tile_group, const Packing packing, int activation) {
     const int tile = blockIdx.z;
     const int group = tile_group == nullptr ? 0 : tile_group[tile];      // (no table: one matrix for all tiles)
     if (group < 0) return;
-    // (grid rows split k among them, and gemm_tile puts row y's sums BM * N elements further on: a tile's parts lie one
+    // (grid rows split k among them, and the tile puts row y's sums BM * N elements further on: a tile's parts lie one
     // after the other, tile after tile)
-    gemm_tile<BM, GROUPED_BN, 2, 4, MODE, 64, 2, TO>(a + (long)tile * BM * lda, w + (long)group * w_stride,
-                                                     out + (long)tile * gridDim.y * BM * N, BM, N, K, blockIdx.x, 1, tiles_n,
-                                                     0, K / (int)gridDim.y, packing, scale, lda, ldw);
+    const TilePlace place = tile_place(blockIdx.x, 1, tiles_n);
+    if (place.m < 0) return;
+    gemm_large_tile<BM, MODE, TO>(a + (long)tile * BM * lda, w + (long)group * w_stride, out + (long)tile * gridDim.y * BM * N, BM, N, K, place,
+                                  0, K / (int)gridDim.y, packing, activation, lda, ldw);
 }
 
 template <int BM, int MODE, typename TO>
 int launch_grouped(const bf16* a, const bf16* w, long w_stride, TO* out, int tiles_m, int N, int K, int lda, int ldw, const int* tile_group,
                    const Packing& packing, int activation, int splits, hipStream_t s) {
-    constexpr int BN_OUT = MODE == MODE_GATED ? GROUPED_BN / 2 : GROUPED_BN;
-    constexpr size_t lds = (size_t)2 * (BM + GROUPED_BN) * 64 * sizeof(bf16);
+    constexpr int BN_OUT = MODE == MODE_GATED ? LARGE_BN / 2 : LARGE_BN;
+    constexpr size_t lds = (size_t)2 * (BM + LARGE_BN) * 64 * sizeof(bf16);
     auto kernel = gemm_grouped_kernel<BM, MODE, TO>;
     static bool configured = false;          // per instantiation
     if (!configured) {
@@ -521,7 +903,7 @@ int launch_grouped(const bf16* a, const bf16* w, long w_stride, TO* out, int til
     XRT_REQUIRE(tiles_m > 0 && tiles_m <= 65535, "linear (groups): %d tiles of rows", tiles_m);
     XRT_REQUIRE(splits >= 1 && K % (64 * splits) == 0 && (splits == 1 || MODE == MODE_STORE), "linear (groups): k in %d parts", splits);
     kernel<<<dim3((unsigned)((tiles_n + 7) / 8 * 8), (unsigned)splits, (unsigned)tiles_m), 8 * XRT_WAVE, lds, s>>>(
-        a, w, w_stride, out, N, K, lda, ldw, tiles_n, tile_group, packing, RowScale{nullptr, 0, 0, 0.f, activation});
+        a, w, w_stride, out, N, K, lda, ldw, tiles_n, tile_group, packing, activation);
     XRT_LAUNCH_CHECK("linear (groups)");
     return 0;
 }
@@ -564,54 +946,69 @@ int launch_kernel(const bf16* a, const bf16* w, TO* out, int M, int N, int K, in
     return 0;
 }
 
-template <int BM, int BN, int WM, int WN, int MODE, typename TO>
-int launch(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int n_first, int n_count, const Packing& packing, int activation,
-           hipStream_t s) {
-    const RowScale plain = {nullptr, 0, 0, 0.f, activation};
-    // Whole tiles along k go straight into LDS, in two stages of 64; a ragged last tile needs the
-    // path through registers. (Four stages of 32 keep a load in flight for longer but meet at
-    // twice as many barriers, and measured slower: 1.03 against 1.06 to 1.16 PFLOP/s on the large tiles.)
-    if (K % 64 == 0) return launch_kernel<BM, BN, WM, WN, MODE, 64, 2, TO>(a, w, out, M, N, K, n_first, n_count, packing, s, 1, 0, plain);
-    if constexpr (BM == 256 && BN == 256 || BM == 128 && BN == 128) {
-        return launch_kernel<BM, BN, WM, WN, MODE, 0, 0, TO>(a, w, out, M, N, K, n_first, n_count, packing, s, 1, 0, plain);
-    } else {
-        XRT_REQUIRE(false, "linear (mfma): this tile takes only K that is a multiple of 64 (K=%d)", K);
+// The large tiles over all of w; splits > 1: k dealt out among grid rows, each with its copy of out.
+template <int BM, int MODE, typename TO>
+int launch_large(const bf16* a, const bf16* w, TO* out, int M, int N, int K, const Packing& packing, int activation, hipStream_t s,
+                 int splits = 1, int k_per_split = 0) {
+    constexpr int BN_OUT = MODE == MODE_GATED ? LARGE_BN / 2 : LARGE_BN;
+    constexpr size_t lds = (size_t)2 * (BM + LARGE_BN) * 64 * sizeof(bf16);
+    auto kernel = gemm_large_kernel<BM, MODE, TO>;
+    static bool configured = false;          // per instantiation
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        XRT_REQUIRE(e == hipSuccess, "linear (mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+        configured = true;
     }
+    XRT_REQUIRE(K % 64 == 0 && (splits == 1 || k_per_split % 64 == 0), "linear (mfma): the large tiles take whole steps of 64 along k (K=%d)", K);
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;
+    const unsigned grid = (unsigned)((tiles_m * tiles_n + 7) / 8 * 8);               // a whole number of rounds over the XCDs
+    kernel<<<dim3(grid, splits), 8 * XRT_WAVE, lds, s>>>(a, w, out, M, N, K, tiles_m, tiles_n, splits == 1 ? K : k_per_split, packing, activation);
+    XRT_LAUNCH_CHECK("linear (mfma, large tiles)");
+    return 0;
 }
 
-// Time of tiles of `tile_elements` outputs, in units of tile elements per compute unit: the tiles
-// run in rounds over the 256 compute units (`share` workgroups of that tile fit one unit and
-// share its matrix cores), and a partly filled last round costs a whole one. `penalty` is what a
-// tile shape loses against the largest, in percent, from reading its operands more often.
-long rounds_cost(long tiles, int tile_elements, int share, int penalty) {
-    const long rounds = (tiles + (long)XRT_COMPUTE_UNITS * share - 1) / ((long)XRT_COMPUTE_UNITS * share);
-    return rounds * share * tile_elements * (100 + penalty) / 100;
+// Time of `tiles` tiles that run in rounds over `places`, in units of a tenth of a microsecond or so: `round` is what a full
+// round takes, a last round that is partly filled takes its share of that, but `least` percent of it: the chip is bound by its
+// power, and with fewer compute units at work their clock rises (256 x 256 tiles, k = 4096: 106 us a full round, 84 us 0.75 of
+// one; 28672 rows of w and 2048 rows of x, 3.5 rounds: 372 us).
+long rounds_cost(long tiles, int places, int round, int least) {
+    const long whole = tiles / places, rest = tiles % places;
+    return whole * round * 100L + (rest == 0 ? 0 : (rest * 100 / places > least ? rest * 100 / places : least) * (long)round);
 }
+enum { LARGE_ROUND = 106, HALF_ROUND = 66, SMALL_ROUND = 75 };      // 256 x 256, 128 x 256 and 128 x 128 tiles (two to a compute unit), k = 4096
 
 template <int MODE, typename TO>
 int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, const Packing& packing, int activation, hipStream_t s) {
     // output columns per tile are half the tile's w rows in the gated mode
     constexpr int DIV = MODE == MODE_GATED ? 2 : 1;
+    const RowScale plain = {nullptr, 0, 0, 0.f, activation};
     auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn / DIV - 1) / (bn / DIV)); };
-    const bool whole_k = K % 64 == 0;
+    if (K % 64 != 0) {                 // a ragged last tile along k: the path through registers
+        const long large = ((tiles(256, 256) + XRT_COMPUTE_UNITS - 1) / XRT_COMPUTE_UNITS) * 100;
+        const long small = ((tiles(128, 128) + 2 * XRT_COMPUTE_UNITS - 1) / (2 * XRT_COMPUTE_UNITS)) * 59;
+        if (large <= small) return launch_kernel<256, 256, 2, 4, MODE, 0, 0, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
+        return launch_kernel<128, 128, 2, 2, MODE, 0, 0, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
+    }
     // Up to 128 rows of a, gated: one round of tiles of 128 x 128 (or nearly), bound by reading w: three stages keep more of
     // it on its way than the two that the tiles below have (gate/up of 14336 pairs and 128 rows: 76 us split in three
     // with a second kernel, 49 us so).
     if constexpr (MODE == MODE_GATED)
-        if (whole_k && M <= 128) return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, RowScale{nullptr, 0, 0, 0.f, activation});
-    const long large = rounds_cost(tiles(256, 256), 256 * 256, 1, 0);
-    const long medium = whole_k && MODE != MODE_GATED ? rounds_cost(tiles(256, 192), 256 * 192, 1, 5) : LONG_MAX;
-    const long small = rounds_cost(tiles(128, 128), 128 * 128, 2, 18);
-    // Large tiles for as many columns as make whole rounds, and tiles of half the height for the
-    // rest, if those then fit one round: the last round is full of half-sized work instead of
-    // half empty.
+        if (M <= 128) return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
+    // 256 x 256 tiles cost the least energy a product, and tiles of half the height somewhat more (2048 rows of x, 4096 rows of
+    // w, k = 4096: 128 tiles of the one 93 us, 256 of the other 69; 6144 rows of w: 84 and 103); tiles of 128 x 128 only
+    // where neither fills the chip (1024 rows of x, 4096 rows of w: 55 against 58 and 86 us).
+    const long large = rounds_cost(tiles(256, 256), XRT_COMPUTE_UNITS, LARGE_ROUND, 72);
+    const long half = rounds_cost(tiles(128, 256), XRT_COMPUTE_UNITS, HALF_ROUND, 80);
+    const long small = rounds_cost(tiles(128, 128), 2 * XRT_COMPUTE_UNITS, SMALL_ROUND, 68);
+    // Large tiles for as many columns as make whole rounds, and tiles of half the height for the rest, if those then fit
+    // one round: the last round is full of half-sized work instead of half empty (3.5 rounds: 366 against 372 us).
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 256 / DIV - 1) / (256 / DIV);
     const int whole_columns = (int)((long)tiles_m * tiles_n / XRT_COMPUTE_UNITS * XRT_COMPUTE_UNITS / tiles_m);     // n-tiles that run in full rounds
     const long rest_tiles = (long)((M + 127) / 128) * (tiles_n - whole_columns);
     long mixed = LONG_MAX;
-    if (whole_k && whole_columns > 0 && whole_columns < tiles_n && rest_tiles <= XRT_COMPUTE_UNITS)
-        mixed = rounds_cost((long)tiles_m * whole_columns, 256 * 256, 1, 0) + rounds_cost(rest_tiles, 128 * 256, 1, 8);
-    if (mixed < large && mixed <= medium && mixed <= small) {
+    if (whole_columns > 0 && whole_columns < tiles_n && rest_tiles <= XRT_COMPUTE_UNITS)
+        mixed = rounds_cost((long)tiles_m * whole_columns, XRT_COMPUTE_UNITS, LARGE_ROUND, 72) + rounds_cost(rest_tiles, XRT_COMPUTE_UNITS, HALF_ROUND, 80);
+    if (mixed < large && mixed <= half && mixed <= small) {
         const int split = whole_columns * (256 / DIV);
         const int small_tiles_m = (M + 127) / 128, small_tiles_n = tiles_n - whole_columns;
         const int large_blocks = (tiles_m * whole_columns + 7) / 8 * 8;      // whole rounds over the XCDs
@@ -625,14 +1022,14 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
             configured = true;
         }
         kernel<<<large_blocks + small_blocks, 8 * XRT_WAVE, lds, s>>>(a, w, out, M, N, K, large_blocks, tiles_m, whole_columns,
-                                                                      split, small_tiles_m, small_tiles_n, packing, RowScale{nullptr, 0, 0, 0.f, activation});
+                                                                      split, small_tiles_m, small_tiles_n, packing, activation);
         XRT_LAUNCH_CHECK("linear (mfma, two tile shapes)");
         return 0;
     }
-    if (large <= medium && large <= small) return launch<256, 256, 2, 4, MODE, TO>(a, w, out, M, N, K, 0, N, packing, activation, s);
-    if constexpr (MODE != MODE_GATED)
-        if (medium <= small) return launch<256, 192, 4, 2, MODE, TO>(a, w, out, M, N, K, 0, N, packing, activation, s);
-    return launch<128, 128, 2, 2, MODE, TO>(a, w, out, M, N, K, 0, N, packing, activation, s);
+    if (large <= half && large <= small) return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+    if (half <= small) return launch_large<128, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+    // (four stages of 32 keep a load in flight for longer but meet at twice as many barriers, and measured slower)
+    return launch_kernel<128, 128, 2, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
 }
 
 template <typename TO>
@@ -794,9 +1191,9 @@ __global__ void __launch_bounds__(256) split_reduce_wide_kernel(const float* __r
     if constexpr (sizeof(TO) == 4) {
         *reinterpret_cast<float4*>(out + index) = sum;
     } else {
-        struct alignas(8) Four { TO e[4]; } four;
+        Four<TO> four;
         four.e[0] = from_float<TO>(sum.x); four.e[1] = from_float<TO>(sum.y); four.e[2] = from_float<TO>(sum.z); four.e[3] = from_float<TO>(sum.w);
-        *reinterpret_cast<Four*>(out + index) = four;
+        *reinterpret_cast<Four<TO>*>(out + index) = four;
     }
 }
 
@@ -804,7 +1201,6 @@ __global__ void __launch_bounds__(256) split_reduce_wide_kernel(const float* __r
 // parts onto the residual and writes the row's norm as well. The norm is the norm kernel's (elementwise.hip) to the bit: the same
 // four columns a thread, the same order of the sum of squares, (x * 1/rms) * gain.
 constexpr int NORM_QUADS = 8;                      // four-column pieces a thread holds: rows of up to 8 * 256 * 4 columns
-template <typename T> struct alignas(sizeof(T) * 4) Four { T e[4]; };
 template <typename TW>
 __global__ void __launch_bounds__(256) split_reduce_rmsnorm_kernel(const float* __restrict__ parts, int splits, long count, int N,
                                                                     float* __restrict__ out, const TW* __restrict__ gain, float eps,
@@ -955,8 +1351,7 @@ int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int
         ? launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, float>(
               a, w, workspace, M, (int)plan.rows_w, K, 0, (int)plan.rows_w, packing, s, plan.splits, plan.k_per_split)
         : plan.tile == 256
-        ? launch_kernel<256, 256, 2, 4, MODE_STORE, 64, 2, float>(
-              a, w, workspace, M, (int)plan.rows_w, K, 0, (int)plan.rows_w, packing, s, plan.splits, plan.k_per_split)
+        ? launch_large<256, MODE_STORE, float>(a, w, workspace, M, (int)plan.rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split)
         : plan.columns == 64
         ? launch_kernel<128, 64, 2, 2, MODE_STORE, 64, 3, float>(
               a, w, workspace, M, (int)plan.rows_w, K, 0, (int)plan.rows_w, packing, s, plan.splits, plan.k_per_split)
@@ -1041,7 +1436,7 @@ bool xrt_linear_groups_mfma_accepts(const void* a, int lda, const void* w, int l
 // How many parts k is best split into: two where the tiles are too few to fill the chip twice over (a last round that is mostly
 // empty costs a whole one), one otherwise. Only plain sums can be split (their parts are added by whoever reads them).
 int xrt_linear_groups_splits(int tiles_m, int N, int K, int mode) {
-    const int tiles_n = (N + GROUPED_BN - 1) / GROUPED_BN;
+    const int tiles_n = (N + LARGE_BN - 1) / LARGE_BN;
     return mode == MODE_STORE && K % 128 == 0 && (long)tiles_m * tiles_n < 2L * XRT_COMPUTE_UNITS ? 2 : 1;
 }
 
