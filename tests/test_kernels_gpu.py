@@ -120,6 +120,30 @@ def test_linear(ops, dtype, m, n, k):
     assert rel(acc.cpu(), base.double().cpu() + want) < 1e-5
 
 
+# float32: the matrix cores' product of many rows gives the bits of the kernels of few rows (the sums of 16 consecutive k, in order),
+# also where k ends inside 16 or 32 columns, with rows and columns that fill no tile, denormals and infinities.
+@pytest.mark.parametrize("m,n,k", [(17, 64, 4), (33, 176, 64), (64, 65, 20), (70, 130, 36), (130, 40, 100), (200, 333, 1040), (65, 256, 176)])
+def test_linear_float32_has_the_same_bits_with_few_rows_and_with_many(ops, m, n, k):
+    a, w = rand(m, k, seed=m), rand(2 * n, k, seed=n, scale=0.3)
+    a[3] *= 1e-36
+    w[1] *= 1e-6
+    a[5, k // 2] = float("inf")
+    base = rand(m, 2 * n, seed=5)
+    for rows in (16, 5):
+        many, few = base.clone(), base.clone()
+        stored, stored_few = torch.empty_like(base), torch.empty_like(base)
+        gated, gated_few = torch.empty(m, n, device=DEV), torch.empty(m, n, device=DEV)
+        ops.linear(a, w, many, accumulate=True)
+        ops.linear(a, w, stored)
+        ops.linear_glu(a, w, gated)
+        for at in range(0, m, rows):
+            ops.linear(a[at:at + rows], w, few[at:at + rows], accumulate=True)
+            ops.linear(a[at:at + rows], w, stored_few[at:at + rows])
+            ops.linear_glu(a[at:at + rows], w, gated_few[at:at + rows])
+        for got, want in ((many, few), (stored, stored_few), (gated, gated_few)):
+            assert torch.equal(torch.nan_to_num(got, nan=7.0), torch.nan_to_num(want, nan=7.0))
+
+
 # The tiles of eight wavefronts (256 and 128 rows by 256) at the edges of tiles, with one, two and three steps along k, columns that
 # do and do not allow 16 bytes a store; by the rule of the launcher: large tiles alone, half tiles alone, both in one launch.
 @pytest.mark.parametrize("kind", ["plain", "packed", "rotary"])
