@@ -106,6 +106,11 @@ __device__ __forceinline__ void load_to_lds(const void* base, unsigned byte_offs
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
                  :: "s"(lds_base), "v"(byte_offset), "s"(base) : "memory", "m0");
 }
+// The same for bytes that nobody else reads: past the caches (whole cache lines an instruction only).
+__device__ __forceinline__ void stream_to_lds(const void* base, unsigned byte_offset, unsigned lds_base) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                 :: "s"(lds_base), "v"(byte_offset), "s"(base) : "memory", "m0");
+}
 // The same with 4 bytes per lane: lane l writes LDS byte address lds_base + 4 * l.
 __device__ __forceinline__ void load_dword_to_lds(const void* base, unsigned byte_offset, unsigned lds_base) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"

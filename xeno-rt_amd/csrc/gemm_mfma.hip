@@ -180,6 +180,10 @@ __device__ __forceinline__ void gemm_tile(
         const unsigned w_step = packed_b ? 32u : 2u;                // bytes per column of k
         const int wave_uniform = __builtin_amdgcn_readfirstlane(wave);
         const unsigned lds_a0 = lds_address(stage_a), lds_b0 = lds_address(stage_b);
+        // Up to 64 rows of a, k not split: every byte of w is read by one workgroup, in one long run, and passes the caches by
+        // (64 rows: gate/up 47.2 -> 44.1 us, an output head of 128256 rows 212 -> 197). Split along k the runs are short, and so marked
+        // they are read more slowly (4096 x 4096 in eight parts 16.3 -> 18.1 us).
+        const bool past_caches = gridDim.y == 1;
         auto issue = [&](int stage, int k0) {
 #pragma unroll
             for (int i = 0; i < LOADS_A; ++i) {
@@ -189,7 +193,9 @@ __device__ __forceinline__ void gemm_tile(
 #pragma unroll
             for (int i = 0; i < LOADS_B; ++i) {
                 const int block = min(i * WAVES + wave_uniform, BLOCKS_B - 1);
-                load_to_lds(w, off_b[i] + (unsigned)k0 * w_step, lds_b0 + (unsigned)((stage * BN + block * ROWS) * DK * 2));
+                const unsigned to = lds_b0 + (unsigned)((stage * BN + block * ROWS) * DK * 2);
+                if (BM <= 64 && past_caches) stream_to_lds(w, off_b[i] + (unsigned)k0 * w_step, to);
+                else load_to_lds(w, off_b[i] + (unsigned)k0 * w_step, to);
             }
         };
         const int swizzle = swizzle_of(lane % 16);                 // of every row this lane reads: they differ by multiples of 32
@@ -1131,10 +1137,20 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const float* __restri
     }
     float sum = 0.f, up = 0.f;
     if (inside) {
-        for (int p = 0; p < splits; ++p) {
-            const float* part = parts + ((long)p * M + m) * rows_w;
-            sum += part[n];
-            if constexpr (MODE == MODE_GATED) up += part[N + n];
+        // eight parts at a time are asked for at once (those beyond the last: that one again), then added in order
+        for (int p0 = 0; p0 < splits; p0 += 8) {
+            float of[8], of_up[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const float* part = parts + ((long)min(p0 + u, splits - 1) * M + m) * rows_w;
+                of[u] = part[n];
+                if constexpr (MODE == MODE_GATED) of_up[u] = part[N + n];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                sum = p0 + u < splits ? sum + of[u] : sum;
+                if constexpr (MODE == MODE_GATED) up = p0 + u < splits ? up + of_up[u] : up;
+            }
         }
     }
     float by = 1.0f;
@@ -1276,10 +1292,19 @@ __global__ void __launch_bounds__(256) split_reduce_qkv_kernel(const float* __re
             for (int t = 0; t < norm.tiles_in; ++t) mine += norm.squares_in[(long)t * XRT_SQUARES_STRIDE + m];
     }
     float lower = 0.f, upper = 0.f;
-    for (int p = 0; p < splits; ++p) {
-        const float* part = parts + ((long)p * M + m) * N;
-        lower += part[n];
-        upper += part[n + half];
+    for (int p0 = 0; p0 < splits; p0 += 8) {                    // (as above: eight parts at once, added in order)
+        float of_lower[8], of_upper[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const float* part = parts + ((long)min(p0 + u, splits - 1) * M + m) * N;
+            of_lower[u] = part[n];
+            of_upper[u] = part[n + half];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            lower = p0 + u < splits ? lower + of_lower[u] : lower;
+            upper = p0 + u < splits ? upper + of_upper[u] : upper;
+        }
     }
     const int pos = after.positions[m];
     const bool is_q = head < after.n_heads, is_v = head >= after.n_heads + after.n_kv_heads;
