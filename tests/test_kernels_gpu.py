@@ -859,6 +859,25 @@ def test_attention_prefill_on_matrix_cores(ops, nh, nkv, hd):
     assert rel(out.cpu(), want) < 1e-2
 
 
+# Few new tokens on a long cache: the keys of a tile are cut into runs that a second kernel merges. Runs that end inside, before and
+# behind what a tile of queries sees, one token to three tiles, sequences of unequal lengths (some of whose runs hold no keys).
+@pytest.mark.parametrize("nh,nkv,hd", [(4, 4, 64), (8, 2, 128), (32, 8, 128)])
+@pytest.mark.parametrize("starts,counts", [([1100], [333]), ([1023], [2]), ([1990], [129]), ([1500, 3, 700], [40, 2, 300]), ([2300, 64], [257, 1])])
+def test_attention_of_few_new_tokens_on_a_long_cache(ops, nh, nkv, hd, starts, counts):
+    lengths = [s + n for s, n in zip(starts, counts)]
+    kv, keys, values = filled_cache(nkv, hd, torch.bfloat16, lengths, seed=hd + nh)
+    batch = described(list(range(len(counts))), counts, starts)
+    tokens = sum(counts)
+    if nh < 32:                                              # (with 32 heads the larger steps fill the chip without)
+        assert ops.lib.xrt_attention_workspace(1, tokens, nh, nkv, hd, 0, max(counts), max(lengths)) > 0
+    qkv = rand(tokens, (nh + 2 * nkv) * hd, dtype=torch.bfloat16, seed=5, scale=2.0)
+    out = torch.full((tokens, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.attention(qkv, nh, nkv, hd, kv, batch, out, scale=1.0 / math.sqrt(hd))
+    want = expected_attention(qkv, batch.slots.tolist(), batch.positions.tolist(), keys, values, nh, nkv, hd)
+    assert torch.isfinite(out).all()
+    assert rel(out.cpu(), want) < 1e-2                       # probabilities and results in bfloat16, as without the cut
+
+
 def test_matrix_core_attention_finds_a_far_key(ops):
     nh, nkv, hd = 8, 2, 128
     kv, keys, values = filled_cache(nkv, hd, torch.bfloat16, [900], seed=1)

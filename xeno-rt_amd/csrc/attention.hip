@@ -22,6 +22,12 @@ int xrt_attention_prefill(const void* qkv, long q_stride, int tokens, int n_head
                           const int* seq_offsets, const int* seq_slots, const int* seq_starts, int n_seqs, void* out,
                           float scale, int stretch, bool fine, const float* bias, int span, const float* sinks, hipStream_t s);
 
+long xrt_attention_prefill_workspace(int tokens, int n_heads, int head_dim, int max_count, int max_context);
+int xrt_attention_prefill_split(const void* qkv, int tokens, int n_heads, int n_kv_heads, int head_dim, const void* k_cache, const void* v_cache,
+                                const int* block_table, int table_stride, int n_blocks, const int* seq_offsets, const int* seq_slots,
+                                const int* seq_starts, int n_seqs, void* out, float scale, int max_count, int max_context, float* workspace,
+                                hipStream_t s);
+
 static bool takes_decode_kernel(int dtype, int n_heads, int n_kv_heads, int head_dim, int window, int max_count, int max_context) {
     return dtype == XRT_BF16 && window == 0 && max_count == 1 && max_context > 0 && n_heads > 0 && n_kv_heads > 0 &&
            n_heads % n_kv_heads == 0 && xrt_attention_decode_accepts(head_dim);
@@ -29,7 +35,10 @@ static bool takes_decode_kernel(int dtype, int n_heads, int n_kv_heads, int head
 
 extern "C" long xrt_attention_workspace(int dtype, int tokens, int n_heads, int n_kv_heads, int head_dim, int window,
                                         int max_count, int max_context) {
-    if (tokens <= 0 || !takes_decode_kernel(dtype, n_heads, n_kv_heads, head_dim, window, max_count, max_context)) return 0;
+    if (tokens <= 0) return 0;
+    if (dtype == XRT_BF16 && window == 0 && max_count > 1 && max_context > 0 && n_heads > 0 && xrt_attention_prefill_accepts(head_dim))
+        return xrt_attention_prefill_workspace(tokens, n_heads, head_dim, max_count, max_context);
+    if (!takes_decode_kernel(dtype, n_heads, n_kv_heads, head_dim, window, max_count, max_context)) return 0;
     return xrt_attention_decode_workspace(tokens, n_heads, n_kv_heads, head_dim, max_context);
 }
 
@@ -60,6 +69,11 @@ extern "C" int xrt_attention(const void* qkv, int dtype, int tokens, int n_heads
             // tokens beyond the sequences (padding) get zeros
             // (their rows are read by nothing, but must not hold what a later product could choke on)
             XRT_REQUIRE(n_seqs <= tokens, "attention: more sequences than tokens");
+            // few new tokens on a long cache, and room for what the runs of their keys make: cut (without the room: not)
+            if (need > 0 && workspace != nullptr && workspace_floats >= need && (uintptr_t)workspace % 16 == 0)
+                return xrt_attention_prefill_split(qkv, tokens, n_heads, n_kv_heads, head_dim, k_cache, v_cache, block_table, table_stride,
+                                                   n_blocks, seq_offsets, seq_slots, seq_starts, n_seqs, out, scale, max_count, max_context,
+                                                   workspace, s);
             return xrt_attention_prefill(qkv, 0, tokens, n_heads, n_kv_heads, head_dim, k_cache, v_cache, block_table,
                                          table_stride, n_blocks, seq_offsets, seq_slots, seq_starts, n_seqs, out,
                                          scale, 0, false, nullptr, 0, nullptr, s);

@@ -32,6 +32,7 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 constexpr int QT = 32;                 // query tokens per wavefront
 constexpr int BT = XRT_BLOCK_TOKENS;   // keys per cache block
 constexpr int PER_STAGE = 2;           // cache blocks between two barriers
+constexpr int MOST_RUNS = 8;           // runs that the keys of a tile are cut into, at most
 constexpr float LOG2E = 1.4426950408889634f;
 
 // Key (0..31 within a tile of 32 keys) that row r of the score tile stands for. Accumulator
@@ -58,12 +59,22 @@ constexpr int QW = GROUPS * QT;        // queries of a tile
 struct PrefillExtras {
     const float* bias; int span; float inv_scale; const float* sinks;
 };
-template <int HD, bool FINE, bool EXTRAS = false>
+// SPLIT: a step of few new tokens on a long cache has too few pairs of tiles to fill the chip (333 tokens of 32 heads: 64
+// workgroups), and each walks thousands of keys. Then grid z cuts the blocks of a pair's keys into runs of equal length, and
+// every workgroup leaves what its run makes (sum of weighted values, maximum, sum) in a workspace, from which a second kernel
+// merges the runs in order. (333 tokens behind 3001: 97 us, with four runs and the second kernel 41 + 8.)
+struct PrefillParts {
+    float* o;                          // [runs][tokens][heads][HD], relative to the maximum
+    float* ml;                         // [runs][tokens][heads][2]: maximum (-inf: no key of this run is seen) and sum
+    int tokens;
+};
+template <int HD, bool FINE, bool EXTRAS = false, bool SPLIT = false>
 __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
     const bf16* __restrict__ qkv, int row_width, int n_heads, int n_kv_heads,
     const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache, const int* __restrict__ block_table,
     int table_stride, int n_blocks, const int* __restrict__ seq_offsets, const int* __restrict__ seq_slots,
-    const int* __restrict__ seq_starts, int n_seqs, bf16* __restrict__ out, float scale, int stretch, const PrefillExtras extras) {
+    const int* __restrict__ seq_starts, int n_seqs, bf16* __restrict__ out, float scale, int stretch, const PrefillExtras extras,
+    const PrefillParts parts) {
     constexpr int KS = HD / 16;            // K steps of the score product
     constexpr int DT = HD / 32;            // 32-row tiles of the value product
     constexpr int K_CHUNKS = HD / 8;       // 16-byte chunks of a key row (16 or 8)
@@ -121,6 +132,13 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
     const int early_blocks = has_early ? (start + (early_tile + 1) * QW - 1) / BT + 1 : 0;
     const int kv_head = head / (n_heads / n_kv_heads);
     const float scale2 = scale * LOG2E;
+    // the blocks that this workgroup walks: all of the late tile's, or its run of them (whole stages)
+    int walk_from = 0, walk_to = late_blocks;
+    if constexpr (SPLIT) {
+        const int run = ((late_blocks + (int)gridDim.z - 1) / (int)gridDim.z + PER_STAGE - 1) / PER_STAGE * PER_STAGE;
+        walk_from = min((int)blockIdx.z * run, late_blocks);
+        walk_to = min(walk_from + run, late_blocks);
+    }
 
     // ---- the queries a wavefront is working on
     long token = 0;                                          // row of qkv and out (clamped: loads need no guard)
@@ -171,8 +189,31 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
                 *reinterpret_cast<Four*>(dst + dt * 32 + g * 8 + half * 4) = four;
             }
     };
+    // What a run of keys makes of the queries at hand (l summed over the pair of lanes); nothing seen: the maximum says so.
+    auto write_part = [&]() {
+        if constexpr (SPLIT) {
+            if (!q_valid) return;
+            const long index = ((long)blockIdx.z * parts.tokens + token) * n_heads + head;
+            if (half == 0) *reinterpret_cast<float2*>(parts.ml + index * 2) = make_float2(m, l);
+            if (m == -INFINITY) return;
+            float* dst = parts.o + index * HD;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<float4*>(dst + dt * 32 + g * 8 + half * 4) =
+                        make_float4(o[dt][g * 4], o[dt][g * 4 + 1], o[dt][g * 4 + 2], o[dt][g * 4 + 3]);
+        }
+    };
     take(helper && has_early ? early_tile : late_tile);
     bool on_early = helper && has_early;
+    if constexpr (SPLIT) {
+        if (on_early && early_blocks <= walk_from) {         // no key of this run is seen by the early tile
+            write_part();
+            take(late_tile);
+            on_early = false;
+        }
+    }
 
     // ---- moving a cache block into LDS: it goes straight there (global_load_lds_dwordx4): lane l of an
     // instruction fills the l-th 16 bytes of a 1024-byte stretch with the chunk that belongs in that place,
@@ -330,18 +371,18 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
     };
 
     // ---- the blocks of the sequence, in order: the next stage's blocks travel while this stage's are used
-    const int last_block = late_blocks - 1;
+    const int last_block = walk_to - 1;
     // the early tile's blocks end at a stage's end for the helpers: up to there every wavefront takes every block
     // (those beyond its queries' last key fall away by themselves), from there on they take turns
-    const int turns_from = (early_blocks + PER_STAGE - 1) / PER_STAGE * PER_STAGE;
+    const int turns_from = max(walk_from, (early_blocks + PER_STAGE - 1) / PER_STAGE * PER_STAGE);
     int coming[PER_STAGE];                                   // the blocks that the next fetch asks for
 #pragma unroll
     for (int i = 0; i < PER_STAGE; ++i) {
-        if (i <= last_block) fetch(block_of(i), i);
-        coming[i] = block_of(PER_STAGE + i);
+        if (walk_from + i <= last_block) fetch(block_of(walk_from + i), walk_from % (2 * PER_STAGE) + i);
+        coming[i] = block_of(walk_from + PER_STAGE + i);
     }
     wait_loads_and_barrier<0>();
-    for (int first = 0; first <= last_block; first += PER_STAGE) {
+    for (int first = walk_from; first <= last_block; first += PER_STAGE) {
         const int stage = (first / PER_STAGE) & 1;
         // the other stage's buffers were read in the step before, ahead of the last barrier
         pieces_wanted = max(0, min(PER_STAGE, last_block - first - PER_STAGE + 1)) * LOADS;
@@ -371,7 +412,8 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
         }
         if (on_early && first + PER_STAGE >= early_blocks) {  // the early tile is done: its result goes out, the late tile's queries come in
             l += __shfl_xor(l, 32, XRT_WAVE);
-            write_out();
+            if constexpr (SPLIT) write_part();
+            else write_out();
             take(late_tile);
             on_early = false;
         }
@@ -379,6 +421,13 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
         wait_loads_and_barrier<0>();                         // the next blocks have arrived from every wavefront, these have been read by all
     }
 
+    if constexpr (SPLIT) {
+        if (on_early) {                                      // the early tile sees keys beyond this run: it has had all of it
+            l += __shfl_xor(l, 32, XRT_WAVE);
+            write_part();
+            take(late_tile);                                 // and the late tile got nothing from this wavefront
+        }
+    }
     // ---- the two wavefronts of a group of queries merge what they have, through LDS (the blocks' buffers are free now)
     float (*merge_o)[DT * 16][XRT_WAVE] = reinterpret_cast<float (*)[DT * 16][XRT_WAVE]>(lds_raw);          // [GROUPS]
     float (*merge_ml)[2][XRT_WAVE] = reinterpret_cast<float (*)[2][XRT_WAVE]>(lds_raw + GROUPS * DT * 16 * XRT_WAVE * sizeof(float));
@@ -405,7 +454,83 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
         m = m_all;                                           // what l and o are relative to now
     }
     l += __shfl_xor(l, 32, XRT_WAVE);
-    write_out();
+    if constexpr (SPLIT) write_part();
+    else write_out();
+}
+
+// Merges the runs of keys of one (token, head), in order: a wavefront each, HD / 64 dims a lane.
+template <int HD>
+__global__ void __launch_bounds__(4 * XRT_WAVE) attention_prefill_merge_kernel(const PrefillParts parts, int runs, int n_heads,
+                                                                               const int* __restrict__ seq_offsets, int n_seqs,
+                                                                               bf16* __restrict__ out) {
+    constexpr int PER_LANE = HD / XRT_WAVE;
+    const int lane = threadIdx.x % XRT_WAVE;
+    const long row = (long)blockIdx.x * 4 + threadIdx.x / XRT_WAVE, rows = (long)parts.tokens * n_heads;      // (token, head)
+    if (row >= rows || row / n_heads >= seq_offsets[n_seqs]) return;      // (tokens beyond the sequences are nobody's)
+    float m_of[MOST_RUNS], l_of[MOST_RUNS], o_of[MOST_RUNS][PER_LANE];
+#pragma unroll
+    for (int r = 0; r < MOST_RUNS; ++r) {                     // all runs are asked for at once (those beyond the last: that one again)
+        const long index = (long)min(r, runs - 1) * rows + row;
+        const float2 ml = *reinterpret_cast<const float2*>(parts.ml + index * 2);
+        m_of[r] = r < runs ? ml.x : -INFINITY;
+        l_of[r] = ml.y;
+#pragma unroll
+        for (int d = 0; d < PER_LANE; ++d) o_of[r][d] = parts.o[index * HD + lane * PER_LANE + d];
+    }
+    float m = m_of[0];
+#pragma unroll
+    for (int r = 1; r < MOST_RUNS; ++r) m = fmaxf(m, m_of[r]);
+    float l = 0.f, o[PER_LANE] = {};
+#pragma unroll
+    for (int r = 0; r < MOST_RUNS; ++r) {
+        if (m_of[r] == -INFINITY) continue;                  // this run wrote nothing else
+        const float weight = __builtin_amdgcn_exp2f(m_of[r] - m);
+        l = fmaf(weight, l_of[r], l);
+#pragma unroll
+        for (int d = 0; d < PER_LANE; ++d) o[d] = fmaf(weight, o_of[r][d], o[d]);
+    }
+    const float inv = l > 0.f ? 1.0f / l : 0.f;
+    struct alignas(2 * PER_LANE) Dims { bf16 e[PER_LANE]; } made;
+#pragma unroll
+    for (int d = 0; d < PER_LANE; ++d) made.e[d] = (bf16)(o[d] * inv);
+    *reinterpret_cast<Dims*>(out + row * HD + lane * PER_LANE) = made;
+}
+
+// Into how many runs a step's keys are cut (1: not at all): as many as fill the compute units that its pairs of tiles leave idle,
+// each of eight blocks of keys at least (a shorter one costs more than it saves: start, merge and 520 bytes a query, head and run).
+int prefill_runs(int tokens, int n_heads, int head_dim, int max_count, int max_context) {
+    const long sequences = (tokens + max_count - 1) / max_count, by_tokens = (tokens + 2 * QW - 1) / (2 * QW);
+    const long workgroups = n_heads * (sequences > by_tokens ? sequences : by_tokens);
+    const long places = XRT_COMPUTE_UNITS * (head_dim == 64 ? 2 : 1);              // what the LDS of a workgroup leaves room for
+    const long blocks = (max_context + BT - 1) / BT;
+    long runs = places / workgroups;
+    runs = runs > blocks / 8 ? blocks / 8 : runs;
+    return runs < 2 ? 1 : runs > MOST_RUNS ? MOST_RUNS : (int)runs;
+}
+
+template <int HD>
+int launch_split(const bf16* qkv, int tokens, int n_heads, int n_kv_heads, const bf16* k_cache, const bf16* v_cache, const int* block_table,
+                 int table_stride, int n_blocks, const int* seq_offsets, const int* seq_slots, const int* seq_starts, int n_seqs, bf16* out,
+                 float scale, int runs, float* workspace, hipStream_t s) {
+    const long pairs = ((tokens + QW - 1) / QW + (long)n_seqs) / 2 + n_seqs;
+    XRT_REQUIRE(pairs <= 65535, "attention (prefill): too many query tiles for the grid");
+    constexpr size_t lds = (size_t)2 * PER_STAGE * (BT * HD + HD * BT) * sizeof(bf16);
+    auto kernel = attention_prefill_kernel<HD, false, false, true>;
+    static bool configured = false;          // per instantiation
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        XRT_REQUIRE(e == hipSuccess, "attention (prefill): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+        configured = true;
+    }
+    const PrefillParts parts{workspace, workspace + (long)runs * tokens * n_heads * HD, tokens};
+    kernel<<<dim3(n_heads, (unsigned)pairs, runs), WAVES * XRT_WAVE, lds, s>>>(
+        qkv, (n_heads + 2 * n_kv_heads) * HD, n_heads, n_kv_heads, k_cache, v_cache, block_table, table_stride, n_blocks, seq_offsets, seq_slots,
+        seq_starts, n_seqs, out, scale, 0, PrefillExtras{}, parts);
+    XRT_LAUNCH_CHECK("attention (prefill, runs of keys)");
+    const long rows = (long)tokens * n_heads;
+    attention_prefill_merge_kernel<HD><<<(unsigned)((rows + 3) / 4), 4 * XRT_WAVE, 0, s>>>(parts, runs, n_heads, seq_offsets, n_seqs, out);
+    XRT_LAUNCH_CHECK("attention (prefill, merge)");
+    return 0;
 }
 
 template <int HD, bool FINE, bool EXTRAS = false>
@@ -430,7 +555,7 @@ int launch_waves(const bf16* qkv, long q_stride, int tokens, int n_heads, int n_
     }
     attention_prefill_kernel<HD, FINE, EXTRAS><<<grid, WAVES * XRT_WAVE, lds, s>>>(
         qkv, row_width, n_heads, n_kv_heads, k_cache, v_cache, block_table, table_stride, n_blocks, seq_offsets,
-        seq_slots, seq_starts, n_seqs, out, scale, stretch, extras);
+        seq_slots, seq_starts, n_seqs, out, scale, stretch, extras, PrefillParts{});
     XRT_LAUNCH_CHECK("attention (prefill)");
     return 0;
 }
@@ -438,6 +563,24 @@ int launch_waves(const bf16* qkv, long q_stride, int tokens, int n_heads, int n_
 }  // namespace
 
 bool xrt_attention_prefill_accepts(int head_dim) { return head_dim == 64 || head_dim == 128; }
+
+// Floats of workspace for the runs of keys that a step would be cut into (0: it is not cut), and such a step.
+long xrt_attention_prefill_workspace(int tokens, int n_heads, int head_dim, int max_count, int max_context) {
+    const int runs = prefill_runs(tokens, n_heads, head_dim, max_count, max_context);
+    return runs == 1 ? 0 : (long)runs * tokens * n_heads * (head_dim + 2);
+}
+
+int xrt_attention_prefill_split(const void* qkv, int tokens, int n_heads, int n_kv_heads, int head_dim, const void* k_cache, const void* v_cache,
+                                const int* block_table, int table_stride, int n_blocks, const int* seq_offsets, const int* seq_slots,
+                                const int* seq_starts, int n_seqs, void* out, float scale, int max_count, int max_context, float* workspace,
+                                hipStream_t s) {
+    const int runs = prefill_runs(tokens, n_heads, head_dim, max_count, max_context);
+    auto run = [&](auto launcher) {
+        return launcher((const bf16*)qkv, tokens, n_heads, n_kv_heads, (const bf16*)k_cache, (const bf16*)v_cache, block_table, table_stride,
+                        n_blocks, seq_offsets, seq_slots, seq_starts, n_seqs, (bf16*)out, scale, runs, workspace, s);
+    };
+    return head_dim == 64 ? run(launch_split<64>) : run(launch_split<128>);
+}
 
 // q_stride: 0, or how far the rows of q lie apart when they hold the queries alone. stretch: 0, or the size of the stretches
 // that positions are cut into (a multiple of the cache block), of which a query sees its own. fine: probabilities of sixteen bits.

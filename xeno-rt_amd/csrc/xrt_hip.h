@@ -150,7 +150,8 @@ int xrt_linear_qkv(const void* a, const void* w, const xrt_packing* packing, int
 // step may be described (seq_* arrays, n_seqs, the largest token count of a sequence and the
 // longest sequence after the step): then the matrix-core kernels can be used; a decode step (max_count 1)
 // then needs a workspace of xrt_attention_workspace(...) floats for the partial results of the parts that
-// its keys are cut into (0: none), and takes the general kernel without it. distance_slopes (null: none): one
+// its keys are cut into (0: none), and takes the general kernel without it; with few new tokens on a long cache
+// the keys are cut too (without the workspace: not). distance_slopes (null: none): one
 // float per query head; a key at position j then adds slope * (j - P) to the scaled score of the query at
 // position P, for position encodings that act on the scores (the general kernel serves them).
 long xrt_attention_workspace(int dtype, int tokens, int n_heads, int n_kv_heads, int head_dim, int window,
