@@ -16,15 +16,19 @@ from . import build as _build
 
 _CODES = {torch.float32: 0, torch.bfloat16: 1}
 
+# the handle of the current stream of a device (by its index)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda index: torch.cuda.current_stream(index).cuda_stream)
+
 
 class KernelError(RuntimeError):
     """The kernel library refused an operation, or could not be loaded."""
 
 
 def _code(tensor: torch.Tensor) -> int:
-    if tensor.dtype not in _CODES:
+    code = _CODES.get(tensor.dtype)
+    if code is None:
         raise KernelError(f"unsupported element type {tensor.dtype}")
-    return _CODES[tensor.dtype]
+    return code
 
 
 def _ptr(tensor: Optional[torch.Tensor]):
@@ -230,21 +234,24 @@ class HipOps:
         if status != 0:
             raise KernelError(self.lib.xrt_last_error().decode())
 
+    # (A step that is launched kernel by kernel asks for its stream a hundred times and for its tensors' shapes five hundred
+    # times: a prompt of 100 tokens through 16 layers was bound by this file. So the stream's handle comes from torch without
+    # a Stream object around it, and devices and shapes are compared as numbers and as they are.)
     @staticmethod
     def _stream(tensor: torch.Tensor):
-        return ctypes.c_void_p(torch.cuda.current_stream(tensor.device).cuda_stream)
+        return ctypes.c_void_p(_raw_stream(tensor.get_device()))
 
     @staticmethod
     def _require(tensor: torch.Tensor, what: str, dtype=None, shape=None, like=None) -> None:
         if not isinstance(tensor, torch.Tensor) or not tensor.is_cuda:
             raise KernelError(f"{what}: expected a tensor on the GPU")
-        if like is not None and tensor.device != like.device:
+        if like is not None and tensor.get_device() != like.get_device():
             raise KernelError(f"{what}: on {tensor.device}, expected {like.device}")
         if not tensor.is_contiguous():
             raise KernelError(f"{what}: must be contiguous")
         if dtype is not None and tensor.dtype != dtype:
             raise KernelError(f"{what}: dtype {tensor.dtype}, expected {dtype}")
-        if shape is not None and tuple(tensor.shape) != tuple(shape):
+        if shape is not None and tensor.shape != (shape if type(shape) is tuple else tuple(shape)):
             raise KernelError(f"{what}: shape {tuple(tensor.shape)}, expected {tuple(shape)}")
 
     # -- operations ----------------------------------------------------------
@@ -353,8 +360,9 @@ class HipOps:
         if w.shape[0] != (2 * n if mode == 2 else n):
             raise KernelError(f"linear: w has {w.shape[0]} rows for {n} outputs")
         self._require(out, "linear out", None, (m, n), a)
-        sizes = (_ptr(a), _ptr(data), _code(a))
-        packed = (_ptr(a), _ptr(data), packing, _code(a))
+        at_a, at_w, code = _ptr(a), _ptr(data), _code(a)
+        sizes = (at_a, at_w, code)
+        packed = (at_a, at_w, packing, code)
         # the norm after an accumulating product: only if that product, and one of the same rows
         # over the n columns it writes, can take it
         emit = None
@@ -468,9 +476,10 @@ class HipOps:
             self._require(scaled.squares, "sums of squares", torch.float32, (tiles, SQUARES_STRIDE), a)
             norm = _LinearNorm()
             norm.squares_in, norm.tiles_in, norm.width_in, norm.eps = scaled.squares.data_ptr(), tiles, k, scaled.eps
-        need = int(self.lib.xrt_linear_workspace(_ptr(a), _ptr(data), _code(a), m, w.shape[0], k, 0))
+        at_a, at_w, code = _ptr(a), _ptr(data), _code(a)
+        need = int(self.lib.xrt_linear_workspace(at_a, at_w, code, m, w.shape[0], k, 0))
         workspace = self._empty(need, torch.float32, a.device) if need > 0 else None
-        self._check(self.lib.xrt_linear_qkv(_ptr(a), _ptr(data), packing, _code(a), _ptr(qkv), m, k,
+        self._check(self.lib.xrt_linear_qkv(at_a, at_w, packing, code, _ptr(qkv), m, k,
                                             None if norm is None else ctypes.byref(norm), *prepare,
                                             _ptr(workspace), ctypes.c_long(need), self._stream(a)))
 

@@ -102,6 +102,7 @@ class StepArena:
     def __init__(self, device):
         self.device = torch.device(device)
         self.buffer: Optional[torch.Tensor] = None
+        self.typed: Dict[torch.dtype, torch.Tensor] = {}     # the stretch as elements of a type
         self.at = 0                 # bytes handed out in this step, those that did not fit included
         self.wanted = 0             # the most a step has needed
         self.active = False
@@ -110,7 +111,8 @@ class StepArena:
         capacity = 0 if self.buffer is None else self.buffer.numel()
         if self.wanted > capacity:
             self.buffer = None                                   # (given back before the longer one is taken)
-            self.buffer = torch.empty(self.wanted + self.wanted // 8, dtype=torch.uint8, device=self.device)
+            self.typed.clear()
+            self.buffer = torch.empty((self.wanted + self.wanted // 8 + self.ALIGN - 1) // self.ALIGN * self.ALIGN, dtype=torch.uint8, device=self.device)
         self.at = 0
         self.active = True
 
@@ -120,15 +122,21 @@ class StepArena:
 
     def take(self, shape, dtype: torch.dtype) -> Optional[torch.Tensor]:
         """A tensor of this shape from the stretch, or None if it does not fit (the caller takes it from torch)."""
-        count = 1
-        for size in (shape if isinstance(shape, (tuple, list, torch.Size)) else (shape,)):
+        shape = tuple(shape) if isinstance(shape, (tuple, list)) else (shape,)
+        strides, count = [], 1
+        for size in reversed(shape):
+            strides.append(count)
             count *= int(size)
-        size = count * torch.empty(0, dtype=dtype).element_size()
+        item = dtype.itemsize
         start = (self.at + self.ALIGN - 1) // self.ALIGN * self.ALIGN
-        self.at = start + size
+        self.at = start + count * item
         if self.buffer is None or self.at > self.buffer.numel():
             return None
-        return self.buffer[start:start + size].view(dtype).view(shape)
+        whole = self.typed.get(dtype)
+        if whole is None:
+            whole = self.typed[dtype] = self.buffer.view(dtype)
+        # (one call instead of a slice and two views, which a step makes some hundred times)
+        return whole.as_strided(shape, strides[::-1], start // item)
 
 
 class Runtime:
