@@ -181,6 +181,22 @@ def test_linear_glu_large_tiles(ops, m, n, k, packed):
         assert rel(out.cpu(), want) < (ULP["bfloat16"] * 2 if dtype == torch.bfloat16 else 1e-5)
 
 
+# Gates so negative that their sigmoid is a denormal number, and far beyond: in the quick epilogues of few and of many rows too.
+@pytest.mark.parametrize("m", [1, 40, 250])
+def test_linear_glu_of_very_negative_gates(ops, m):
+    n, k = 4096, 64
+    gates = torch.tensor([-80.0, -86.0, -87.5, -88.0, -200.0, 0.0, 3.0, -1e-3], dtype=torch.float64).repeat(n // 8)
+    w = torch.cat([(gates / k)[:, None].expand(n, k), torch.full((n, k), 1.0 / k)]).to(torch.bfloat16).to(DEV)
+    a = torch.ones(m, k, dtype=torch.bfloat16, device=DEV)
+    both = a.double() @ w.double().t()
+    want = P.swiglu(both[:, :n], both[:, n:]).cpu()
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops.linear_glu(a, ops.pack(w, "gated", gated_n=n), out)
+    error = (out.cpu().double() - want).abs()
+    # relative, element by element: the rounding of the result, and what float32 leaves of exp(88) (88 * 2^-24 relative); down to what float32 exp can reach
+    assert bool((error <= want.abs() * 2 * ULP["bfloat16"] + 1e-38).all())
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16", "bfloat16 packed"])
 @pytest.mark.parametrize("m,n,k", [(1, 176, 64), (9, 100, 96), (64, 520, 200), (200, 1000, 72), (48, 2000, 520),
                                    (3, 8, 32), (16, 24, 160), (30, 1000, 96), (64, 4104, 224), (8, 14336, 4096),

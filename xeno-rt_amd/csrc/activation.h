@@ -20,7 +20,9 @@ __device__ __forceinline__ float gate_activation(float z, int activation) {
     switch (activation) {
         case XRT_ACT_SILU:
         default:                                    // silu(z) = z / (1 + exp(-z)): crates/xrt-kernels/src/cpu/silu.rs:1-3 of the reference
-            if constexpr (QUICK) return z * __builtin_amdgcn_rcpf(1.0f + __expf(-z));
+            // (numerator and denominator times 2^-24: the hardware's reciprocal has no denormal results, and without the factor
+            // it would make 0 of the gates below -87)
+            if constexpr (QUICK) return (z * 0x1p-24f) * __builtin_amdgcn_rcpf(fmaf(__expf(-z), 0x1p-24f, 0x1p-24f));
             else return z / (1.0f + expf(-z));
     }
 }
