@@ -894,6 +894,13 @@ def test_attention_of_few_new_tokens_on_a_long_cache(ops, nh, nkv, hd, starts, c
     assert rel(out.cpu(), want) < 1e-2                       # probabilities and results in bfloat16, as without the cut
 
 
+@pytest.mark.parametrize("nh,nkv,hd,count", [(16, 8, 128, 1024), (32, 8, 128, 1024), (32, 8, 64, 2048), (16, 8, 128, 2048)])
+def test_prompts_that_begin_are_not_cut_and_those_far_behind_are(ops, nh, nkv, hd, count):
+    assert ops.lib.xrt_attention_workspace(1, count, nh, nkv, hd, 0, count, count) == 0
+    runs, rest = divmod(ops.lib.xrt_attention_workspace(1, 100, nh, nkv, hd, 0, 100, count + 4000), 100 * nh * (hd + 2))
+    assert 2 <= runs <= 8 and rest == 0
+
+
 def test_matrix_core_attention_finds_a_far_key(ops):
     nh, nkv, hd = 8, 2, 128
     kv, keys, values = filled_cache(nkv, hd, torch.bfloat16, [900], seed=1)

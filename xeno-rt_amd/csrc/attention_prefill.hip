@@ -458,8 +458,8 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
     else write_out();
 }
 
-// Merges the runs of keys of one (token, head), in order: a wavefront each, HD / 64 dims a lane.
-template <int HD>
+// Merges the runs of keys of one (token, head), in order: a wavefront each, HD / 64 dims a lane. At most MOST runs.
+template <int HD, int MOST>
 __global__ void __launch_bounds__(4 * XRT_WAVE) attention_prefill_merge_kernel(const PrefillParts parts, int runs, int n_heads,
                                                                                const int* __restrict__ seq_offsets, int n_seqs,
                                                                                bf16* __restrict__ out) {
@@ -467,9 +467,9 @@ __global__ void __launch_bounds__(4 * XRT_WAVE) attention_prefill_merge_kernel(c
     const int lane = threadIdx.x % XRT_WAVE;
     const long row = (long)blockIdx.x * 4 + threadIdx.x / XRT_WAVE, rows = (long)parts.tokens * n_heads;      // (token, head)
     if (row >= rows || row / n_heads >= seq_offsets[n_seqs]) return;      // (tokens beyond the sequences are nobody's)
-    float m_of[MOST_RUNS], l_of[MOST_RUNS], o_of[MOST_RUNS][PER_LANE];
+    float m_of[MOST], l_of[MOST], o_of[MOST][PER_LANE];
 #pragma unroll
-    for (int r = 0; r < MOST_RUNS; ++r) {                     // all runs are asked for at once (those beyond the last: that one again)
+    for (int r = 0; r < MOST; ++r) {                     // all runs are asked for at once (those beyond the last: that one again)
         const long index = (long)min(r, runs - 1) * rows + row;
         const float2 ml = *reinterpret_cast<const float2*>(parts.ml + index * 2);
         m_of[r] = r < runs ? ml.x : -INFINITY;
@@ -479,10 +479,10 @@ __global__ void __launch_bounds__(4 * XRT_WAVE) attention_prefill_merge_kernel(c
     }
     float m = m_of[0];
 #pragma unroll
-    for (int r = 1; r < MOST_RUNS; ++r) m = fmaxf(m, m_of[r]);
+    for (int r = 1; r < MOST; ++r) m = fmaxf(m, m_of[r]);
     float l = 0.f, o[PER_LANE] = {};
 #pragma unroll
-    for (int r = 0; r < MOST_RUNS; ++r) {
+    for (int r = 0; r < MOST; ++r) {
         if (m_of[r] == -INFINITY) continue;                  // this run wrote nothing else
         const float weight = __builtin_amdgcn_exp2f(m_of[r] - m);
         l = fmaf(weight, l_of[r], l);
@@ -496,16 +496,31 @@ __global__ void __launch_bounds__(4 * XRT_WAVE) attention_prefill_merge_kernel(c
     *reinterpret_cast<Dims*>(out + row * HD + lane * PER_LANE) = made;
 }
 
-// Into how many runs a step's keys are cut (1: not at all): as many as fill the compute units that its pairs of tiles leave idle,
-// each of eight blocks of keys at least (a shorter one costs more than it saves: start, merge and 520 bytes a query, head and run).
+// Into how many runs a step's keys are cut (1: not at all). At most as many as fill the compute units that its pairs of tiles leave
+// idle: a second workgroup on a compute unit, which heads of 64 have LDS for, gains nothing (256 pairs on 2048 new tokens 35 -> 54 us).
+// A run takes its share off the time that a pair of tiles spends on its keys (0.58 us a block and tile at heads of 64, 0.78 at 128;
+// half of it where a sequence has one tile, whose wavefronts share its keys), and costs the second kernel and 8 bytes of traffic a dim, query
+// and head. Measured, uncut -> cut, in us: 333 tokens on 2000, 32 heads of 128 in four 70 -> 38; 1024 on 1000 in two 59 -> 55,
+// on 500 46 -> 48, on none 30 -> 36; 2048 on 500, 16 heads of 128 in two 62 -> 58, on none 47 -> 49; 32 on 500 17 -> 20. The estimate cuts
+// those that gain.
 int prefill_runs(int tokens, int n_heads, int head_dim, int max_count, int max_context) {
     const long sequences = (tokens + max_count - 1) / max_count, by_tokens = (tokens + 2 * QW - 1) / (2 * QW);
     const long workgroups = n_heads * (sequences > by_tokens ? sequences : by_tokens);
-    const long places = XRT_COMPUTE_UNITS * (head_dim == 64 ? 2 : 1);              // what the LDS of a workgroup leaves room for
-    const long blocks = (max_context + BT - 1) / BT;
-    long runs = places / workgroups;
-    runs = runs > blocks / 8 ? blocks / 8 : runs;
-    return runs < 2 ? 1 : runs > MOST_RUNS ? MOST_RUNS : (int)runs;
+    const long blocks = (max_context + BT - 1) / BT, seen = (long)max_context - max_count / 2;       // keys of a query, about
+    long most = XRT_COMPUTE_UNITS / workgroups;
+    most = most > blocks / 2 ? blocks / 2 : most;
+    most = most > MOST_RUNS ? MOST_RUNS : most;
+    const long whole = (head_dim == 64 ? 580L : 780L) * (max_count > QW ? 2 : 1) * seen / BT;          // ns
+    long gained = 0;
+    int best = 1;
+    for (int runs = 2; runs <= most; ++runs) {
+        const long gain = whole - whole / runs - 6000 - (long)runs * tokens * n_heads * (head_dim + 2) * 12 / 10000;
+        if (gain > gained) {
+            gained = gain;
+            best = runs;
+        }
+    }
+    return best;
 }
 
 template <int HD>
@@ -528,7 +543,9 @@ int launch_split(const bf16* qkv, int tokens, int n_heads, int n_kv_heads, const
         seq_starts, n_seqs, out, scale, 0, PrefillExtras{}, parts);
     XRT_LAUNCH_CHECK("attention (prefill, runs of keys)");
     const long rows = (long)tokens * n_heads;
-    attention_prefill_merge_kernel<HD><<<(unsigned)((rows + 3) / 4), 4 * XRT_WAVE, 0, s>>>(parts, runs, n_heads, seq_offsets, n_seqs, out);
+    auto merge = runs == 2 ? attention_prefill_merge_kernel<HD, 2> : runs <= 4 ? attention_prefill_merge_kernel<HD, 4>
+                                                                               : attention_prefill_merge_kernel<HD, MOST_RUNS>;
+    merge<<<(unsigned)((rows + 3) / 4), 4 * XRT_WAVE, 0, s>>>(parts, runs, n_heads, seq_offsets, n_seqs, out);
     XRT_LAUNCH_CHECK("attention (prefill, merge)");
     return 0;
 }
