@@ -197,6 +197,23 @@ def test_linear_glu_of_very_negative_gates(ops, m):
     assert bool((error <= want.abs() * 2 * ULP["bfloat16"] + 1e-38).all())
 
 
+# Gates down to the smallest normal number, against up values that bring them back: silu(z) = z / 2 to the rounding of the result.
+@pytest.mark.parametrize("m", [1, 40, 250])
+def test_linear_glu_of_very_small_gates(ops, m):
+    n, k = 4096, 64
+    gates = torch.tensor([1e-30, -1e-35, 6e-36, -1e-36, 1e-37, -1.3e-37, 3e-38, 1.0], dtype=torch.float64).repeat(n // 8)
+    w = torch.zeros(2 * n, k, dtype=torch.float64)
+    w[:n, 0], w[n:, 1] = gates * 2.0 ** 60, 1e30                # one product a sum, so that nothing but the gate itself is small
+    w = w.to(torch.bfloat16).to(DEV)
+    a = torch.zeros(m, k, dtype=torch.bfloat16, device=DEV)
+    a[:, 0], a[:, 1] = 2.0 ** -60, 1.0
+    both = a.double() @ w.double().t()
+    want = P.swiglu(both[:, :n], both[:, n:]).cpu()
+    out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops.linear_glu(a, ops.pack(w, "gated", gated_n=n), out)
+    assert bool(((out.cpu().double() - want).abs() <= want.abs() * ULP["bfloat16"]).all())
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16", "bfloat16 packed"])
 @pytest.mark.parametrize("m,n,k", [(1, 176, 64), (9, 100, 96), (64, 520, 200), (200, 1000, 72), (48, 2000, 520),
                                    (3, 8, 32), (16, 24, 160), (30, 1000, 96), (64, 4104, 224), (8, 14336, 4096),
