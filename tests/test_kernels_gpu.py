@@ -918,6 +918,18 @@ def test_prompts_that_begin_are_not_cut_and_those_far_behind_are(ops, nh, nkv, h
     assert 2 <= runs <= 8 and rest == 0
 
 
+@pytest.mark.parametrize("start", [0, 4000])                # keys that are not cut and keys that are
+@pytest.mark.parametrize("scale", [0.0, -0.125, float("nan")])
+def test_prompts_want_a_positive_scale(ops, start, scale):
+    from xeno_rt_amd.ops.hip import KernelError
+    nh, nkv, hd, count = 8, 2, 128, 20
+    kv, _, _ = filled_cache(nkv, hd, torch.bfloat16, [start + count])
+    assert (ops.lib.xrt_attention_workspace(1, count, nh, nkv, hd, 0, count, start + count) > 0) == (start > 0)
+    qkv = rand(count, (nh + 2 * nkv) * hd, dtype=torch.bfloat16)
+    with pytest.raises(KernelError, match="positive"):
+        ops.attention(qkv, nh, nkv, hd, kv, described([0], [count], [start]), torch.empty(count, nh * hd, dtype=torch.bfloat16, device=DEV), scale=scale)
+
+
 def test_matrix_core_attention_finds_a_far_key(ops):
     nh, nkv, hd = 8, 2, 128
     kv, keys, values = filled_cache(nkv, hd, torch.bfloat16, [900], seed=1)

@@ -591,6 +591,7 @@ int xrt_attention_prefill_split(const void* qkv, int tokens, int n_heads, int n_
                                 const int* block_table, int table_stride, int n_blocks, const int* seq_offsets, const int* seq_slots,
                                 const int* seq_starts, int n_seqs, void* out, float scale, int max_count, int max_context, float* workspace,
                                 hipStream_t s) {
+    XRT_REQUIRE(scale > 0.f, "attention (prefill): the scale is positive");          // (the maximum is taken of the raw products)
     const int runs = prefill_runs(tokens, n_heads, head_dim, max_count, max_context);
     auto run = [&](auto launcher) {
         return launcher((const bf16*)qkv, tokens, n_heads, n_kv_heads, (const bf16*)k_cache, (const bf16*)v_cache, block_table, table_stride,
