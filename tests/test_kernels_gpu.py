@@ -918,6 +918,42 @@ def test_prompts_that_begin_are_not_cut_and_those_far_behind_are(ops, nh, nkv, h
     assert 2 <= runs <= 8 and rest == 0
 
 
+# NaN and infinities in queries, keys and values (whole runs of keys, a run's edge, keys behind some of the queries): cut and not cut
+# the same outputs are finite, and those agree.
+@pytest.mark.parametrize("nh,nkv,hd", [(4, 4, 64), (8, 2, 128)])
+@pytest.mark.parametrize("start,count", [(1100, 200), (2000, 130), (1500, 20)])
+def test_attention_cut_into_runs_keeps_what_is_not_finite(ops, monkeypatch, nh, nkv, hd, start, count):
+    length = start + count
+    kv, _, _ = filled_cache(nkv, hd, torch.bfloat16, [length], seed=hd)
+    blocks = kv.block_table[0].tolist()
+    assert ops.lib.xrt_attention_workspace(1, count, nh, nkv, hd, 0, count, length) > 0
+    nan, inf = float("nan"), float("inf")
+    qkv = rand(count, (nh + 2 * nkv) * hd, dtype=torch.bfloat16, seed=5)
+    qkv[3, :hd] = nan                                        # a query without any score that is a number
+    qkv[7, hd:2 * hd] = inf                                  # scores of either infinity
+    qkv[11, hd] = 3e38
+    clean = kv
+    for head, poison in ((0, lambda k, v: k[blocks[0], 0].fill_(nan)),                                  # the first block's keys
+                         (0, lambda k, v: [k[blocks[b], 0].fill_(nan) for b in range(length // 64)]),     # all keys but the last block's
+                         (0, lambda k, v: [k[blocks[b], 0].fill_(inf) for b in range(2, 4)]),
+                         (0, lambda k, v: v[blocks[length // 64 - 1], 0].fill_(inf)),                     # values, seen by some of the queries
+                         (0, lambda k, v: v[blocks[1], 0].fill_(nan)), (0, lambda k, v: None)):
+        kv = clone_cache(clean)
+        poison(kv.k, kv.v)
+        outs = []
+        for cut in (True, False):
+            with monkeypatch.context() as patch:
+                if not cut:
+                    patch.setattr(ops.lib, "xrt_attention_workspace", lambda *sizes: 0)
+                out = torch.full((count, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV)
+                ops.attention(qkv, nh, nkv, hd, kv, described([0], [count], [start]), out, scale=1.0 / math.sqrt(hd))
+            outs.append(out.float())
+        finite = outs[1].isfinite()
+        assert torch.equal(outs[0][~finite].nan_to_num(nan=7.0), outs[1][~finite].nan_to_num(nan=7.0))
+        assert outs[0][3, :hd].isnan().all() and finite[4, -hd:].all()
+        assert rel(outs[0][finite].cpu(), outs[1][finite].cpu()) < 1e-2          # probabilities and results in bfloat16
+
+
 @pytest.mark.parametrize("start", [0, 4000])                # keys that are not cut and keys that are
 @pytest.mark.parametrize("scale", [0.0, -0.125, float("nan")])
 def test_prompts_want_a_positive_scale(ops, start, scale):

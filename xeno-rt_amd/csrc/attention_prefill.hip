@@ -65,7 +65,7 @@ struct PrefillExtras {
 // merges the runs in order. (333 tokens behind 3001: 97 us, with four runs and the second kernel 41 + 8.)
 struct PrefillParts {
     float* o;                          // [runs][tokens][heads][HD], relative to the maximum
-    float* ml;                         // [runs][tokens][heads][2]: maximum (-inf: no key of this run is seen) and sum
+    float* ml;                         // [runs][tokens][heads][2]: maximum (-inf: no key of this run has a score above that) and sum
     int tokens;
 };
 template <int HD, bool FINE, bool EXTRAS = false, bool SPLIT = false>
@@ -189,13 +189,13 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
                 *reinterpret_cast<Four*>(dst + dt * 32 + g * 8 + half * 4) = four;
             }
     };
-    // What a run of keys makes of the queries at hand (l summed over the pair of lanes); nothing seen: the maximum says so.
+    // What a run of keys makes of the queries at hand (l summed over the pair of lanes). A maximum of -inf does not say that no
+    // key was seen (scores that are all NaN leave it there too), so the sums are written whatever it is.
     auto write_part = [&]() {
         if constexpr (SPLIT) {
             if (!q_valid) return;
             const long index = ((long)blockIdx.z * parts.tokens + token) * n_heads + head;
             if (half == 0) *reinterpret_cast<float2*>(parts.ml + index * 2) = make_float2(m, l);
-            if (m == -INFINITY) return;
             float* dst = parts.o + index * HD;
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt)
@@ -458,33 +458,32 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) attention_prefill_kernel(
     else write_out();
 }
 
-// Merges the runs of keys of one (token, head), in order: a wavefront each, HD / 64 dims a lane. At most MOST runs.
-template <int HD, int MOST>
-__global__ void __launch_bounds__(4 * XRT_WAVE) attention_prefill_merge_kernel(const PrefillParts parts, int runs, int n_heads,
-                                                                               const int* __restrict__ seq_offsets, int n_seqs,
-                                                                               bf16* __restrict__ out) {
+// Merges the RUNS runs of keys of one (token, head), in order: a wavefront each, HD / 64 dims a lane.
+template <int HD, int RUNS>
+__global__ void __launch_bounds__(4 * XRT_WAVE) attention_prefill_merge_kernel(const PrefillParts parts, int n_heads, const int* __restrict__ seq_offsets,
+                                                                               int n_seqs, bf16* __restrict__ out) {
     constexpr int PER_LANE = HD / XRT_WAVE;
     const int lane = threadIdx.x % XRT_WAVE;
     const long row = (long)blockIdx.x * 4 + threadIdx.x / XRT_WAVE, rows = (long)parts.tokens * n_heads;      // (token, head)
     if (row >= rows || row / n_heads >= seq_offsets[n_seqs]) return;      // (tokens beyond the sequences are nobody's)
-    float m_of[MOST], l_of[MOST], o_of[MOST][PER_LANE];
+    float m_of[RUNS], l_of[RUNS], o_of[RUNS][PER_LANE];
 #pragma unroll
-    for (int r = 0; r < MOST; ++r) {                     // all runs are asked for at once (those beyond the last: that one again)
-        const long index = (long)min(r, runs - 1) * rows + row;
+    for (int r = 0; r < RUNS; ++r) {                     // all runs are asked for at once
+        const long index = (long)r * rows + row;
         const float2 ml = *reinterpret_cast<const float2*>(parts.ml + index * 2);
-        m_of[r] = r < runs ? ml.x : -INFINITY;
+        m_of[r] = ml.x;
         l_of[r] = ml.y;
 #pragma unroll
         for (int d = 0; d < PER_LANE; ++d) o_of[r][d] = parts.o[index * HD + lane * PER_LANE + d];
     }
     float m = m_of[0];
 #pragma unroll
-    for (int r = 1; r < MOST; ++r) m = fmaxf(m, m_of[r]);
+    for (int r = 1; r < RUNS; ++r) m = fmaxf(m, m_of[r]);
+    const float m_safe = m == -INFINITY ? 0.f : m;           // (as the wavefronts of a tile merge: a NaN of any run stays one)
     float l = 0.f, o[PER_LANE] = {};
 #pragma unroll
-    for (int r = 0; r < MOST; ++r) {
-        if (m_of[r] == -INFINITY) continue;                  // this run wrote nothing else
-        const float weight = __builtin_amdgcn_exp2f(m_of[r] - m);
+    for (int r = 0; r < RUNS; ++r) {
+        const float weight = __builtin_amdgcn_exp2f(m_of[r] - m_safe);       // 0 for a run that saw no key
         l = fmaf(weight, l_of[r], l);
 #pragma unroll
         for (int d = 0; d < PER_LANE; ++d) o[d] = fmaf(weight, o_of[r][d], o[d]);
@@ -543,9 +542,19 @@ int launch_split(const bf16* qkv, int tokens, int n_heads, int n_kv_heads, const
         seq_starts, n_seqs, out, scale, 0, PrefillExtras{}, parts);
     XRT_LAUNCH_CHECK("attention (prefill, runs of keys)");
     const long rows = (long)tokens * n_heads;
-    auto merge = runs == 2 ? attention_prefill_merge_kernel<HD, 2> : runs <= 4 ? attention_prefill_merge_kernel<HD, 4>
-                                                                               : attention_prefill_merge_kernel<HD, MOST_RUNS>;
-    merge<<<(unsigned)((rows + 3) / 4), 4 * XRT_WAVE, 0, s>>>(parts, runs, n_heads, seq_offsets, n_seqs, out);
+    const auto merge = [&] {
+        static_assert(MOST_RUNS == 8, "a kernel for every number of runs");
+        switch (runs) {
+            case 2: return attention_prefill_merge_kernel<HD, 2>;
+            case 3: return attention_prefill_merge_kernel<HD, 3>;
+            case 4: return attention_prefill_merge_kernel<HD, 4>;
+            case 5: return attention_prefill_merge_kernel<HD, 5>;
+            case 6: return attention_prefill_merge_kernel<HD, 6>;
+            case 7: return attention_prefill_merge_kernel<HD, 7>;
+            default: return attention_prefill_merge_kernel<HD, 8>;
+        }
+    }();
+    merge<<<(unsigned)((rows + 3) / 4), 4 * XRT_WAVE, 0, s>>>(parts, n_heads, seq_offsets, n_seqs, out);
     XRT_LAUNCH_CHECK("attention (prefill, merge)");
     return 0;
 }
