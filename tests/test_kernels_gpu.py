@@ -738,6 +738,20 @@ def test_attention_with_scores_biased_by_distance(ops, cpp, dtype, nh, nkv, hd):
                 assert rel(plain[t].cpu(), want) > 10 * limit        # the slopes do change the result
 
 
+@pytest.mark.parametrize("count", [1, 20])
+def test_attention_with_scores_biased_by_distance_takes_no_workspace(ops, monkeypatch, count):
+    nh, nkv, hd, start = 8, 2, 128, 4000
+    kv, _, _ = filled_cache(nkv, hd, torch.bfloat16, [start + count])
+    assert ops.lib.xrt_attention_workspace(1, count, nh, nkv, hd, 0, count, start + count) > 0
+    qkv = rand(count, (nh + 2 * nkv) * hd, dtype=torch.bfloat16)
+    taken = []
+    monkeypatch.setattr(ops, "allocate", lambda shape, dtype, device: taken.append(shape) or torch.empty(shape, dtype=dtype, device=device))
+    for slopes in (None, torch.full((nh,), 0.1, device=DEV)):
+        out = torch.empty(count, nh * hd, dtype=torch.bfloat16, device=DEV)
+        ops.attention(qkv, nh, nkv, hd, kv, described([0], [count], [start]), out, scale=1.0 / math.sqrt(hd), distance_slopes=slopes)
+        assert len(taken) == 1                               # the one of the kernels without slopes
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_attention_window_edge(ops, dtype):
     """With a window of W a query at P sees keys P-W+1..P: a loud key just outside must be

@@ -574,8 +574,9 @@ class HipOps:
             self._require(starts, "sequence starts", torch.int32, (n_seqs,), qkv)
             if max_context > stride * BLOCK_TOKENS:
                 raise KernelError(f"attention: a sequence of {max_context} tokens exceeds the block table")
-            workspace_floats = int(self.lib.xrt_attention_workspace(_code(qkv), tokens, n_heads, n_kv_heads, head_dim,
-                                                                    int(window or 0), max_count, max_context))
+            if distance_slopes is None:                         # (the general kernel, which serves those, needs none)
+                workspace_floats = int(self.lib.xrt_attention_workspace(_code(qkv), tokens, n_heads, n_kv_heads, head_dim,
+                                                                        int(window or 0), max_count, max_context))
             if workspace_floats > 0:
                 workspace = self._empty(workspace_floats, torch.float32, qkv.device)
         self._check(self.lib.xrt_attention(
