@@ -181,6 +181,28 @@ def test_linear_glu_large_tiles(ops, m, n, k, packed):
         assert rel(out.cpu(), want) < (ULP["bfloat16"] * 2 if dtype == torch.bfloat16 else 1e-5)
 
 
+# 17 to 64 rows: a w that the last cache cannot keep passes the caches by; the halves of it, which do not, give the same bits.
+@pytest.mark.parametrize("m", [17, 64])
+def test_linear_of_a_w_beyond_the_caches(ops, m):
+    for n, k, kind in ((140000, 1024, "tiles"), (24000, 2048, "gated")):
+        rows = n if kind == "tiles" else 2 * n
+        a, w = rand(m, k, dtype=torch.bfloat16, seed=m), rand(rows, k, dtype=torch.bfloat16, seed=n, scale=0.1)
+        wholes, halves = [], []
+        for part, into in ((w, wholes), (w.view(rows // n, 2, n // 2, k)[:, 0], halves), (w.view(rows // n, 2, n // 2, k)[:, 1], halves)):
+            part = part.reshape(-1, k)
+            of = part.shape[0] * n // rows
+            out = torch.empty(m, of, dtype=torch.bfloat16, device=DEV)
+            if kind == "gated":
+                ops.linear_glu(a, ops.pack(part, "gated", gated_n=of), out)
+            else:
+                ops.linear(a, ops.pack(part, "tiles"), out)
+            into.append(out)
+        assert torch.equal(wholes[0], torch.cat(halves, dim=1))
+        both = a.float() @ w.float().t()
+        want = both if kind == "tiles" else P.swiglu(both[:, :n], both[:, n:])
+        assert rel(wholes[0].cpu(), want.cpu()) < ULP["bfloat16"] * 2
+
+
 # Gates so negative that their sigmoid is a denormal number, and far beyond: in the quick epilogues of few and of many rows too.
 @pytest.mark.parametrize("m", [1, 40, 250])
 def test_linear_glu_of_very_negative_gates(ops, m):

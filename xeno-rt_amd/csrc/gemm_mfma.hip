@@ -58,8 +58,8 @@ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, int tiles_n
 struct RowScale { const float* squares; int tiles; int width; float eps; int activation; };     // (activation: of a gated epilogue)
 
 // One tile of the product, by one workgroup: `id` is the workgroup's number among those that work
-// on the output columns from n_first on, tiles_m x tiles_n of them.
-template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO>
+// on the output columns from n_first on, tiles_m x tiles_n of them. PAST_CACHES: w is asked for past the caches.
+template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES = false>
 __device__ __forceinline__ void gemm_tile(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
     int id, int tiles_m, int tiles_n, int n_first, int k_per_split, const Packing packing, const RowScale scale = RowScale{},
@@ -180,10 +180,6 @@ __device__ __forceinline__ void gemm_tile(
         const unsigned w_step = packed_b ? 32u : 2u;                // bytes per column of k
         const int wave_uniform = __builtin_amdgcn_readfirstlane(wave);
         const unsigned lds_a0 = lds_address(stage_a), lds_b0 = lds_address(stage_b);
-        // Up to 64 rows of a, k not split: every byte of w is read by one workgroup, in one long run, and passes the caches by
-        // (64 rows: gate/up 47.2 -> 44.1 us, an output head of 128256 rows 212 -> 197). Split along k the runs are short, and so marked
-        // they are read more slowly (4096 x 4096 in eight parts 16.3 -> 18.1 us).
-        const bool past_caches = gridDim.y == 1;
         auto issue = [&](int stage, int k0) {
 #pragma unroll
             for (int i = 0; i < LOADS_A; ++i) {
@@ -194,7 +190,7 @@ __device__ __forceinline__ void gemm_tile(
             for (int i = 0; i < LOADS_B; ++i) {
                 const int block = min(i * WAVES + wave_uniform, BLOCKS_B - 1);
                 const unsigned to = lds_b0 + (unsigned)((stage * BN + block * ROWS) * DK * 2);
-                if (BM <= 64 && past_caches) stream_to_lds(w, off_b[i] + (unsigned)k0 * w_step, to);
+                if constexpr (PAST_CACHES) stream_to_lds(w, off_b[i] + (unsigned)k0 * w_step, to);
                 else load_to_lds(w, off_b[i] + (unsigned)k0 * w_step, to);
             }
         };
@@ -845,11 +841,11 @@ __global__ void __launch_bounds__(8 * XRT_WAVE) gemm_large_kernel(
     gemm_large_tile<BM, MODE, TO>(a, w, out, M, N, K, place, 0, k_per_split, packing, activation);
 }
 
-template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO>
+template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES>
 __global__ void __launch_bounds__(WM * WN * XRT_WAVE) gemm_mfma_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
     int tiles_m, int tiles_n, int n_first, int k_per_split, const Packing packing, const RowScale scale) {
-    gemm_tile<BM, BN, WM, WN, MODE, DK, STAGES, TO>(a, w, out, M, N, K, blockIdx.x, tiles_m, tiles_n, n_first, k_per_split, packing, scale);
+    gemm_tile<BM, BN, WM, WN, MODE, DK, STAGES, TO, PAST_CACHES>(a, w, out, M, N, K, blockIdx.x, tiles_m, tiles_n, n_first, k_per_split, packing, scale);
 }
 
 // Two tile shapes in one launch: the first `large_blocks` workgroups take 256 x 256 tiles of the
@@ -925,16 +921,31 @@ int launch_grouped_of(const bf16* x, const bf16* m, long w_stride, void* out, in
     return launch_grouped<BM, MODE_STORE, bf16>(x, m, w_stride, (bf16*)out, tiles_m, N, K, lda, ldw, tile_group, packing, activation, splits, s);
 }
 
+// Up to 64 rows of a, k not split: every byte of w is read by one workgroup, in one long run, and is asked for past the caches
+// where it cannot stay in the last one (256 MB) until the next step. (Among other matrices, 64 rows: gate/up of 28672 rows
+// of w and k = 4096 46.6 -> 44.1 us, an output head of 128256 rows and k = 2048 105.0 -> 98.5. A w that does stay is read faster from
+// there: 17408 rows and k = 1024, 214 MB of such matrices in turn, 11.3 us as it is, 12.8 past the caches.) A gated matrix counts one
+// and a half times: a model has the one back from that width too. Split along k the runs are short, and so marked they are
+// read more slowly (4096 x 4096 in eight parts 16.3 -> 18.1 us).
+template <int BM, int MODE>
+bool reads_past_caches(int N, int K, int splits) {
+    constexpr long LAST_CACHE = 256L << 20;
+    return BM <= 64 && splits == 1 && (MODE == MODE_GATED ? 3L * N : (long)N) * K * (long)sizeof(bf16) > LAST_CACHE;
+}
+
 // Launches the tiles of output columns [n_first, n_first + n_count).
-template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO>
+template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES = false>
 int launch_kernel(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int n_first, int n_count, const Packing& packing,
                   hipStream_t s, int splits = 1, int k_per_split = 0, const RowScale scale = RowScale{}) {
+    if constexpr (BM <= 64 && !PAST_CACHES)
+        if (reads_past_caches<BM, MODE>(N, K, splits))
+            return launch_kernel<BM, BN, WM, WN, MODE, DK, STAGES, TO, true>(a, w, out, M, N, K, n_first, n_count, packing, s, splits, k_per_split, scale);
     constexpr int BN_OUT = MODE == MODE_GATED ? BN / 2 : BN;
     constexpr int THREADS = WM * WN * XRT_WAVE;
     constexpr size_t staging = DK != 0 ? (size_t)STAGES * (BM + BN) * DK * sizeof(bf16) : (size_t)2 * (BM + BN) * PITCH * sizeof(bf16);
     constexpr size_t lds = staging;
     static_assert(lds <= 160 * 1024, "tile does not fit the LDS of a compute unit");
-    auto kernel = gemm_mfma_kernel<BM, BN, WM, WN, MODE, DK, STAGES, TO>;
+    auto kernel = gemm_mfma_kernel<BM, BN, WM, WN, MODE, DK, STAGES, TO, PAST_CACHES>;
     static bool configured = false;          // per instantiation
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
