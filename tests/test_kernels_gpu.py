@@ -144,10 +144,12 @@ def test_linear_float32_has_the_same_bits_with_few_rows_and_with_many(ops, m, n,
             assert torch.equal(torch.nan_to_num(got, nan=7.0), torch.nan_to_num(want, nan=7.0))
 
 
-# The tiles of eight wavefronts (256 and 128 rows by 256) at the edges of tiles, with one, two and three steps along k, columns that
-# do and do not allow 16 bytes a store; by the rule of the launcher: large tiles alone, half tiles alone, both in one launch.
+# The tiles of eight wavefronts (256 and 128 rows by 256) and those of 256 x 192 at the edges of tiles, with one, two and three steps along
+# k and more, columns that do and do not allow 16 bytes a store. By the rule of the launcher, stored (added): large (large), half (narrow),
+# large (large), narrow (narrow), mixed (narrow), mixed (narrow); then half (half) twice, mixed (mixed), narrow (narrow) twice, large (large).
 @pytest.mark.parametrize("kind", ["plain", "packed", "rotary"])
-@pytest.mark.parametrize("m,n,k", [(250, 61001, 64), (257, 47104, 128), (130, 61440, 192), (520, 16128, 320), (1100, 16000, 128), (2048, 11008, 64)])
+@pytest.mark.parametrize("m,n,k", [(250, 61001, 64), (257, 47104, 128), (130, 61440, 192), (520, 16128, 320), (1100, 16000, 128), (2048, 11008, 64),
+                                   (270, 14990, 1984), (1900, 4090, 1472), (1030, 19616, 256), (393, 16400, 64), (2816, 3070, 512), (520, 16400, 192)])
 def test_linear_large_tiles(ops, m, n, k, kind):
     if kind == "rotary" and n % 256 != 0:
         pytest.skip("whole heads")
@@ -167,8 +169,10 @@ def test_linear_large_tiles(ops, m, n, k, kind):
     assert rel(out32.cpu(), want) < 1e-5
 
 
+# (large, mixed, large, large, mixed; then half three times, mixed)
 @pytest.mark.parametrize("packed", [False, True])
-@pytest.mark.parametrize("m,n,k", [(250, 30504, 64), (257, 24000, 128), (140, 31000, 192), (520, 8200, 320), (2048, 5504, 64)])
+@pytest.mark.parametrize("m,n,k", [(250, 30504, 64), (257, 24000, 128), (140, 31000, 192), (520, 8200, 320), (2048, 5504, 64),
+                                   (140, 5072, 128), (2040, 2040, 64), (700, 5000, 1024), (790, 9352, 64)])
 def test_linear_glu_large_tiles(ops, m, n, k, packed):
     a = rand(m, k, dtype=torch.bfloat16, seed=m)
     w = rand(2 * n, k, dtype=torch.bfloat16, seed=n, scale=0.3)

@@ -984,15 +984,19 @@ int launch_large(const bf16* a, const bf16* w, TO* out, int M, int N, int K, con
     return 0;
 }
 
-// Time of `tiles` tiles that run in rounds over `places`, in units of a tenth of a microsecond or so: `round` is what a full
-// round takes, a last round that is partly filled takes its share of that, but `least` percent of it: the chip is bound by its
-// power, and with fewer compute units at work their clock rises (256 x 256 tiles, k = 4096: 106 us a full round, 84 us 0.75 of
-// one; 28672 rows of w and 2048 rows of x, 3.5 rounds: 372 us).
-long rounds_cost(long tiles, int places, int round, int least) {
-    const long whole = tiles / places, rest = tiles % places;
-    return whole * round * 100L + (rest == 0 ? 0 : (rest * 100 / places > least ? rest * 100 / places : least) * (long)round);
+// What a tile shape costs: a full round over `places` takes `products` microseconds for each 4096 of k and ends[mode] for its
+// first loads and its epilogue. A last round that is partly filled takes `least` percent of a full one and its share of the
+// rest: the chip is bound by its power, and with fewer compute units at work their clock rises. The numbers are fitted to 608
+// products (layers of seven sizes and sizes drawn at random, k from 512 to 25600, 129 to 8192 rows of x), every tile shape
+// of each of them timed: what the estimate chooses is 0.3 % off the best of them on average.
+struct TileTime { int bm, bn, places, products, ends[3], least; };
+constexpr TileTime LARGE_TILE = {256, 256, XRT_COMPUTE_UNITS, 88, {10, 14, 16}, 56}, HALF_TILE = {128, 256, XRT_COMPUTE_UNITS, 57, {5, 10, 9}, 56},
+                   NARROW_TILE = {256, 192, XRT_COMPUTE_UNITS, 80, {8, 8, 0}, 56}, SMALL_TILE = {128, 128, 2 * XRT_COMPUTE_UNITS, 64, {6, 8, 10}, 45};
+long rounds_cost(long tiles, const TileTime& tile, int K, int mode) {        // in nanoseconds or so
+    const long round = tile.products * 1000L * K / 4096 + tile.ends[mode] * 1000L;
+    const long whole = tiles / tile.places, rest = tiles % tile.places;
+    return whole * round + (rest == 0 ? 0 : (tile.least + (100 - tile.least) * rest / tile.places) * round / 100);
 }
-enum { LARGE_ROUND = 106, HALF_ROUND = 66, SMALL_ROUND = 75 };      // 256 x 256, 128 x 256 and 128 x 128 tiles (two to a compute unit), k = 4096
 
 template <int MODE, typename TO>
 int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, const Packing& packing, int activation, hipStream_t s) {
@@ -1012,20 +1016,27 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
     if constexpr (MODE == MODE_GATED)
         if (M <= 128) return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
     // 256 x 256 tiles cost the least energy a product, and tiles of half the height somewhat more (2048 rows of x, 4096 rows of
-    // w, k = 4096: 128 tiles of the one 93 us, 256 of the other 69; 6144 rows of w: 84 and 103); tiles of 128 x 128 only
-    // where neither fills the chip (1024 rows of x, 4096 rows of w: 55 against 58 and 86 us).
-    const long large = rounds_cost(tiles(256, 256), XRT_COMPUTE_UNITS, LARGE_ROUND, 72);
-    const long half = rounds_cost(tiles(128, 256), XRT_COMPUTE_UNITS, HALF_ROUND, 80);
-    const long small = rounds_cost(tiles(128, 128), 2 * XRT_COMPUTE_UNITS, SMALL_ROUND, 68);
+    // w, k = 4096: 128 tiles of the one 85 us, 256 of the other 58; 6144 rows of w: 82 and 102); tiles of 128 x 128, two to a compute
+    // unit, where neither fills the chip, or where k is so short that one's epilogue wants another's products beside it (200 rows of x,
+    // 9632 rows of w, k = 1728, adding: 25 against 31 us). The tiles of 256 x 192, which are gemm_tile's, where they make one round that
+    // the large ones leave half empty and those of half the height need two for (3072 rows of w, k = 3072, 2816 rows of x: 63
+    // against 73 and 90 us; 4096 rows, k = 14336, 2300 rows of x: 250, 259 and 327). They read their operands more often, which a w
+    // beyond the caches does not stand (5120 rows of w, k = 25600, 2048 rows of x: 572 against 447 us; 13536 rows, k = 10624,
+    // 724 rows of x: 240 against 188).
+    constexpr long NARROW_W = 150L * 1000 * 1000;              // bytes
+    auto cost = [&](const TileTime& tile) { return rounds_cost(tiles(tile.bm, tile.bn), tile, K, MODE); };
+    const long large = cost(LARGE_TILE), half = cost(HALF_TILE), small = cost(SMALL_TILE);
+    const long narrow = MODE != MODE_GATED && (long)N * K * (long)sizeof(bf16) <= NARROW_W ? cost(NARROW_TILE) : LONG_MAX;
     // Large tiles for as many columns as make whole rounds, and tiles of half the height for the rest, if those then fit
-    // one round: the last round is full of half-sized work instead of half empty (3.5 rounds: 366 against 372 us).
+    // one round: the last round is full of half-sized work instead of half empty (28672 rows of w, k = 4096, 2048 rows of x:
+    // 366 against 372 us).
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 256 / DIV - 1) / (256 / DIV);
     const int whole_columns = (int)((long)tiles_m * tiles_n / XRT_COMPUTE_UNITS * XRT_COMPUTE_UNITS / tiles_m);     // n-tiles that run in full rounds
     const long rest_tiles = (long)((M + 127) / 128) * (tiles_n - whole_columns);
     long mixed = LONG_MAX;
     if (whole_columns > 0 && whole_columns < tiles_n && rest_tiles <= XRT_COMPUTE_UNITS)
-        mixed = rounds_cost((long)tiles_m * whole_columns, XRT_COMPUTE_UNITS, LARGE_ROUND, 72) + rounds_cost(rest_tiles, XRT_COMPUTE_UNITS, HALF_ROUND, 80);
-    if (mixed < large && mixed <= half && mixed <= small) {
+        mixed = rounds_cost((long)tiles_m * whole_columns, LARGE_TILE, K, MODE) + rounds_cost(rest_tiles, HALF_TILE, K, MODE);
+    if (mixed < large && mixed <= half && mixed <= small && mixed <= narrow) {
         const int split = whole_columns * (256 / DIV);
         const int small_tiles_m = (M + 127) / 128, small_tiles_n = tiles_n - whole_columns;
         const int large_blocks = (tiles_m * whole_columns + 7) / 8 * 8;      // whole rounds over the XCDs
@@ -1043,8 +1054,10 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
         XRT_LAUNCH_CHECK("linear (mfma, two tile shapes)");
         return 0;
     }
-    if (large <= half && large <= small) return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
-    if (half <= small) return launch_large<128, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+    if (large <= half && large <= small && large <= narrow) return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+    if (half <= small && half <= narrow) return launch_large<128, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+    if constexpr (MODE != MODE_GATED)
+        if (narrow <= small) return launch_kernel<256, 192, 4, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
     // (four stages of 32 keep a load in flight for longer but meet at twice as many barriers, and measured slower)
     return launch_kernel<128, 128, 2, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
 }
