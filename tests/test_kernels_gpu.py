@@ -185,6 +185,28 @@ def test_linear_glu_large_tiles(ops, m, n, k, packed):
         assert rel(out.cpu(), want) < (ULP["bfloat16"] * 2 if dtype == torch.bfloat16 else 1e-5)
 
 
+# Results that do not begin at a multiple of 16 bytes go out in single elements: the same bits (large tiles, both halves of a launch, half
+# tiles; the padding around the result stays).
+@pytest.mark.parametrize("m,n,k,kind", [(520, 16400, 192, "store"), (1030, 19616, 256, "store"), (270, 15000, 1984, "store"), (520, 8200, 320, "gated"),
+                                        (790, 9352, 64, "gated"), (140, 5072, 128, "gated"), (520, 16400, 192, "add")])
+@pytest.mark.parametrize("packed", [False, True])
+def test_large_tiles_into_a_result_that_is_not_aligned(ops, m, n, k, kind, packed):
+    a, w = rand(m, k, dtype=torch.bfloat16, seed=m), rand(2 * n if kind == "gated" else n, k, dtype=torch.bfloat16, seed=n, scale=0.1)
+    w = packed_or_not(ops, w, packed, "gated" if kind == "gated" else "tiles", **({"gated_n": n} if kind == "gated" else {}))
+    dtype = torch.float32 if kind == "add" else torch.bfloat16
+    results = []
+    for at in (8, 9):                                            # elements: a multiple of 16 bytes, and not
+        room = torch.full((m * n + 32,), 7.0, dtype=dtype, device=DEV)
+        out = room[at:at + m * n].view(m, n)
+        if kind == "gated":
+            ops.linear_glu(a, w, out)
+        else:
+            ops.linear(a, w, out, accumulate=kind == "add")
+        assert bool((room[:at] == 7.0).all()) and bool((room[at + m * n:] == 7.0).all())
+        results.append(out)
+    assert torch.equal(results[0], results[1]) and not bool((results[0] == 7.0).all())
+
+
 # 17 to 64 rows: a w that the last cache cannot keep passes the caches by; the halves of it, which do not, give the same bits.
 @pytest.mark.parametrize("m", [17, 64])
 def test_linear_of_a_w_beyond_the_caches(ops, m):
@@ -992,6 +1014,36 @@ def test_attention_cut_into_runs_keeps_what_is_not_finite(ops, monkeypatch, nh, 
         assert torch.equal(outs[0][~finite].nan_to_num(nan=7.0), outs[1][~finite].nan_to_num(nan=7.0))
         assert outs[0][3, :hd].isnan().all() and finite[4, -hd:].all()
         assert rel(outs[0][finite].cpu(), outs[1][finite].cpu()) < 1e-2          # probabilities and results in bfloat16
+
+
+# A step whose keys would be cut, with tokens behind the sequences (padding, whose rows nobody writes), and with a workspace that is missing,
+# a float too small or not aligned to 16 bytes: the kernel that does not cut then serves it.
+@pytest.mark.parametrize("nh,nkv,hd", [(4, 4, 64), (8, 2, 128)])
+def test_attention_of_few_new_tokens_with_padding_or_without_its_workspace(ops, monkeypatch, nh, nkv, hd):
+    starts, counts, padding = [1500, 700], [40, 100], 5
+    lengths = [s + n for s, n in zip(starts, counts)]
+    kv, keys, values = filled_cache(nkv, hd, torch.bfloat16, lengths, seed=hd)
+    batch = described([0, 1], counts, starts)
+    tokens = sum(counts)
+    batch.slots, batch.positions = (torch.cat([x, x.new_full((padding,), fill)]) for x, fill in ((batch.slots, -1), (batch.positions, 0)))
+    qkv = rand(tokens + padding, (nh + 2 * nkv) * hd, dtype=torch.bfloat16, seed=5, scale=2.0)
+    need = ops.lib.xrt_attention_workspace(1, tokens + padding, nh, nkv, hd, 0, max(counts), max(lengths))
+    assert need > 0
+    want = expected_attention(qkv[:tokens], batch.slots[:tokens].tolist(), batch.positions[:tokens].tolist(), keys, values, nh, nkv, hd)
+    outs = {}
+    for kind in ("cut", "none", "small", "unaligned"):
+        with monkeypatch.context() as patch:
+            if kind in ("none", "small"):
+                patch.setattr(ops.lib, "xrt_attention_workspace", lambda *sizes: 0 if kind == "none" else need - 1)
+            if kind == "unaligned":
+                patch.setattr(ops, "allocate", lambda count, dtype, device: torch.empty(count + 1, dtype=dtype, device=device)[1:])
+            out = torch.full((tokens + padding, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV)
+            ops.attention(qkv, nh, nkv, hd, kv, batch, out, scale=1.0 / math.sqrt(hd))
+        assert rel(out[:tokens].cpu(), want) < 1e-2              # probabilities and results in bfloat16
+        assert bool((out[tokens:] == 7.0).all())
+        outs[kind] = out
+    assert torch.equal(outs["none"], outs["small"]) and torch.equal(outs["none"], outs["unaligned"])
+    assert not torch.equal(outs["none"], outs["cut"])            # (another order of the sums: the cut was taken)
 
 
 @pytest.mark.parametrize("start", [0, 4000])                # keys that are not cut and keys that are
