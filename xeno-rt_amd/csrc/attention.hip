@@ -66,8 +66,7 @@ extern "C" int xrt_attention(const void* qkv, int dtype, int tokens, int n_heads
                                         table_stride, n_blocks, positions, slots, out, scale, max_context, workspace,
                                         workspace_floats, nullptr, s);
         if (max_count > 1 && xrt_attention_prefill_accepts(head_dim)) {
-            // tokens beyond the sequences (padding) get zeros
-            // (their rows are read by nothing, but must not hold what a later product could choke on)
+            // (tokens beyond the sequences, padding, are nobody's: their rows of out stay as they are, and nothing reads them)
             XRT_REQUIRE(n_seqs <= tokens, "attention: more sequences than tokens");
             // few new tokens on a long cache, and room for what the runs of their keys make: cut (without the room: not)
             if (need > 0 && workspace != nullptr && workspace_floats >= need && (uintptr_t)workspace % 16 == 0)

@@ -57,13 +57,12 @@ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, int tiles_n
 // multiplies its sums by it before the epilogue. squares null: nothing of the kind.
 struct RowScale { const float* squares; int tiles; int width; float eps; int activation; };     // (activation: of a gated epilogue)
 
-// One tile of the product, by one workgroup: `id` is the workgroup's number among those that work
-// on the output columns from n_first on, tiles_m x tiles_n of them. PAST_CACHES: w is asked for past the caches.
+// One tile of the product, by one workgroup: `id` is the workgroup's number among the tiles_m x tiles_n tiles.
+// PAST_CACHES: w is asked for past the caches.
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES = false>
 __device__ __forceinline__ void gemm_tile(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
-    int id, int tiles_m, int tiles_n, int n_first, int k_per_split, const Packing packing, const RowScale scale = RowScale{},
-    const int lda = 0, const int ldw = 0) {      // lda, ldw: how far the rows of a and of w lie apart, if not K (whole tiles along k only)
+    int id, int tiles_m, int tiles_n, int k_per_split, const Packing packing, const RowScale scale) {
     constexpr int THREADS = WM * WN * XRT_WAVE;
     constexpr int WAVE_M = BM / WM, WAVE_N = BN / WN;        // part of the tile owned by one wavefront
     constexpr int TM = WAVE_M / 32, TN = WAVE_N / 32;        // 32x32 accumulator tiles of a wavefront
@@ -78,7 +77,7 @@ __device__ __forceinline__ void gemm_tile(
     if (place.m < 0) return;
     const long m0 = (long)place.m * BM;
     constexpr int BN_OUT = MODE == MODE_GATED ? BN / 2 : BN;          // output columns of a tile
-    const long n0 = n_first + (long)place.n * BN_OUT;      // this launch covers output columns from n_first on
+    const long n0 = (long)place.n * BN_OUT;
 
     const int tid = threadIdx.x, lane = tid % XRT_WAVE, wave = tid / XRT_WAVE;
     const int wave_m = wave / WN, wave_n = wave % WN;
@@ -150,11 +149,10 @@ __device__ __forceinline__ void gemm_tile(
         const int sub = lane / CHUNKS;                             // row within the rows of one instruction
         auto chunk_of = [&](int row) { return ((lane % CHUNKS) ^ swizzle_of(row)) * 8; };   // what belongs in this lane's place
         unsigned off_a[LOADS_A], off_b[LOADS_B];                   // bytes
-        const long row_a = lda > 0 ? lda : K, row_w = ldw > 0 ? ldw : K;
 #pragma unroll
         for (int i = 0; i < LOADS_A; ++i) {
             const int r = min(i * WAVES + wave, BLOCKS_A - 1) * ROWS + sub;
-            off_a[i] = (unsigned)(min(m0 + r, (long)M - 1) * row_a + chunk_of(r)) * 2u;
+            off_a[i] = (unsigned)(min(m0 + r, (long)M - 1) * K + chunk_of(r)) * 2u;
         }
         // A packed w is copied as it lies: an instruction takes one whole tile of the packing (16 packed rows x 32
         // columns, a contiguous kilobyte, lane by lane), and the stage holds the tile's groups of 16 packed rows
@@ -170,10 +168,10 @@ __device__ __forceinline__ void gemm_tile(
             const int block = min(i * WAVES + wave, BLOCKS_B - 1);
             if (packed_b) {
                 const long group = min(first_packed / 16 + block / 2, last_group);       // groups beyond the matrix: the last one again
-                off_b[i] = (unsigned)(((group * (row_w / 32) + block % 2) * 512 + lane * 8) * 2);
+                off_b[i] = (unsigned)(((group * (K / 32) + block % 2) * 512 + lane * 8) * 2);
             } else {
                 const int r = block * ROWS + sub;
-                off_b[i] = (unsigned)(w_row(r) * row_w + chunk_of(r)) * 2u;
+                off_b[i] = (unsigned)(w_row(r) * K + chunk_of(r)) * 2u;
             }
         }
         // a step of k0 columns along k moves a row contiguous along k by k0 elements, a packed one by k0 / 32 tiles
@@ -844,8 +842,8 @@ __global__ void __launch_bounds__(8 * XRT_WAVE) gemm_large_kernel(
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES>
 __global__ void __launch_bounds__(WM * WN * XRT_WAVE) gemm_mfma_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
-    int tiles_m, int tiles_n, int n_first, int k_per_split, const Packing packing, const RowScale scale) {
-    gemm_tile<BM, BN, WM, WN, MODE, DK, STAGES, TO, PAST_CACHES>(a, w, out, M, N, K, blockIdx.x, tiles_m, tiles_n, n_first, k_per_split, packing, scale);
+    int tiles_m, int tiles_n, int k_per_split, const Packing packing, const RowScale scale) {
+    gemm_tile<BM, BN, WM, WN, MODE, DK, STAGES, TO, PAST_CACHES>(a, w, out, M, N, K, blockIdx.x, tiles_m, tiles_n, k_per_split, packing, scale);
 }
 
 // Two tile shapes in one launch: the first `large_blocks` workgroups take 256 x 256 tiles of the
@@ -933,13 +931,12 @@ bool reads_past_caches(int N, int K, int splits) {
     return BM <= 64 && splits == 1 && (MODE == MODE_GATED ? 3L * N : (long)N) * K * (long)sizeof(bf16) > LAST_CACHE;
 }
 
-// Launches the tiles of output columns [n_first, n_first + n_count).
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES = false>
-int launch_kernel(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int n_first, int n_count, const Packing& packing,
+int launch_kernel(const bf16* a, const bf16* w, TO* out, int M, int N, int K, const Packing& packing,
                   hipStream_t s, int splits = 1, int k_per_split = 0, const RowScale scale = RowScale{}) {
     if constexpr (BM <= 64 && !PAST_CACHES)
         if (reads_past_caches<BM, MODE>(N, K, splits))
-            return launch_kernel<BM, BN, WM, WN, MODE, DK, STAGES, TO, true>(a, w, out, M, N, K, n_first, n_count, packing, s, splits, k_per_split, scale);
+            return launch_kernel<BM, BN, WM, WN, MODE, DK, STAGES, TO, true>(a, w, out, M, N, K, packing, s, splits, k_per_split, scale);
     constexpr int BN_OUT = MODE == MODE_GATED ? BN / 2 : BN;
     constexpr int THREADS = WM * WN * XRT_WAVE;
     constexpr size_t staging = DK != 0 ? (size_t)STAGES * (BM + BN) * DK * sizeof(bf16) : (size_t)2 * (BM + BN) * PITCH * sizeof(bf16);
@@ -952,12 +949,12 @@ int launch_kernel(const bf16* a, const bf16* w, TO* out, int M, int N, int K, in
         XRT_REQUIRE(e == hipSuccess, "linear (mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
         configured = true;
     }
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (n_count + BN_OUT - 1) / BN_OUT;
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;
     const int total = tiles_m * tiles_n;
     const unsigned grid = (unsigned)(((total + 7) / 8) * 8);           // a whole number of rounds over the XCDs
     XRT_REQUIRE(splits == 1 || DK != 0, "linear (mfma): only whole tiles along k can be split");
     XRT_REQUIRE(scale.squares == nullptr || (BM <= 64 && splits == 1), "linear (mfma): rows are scaled by tiles of up to 64 rows that see all of k");
-    kernel<<<dim3(grid, splits), THREADS, lds, s>>>(a, w, out, M, N, K, tiles_m, tiles_n, n_first,
+    kernel<<<dim3(grid, splits), THREADS, lds, s>>>(a, w, out, M, N, K, tiles_m, tiles_n,
                                                     splits == 1 ? K : k_per_split, packing, scale);
     XRT_LAUNCH_CHECK("linear (mfma)");
     return 0;
@@ -1007,14 +1004,14 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
     if (K % 64 != 0) {                 // a ragged last tile along k: the path through registers
         const long large = ((tiles(256, 256) + XRT_COMPUTE_UNITS - 1) / XRT_COMPUTE_UNITS) * 100;
         const long small = ((tiles(128, 128) + 2 * XRT_COMPUTE_UNITS - 1) / (2 * XRT_COMPUTE_UNITS)) * 59;
-        if (large <= small) return launch_kernel<256, 256, 2, 4, MODE, 0, 0, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
-        return launch_kernel<128, 128, 2, 2, MODE, 0, 0, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
+        if (large <= small) return launch_kernel<256, 256, 2, 4, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+        return launch_kernel<128, 128, 2, 2, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
     }
     // Up to 128 rows of a, gated: one round of tiles of 128 x 128 (or nearly), bound by reading w: three stages keep more of
     // it on its way than the two that the tiles below have (gate/up of 14336 pairs and 128 rows: 76 us split in three
     // with a second kernel, 49 us so).
     if constexpr (MODE == MODE_GATED)
-        if (M <= 128) return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
+        if (M <= 128) return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
     // 256 x 256 tiles cost the least energy a product, and tiles of half the height somewhat more (2048 rows of x, 4096 rows of
     // w, k = 4096: 128 tiles of the one 85 us, 256 of the other 58; 6144 rows of w: 82 and 102); tiles of 128 x 128, two to a compute
     // unit, where neither fills the chip, or where k is so short that one's epilogue wants another's products beside it (200 rows of x,
@@ -1057,9 +1054,9 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
     if (large <= half && large <= small && large <= narrow) return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
     if (half <= small && half <= narrow) return launch_large<128, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
     if constexpr (MODE != MODE_GATED)
-        if (narrow <= small) return launch_kernel<256, 192, 4, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
+        if (narrow <= small) return launch_kernel<256, 192, 4, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
     // (four stages of 32 keep a load in flight for longer but meet at twice as many barriers, and measured slower)
-    return launch_kernel<128, 128, 2, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, plain);
+    return launch_kernel<128, 128, 2, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
 }
 
 template <typename TO>
@@ -1391,27 +1388,27 @@ int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int
                 "linear (mfma): only a bfloat16 product split along k does what follows a q/k/v projection");
     if (M <= SPLIT_BM && plan.splits == 1) {                   // tiles enough: each applies the epilogue itself
         XRT_REQUIRE(!emits, "linear (mfma): only a product split along k writes what the norm after it needs");
-        if (mode == MODE_STORE) return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, scale);
-        if (mode == MODE_GATED) return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 2, MODE_GATED, 64, 3, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, scale);
+        if (mode == MODE_STORE) return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
+        if (mode == MODE_GATED) return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 2, MODE_GATED, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
         if constexpr (sizeof(TO) == 4)
-            return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_ACCUMULATE, 64, 3, TO>(a, w, out, M, N, K, 0, N, packing, s, 1, 0, scale);
+            return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_ACCUMULATE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
         XRT_REQUIRE(false, "linear (mfma): accumulation needs a float32 output");
     }
     XRT_REQUIRE(workspace != nullptr, "linear (mfma): a product split along k needs its workspace");
     // the product of all rows of w, ungated, into the workspace: [splits][M][rows_w]
     const int status = M <= SPLIT_BM
         ? launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, float>(
-              a, w, workspace, M, (int)plan.rows_w, K, 0, (int)plan.rows_w, packing, s, plan.splits, plan.k_per_split)
+              a, w, workspace, M, (int)plan.rows_w, K, packing, s, plan.splits, plan.k_per_split)
         : plan.tile == 256
         ? launch_large<256, MODE_STORE, float>(a, w, workspace, M, (int)plan.rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split)
         : plan.columns == 64
         ? launch_kernel<128, 64, 2, 2, MODE_STORE, 64, 3, float>(
-              a, w, workspace, M, (int)plan.rows_w, K, 0, (int)plan.rows_w, packing, s, plan.splits, plan.k_per_split)
+              a, w, workspace, M, (int)plan.rows_w, K, packing, s, plan.splits, plan.k_per_split)
         : M <= 256          // (one workgroup to a compute unit anyway: a third stage keeps more of w on its way; with more, two share a unit)
         ? launch_kernel<128, 128, 2, 2, MODE_STORE, 64, 3, float>(
-              a, w, workspace, M, (int)plan.rows_w, K, 0, (int)plan.rows_w, packing, s, plan.splits, plan.k_per_split)
+              a, w, workspace, M, (int)plan.rows_w, K, packing, s, plan.splits, plan.k_per_split)
         : launch_kernel<128, 128, 2, 2, MODE_STORE, 64, 2, float>(
-              a, w, workspace, M, (int)plan.rows_w, K, 0, (int)plan.rows_w, packing, s, plan.splits, plan.k_per_split);
+              a, w, workspace, M, (int)plan.rows_w, K, packing, s, plan.splits, plan.k_per_split);
     if (status != 0) return status;
     const unsigned blocks = (unsigned)(((long)M * N + 255) / 256);
     const xrt_linear_norm none = {};
