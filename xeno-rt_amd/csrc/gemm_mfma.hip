@@ -981,18 +981,19 @@ int launch_large(const bf16* a, const bf16* w, TO* out, int M, int N, int K, con
     return 0;
 }
 
-// What a tile shape costs: a full round over `places` takes `products` microseconds for each 4096 of k and ends[mode] for its
+// What a tile shape costs: a full round over `places` takes `products` microseconds for each 4096 of k and ends[kind] for its
 // first loads and its epilogue. A last round that is partly filled takes `least` percent of a full one and its share of the
-// rest: the chip is bound by its power, and with fewer compute units at work their clock rises. The numbers are fitted to 608
-// products (layers of seven sizes and sizes drawn at random, k from 512 to 25600, 129 to 8192 rows of x), every tile shape
-// of each of them timed: what the estimate chooses is 0.3 % off the best of them on average.
-struct TileTime { int bm, bn, places, products, ends[3], least; };
-constexpr TileTime LARGE_TILE = {256, 256, XRT_COMPUTE_UNITS, 88, {10, 14, 16}, 56}, HALF_TILE = {128, 256, XRT_COMPUTE_UNITS, 57, {5, 10, 9}, 56},
-                   NARROW_TILE = {256, 192, XRT_COMPUTE_UNITS, 80, {8, 8, 0}, 56}, SMALL_TILE = {128, 128, 2 * XRT_COMPUTE_UNITS, 64, {6, 8, 10}, 45};
-long rounds_cost(long tiles, const TileTime& tile, int K, int mode) {        // in nanoseconds or so
-    const long round = tile.products * 1000L * K / 4096 + tile.ends[mode] * 1000L;
+// rest: the chip is bound by its power, and with fewer compute units at work their clock rises. The numbers are fitted to 1985
+// products (layers of seven sizes and sizes drawn at random, k from 64 to 25600, 129 to 8192 rows of x), every tile shape of
+// each of them timed: what the estimate chooses is 0.6 % off the best of them on average, which is within the runs' differences.
+enum { ENDS_BF16 = 0, ENDS_F32 = 1, ENDS_ADDING = 2, ENDS_GATED = 3 };
+struct TileTime { int bm, bn, places, products, ends[4], least; };
+constexpr TileTime LARGE_TILE = {256, 256, XRT_COMPUTE_UNITS, 88, {10, 16, 15, 16}, 55}, HALF_TILE = {128, 256, XRT_COMPUTE_UNITS, 54, {6, 8, 9, 9}, 62},
+                   NARROW_TILE = {256, 192, XRT_COMPUTE_UNITS, 81, {0, 11, 8, 0}, 55}, SMALL_TILE = {128, 128, 2 * XRT_COMPUTE_UNITS, 67, {7, 7, 5, 10}, 41};
+long rounds_cost(long tiles, const TileTime& tile, int K, int kind) {        // in nanoseconds or so
+    const long round = tile.products * 1000L * K / 4096 + tile.ends[kind] * 1000L;
     const long whole = tiles / tile.places, rest = tiles % tile.places;
-    return whole * round + (rest == 0 ? 0 : (tile.least + (100 - tile.least) * rest / tile.places) * round / 100);
+    return whole * round + (rest == 0 ? 0 : (tile.least * (long)tile.places + (100 - tile.least) * rest) * round / (100L * tile.places));
 }
 
 template <int MODE, typename TO>
@@ -1016,14 +1017,17 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
     // w, k = 4096: 128 tiles of the one 85 us, 256 of the other 58; 6144 rows of w: 82 and 102); tiles of 128 x 128, two to a compute
     // unit, where neither fills the chip, or where k is so short that one's epilogue wants another's products beside it (200 rows of x,
     // 9632 rows of w, k = 1728, adding: 25 against 31 us). The tiles of 256 x 192, which are gemm_tile's, where they make one round that
-    // the large ones leave half empty and those of half the height need two for (3072 rows of w, k = 3072, 2816 rows of x: 63
-    // against 73 and 90 us; 4096 rows, k = 14336, 2300 rows of x: 250, 259 and 327). They read their operands more often, which a w
+    // the large ones leave half empty and those of half the height need two for, and results are float32, which they write faster
+    // (adding, 3072 rows of w, k = 3072, 2816 rows of x: 63 against 73 and 90 us; 4096 rows, k = 14336, 2300 rows of x: 250, 259 and
+    // 327; bfloat16 results, 3072 rows, k = 2048, 2048 rows of x: 53 against 46 us). They read their operands more often, which a w
     // beyond the caches does not stand (5120 rows of w, k = 25600, 2048 rows of x: 572 against 447 us; 13536 rows, k = 10624,
     // 724 rows of x: 240 against 188).
     constexpr long NARROW_W = 150L * 1000 * 1000;              // bytes
-    auto cost = [&](const TileTime& tile) { return rounds_cost(tiles(tile.bm, tile.bn), tile, K, MODE); };
+    constexpr int KIND = MODE == MODE_GATED ? ENDS_GATED : MODE == MODE_ACCUMULATE ? ENDS_ADDING : sizeof(TO) == 4 ? ENDS_F32 : ENDS_BF16;
+    auto cost = [&](const TileTime& tile) { return rounds_cost(tiles(tile.bm, tile.bn), tile, K, KIND); };
     const long large = cost(LARGE_TILE), half = cost(HALF_TILE), small = cost(SMALL_TILE);
-    const long narrow = MODE != MODE_GATED && (long)N * K * (long)sizeof(bf16) <= NARROW_W ? cost(NARROW_TILE) : LONG_MAX;
+    constexpr bool NARROW = MODE != MODE_GATED && sizeof(TO) == 4;
+    const long narrow = NARROW && (long)N * K * (long)sizeof(bf16) <= NARROW_W ? cost(NARROW_TILE) : LONG_MAX;
     // Large tiles for as many columns as make whole rounds, and tiles of half the height for the rest, if those then fit
     // one round: the last round is full of half-sized work instead of half empty (28672 rows of w, k = 4096, 2048 rows of x:
     // 366 against 372 us).
@@ -1032,7 +1036,7 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
     const long rest_tiles = (long)((M + 127) / 128) * (tiles_n - whole_columns);
     long mixed = LONG_MAX;
     if (whole_columns > 0 && whole_columns < tiles_n && rest_tiles <= XRT_COMPUTE_UNITS)
-        mixed = rounds_cost((long)tiles_m * whole_columns, LARGE_TILE, K, MODE) + rounds_cost(rest_tiles, HALF_TILE, K, MODE);
+        mixed = rounds_cost((long)tiles_m * whole_columns, LARGE_TILE, K, KIND) + rounds_cost(rest_tiles, HALF_TILE, K, KIND);
     if (mixed < large && mixed <= half && mixed <= small && mixed <= narrow) {
         const int split = whole_columns * (256 / DIV);
         const int small_tiles_m = (M + 127) / 128, small_tiles_n = tiles_n - whole_columns;
@@ -1053,7 +1057,7 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
     }
     if (large <= half && large <= small && large <= narrow) return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
     if (half <= small && half <= narrow) return launch_large<128, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
-    if constexpr (MODE != MODE_GATED)
+    if constexpr (NARROW)
         if (narrow <= small) return launch_kernel<256, 192, 4, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
     // (four stages of 32 keep a load in flight for longer but meet at twice as many barriers, and measured slower)
     return launch_kernel<128, 128, 2, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
