@@ -698,6 +698,49 @@ def test_attention(ops, dtype, nh, nkv, hd):
         assert rel(out[t:t + 1].cpu(), want) < (2e-5 if dtype == "float32" else 1e-2), (t, slot, pos)
 
 
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 64), (5, 5, 64), (6, 2, 128), (16, 2, 64), (32, 1, 128)])
+def test_float32_attention_of_many_tokens_gives_the_bits_of_few(ops, nh, nkv, hd):
+    """A step of many tokens takes the matrix cores in tiles of 16 tokens, four of them a workgroup (groups of 4, 1, 3, 8 and 32 heads
+    here); the same tokens as a step that nothing describes take the general kernel. Runs of a sequence that begin and end inside tiles, padding
+    behind them, queries at the edges of blocks and of chunks of 512 keys; infinite and NaN keys and values, which only those who see them may feel."""
+    lengths = [700, 130, 1, 64, 1100]          # (one, two and three chunks of 512 keys)
+    kv, keys, values = filled_cache(nkv, hd, torch.float32, lengths, seed=hd + nh)
+    of_values, of_keys = kv.v.view(-1, nkv, 64 * hd), kv.k.view(-1, nkv, 64 * hd)
+    for slot, at, what in ((0, 650, float("nan")), (0, 37, float("inf")), (1, 100, float("-inf")), (4, 1090, float("nan"))):
+        block = int(kv.block_table[slot, at // 64])
+        of_values[block, 0, int(cache_order.value_places(hd)[3, at % 64])] = what
+        if slot == 1:
+            of_keys[block, nkv - 1, int(cache_order.key_places(hd)[at % 64, 5])] = what
+    runs = [(0, 590, 110), (3, 0, 64), (1, 0, 130), (4, 505, 13), (4, 1000, 100), (2, 0, 1), (0, 60, 8), (4, 1020, 9)]
+    where = [(slot, start + i) for slot, start, count in runs for i in range(count)] + [(-1, 0)] * 5      # (the rule asks for eight to 64 tokens a sequence, the kernel serves one)
+    while len(where) * nh <= 2048:
+        where = where + where
+    qkv = rand(len(where), (nh + 2 * nkv) * hd, seed=nh)
+
+    def attend(rows, described):
+        out = torch.full((len(rows), nh * hd), 7.0, device=DEV)
+        batch = SimpleNamespace(slots=i32([where[r][0] for r in rows]), positions=i32([where[r][1] for r in rows]))
+        if described:
+            offsets = [0]
+            for _, _, count in runs:
+                offsets.append(offsets[-1] + count)
+            batch.sequence_offsets, batch.sequence_slots, batch.sequence_starts = i32(offsets), i32([r[0] for r in runs]), i32([r[1] for r in runs])
+            batch.n_sequences, batch.max_count, batch.max_context, batch.host_counts = len(runs), 130, 1100, [64] * len(runs)
+        before = ops.lib.xrt_attention_float_prompts
+        taken = []
+        ops.lib.xrt_attention_float_prompts = lambda *arguments: (taken.append(1), before(*arguments))[1]
+        try:
+            ops.attention(qkv[rows], nh, nkv, hd, kv, batch, out, scale=1.0 / math.sqrt(hd))
+        finally:
+            ops.lib.xrt_attention_float_prompts = before
+        assert bool(taken) == described
+        return out
+
+    many, few = attend(list(range(len(where))), True), attend(list(range(len(where))), False)
+    assert bool(torch.isnan(few).any()) and bool(torch.isinf(few).any())
+    assert torch.equal(torch.nan_to_num(many, nan=7.0), torch.nan_to_num(few, nan=7.0))
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("nh,nkv,hd,window", [(4, 2, 48, None), (8, 2, 128, None), (2, 1, 100, None), (4, 4, 32, 700)])
 def test_general_attention_gives_the_same_bits_with_few_tokens_and_with_many(ops, dtype, nh, nkv, hd, window):

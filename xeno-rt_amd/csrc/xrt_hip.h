@@ -309,6 +309,15 @@ int xrt_attention_stretches(const void* q, long q_stride, int dtype, int tokens,
                             const int* seq_offsets, const int* seq_slots, const int* seq_starts, int n_seqs, void* out,
                             float scale, int chunk, const float* distance_bias, int bias_span, const float* sink_scores, void* stream);
 
+// Plain causal attention of a float32 step that brings every sequence `fewest` tokens at least, on the matrix cores, to the bits of
+// xrt_attention (rows of qkv as there). `accepts` says which steps: heads of 64 or 128 dims, more (token, head) pairs than a
+// decode step has, aligned operands.
+int xrt_attention_float_prompts_accepts(const void* qkv, int tokens, int n_heads, int n_kv_heads, int head_dim, const void* k_cache,
+                                        const void* v_cache, const void* out, int fewest);
+int xrt_attention_float_prompts(const void* qkv, int tokens, int n_heads, int n_kv_heads, int head_dim, const void* k_cache,
+                                const void* v_cache, const int* block_table, int table_stride, int n_blocks, const int* positions,
+                                const int* slots, void* out, float scale, int fewest, void* stream);
+
 // Attention without a softmax: the weight of a visible key is sigmoid(score_h + head_bias[h]), not normalised over the keys;
 // before that the heads' scaled scores of a (query, key) pair are mixed, score_h <- sum_g head_mix[h][g] score_g
 // (head_mix float32 [n_heads][n_heads], or null); a head's summed values are multiplied by sigmoid(gate[token][h]) (float32

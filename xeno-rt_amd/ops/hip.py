@@ -209,6 +209,7 @@ class HipOps:
                      "xrt_layernorm", "xrt_layernorm_shift", "xrt_add_layernormed", "xrt_short_conv_with", "xrt_selective_scan",
                      "xrt_bigram_add", "xrt_gated_rows", "xrt_add_weighted", "xrt_glu_clamped", "xrt_softcap", "xrt_cast",
                      "xrt_route_experts", "xrt_scale_blocks", "xrt_attention_stretches", "xrt_attention_stretches_accepts",
+                     "xrt_attention_float_prompts", "xrt_attention_float_prompts_accepts",
                      "xrt_experts_sort", "xrt_gather_rows", "xrt_linear_groups", "xrt_linear_groups_accepts", "xrt_experts_combine",
                      "xrt_linear_groups_tile_rows", "xrt_linear_groups_parts", "xrt_streams_open", "xrt_streams_read", "xrt_streams_write",
                      "xrt_latent_complete", "xrt_latent_queries", "xrt_linear_heads", "xrt_causal_softmax", "xrt_transpose", "xrt_attention_latent",
@@ -574,6 +575,15 @@ class HipOps:
             self._require(starts, "sequence starts", torch.int32, (n_seqs,), qkv)
             if max_context > stride * BLOCK_TOKENS:
                 raise KernelError(f"attention: a sequence of {max_context} tokens exceeds the block table")
+            counts = getattr(batch, "host_counts", None)
+            if qkv.dtype == torch.float32 and not window and distance_slopes is None and counts:
+                # float32 prompts: the matrix cores, to the bits of the general kernel
+                fewest, k_at, v_at, q_at, out_at = min(counts), _ptr(k_cache), _ptr(v_cache), _ptr(qkv), _ptr(out)
+                if self.lib.xrt_attention_float_prompts_accepts(q_at, tokens, n_heads, n_kv_heads, head_dim, k_at, v_at, out_at, fewest):
+                    self._check(self.lib.xrt_attention_float_prompts(
+                        q_at, tokens, n_heads, n_kv_heads, head_dim, k_at, v_at, _ptr(table), stride, n_blocks, _ptr(batch.positions), _ptr(batch.slots),
+                        out_at, ctypes.c_float(scale), fewest, self._stream(qkv)))
+                    return None
             if distance_slopes is None:                         # (the general kernel, which serves those, needs none)
                 workspace_floats = int(self.lib.xrt_attention_workspace(_code(qkv), tokens, n_heads, n_kv_heads, head_dim,
                                                                         int(window or 0), max_count, max_context))
