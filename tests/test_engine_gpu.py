@@ -276,6 +276,45 @@ def test_a_step_may_mix_sequences_that_start_with_sequences_that_go_on(name, dty
     engine.cache.check()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", ["llama", "qwen3"])
+def test_rows_that_nobody_wants_stop_behind_the_last_attention(name, dtype, models, engines, monkeypatch):
+    """Steps of 17 to some hundred tokens of which few rows are wanted, in any order, some twice, or none: the logits of the wanted rows, and what the
+    sequences' later tokens see of the others in the cache."""
+    from xeno_rt_amd.parts.attention import Attention
+    monkeypatch.setattr(Attention, "WANTED_FROM", 0)                       # (these models' layers are too small to gain by it)
+    engine = engines(name, dtype)
+    _, _, cases = models[name]
+    lengths = LENGTHS[name]
+    a, b, c = (cases[n] for n in (lengths[3], lengths[4], lengths[5]))     # (ids, plain logits)
+    want = {"float32": lambda ids, plain, rows: run_whole(engine, ids)[rows], "bfloat16": lambda ids, plain, rows: plain[rows]}[dtype]
+    slots = [engine.alloc_slot() for _ in range(3)]
+    cuts = [17, len(b[0]) - 21, len(c[0]) - 2]
+    steps = [[(slots[0], a[0][:17], [16, 0, 16, 3])],                        # 17 tokens, four of them (one twice)
+             [(slots[1], b[0][:cuts[1]], []), (slots[2], c[0][:cuts[2]], [])],                 # none at all
+             [(slots[0], a[0][17:], []), (slots[1], b[0][cuts[1]:], [20, 5]), (slots[2], c[0][cuts[2]:], [1])]]
+    rows = [[(a, [16, 0, 16, 3])], [], [(b, [cuts[1] + 20, cuts[1] + 5]), (c, [cuts[2] + 1])]]
+    taken = []
+    before = engine.ops.lib.xrt_take_rows
+    engine.ops.lib.xrt_take_rows = lambda *arguments: (taken.append(1), before(*arguments))[1]
+    try:
+        got = [engine.step(step) for step in steps]
+    finally:
+        engine.ops.lib.xrt_take_rows = before
+    assert len(taken) == 2 and got[1].shape == (0, engine.vocab_size)
+    for slot in slots:
+        engine.free_slot(slot)
+    for logits, wanted in zip(got, rows):
+        expected = [want(ids, plain, some) for (ids, plain), some in wanted]
+        if not expected:
+            continue
+        expected = torch.cat([part.cpu() for part in expected])
+        assert_logits(logits, expected, dtype, f"{name}, few rows wanted")
+        if dtype == "float32":
+            assert torch.equal(logits.cpu(), expected), f"{name}: float32 bits depend on how many rows are wanted"
+    engine.cache.check()
+
+
 @pytest.mark.parametrize("arch,sizes", [
     ("llama", dict(num_attention_heads=4, num_key_value_heads=1, head_dim=64, max_position_embeddings=1200)),
     # half of a head rotated, positions halved: the projection's epilogue does not rotate such heads, a kernel after it does

@@ -296,6 +296,37 @@ extern "C" int xrt_replace_rows(float* x, const float* base, void* copy, int cop
     return 0;
 }
 
+// The rows of a step whose results somebody wants, brought together: what the layers' last attention and everything behind it go on with.
+// One workgroup a row; a launch of a few kilobytes, bound by its start.
+__global__ void __launch_bounds__(256) take_rows_kernel(const char* __restrict__ a, long a_stride, int a_bytes, char* __restrict__ a_out, long a_out_stride,
+                                                        const char* __restrict__ b, int b_bytes, char* __restrict__ b_out, const int* __restrict__ positions,
+                                                        const int* __restrict__ slots, const int* __restrict__ rows, int count, int tokens,
+                                                        int* __restrict__ described) {
+    const int i = blockIdx.x, row = min(max(rows[i], 0), tokens - 1);
+    for (int at = threadIdx.x * 16; at < a_bytes; at += 256 * 16)
+        *reinterpret_cast<uint4*>(a_out + i * a_out_stride + at) = *reinterpret_cast<const uint4*>(a + row * a_stride + at);
+    for (int at = threadIdx.x * 16; at < b_bytes; at += 256 * 16)
+        *reinterpret_cast<uint4*>(b_out + (long)i * b_bytes + at) = *reinterpret_cast<const uint4*>(b + (long)row * b_bytes + at);
+    if (threadIdx.x == 0) {                                     // [positions | slots | 0 .. count]
+        described[i] = positions[row];
+        described[count + i] = slots[row];
+        described[2 * count + i] = i;
+        if (i == count - 1) described[3 * count] = count;
+    }
+}
+
+extern "C" int xrt_take_rows(const void* a, long a_stride, int a_bytes, void* a_out, long a_out_stride, const void* b, int b_bytes, void* b_out,
+                             const int* positions, const int* slots, const int* rows, int count, int tokens, int* described, void* stream) {
+    XRT_REQUIRE(a && a_out && b && b_out && positions && slots && rows && described && count > 0 && tokens > 0, "take_rows: bad operands");
+    XRT_REQUIRE(a_bytes >= 0 && b_bytes >= 0 && a_bytes % 16 == 0 && b_bytes % 16 == 0 && a_stride % 16 == 0 && a_out_stride % 16 == 0 && a_stride >= a_bytes &&
+                a_out_stride >= a_bytes && (uintptr_t)a % 16 == 0 && (uintptr_t)a_out % 16 == 0 && (uintptr_t)b % 16 == 0 && (uintptr_t)b_out % 16 == 0,
+                "take_rows: rows of whole 16 bytes, aligned to them");
+    take_rows_kernel<<<count, 256, 0, (hipStream_t)stream>>>((const char*)a, a_stride, a_bytes, (char*)a_out, a_out_stride, (const char*)b, b_bytes,
+                                                             (char*)b_out, positions, slots, rows, count, tokens, described);
+    XRT_LAUNCH_CHECK("take_rows");
+    return 0;
+}
+
 extern "C" int xrt_embed(const void* table, int table_dtype, const xrt_packing* packing, const int* ids, float* out, int tokens,
                          int hidden, int vocab, float scale, void* stream) {
     XRT_REQUIRE(tokens >= 0 && hidden > 0 && vocab > 0, "embed: bad sizes tokens=%d hidden=%d vocab=%d", tokens, hidden, vocab);

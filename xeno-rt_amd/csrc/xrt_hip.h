@@ -69,6 +69,11 @@ int xrt_rmsnorm_two(const float* x, const void* weight_a, const void* weight_b, 
 // copy[i] = x[i] in copy_dtype, then x[i] = base[i]
 int xrt_replace_rows(float* x, const float* base, void* copy, int copy_dtype, long count, void* stream);
 
+// Rows `rows` (indices below `tokens`) of a step: a_out[i] = the first a_bytes of row rows[i] of a (strides in bytes), b_out[i] = row rows[i] of
+// b (b_bytes each, dense), described = [positions of those rows | their slots | 0 .. count]: a step in which every row is a sequence with one token.
+int xrt_take_rows(const void* a, long a_stride, int a_bytes, void* a_out, long a_out_stride, const void* b, int b_bytes, void* b_out,
+                  const int* positions, const int* slots, const int* rows, int count, int tokens, int* described, void* stream);
+
 // xrt_rmsnorm of every row, then xrt_short_conv of the normed rows (plain, or plus the input), for a step in which row r is the
 // one new token of the sequence in slot token_slots[r] (negative: padding, the row becomes zeros): one kernel, the same bits.
 int xrt_rmsnorm_conv_step(const float* x, const void* weight, int weight_dtype, float eps, void* out, int out_dtype, int n_rows,

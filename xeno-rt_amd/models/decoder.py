@@ -130,6 +130,7 @@ class DecoderModel:
             x = spec.embedding.forward(batch.token_ids, batch.positions)
         if spec.streams is not None:                             # the blocks then work on the copies [tokens, copies, hidden]
             x = spec.streams.open(x)
+        wanted = batch.logit_rows
         opened = spec.entry.open(x) if spec.entry is not None else None      # (before any layer: the stream still is what the embedding left)
         for index, call in enumerate(spec.schedule):
             block = spec.layers[call.layer]
@@ -138,6 +139,11 @@ class DecoderModel:
             if not getattr(block, "passes_norms", False):
                 block.forward(x, batch, cache.layer_cache(index))
                 h = None
+                continue
+            if index + 1 == len(spec.schedule) and spec.streams is None and hasattr(block, "goes_on_with") and block.goes_on_with(batch):
+                # behind the last attention only the wanted tokens count: the others' keys and values are all that is left of them
+                x = block.forward_wanted(x, batch, cache.layer_cache(index), h=h)
+                wanted = None
                 continue
             last = index + 1 == len(spec.schedule) or spec.schedule[index + 1].enters      # (what follows does not read the stream as this block leaves it)
             after = None if last else spec.layers[spec.schedule[index + 1].layer]
@@ -148,5 +154,5 @@ class DecoderModel:
         if spec.streams is not None:
             y = spec.streams.close(x, spec.final_norm, rows=batch.logit_rows)
         else:
-            y = spec.final_norm.forward(x, rows=batch.logit_rows)
+            y = spec.final_norm.forward(x, rows=wanted)
         return spec.head.forward(y)

@@ -213,7 +213,7 @@ class HipOps:
                      "xrt_experts_sort", "xrt_gather_rows", "xrt_linear_groups", "xrt_linear_groups_accepts", "xrt_experts_combine",
                      "xrt_linear_groups_tile_rows", "xrt_linear_groups_parts", "xrt_streams_open", "xrt_streams_read", "xrt_streams_write",
                      "xrt_latent_complete", "xrt_latent_queries", "xrt_linear_heads", "xrt_causal_softmax", "xrt_transpose", "xrt_attention_latent",
-                     "xrt_attention_latent_accepts", "xrt_attention_latent_prompts", "xrt_latent_prepare", "xrt_glu_experts", "xrt_embed_normed", "xrt_rmsnorm_two", "xrt_replace_rows"):
+                     "xrt_attention_latent_accepts", "xrt_attention_latent_prompts", "xrt_latent_prepare", "xrt_glu_experts", "xrt_embed_normed", "xrt_rmsnorm_two", "xrt_replace_rows", "xrt_take_rows"):
             getattr(self.lib, name).restype = ctypes.c_int
         from ..cache.allocator import BLOCK_TOKENS
         if int(self.lib.xrt_block_tokens()) != BLOCK_TOKENS:
@@ -344,6 +344,25 @@ class HipOps:
         self._require(base, "replace_rows base", torch.float32, x.shape, x)
         self._require(copy, "replace_rows copy", None, x.shape, x)
         self._check(self.lib.xrt_replace_rows(_ptr(x), _ptr(base), _ptr(copy), _code(copy), ctypes.c_long(x.numel()), self._stream(x)))
+
+    def take_rows(self, qkv, q_width, x, positions, slots, rows):
+        """Rows `rows` (int32, indices of the step's tokens) of a step: (the queries qkv[rows, :q_width], in rows as wide as qkv's whose rest holds
+        nothing, x[rows], positions[rows], slots[rows], 0 .. count as int32)."""
+        tokens, width = qkv.shape
+        count, hidden = rows.shape[0], x.shape[1]
+        self._require(qkv, "take_rows qkv")
+        self._require(x, "take_rows x", torch.float32, (tokens, hidden), qkv)
+        self._require(positions, "take_rows positions", torch.int32, (tokens,), qkv)
+        self._require(slots, "take_rows slots", torch.int32, (tokens,), qkv)
+        self._require(rows, "take_rows rows", torch.int32, (count,), qkv)
+        if not 0 < q_width <= width:
+            raise KernelError(f"take_rows: {q_width} columns of {width}")
+        size = qkv.element_size()
+        q, taken = self._empty((count, width), qkv.dtype, qkv.device), self._empty((count, hidden), torch.float32, qkv.device)
+        described = self._empty((3 * count + 1,), torch.int32, qkv.device)
+        self._check(self.lib.xrt_take_rows(_ptr(qkv), ctypes.c_long(width * size), q_width * size, _ptr(q), ctypes.c_long(width * size), _ptr(x), hidden * 4,
+                                           _ptr(taken), _ptr(positions), _ptr(slots), _ptr(rows), count, tokens, _ptr(described), self._stream(qkv)))
+        return q, taken, described[:count], described[count:2 * count], described[2 * count:]
 
     def _linear(self, a, w, out, coded_mode, n, then_norm=None):
         mode = coded_mode & 255                 # what rides above is a gated product's activation

@@ -42,6 +42,7 @@ keys, at or before it, which the cache then never lets go of); and a layer witho
 from __future__ import annotations
 
 import math
+from dataclasses import replace
 from typing import Dict, Optional
 
 import torch
@@ -317,6 +318,51 @@ class Attention(Mixer):
         rt.ops.rows_add(self.bias_o.reshape(1, -1), row, out)
         return None
 
+    # Tokens whose results nobody wants need go no further than the cache behind the model's last attention: for the others alone the step
+    # goes on from there with their queries, which costs a kernel that brings them together. Up to 16 rows a product is bound by reading its weights, and where
+    # the output projection has fewer than WANTED_FROM elements a layer is all launches: tiny models 305 -> 330 us a prompt by it, 1024 x 2048
+    # the same up to 200 tokens and 3220 -> 3168 us at 400, 4096 x 4096 (4 layers) 633 -> 618 at 17 tokens, 822 -> 780 at 100, 1304 -> 1171 at 400; a prompt
+    # of 2048 tokens through 6 layers 4847 -> 4260, of 8192 through 4 13374 -> 10535. (One layer of a model's: of 32 layers 2 to 3 %.)
+    WANTED_FROM = 1 << 20
+
+    def goes_on_with(self, batch) -> bool:
+        """Whether `forward_wanted` serves this step (rows must be whole pieces of 16 bytes)."""
+        if self.general or not hasattr(self.runtime.ops, "take_rows") or (self.position is not None and self.position.rotation() is None):
+            return False
+        size = 4 if self.runtime.dtype == torch.float32 else 2
+        return batch.n_logit_rows == 0 or (batch.n_tokens > 16 and 4 * batch.n_logit_rows <= batch.n_tokens and self.q_width * self.hidden >= self.WANTED_FROM
+                                           and self.q_width * size % 16 == 0 and self.kv_width * size % 8 == 0 and self.hidden % 4 == 0)
+
+    def forward_wanted(self, h, batch, cache, residual: torch.Tensor, then=None):
+        """`forward` of which only the rows `batch.logit_rows` are wanted: every token's key and value reach the cache, the attention and the output
+        projection run for the wanted rows alone. Returns (those rows of the residual stream, updated, what `forward` returns for them),
+        or (None, None) where no row is wanted."""
+        rt = self.runtime
+        qkv = self._project(h, batch, cache)
+        if batch.n_logit_rows == 0:
+            return None, None
+        q, residual, positions, slots, offsets = rt.ops.take_rows(qkv, self.q_width, residual, batch.positions, batch.slots, batch.logit_rows)
+        count = batch.n_logit_rows
+        alone = replace(batch, n_tokens=count, n_sequences=count, positions=positions, slots=slots, sequence_slots=slots, sequence_offsets=offsets,
+                        sequence_starts=positions, host_slots=None, host_counts=[1] * count, host_starts=None, is_decode=True, max_count=1)
+        out = rt.empty((count, self.q_width))
+        rt.ops.attention(q, self.n_heads, self.n_kv_heads, self.head_dim, cache.kv, alone, out, scale=self.scale, window=self.window)
+        return residual, rt.ops.linear(out, self.w_o, residual, accumulate=True, then_norm=None if then is None else then.row_scale())
+
+    def _project(self, h, batch, cache):
+        """q, k and v of the step's tokens, rotated, keys and values in the cache: the projection, then in one pass (in the same kernel, where a
+        step is short) head norms, rotation, cache write."""
+        qkv = self.runtime.empty((h.shape[0], self.q_width + 2 * self.kv_width))
+        rotation = None if self.position is None else self.position.rotation()
+        self.runtime.ops.linear_qkv(h, self.w_qkv, qkv, self.n_heads, self.n_kv_heads, self.head_dim, batch.positions, batch.slots,
+                                    q_norm=self.q_norm, k_norm=self.k_norm, norm_eps=self.qk_norm_eps,
+                                    rope_theta=None if rotation is None else rotation.theta,
+                                    rope_dim=0 if rotation is None else rotation.rope_dim,
+                                    rope_scale=1.0 if rotation is None else rotation.scale,
+                                    kv=cache.kv if cache.writable else None,
+                                    longest_run=int(getattr(batch, "max_count", 0) or 0))      # picks how the values are written; 0: unknown
+        return qkv
+
     def forward(self, h, batch, cache, residual: torch.Tensor, then=None):
         if self.completed and self.bias_o is None:
             self.runtime.ops.linear(self._attend_completed(h, batch, cache), self.w_o, residual, accumulate=True)
@@ -333,11 +379,8 @@ class Attention(Mixer):
         ops = rt.ops
         tokens = h.shape[0]
         kv = cache.kv
-        qkv = rt.empty((tokens, self.q_width + 2 * self.kv_width))
-
         dims = (self.n_heads, self.n_kv_heads, self.head_dim)
         write_to = kv if cache.writable else None
-        longest_run = int(getattr(batch, "max_count", 0) or 0)      # picks how the values are written; 0: unknown
         rotation = None if self.position is None else self.position.rotation()
         slopes = None if self.position is None else self.position.score_slopes()
         out = rt.empty((tokens, self.q_width))
@@ -345,30 +388,26 @@ class Attention(Mixer):
         # itself (norms, rotation, cache write) where it can; without head norms the projection's own kernel does that.
         finishes = getattr(ops, "attention_finishes_qkv", None)
         if (self.qk_norm and write_to is not None and slopes is None and (rotation is not None or self.position is None)
-                and finishes is not None and finishes(qkv.dtype, *dims, batch, self.window, 0 if rotation is None else rotation.rope_dim,
+                and finishes is not None and finishes(rt.dtype, *dims, batch, self.window, 0 if rotation is None else rotation.rope_dim,
                                                        None if rotation is None else rotation.table)):
+            qkv = rt.empty((tokens, self.q_width + 2 * self.kv_width))
             ops.linear(h, self.w_qkv, qkv)
             ops.attention(qkv, *dims, kv, batch, out, scale=self.scale,
                           finish=ops.QkvFinish(self.q_norm, self.k_norm, self.qk_norm_eps, None if rotation is None else rotation.table))
             return ops.linear(out, self.w_o, residual, accumulate=True,
                               then_norm=None if then is None else then.row_scale())
         if rotation is not None or self.position is None:
-            # the projection, then in one pass (in the same kernel, where a step is short): head norms, rotation, cache write
-            ops.linear_qkv(h, self.w_qkv, qkv, *dims, batch.positions, batch.slots,
-                            q_norm=self.q_norm, k_norm=self.k_norm, norm_eps=self.qk_norm_eps,
-                            rope_theta=None if rotation is None else rotation.theta,
-                            rope_dim=0 if rotation is None else rotation.rope_dim,
-                            rope_scale=1.0 if rotation is None else rotation.scale,
-                            kv=write_to, longest_run=longest_run)
+            qkv = self._project(h, batch, cache)
         else:
             # any other position encoding: norms, then the encoding, then the cache write
+            qkv = rt.empty((tokens, self.q_width + 2 * self.kv_width))
             ops.linear(h, self.w_qkv, qkv)
             if self.qk_norm:
                 ops.qkv_prepare(qkv, *dims, batch.positions, batch.slots,
                                 q_norm=self.q_norm, k_norm=self.k_norm, norm_eps=self.qk_norm_eps)
             self.position.apply(qkv, *dims, batch)
             if write_to is not None:
-                ops.qkv_prepare(qkv, *dims, batch.positions, batch.slots, kv=write_to, longest_run=longest_run)
+                ops.qkv_prepare(qkv, *dims, batch.positions, batch.slots, kv=write_to, longest_run=int(getattr(batch, "max_count", 0) or 0))
 
         ops.attention(qkv, *dims, kv, batch, out, scale=self.scale, window=self.window,
                       **({} if slopes is None else {"distance_slopes": slopes}))

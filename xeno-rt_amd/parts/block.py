@@ -93,6 +93,22 @@ class PreNormBlock(Block):
         self.feed_forward.forward(h, batch, x)
         return None
 
+    def goes_on_with(self, batch) -> bool:
+        """Whether `forward_wanted` serves this step: behind the mixer every part takes a token's row for itself."""
+        return (self.passes_norms and getattr(self.feed_forward, "passes_norms", False)
+                and getattr(self.mixer, "goes_on_with", lambda batch: False)(batch))
+
+    def forward_wanted(self, x, batch, cache, h=None):
+        """`forward` for the last block of a model, of which only the rows `batch.logit_rows` are wanted: returns those rows of the stream (None if
+        there are none); x itself is not what `forward` leaves."""
+        if h is None:
+            h = self.mixer_norm.forward(x)
+        x, h = self.mixer.forward_wanted(h, batch, cache, x, then=self.feed_forward_norm)
+        if x is None:
+            return None
+        self.feed_forward.forward(self.feed_forward_norm.forward(x) if h is None else h, batch, x)
+        return x
+
 
 class SandwichBlock(Block):
     """A norm before and a norm after each sublayer, and a number m that multiplies what a sublayer adds:
