@@ -962,6 +962,32 @@ def test_attention_decode_that_finishes_q_k_and_v_itself(ops, nh, nkv, hd, rotat
     assert float(same.float().mean()) > 0.999               # only the newest keys can differ at all, by a rounding
 
 
+@pytest.mark.parametrize("longest", [64, 65, 256, 257, 512, 513])
+@pytest.mark.parametrize("nh,nkv,hd,tokens", [(8, 4, 128, 2), (8, 4, 128, 65), (12, 4, 64, 64), (20, 1, 64, 3)])
+def test_attention_decode_of_short_contexts(ops, nh, nkv, hd, tokens, longest):
+    """The longest sequence at the edges of four and eight blocks of keys: workgroups of four wavefronts, of eight (a block each, up to 256 pairs of
+    sequence and key/value head, 256 of them here and 260), of four with two blocks each, and keys in parts. Beside it sequences of any shorter
+    length; the kernel that finishes q and k itself as well."""
+    from xeno_rt_amd.ops.hip import QkvFinish
+    lengths = [longest] + [1 + (53 * i) % longest for i in range(1, tokens)]
+    kv, keys, values = filled_cache(nkv, hd, torch.bfloat16, lengths, seed=hd + longest)
+    slots, positions = list(range(tokens)), [n - 1 for n in lengths]
+    batch = described(slots, [1] * tokens, positions)
+    qkv = rand(tokens, (nh + 2 * nkv) * hd, dtype=torch.bfloat16, seed=3)
+    out = torch.full((tokens, nh * hd), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.attention(qkv, nh, nkv, hd, kv, batch, out, scale=1.0 / math.sqrt(hd))
+    want = expected_attention(qkv, slots, positions, keys, values, nh, nkv, hd)
+    assert torch.isfinite(out).all() and rel(out.cpu(), want) < 1e-2
+    for row in range(min(tokens, 4)):
+        assert rel(out[row].cpu(), want[row]) < 2e-2, row
+    two, finished = clone_cache(kv), torch.full_like(out, 7.0)
+    raw = qkv.clone()
+    ops.qkv_prepare(raw, nh, nkv, hd, batch.positions, batch.slots, kv=two)
+    ops.attention(raw, nh, nkv, hd, two, batch, out, scale=1.0 / math.sqrt(hd))
+    ops.attention(qkv, nh, nkv, hd, kv, batch, finished, scale=1.0 / math.sqrt(hd), finish=QkvFinish(None, None, 0.0, None))
+    assert torch.equal(out, finished)                       # (nothing to norm or rotate: the same operands, the same sums)
+
+
 @pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (24, 8, 64)])
 def test_attention_decode_of_many_sequences(ops, nh, nkv, hd):
     """Seventy sequences: with so many (sequence, key/value head) pairs a workgroup takes all keys of its pair

@@ -16,7 +16,7 @@
 // contiguous kilobyte, which nobody else reads, and passes the caches by (non-temporal; with
 // keys as rows of head_dim elements an instruction took half a line of each of 16 keys and the
 // kernel read 6.1 TB/s where it now reads 6.9). A block's values are asked for before its
-// scores are computed, the next block's keys right after. The four wavefronts of a workgroup
+// scores are computed, the next block's keys right after. The four (or eight) wavefronts of a workgroup
 // merge their results (maximum, sum, O) through LDS into one partial result; a second kernel
 // merges the partial results of a token, in order.
 //
@@ -43,7 +43,6 @@ struct Finish {                       // xrt_qkv_finish with its pointers typed
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr int WAVES = 4;
 constexpr float LOG2E = 1.4426950408889634f;
 
 // Row r of score tile t (0 or 1) of a group of 32 keys stands for key 8 (r / 4) + 4 t + r % 4: accumulator
@@ -108,7 +107,7 @@ __device__ __forceinline__ void finish_head(bf16x8 (&x)[HD / 32], const TW* __re
 }
 
 // FINISH: q, k and v come as the projection left them, and `finish` says what is still to do (see the head of this file).
-template <int HD, bool FINISH>
+template <int HD, bool FINISH, int WAVES>
 __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
     const bf16* __restrict__ qkv, int row_width, int n_heads, int n_kv_heads,
     const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache, const int* __restrict__ block_table,
@@ -117,12 +116,13 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
     float* __restrict__ part_o, float* __restrict__ part_ml, bf16* __restrict__ out, const Finish finish) {
     constexpr int KS = HD / 32;                    // K steps of the score product
     constexpr int DT = HD / 16;                    // 16-row tiles of the value product
-    __shared__ floatx4 merge_o[WAVES][DT][XRT_WAVE];
-    __shared__ float merge_ml[WAVES][2][16];
+    extern __shared__ __attribute__((aligned(16))) char lds[];
+    floatx4 (*merge_o)[DT][XRT_WAVE] = reinterpret_cast<floatx4 (*)[DT][XRT_WAVE]>(lds);                    // [WAVES]
+    float (*merge_ml)[2][16] = reinterpret_cast<float (*)[2][16]>(lds + sizeof(floatx4) * WAVES * DT * XRT_WAVE);      // [WAVES]
 
     const int lane = threadIdx.x % XRT_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / XRT_WAVE);   // in a scalar register, and with it the blocks' numbers
     const int r = lane % 16, c = lane / 16;
-    const int part = blockIdx.x;                   // this workgroup's four chunks become one partial result
+    const int part = blockIdx.x;                   // this workgroup's chunks become one partial result
     const int chunk = part * WAVES + wave;
     const int kv_head = blockIdx.y / q_tiles, q_tile = blockIdx.y % q_tiles;
     const int token = blockIdx.z;
@@ -313,7 +313,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
         l += __shfl_xor(l, 32, XRT_WAVE);
     }
 
-    // ---- the four wavefronts' results become one, in wavefront order
+    // ---- the wavefronts' results become one, in wavefront order
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) merge_o[wave][dt][lane] = o[dt];
     if (c == 0) {
@@ -321,43 +321,36 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
         merge_ml[wave][1][r] = l;
     }
     __syncthreads();
-    if (wave == 0 && head_valid) {
-        float m_all = merge_ml[0][0][r];
+    if (!head_valid) return;
+    float m_all = merge_ml[0][0][r];
 #pragma unroll
-        for (int w = 1; w < WAVES; ++w) m_all = fmaxf(m_all, merge_ml[w][0][r]);
-        float l_all = 0.f;
-        floatx4 total[DT];
+    for (int w = 1; w < WAVES; ++w) m_all = fmaxf(m_all, merge_ml[w][0][r]);
+    float l_all = 0.f, weight[WAVES];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) total[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int w = 0; w < WAVES; ++w) {
+        weight[w] = __builtin_amdgcn_exp2f(merge_ml[w][0][r] - m_all);      // 0 for a wavefront without keys
+        l_all += weight[w] * merge_ml[w][1][r];
+    }
+    const float inv = l_all > 0.f ? 1.0f / l_all : 0.f;
+    const long row = (long)token * n_heads + head, index = row * n_parts + part;
+    // every wavefront adds up some of the tiles of dims; accumulator register i of tile dt is dimension dt*16 + c*4 + i, for query head r
+    for (int dt = wave; dt < DT; dt += WAVES) {
+        floatx4 total = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int w = 0; w < WAVES; ++w) {
-            const float weight = __builtin_amdgcn_exp2f(merge_ml[w][0][r] - m_all);     // 0 for a wavefront without keys
-            l_all += weight * merge_ml[w][1][r];
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) total[dt] += merge_o[w][dt][lane] * weight;
-        }
+        for (int w = 0; w < WAVES; ++w) total += merge_o[w][dt][lane] * weight[w];
         if (n_parts == 1) {
             // the workgroup has seen all keys of the sequence: this is the result, and no merge kernel follows
-            const float inv = l_all > 0.f ? 1.0f / l_all : 0.f;
-            bf16* final_row = out + ((long)token * n_heads + head) * HD;
+            struct alignas(8) Four { bf16 e[4]; } four;
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-                struct alignas(8) Four { bf16 e[4]; } four;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) four.e[i] = (bf16)(total[dt][i] * inv);
-                *reinterpret_cast<Four*>(final_row + dt * 16 + c * 4) = four;
-            }
-            return;
+            for (int i = 0; i < 4; ++i) four.e[i] = (bf16)(total[i] * inv);
+            *reinterpret_cast<Four*>(out + row * HD + dt * 16 + c * 4) = four;
+        } else {
+            *reinterpret_cast<floatx4*>(part_o + index * HD + dt * 16 + c * 4) = total;
         }
-        const long index = ((long)token * n_heads + head) * n_parts + part;
-        float* dst = part_o + index * HD;
-        // accumulator register i of tile dt is dimension dt*16 + c*4 + i, for query head r
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) *reinterpret_cast<floatx4*>(dst + dt * 16 + c * 4) = total[dt];
-        if (c == 0) {
-            part_ml[index * 2] = m_all;
-            part_ml[index * 2 + 1] = l_all;
-        }
+    }
+    if (n_parts > 1 && wave == 0 && c == 0) {
+        part_ml[index * 2] = m_all;
+        part_ml[index * 2 + 1] = l_all;
     }
 }
 
@@ -427,11 +420,21 @@ __global__ void __launch_bounds__(HD) attention_decode_merge_kernel(
 }
 
 // How the keys of the longest sequence are cut: blocks per wavefront, and partial results
-// (each from the four wavefronts of a workgroup) per (token, head).
-struct Cut { int chunk_blocks, n_parts; };
+// (each from the wavefronts of a workgroup) per (token, head).
+struct Cut { int chunk_blocks, n_parts, waves; };
 
 Cut cut_for(int tokens, int n_kv_heads, int q_tiles, int max_context, int head_dim) {
+    constexpr int WAVES = 4;                       // of a workgroup, but for the short contexts below
     const int max_blocks = (max_context + XRT_BLOCK_TOKENS - 1) / XRT_BLOCK_TOKENS;
+    const long pairs = (long)tokens * n_kv_heads * q_tiles;
+    // Up to eight blocks: one workgroup sees all keys, and nothing is left to merge. From five blocks on it has eight wavefronts, a block
+    // each, where every pair finds a compute unit of its own, and four of two blocks beyond (16 heads of 128 on 8, 334 keys: 1 sequence 7.4 us in two
+    // parts and their merge, 6.0 with four wavefronts, 5.8 with eight; 16 sequences 9.1, 8.4, 7.9; 48 sequences 18.0, 14.4, 15.9; heads of 64 gain
+    // 0.2 to 1 us by the eight). Nine blocks and more: two blocks one after the other cost more than the merge.
+    if (max_blocks <= 8) {
+        const int waves = max_blocks > 4 && pairs <= XRT_COMPUTE_UNITS ? 8 : 4;
+        return Cut{(max_blocks + waves - 1) / waves, 1, waves};
+    }
     // How long the kernel takes is set by the compute unit with the most to do: workgroups are dealt out to
     // the 256 compute units in turn, and a compute unit works off its share at its own pace (two workgroups
     // at a time are no faster than one after the other). Measured at head size 128: 6.3 us for a block of 64
@@ -439,18 +442,17 @@ Cut cut_for(int tokens, int n_kv_heads, int q_tiles, int max_context, int head_d
     // the fewest blocks per compute unit: 384 workgroups of 16 blocks (two on every second compute unit) are
     // slower than 768 of 8. The longer chunk wins among equals (less to merge); with one workgroup per (token,
     // key/value head) pair nothing is left to merge and the merge kernel is not launched.
-    const long pairs = (long)tokens * n_kv_heads * q_tiles;
     const long block_ns = 6300L * head_dim / 128, group_ns = 700, merge_ns = 5000;
     const int longest = (max_blocks + WAVES - 1) / WAVES;
     long best_ns = -1;
-    Cut best{longest, 1};
+    Cut best{longest, 1, WAVES};
     for (int chunk_blocks = longest; chunk_blocks >= 1; --chunk_blocks) {
         const int n_chunks = (max_blocks + chunk_blocks - 1) / chunk_blocks;
         const int n_parts = (n_chunks + WAVES - 1) / WAVES;
         if ((long)(n_parts - 1) * WAVES * chunk_blocks >= max_blocks) continue;         // a part without keys: a shorter chunk does the same
         const long per_unit = (pairs * n_parts + XRT_COMPUTE_UNITS - 1) / XRT_COMPUTE_UNITS;
         const long ns = per_unit * (chunk_blocks * block_ns + group_ns) + (n_parts > 1 ? merge_ns : 0);
-        if (best_ns < 0 || ns < best_ns) { best_ns = ns; best = Cut{chunk_blocks, n_parts}; }
+        if (best_ns < 0 || ns < best_ns) { best_ns = ns; best = Cut{chunk_blocks, n_parts, WAVES}; }
     }
     return best;
 }
@@ -470,17 +472,24 @@ int launch(const bf16* qkv, int tokens, int n_heads, int n_kv_heads, const bf16*
     const int row_width = (n_heads + 2 * n_kv_heads) * HD;
     XRT_REQUIRE(tokens <= 65535 && n_kv_heads * q_tiles <= 65535, "attention (decode): grid too large");
     const dim3 grid(cut.n_parts, n_kv_heads * q_tiles, tokens);
-    if (finish != nullptr)
-        attention_decode_kernel<HD, true><<<grid, WAVES * XRT_WAVE, 0, s>>>(
-            qkv, row_width, n_heads, n_kv_heads, k_cache, v_cache, block_table, table_stride, n_blocks, positions, slots,
-            scale, cut.chunk_blocks, cut.n_parts, q_tiles, part_o, part_ml, out, *finish);
-    else
-        attention_decode_kernel<HD, false><<<grid, WAVES * XRT_WAVE, 0, s>>>(
-            qkv, row_width, n_heads, n_kv_heads, k_cache, v_cache, block_table, table_stride, n_blocks, positions, slots,
-            scale, cut.chunk_blocks, cut.n_parts, q_tiles, part_o, part_ml, out, Finish{});
+    const size_t lds = cut.waves * (sizeof(floatx4) * HD / 16 * XRT_WAVE + 2 * 16 * sizeof(float));
+#define XRT_DECODE(FINISH_, WAVES_, HOW)                                                                                            \
+    do {                                                                                                                            \
+        static const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_decode_kernel<HD, FINISH_, WAVES_>),   \
+                                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                 \
+        XRT_REQUIRE(room == hipSuccess, "attention (decode): cannot reserve LDS: %s", hipGetErrorString(room));                    \
+        attention_decode_kernel<HD, FINISH_, WAVES_><<<grid, WAVES_ * XRT_WAVE, lds, s>>>(                                            \
+            qkv, row_width, n_heads, n_kv_heads, k_cache, v_cache, block_table, table_stride, n_blocks, positions, slots,            \
+            scale, cut.chunk_blocks, cut.n_parts, q_tiles, part_o, part_ml, out, HOW);                                              \
+    } while (0)
+    if (finish != nullptr && cut.waves == 8) XRT_DECODE(true, 8, *finish);
+    else if (finish != nullptr) XRT_DECODE(true, 4, *finish);
+    else if (cut.waves == 8) XRT_DECODE(false, 8, Finish{});
+    else XRT_DECODE(false, 4, Finish{});
+#undef XRT_DECODE
     XRT_LAUNCH_CHECK("attention (decode)");
     if (cut.n_parts == 1) return 0;
-    const int part_keys = cut.chunk_blocks * WAVES * XRT_BLOCK_TOKENS;
+    const int part_keys = cut.chunk_blocks * cut.waves * XRT_BLOCK_TOKENS;
     attention_decode_merge_kernel<HD><<<dim3(n_heads, tokens), HD, cut.n_parts * sizeof(float), s>>>(
         part_o, part_ml, positions, slots, n_heads, part_keys, cut.n_parts, out);
     XRT_LAUNCH_CHECK("attention (decode merge)");
