@@ -1,6 +1,8 @@
 """The engine on the GPU against the plain implementation: whole requests, decoded tails,
 unequal batches with slot reuse, long decoding, first tokens, greedy generation; in 32-bit
 and in bfloat16, for two tiny configurations that differ in every size and option."""
+import ctypes
+
 import pytest
 import torch
 
@@ -276,6 +278,61 @@ def test_a_step_may_mix_sequences_that_start_with_sequences_that_go_on(name, dty
     engine.cache.check()
 
 
+@pytest.mark.parametrize("pack", ["always", False])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", ["llama", "qwen3"])
+def test_layers_launched_by_one_call_do_what_they_do_one_by_one(name, dtype, pack, models):
+    """The same step with its layers launched by one call and part by part: the same kernels, so the same bits. One token, 16 and 17, a long prompt, sequences that
+    go on (unequal counts), a decode step of three; then memory that is missing a byte, or not aligned, and a step that reaches beyond the block table."""
+    from xeno_rt_amd.engine import Engine
+    from xeno_rt_amd.ops.hip import KernelError
+    folder, _, cases = models[name]
+    engine = Engine.load(folder, dtype=dtype, max_tokens=64 * 8, max_slots=3, graphs=False, pack_weights=pack)
+    assert engine.model.one_call
+    ids = cases[LENGTHS[name][5]][0]
+    counts = [[1], [16], [17], [len(ids)], [40, 1, 20], [3, 1, 9], [1, 1, 1]]
+    results = []
+    for one_call in (True, False):
+        engine.model.one_call = one_call
+        got, slots, held = [], [], []
+        for step in counts:
+            if len(step) != len(slots) or len(step) == 1:
+                for slot in slots:
+                    engine.free_slot(slot)
+                slots, held = [engine.alloc_slot() for _ in step], [0] * len(step)
+            got.append(engine.step([(slot, ids[at:at + count], list(range(count))) for slot, at, count in zip(slots, held, step)]))
+            held = [at + count for at, count in zip(held, step)]
+        for slot in slots:
+            engine.free_slot(slot)
+        results.append(got)
+    for step, one, other in zip(counts, *results):
+        assert torch.isfinite(one).all() and torch.equal(one, other), step
+    engine.model.one_call = True
+    before, sizes = engine.ops.lib.xrt_dense_blocks, []
+
+    def spoiled(how):
+        def run(layers, count, step, wanted, memory, size):
+            if memory is None:
+                return before(layers, count, step, wanted, memory, size)
+            sizes.append(size.value)
+            return how(layers, count, step, wanted, memory, size)
+        return run
+    ways = {"too small": lambda l, n, s, w, memory, size: before(l, n, s, w, memory, ctypes.c_long(size.value - 1)),
+            "aligned": lambda l, n, s, w, memory, size: before(l, n, s, w, ctypes.c_void_p(memory.value + 16), size),
+            "block table": lambda l, n, s, w, memory, size: (setattr(s._obj, "max_context", 10 ** 6), before(l, n, s, w, memory, size))[1]}
+    try:
+        for what, how in ways.items():
+            engine.ops.lib.xrt_dense_blocks = spoiled(how)
+            slot = engine.alloc_slot()
+            with pytest.raises(KernelError, match=what):
+                engine.step([(slot, ids[:5], [4])])
+            engine.free_slot(slot)
+    finally:
+        engine.ops.lib.xrt_dense_blocks = before
+    assert len(sizes) == 3 and min(sizes) > 0
+    engine.cache.check()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("name", ["llama", "qwen3"])
 def test_rows_that_nobody_wants_stop_behind_the_last_attention(name, dtype, models, engines, monkeypatch):
@@ -295,13 +352,10 @@ def test_rows_that_nobody_wants_stop_behind_the_last_attention(name, dtype, mode
              [(slots[0], a[0][17:], []), (slots[1], b[0][cuts[1]:], [20, 5]), (slots[2], c[0][cuts[2]:], [1])]]
     rows = [[(a, [16, 0, 16, 3])], [], [(b, [cuts[1] + 20, cuts[1] + 5]), (c, [cuts[2] + 1])]]
     taken = []
-    before = engine.ops.lib.xrt_take_rows
-    engine.ops.lib.xrt_take_rows = lambda *arguments: (taken.append(1), before(*arguments))[1]
-    try:
-        got = [engine.step(step) for step in steps]
-    finally:
-        engine.ops.lib.xrt_take_rows = before
-    assert len(taken) == 2 and got[1].shape == (0, engine.vocab_size)
+    before = engine.ops.dense_blocks
+    monkeypatch.setattr(engine.ops, "dense_blocks", lambda *arguments, rows=None: (taken.append(rows), before(*arguments, rows=rows))[1])
+    got = [engine.step(step) for step in steps]
+    assert [None if rows is None else rows.shape[0] for rows in taken] == [4, 0, 3] and got[1].shape == (0, engine.vocab_size)
     for slot in slots:
         engine.free_slot(slot)
     for logits, wanted in zip(got, rows):

@@ -323,6 +323,28 @@ int xrt_attention_float_prompts(const void* qkv, int tokens, int n_heads, int n_
                                 const void* v_cache, const int* block_table, int table_stride, int n_blocks, const int* positions,
                                 const int* slots, void* out, float scale, int fewest, void* stream);
 
+// The layers of a plain dense decoder from one call (dense_blocks.hip): for each of `count` layers in turn the RMSNorm of the float32 stream x, q/k/v with
+// head norms, rotation and cache write, causal attention, the output projection onto x, the second norm, the gated (silu) product and the one back onto x, with the kernels and operands
+// that the calls above would get one by one. q_norm, k_norm: null without head norms; rope_theta: null without rotation, else float32 [rope_dim / 2]; rope_table: null, or xrt_rope_table's
+// for the first table_positions positions; writable 0: the keys and values are another call's. fewest: the fewest new tokens of a sequence. wanted: null, or the rows of the step that the last
+// layer goes on with behind its keys and values (count 0: none): x is then left as the layers before it made it, and those rows, updated, lie in wanted->x.
+// arena null: returns the bytes of memory the call needs (launches nothing); else memory of at least so many, aligned to 256. Returns that number, or -1 (xrt_last_error).
+typedef struct xrt_dense_matrix { const void* data; xrt_packing packing; } xrt_dense_matrix;
+typedef struct xrt_dense_layer {
+    const void* mixer_gain; const void* ff_gain; int mixer_gain_dtype; int ff_gain_dtype; float mixer_eps; float ff_eps;
+    xrt_dense_matrix qkv; xrt_dense_matrix o; xrt_dense_matrix gate_up; xrt_dense_matrix down;
+    const void* q_norm; const void* k_norm; int head_norm_dtype; float head_norm_eps;
+    int n_heads; int n_kv_heads; int head_dim; int intermediate;
+    const float* rope_theta; const float* rope_table; int rope_dim; int table_positions; float rope_scale; float scale;
+    void* k_cache; void* v_cache; const int* block_table; int table_stride; int n_blocks; int writable;
+} xrt_dense_layer;
+typedef struct xrt_dense_step {
+    float* x; const int* positions; const int* slots; const int* seq_offsets; const int* seq_slots; const int* seq_starts; void* stream;
+    int dtype; int tokens; int hidden; int n_seqs; int max_count; int max_context; int fewest;
+} xrt_dense_step;
+typedef struct xrt_dense_wanted { const int* rows; float* x; int count; } xrt_dense_wanted;
+long xrt_dense_blocks(const xrt_dense_layer* layers, int count, const xrt_dense_step* step, const xrt_dense_wanted* wanted, void* arena, long arena_bytes);
+
 // Attention without a softmax: the weight of a visible key is sigmoid(score_h + head_bias[h]), not normalised over the keys;
 // before that the heads' scaled scores of a (query, key) pair are mixed, score_h <- sum_g head_mix[h][g] score_g
 // (head_mix float32 [n_heads][n_heads], or null); a head's summed values are multiplied by sigmoid(gate[token][h]) (float32

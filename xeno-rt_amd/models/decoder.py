@@ -108,6 +108,19 @@ class DecoderModel:
         self.runtime = runtime
         for part in spec.parts():
             part.bind(tensors, runtime)
+        # every layer a plain dense block: a step's layers are launched by one call
+        self.one_call = (hasattr(runtime.ops, "dense_blocks") and spec.streams is None and spec.entry is None and not getattr(spec.embedding, "keeps_state", False)
+                         and all(getattr(spec.layers[call.layer], "one_call", False) for call in spec.schedule))
+
+    def _layers_by_one_call(self, x, batch, cache):
+        """(the stream behind the layers, the rows of it that are wanted: None for all). Behind the last attention only the wanted tokens count."""
+        spec, ops = self.spec, self.runtime.ops
+        layers = (ops.DenseLayer * len(spec.schedule))()
+        for index, call in enumerate(spec.schedule):
+            spec.layers[call.layer].describe(layers[index], cache.layer_cache(index))
+        if spec.layers[spec.schedule[-1].layer].mixer.goes_on_with(batch):
+            return ops.dense_blocks(layers, x, batch, self.runtime.dtype, rows=batch.logit_rows), None
+        return ops.dense_blocks(layers, x, batch, self.runtime.dtype), batch.logit_rows
 
     def _first_reads_stream(self) -> bool:
         """Whether the first block reads the stream itself in the compute dtype and the embedding can hand it that beside the stream."""
@@ -132,18 +145,15 @@ class DecoderModel:
             x = spec.streams.open(x)
         wanted = batch.logit_rows
         opened = spec.entry.open(x) if spec.entry is not None else None      # (before any layer: the stream still is what the embedding left)
-        for index, call in enumerate(spec.schedule):
+        if self.one_call:
+            x, wanted = self._layers_by_one_call(x, batch, cache)
+        for index, call in enumerate(spec.schedule if not self.one_call else ()):
             block = spec.layers[call.layer]
             if call.enters:
                 spec.entry.forward(x, opened)
             if not getattr(block, "passes_norms", False):
                 block.forward(x, batch, cache.layer_cache(index))
                 h = None
-                continue
-            if index + 1 == len(spec.schedule) and spec.streams is None and hasattr(block, "goes_on_with") and block.goes_on_with(batch):
-                # behind the last attention only the wanted tokens count: the others' keys and values are all that is left of them
-                x = block.forward_wanted(x, batch, cache.layer_cache(index), h=h)
-                wanted = None
                 continue
             last = index + 1 == len(spec.schedule) or spec.schedule[index + 1].enters      # (what follows does not read the stream as this block leaves it)
             after = None if last else spec.layers[spec.schedule[index + 1].layer]

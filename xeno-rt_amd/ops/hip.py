@@ -133,6 +133,39 @@ class _LinearNorm(ctypes.Structure):
                 ("gain_dtype", ctypes.c_int), ("squares_out", ctypes.c_void_p)]
 
 
+class _DenseMatrix(ctypes.Structure):
+    _fields_ = [("data", ctypes.c_void_p), ("packing", _Packing)]
+
+    def set(self, w) -> None:
+        if isinstance(w, PackedMatrix):
+            self.data, self.packing = w.data.data_ptr(), w.packing
+        else:
+            self.data, self.packing.kind = w.data_ptr(), 0
+
+
+class DenseLayer(ctypes.Structure):
+    """A layer of `dense_blocks`, as its parts describe it (`PreNormBlock.describe`)."""
+    _fields_ = [("mixer_gain", ctypes.c_void_p), ("ff_gain", ctypes.c_void_p), ("mixer_gain_dtype", ctypes.c_int), ("ff_gain_dtype", ctypes.c_int),
+                ("mixer_eps", ctypes.c_float), ("ff_eps", ctypes.c_float), ("qkv", _DenseMatrix), ("o", _DenseMatrix), ("gate_up", _DenseMatrix),
+                ("down", _DenseMatrix), ("q_norm", ctypes.c_void_p), ("k_norm", ctypes.c_void_p), ("head_norm_dtype", ctypes.c_int),
+                ("head_norm_eps", ctypes.c_float), ("n_heads", ctypes.c_int), ("n_kv_heads", ctypes.c_int), ("head_dim", ctypes.c_int),
+                ("intermediate", ctypes.c_int), ("rope_theta", ctypes.c_void_p), ("rope_table", ctypes.c_void_p), ("rope_dim", ctypes.c_int),
+                ("table_positions", ctypes.c_int), ("rope_scale", ctypes.c_float), ("scale", ctypes.c_float), ("k_cache", ctypes.c_void_p),
+                ("v_cache", ctypes.c_void_p), ("block_table", ctypes.c_void_p), ("table_stride", ctypes.c_int), ("n_blocks", ctypes.c_int),
+                ("writable", ctypes.c_int)]
+
+
+class _DenseStep(ctypes.Structure):
+    _fields_ = [("x", ctypes.c_void_p), ("positions", ctypes.c_void_p), ("slots", ctypes.c_void_p), ("seq_offsets", ctypes.c_void_p),
+                ("seq_slots", ctypes.c_void_p), ("seq_starts", ctypes.c_void_p), ("stream", ctypes.c_void_p), ("dtype", ctypes.c_int),
+                ("tokens", ctypes.c_int), ("hidden", ctypes.c_int), ("n_seqs", ctypes.c_int), ("max_count", ctypes.c_int),
+                ("max_context", ctypes.c_int), ("fewest", ctypes.c_int)]
+
+
+class _DenseWanted(ctypes.Structure):
+    _fields_ = [("rows", ctypes.c_void_p), ("x", ctypes.c_void_p), ("count", ctypes.c_int)]
+
+
 class _Recurrence(ctypes.Structure):
     _fields_ = [("q", ctypes.c_void_p), ("k", ctypes.c_void_p), ("v", ctypes.c_void_p),
                 ("q_stride", ctypes.c_long), ("k_stride", ctypes.c_long), ("v_stride", ctypes.c_long),
@@ -213,7 +246,7 @@ class HipOps:
                      "xrt_experts_sort", "xrt_gather_rows", "xrt_linear_groups", "xrt_linear_groups_accepts", "xrt_experts_combine",
                      "xrt_linear_groups_tile_rows", "xrt_linear_groups_parts", "xrt_streams_open", "xrt_streams_read", "xrt_streams_write",
                      "xrt_latent_complete", "xrt_latent_queries", "xrt_linear_heads", "xrt_causal_softmax", "xrt_transpose", "xrt_attention_latent",
-                     "xrt_attention_latent_accepts", "xrt_attention_latent_prompts", "xrt_latent_prepare", "xrt_glu_experts", "xrt_embed_normed", "xrt_rmsnorm_two", "xrt_replace_rows", "xrt_take_rows"):
+                     "xrt_attention_latent_accepts", "xrt_attention_latent_prompts", "xrt_latent_prepare", "xrt_glu_experts", "xrt_embed_normed", "xrt_rmsnorm_two", "xrt_replace_rows"):
             getattr(self.lib, name).restype = ctypes.c_int
         from ..cache.allocator import BLOCK_TOKENS
         if int(self.lib.xrt_block_tokens()) != BLOCK_TOKENS:
@@ -222,6 +255,7 @@ class HipOps:
         self.lib.xrt_linear_workspace.restype = ctypes.c_long
         self.lib.xrt_linear_whole_norm_workspace.restype = ctypes.c_long
         self.lib.xrt_attention_workspace.restype = ctypes.c_long
+        self.lib.xrt_dense_blocks.restype = ctypes.c_long
         self.lib.xrt_probe_read_bytes.restype = ctypes.c_long
         self.lib.xrt_sample_workspace.restype = ctypes.c_long
         self.lib.xrt_linear_recurrence_workspace.restype = ctypes.c_long
@@ -345,24 +379,38 @@ class HipOps:
         self._require(copy, "replace_rows copy", None, x.shape, x)
         self._check(self.lib.xrt_replace_rows(_ptr(x), _ptr(base), _ptr(copy), _code(copy), ctypes.c_long(x.numel()), self._stream(x)))
 
-    def take_rows(self, qkv, q_width, x, positions, slots, rows):
-        """Rows `rows` (int32, indices of the step's tokens) of a step: (the queries qkv[rows, :q_width], in rows as wide as qkv's whose rest holds
-        nothing, x[rows], positions[rows], slots[rows], 0 .. count as int32)."""
-        tokens, width = qkv.shape
-        count, hidden = rows.shape[0], x.shape[1]
-        self._require(qkv, "take_rows qkv")
-        self._require(x, "take_rows x", torch.float32, (tokens, hidden), qkv)
-        self._require(positions, "take_rows positions", torch.int32, (tokens,), qkv)
-        self._require(slots, "take_rows slots", torch.int32, (tokens,), qkv)
-        self._require(rows, "take_rows rows", torch.int32, (count,), qkv)
-        if not 0 < q_width <= width:
-            raise KernelError(f"take_rows: {q_width} columns of {width}")
-        size = qkv.element_size()
-        q, taken = self._empty((count, width), qkv.dtype, qkv.device), self._empty((count, hidden), torch.float32, qkv.device)
-        described = self._empty((3 * count + 1,), torch.int32, qkv.device)
-        self._check(self.lib.xrt_take_rows(_ptr(qkv), ctypes.c_long(width * size), q_width * size, _ptr(q), ctypes.c_long(width * size), _ptr(x), hidden * 4,
-                                           _ptr(taken), _ptr(positions), _ptr(slots), _ptr(rows), count, tokens, _ptr(described), self._stream(qkv)))
-        return q, taken, described[:count], described[count:2 * count], described[2 * count:]
+    DenseLayer = DenseLayer
+    dtype_codes = _CODES
+
+    def dense_blocks(self, layers, x, batch, dtype, rows=None):
+        """The layers of a plain dense decoder (an array of DenseLayer) on the float32 stream x, all launched by one call. rows: None, or the rows (int32)
+        of the step's tokens that the last layer goes on with behind its keys and values: those rows, updated, are returned (None without any)
+        and x is left as the layers before made it; without `rows` x itself is returned."""
+        tokens, hidden = x.shape
+        n_seqs = int(batch.n_sequences)
+        self._require(x, "dense blocks x", torch.float32)
+        self._require(batch.positions, "positions", torch.int32, (tokens,), x)
+        self._require(batch.slots, "slots", torch.int32, (tokens,), x)
+        self._require(batch.sequence_offsets, "sequence offsets", torch.int32, (n_seqs + 1,), x)
+        self._require(batch.sequence_slots, "sequence slots", torch.int32, (n_seqs,), x)
+        self._require(batch.sequence_starts, "sequence starts", torch.int32, (n_seqs,), x)
+        step = _DenseStep(x.data_ptr(), batch.positions.data_ptr(), batch.slots.data_ptr(), batch.sequence_offsets.data_ptr(), batch.sequence_slots.data_ptr(),
+                          batch.sequence_starts.data_ptr(), self._stream(x), _CODES[dtype], tokens, hidden, n_seqs, int(batch.max_count), int(batch.max_context),
+                          min(batch.host_counts))
+        wanted, out = None, x
+        if rows is not None:
+            count = rows.shape[0]
+            self._require(rows, "wanted rows", torch.int32, (count,), x)
+            out = self._empty((count, hidden), torch.float32, x.device) if count else None
+            wanted = ctypes.byref(_DenseWanted(rows.data_ptr(), None if out is None else out.data_ptr(), count))
+        run = self.lib.xrt_dense_blocks
+        need = run(layers, len(layers), ctypes.byref(step), wanted, None, ctypes.c_long(0))
+        if need >= 0:
+            memory = self._empty((need,), torch.uint8, x.device)
+            need = run(layers, len(layers), ctypes.byref(step), wanted, _ptr(memory), ctypes.c_long(need))
+        if need < 0:
+            raise KernelError(self.lib.xrt_last_error().decode())
+        return out
 
     def _linear(self, a, w, out, coded_mode, n, then_norm=None):
         mode = coded_mode & 255                 # what rides above is a gated product's activation

@@ -42,7 +42,6 @@ keys, at or before it, which the cache then never lets go of); and a layer witho
 from __future__ import annotations
 
 import math
-from dataclasses import replace
 from typing import Dict, Optional
 
 import torch
@@ -318,36 +317,42 @@ class Attention(Mixer):
         rt.ops.rows_add(self.bias_o.reshape(1, -1), row, out)
         return None
 
+    @property
+    def one_call(self) -> bool:
+        """Whether `describe` says all there is to say of this layer: plain causal attention, positions by rotation or not at all."""
+        return type(self) is Attention and not self.general and self.window is None and (self.position is None or self.position.rotation() is not None) and (
+            self.position is None or self.position.score_slopes() is None)
+
     # Tokens whose results nobody wants need go no further than the cache behind the model's last attention: for the others alone the step
     # goes on from there with their queries, which costs a kernel that brings them together. Up to 16 rows a product is bound by reading its weights, and where
-    # the output projection has fewer than WANTED_FROM elements a layer is all launches: tiny models 305 -> 330 us a prompt by it, 1024 x 2048
-    # the same up to 200 tokens and 3220 -> 3168 us at 400, 4096 x 4096 (4 layers) 633 -> 618 at 17 tokens, 822 -> 780 at 100, 1304 -> 1171 at 400; a prompt
-    # of 2048 tokens through 6 layers 4847 -> 4260, of 8192 through 4 13374 -> 10535. (One layer of a model's: of 32 layers 2 to 3 %.)
+    # the output projection has fewer than WANTED_FROM elements a layer is all launches. Measured with every kernel launched from Python: tiny models 305 -> 330 us
+    # a prompt by it, 1024 x 2048 the same up to 200 tokens and 3220 -> 3168 us at 400, 4096 x 4096 (4 layers) 633 -> 618 at 17 tokens, 822 -> 780 at 100,
+    # 1304 -> 1171 at 400; a prompt of 2048 tokens through 6 layers 4847 -> 4260, of 8192 through 4 13374 -> 10535. (One layer of a model's: of 32 layers 2 to 3 %.)
     WANTED_FROM = 1 << 20
 
     def goes_on_with(self, batch) -> bool:
-        """Whether `forward_wanted` serves this step (rows must be whole pieces of 16 bytes)."""
-        if self.general or not hasattr(self.runtime.ops, "take_rows") or (self.position is not None and self.position.rotation() is None):
-            return False
+        """Whether the model's last layer goes on with the step's wanted rows alone (which must be whole pieces of 16 bytes)."""
         size = 4 if self.runtime.dtype == torch.float32 else 2
         return batch.n_logit_rows == 0 or (batch.n_tokens > 16 and 4 * batch.n_logit_rows <= batch.n_tokens and self.q_width * self.hidden >= self.WANTED_FROM
                                            and self.q_width * size % 16 == 0 and self.kv_width * size % 8 == 0 and self.hidden % 4 == 0)
 
-    def forward_wanted(self, h, batch, cache, residual: torch.Tensor, then=None):
-        """`forward` of which only the rows `batch.logit_rows` are wanted: every token's key and value reach the cache, the attention and the output
-        projection run for the wanted rows alone. Returns (those rows of the residual stream, updated, what `forward` returns for them),
-        or (None, None) where no row is wanted."""
-        rt = self.runtime
-        qkv = self._project(h, batch, cache)
-        if batch.n_logit_rows == 0:
-            return None, None
-        q, residual, positions, slots, offsets = rt.ops.take_rows(qkv, self.q_width, residual, batch.positions, batch.slots, batch.logit_rows)
-        count = batch.n_logit_rows
-        alone = replace(batch, n_tokens=count, n_sequences=count, positions=positions, slots=slots, sequence_slots=slots, sequence_offsets=offsets,
-                        sequence_starts=positions, host_slots=None, host_counts=[1] * count, host_starts=None, is_decode=True, max_count=1)
-        out = rt.empty((count, self.q_width))
-        rt.ops.attention(q, self.n_heads, self.n_kv_heads, self.head_dim, cache.kv, alone, out, scale=self.scale, window=self.window)
-        return residual, rt.ops.linear(out, self.w_o, residual, accumulate=True, then_norm=None if then is None else then.row_scale())
+    def describe(self, record, cache) -> None:
+        """This layer in the record that `ops.dense_blocks` reads."""
+        codes = self.runtime.ops.dtype_codes
+        record.qkv.set(self.w_qkv)
+        record.o.set(self.w_o)
+        if self.qk_norm:
+            record.q_norm, record.k_norm = self.q_norm.data_ptr(), self.k_norm.data_ptr()
+            record.head_norm_dtype, record.head_norm_eps = codes[self.q_norm.dtype], self.qk_norm_eps
+        record.n_heads, record.n_kv_heads, record.head_dim, record.scale = self.n_heads, self.n_kv_heads, self.head_dim, self.scale
+        rotation = None if self.position is None else self.position.rotation()
+        if rotation is not None:
+            record.rope_theta, record.rope_dim, record.rope_scale = rotation.theta.data_ptr(), rotation.rope_dim, rotation.scale
+            if rotation.table is not None:
+                record.rope_table, record.table_positions = rotation.table.data_ptr(), rotation.table.shape[0]
+        k, v, table = cache.kv.k, cache.kv.v, cache.kv.block_table
+        record.k_cache, record.v_cache, record.block_table = k.data_ptr(), v.data_ptr(), table.data_ptr()
+        record.table_stride, record.n_blocks, record.writable = table.shape[1], k.shape[0], cache.writable
 
     def _project(self, h, batch, cache):
         """q, k and v of the step's tokens, rotated, keys and values in the cache: the projection, then in one pass (in the same kernel, where a

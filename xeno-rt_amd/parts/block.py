@@ -93,21 +93,21 @@ class PreNormBlock(Block):
         self.feed_forward.forward(h, batch, x)
         return None
 
-    def goes_on_with(self, batch) -> bool:
-        """Whether `forward_wanted` serves this step: behind the mixer every part takes a token's row for itself."""
-        return (self.passes_norms and getattr(self.feed_forward, "passes_norms", False)
-                and getattr(self.mixer, "goes_on_with", lambda batch: False)(batch))
+    @property
+    def one_call(self) -> bool:
+        """Whether a run of such blocks can be launched by one call (`ops.dense_blocks`): plain attention and a gated feed-forward behind plain RMS norms."""
+        return (type(self) is PreNormBlock and self.passes_norms and getattr(self.mixer, "one_call", False) and getattr(self.feed_forward, "one_call", False)
+                and self.mixer_norm.row_scale() is not None and self.feed_forward_norm.row_scale() is not None)
 
-    def forward_wanted(self, x, batch, cache, h=None):
-        """`forward` for the last block of a model, of which only the rows `batch.logit_rows` are wanted: returns those rows of the stream (None if
-        there are none); x itself is not what `forward` leaves."""
-        if h is None:
-            h = self.mixer_norm.forward(x)
-        x, h = self.mixer.forward_wanted(h, batch, cache, x, then=self.feed_forward_norm)
-        if x is None:
-            return None
-        self.feed_forward.forward(self.feed_forward_norm.forward(x) if h is None else h, batch, x)
-        return x
+    def describe(self, record, cache) -> None:
+        """This block in the record that `ops.dense_blocks` reads, with the cache of the call under way."""
+        codes = self.runtime.ops.dtype_codes
+        gain, record.mixer_eps = self.mixer_norm.row_scale()
+        record.mixer_gain, record.mixer_gain_dtype = gain.data_ptr(), codes[gain.dtype]
+        gain, record.ff_eps = self.feed_forward_norm.row_scale()
+        record.ff_gain, record.ff_gain_dtype = gain.data_ptr(), codes[gain.dtype]
+        self.mixer.describe(record, cache)
+        self.feed_forward.describe(record)
 
 
 class SandwichBlock(Block):

@@ -46,6 +46,17 @@ class GatedMLP(FeedForward):
         self.w_gate_up = runtime.weight([tensors[self.gate_name], tensors[self.up_name]], "gated", gated_n=self.intermediate)
         self.w_down = runtime.weight(tensors[self.down_name])
 
+    @property
+    def one_call(self) -> bool:
+        """Whether `describe` says all there is to say of this feed-forward."""
+        return type(self) is GatedMLP and self.activation == "silu"
+
+    def describe(self, record) -> None:
+        """This feed-forward in the record that `ops.dense_blocks` reads."""
+        record.gate_up.set(self.w_gate_up)
+        record.down.set(self.w_down)
+        record.intermediate = self.intermediate
+
     def forward_into(self, h, batch, out: torch.Tensor) -> None:
         """The feed-forward's output into `out` (float32 [tokens, hidden]) instead of onto the residual stream: for a
         block that puts a norm between the two."""
