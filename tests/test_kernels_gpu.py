@@ -3,6 +3,7 @@ elementary tensor operations), at sizes other than the engine's: head sizes 16 t
 one to eight query heads per key/value head, widths and vocabularies that are no power
 of two. Inputs are built so that a fault shows: a far key that must win, the edge of a
 window, a block boundary of the cache."""
+import ctypes
 import math
 from types import SimpleNamespace
 
@@ -118,6 +119,24 @@ def test_linear(ops, dtype, m, n, k):
     acc = base.clone()
     ops.linear(a, w, acc, accumulate=True)
     assert rel(acc.cpu(), base.double().cpu() + want) < 1e-5
+
+
+# Products of 65 to 1030 rows in parts along k: narrow tiles below and beyond 256 rows and in several row tiles, wide ones of either kind, up to sixteen parts,
+# a last part that is shorter, columns that fill no tile and are no multiple of four.
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("m,n,k", [(65, 520, 1088), (129, 2000, 1024), (333, 1024, 3072), (300, 514, 1088), (777, 1000, 2048), (1030, 1024, 1984), (100, 515, 8192),
+                                   (70, 5120, 8256), (200, 5121, 8192), (400, 2049, 8192)])
+def test_linear_of_some_hundred_rows_in_parts(ops, m, n, k, packed):
+    a, w = rand(m, k, dtype=torch.bfloat16, seed=m), rand(n, k, dtype=torch.bfloat16, seed=n, scale=0.1)
+    assert int(ops.lib.xrt_linear_workspace(ctypes.c_void_p(a.data_ptr()), ctypes.c_void_p(w.data_ptr()), 1, m, n, k, 0)) >= 2 * m * n      # (two parts or more)
+    want = a.double().cpu() @ w.double().cpu().t()
+    w = packed_or_not(ops, w, packed)
+    stored, rounded, base = torch.empty(m, n, device=DEV), torch.empty(m, n, dtype=torch.bfloat16, device=DEV), rand(m, n, seed=5)
+    added = base.clone()
+    ops.linear(a, w, stored)
+    ops.linear(a, w, rounded)
+    ops.linear(a, w, added, accumulate=True)
+    assert rel(stored.cpu(), want) < 1e-5 and rel(rounded.cpu(), want) < ULP["bfloat16"] * 2 and rel(added.cpu(), base.double().cpu() + want) < 1e-5
 
 
 # float32: the matrix cores' product of many rows gives the bits of the kernels of few rows (the sums of 16 consecutive k, in order),

@@ -1083,6 +1083,31 @@ constexpr int SPLIT_BM = 64, SPLIT_BN = 128;
 
 struct SplitPlan { int splits, k_per_split; long rows_w; int tile, columns; };      // tile: rows of x per tile (64, 128 or 256), columns: rows of w
 
+// What a product of some hundred rows of x takes (nanoseconds) in parts along k: tiles of 128 rows of x and `columns` rows of w, `places` of them to a compute
+// unit. A step of 64 along k takes `step`, `share` more for each tile that a compute unit has on average, and `beside` more where some have two; `once` is
+// start, end and the second kernel's start, `part` what a further part costs it, `sums` what a million partial sums cost to write and to read again. Fitted to
+// 10800 products (512 to 8192 rows of w, k from 512 to 14336, 65 to 1700 rows of x, 2 to 16 parts): what the estimate chooses is 1 % off the best on average,
+// where a rule made at the sizes of the 8B models was 19 % off up to 128 rows, 16 % up to 256, 21 % up to 512 and 13 % beyond. 150
+// products drawn at random afterwards ran 1.34 times as fast up to 128 rows, 1.17 up to 256, 1.13 up to 512, 1.1 beyond (worst: 0.84, two
+// more below 0.92): 4096 rows of w, k = 1024, 100 rows of x 14.5 -> 10.6 us, 1024 rows, k = 3072, 333 rows of x 18.1 -> 13.3, 2048 rows, k = 8192, 100 rows
+// of x 20.8 -> 18.3, 5120 rows, k = 25600, 100 rows of x 85.9 -> 61.6; those of the 8B models stay within 4 % of what they were.
+struct PartTime { int columns, places, once, step, share, beside, part, sums; };
+constexpr PartTime NARROW_PARTS = {64, 2, 5950, 256, 166, 95, 250, 1540}, WIDE_PARTS = {128, 1, 6630, 445, 200, 0, 251, 1720},
+                   WIDE_PARTS_TWO = {128, 2, 7190, 592, 237, 0, 268, 1050};          // (two stages instead of three: two to a compute unit, beyond 256 rows)
+long parts_time(const PartTime& shape, int M, long N, int steps, int parts) {
+    const long groups = (long)((M + 127) / 128) * ((N + shape.columns - 1) / shape.columns) * parts, places = (long)shape.places * XRT_COMPUTE_UNITS;
+    const long whole = groups / places, rest = groups % places;
+    const long full = shape.step + shape.share * shape.places + shape.beside;
+    const long last = rest == 0 ? 0 : shape.step + shape.share * rest / XRT_COMPUTE_UNITS + (rest > XRT_COMPUTE_UNITS ? shape.beside : 0);
+    return shape.once + shape.part * parts + steps * (whole * full + last) + shape.sums * parts * ((long)M * N / 1000) / 1000;
+}
+// The same of the tiles without a split (a fit to the same products: their own estimate counts a warm chip's rounds alone).
+long unsplit_time(int M, int N, int K, int mode) {
+    const int kind = mode == MODE_ACCUMULATE ? ENDS_ADDING : ENDS_BF16;
+    auto cost = [&](const TileTime& tile) { return rounds_cost((long)((M + tile.bm - 1) / tile.bm) * ((N + tile.bn - 1) / tile.bn), tile, K, kind); };
+    return 1000 + min(min(cost(LARGE_TILE), cost(HALF_TILE)), cost(SMALL_TILE)) * 127 / 100;
+}
+
 // whole_norm: an RMSNorm follows that the second kernel can do outright, which is worth a split in two where the product alone
 // would do as well without (k from 4096 on instead of from 8192 on).
 SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
@@ -1103,33 +1128,32 @@ SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
         splits = splits > 8 ? 8 : splits;
         least = 24;
         tile = columns = 256;
-    } else {
-        // Some hundred rows of x: still bound by reading w, and too few tiles to fill the chip without a split.
-        // Every part of k writes its sums and the second kernel reads them again (16 parts of a square w and 128 rows
-        // of x: as many bytes as w has), so the parts are few and long (1024 of k at least), and where tiles of 128 x 128
-        // are fewer than the compute units and k is short, tiles of 128 x 64 make up the number instead of further parts.
-        // With a long k the partial sums are small against w and the wider tile, which reads x half as often, is kept
-        // (at the sizes of the 8B models, 128 rows: q/k/v 31 -> 25 us, o 24 -> 18, down 40 -> 37).
-        // Beyond 256 rows the matrix cores begin to count: tiles of 128 x 128, two to a compute unit, in as many parts as
-        // fill those places.
-        long tiles = (long)((M + 127) / 128) * tiles_n;
+    } else if (mode == MODE_GATED) {
+        // Some hundred rows of x, gated: with a round of tiles or nearly so no split, for the tiles then apply the epilogue themselves.
+        // Beyond 256 rows the workgroups run two to a compute unit: as many parts as still fit those 512 places at once.
+        const long tiles = (long)((M + 127) / 128) * tiles_n;
         tile = columns = 128;
-        if (M <= 256) {
-            if (tiles < XRT_COMPUTE_UNITS && mode != MODE_GATED && K < 8192) {
-                columns = 64;
-                tiles = (long)((M + 127) / 128) * ((rows_w + 63) / 64);
+        splits = M <= 256 ? (tiles >= 200 ? 1 : (int)((XRT_COMPUTE_UNITS + tiles - 1) / tiles)) : (int)(2 * XRT_COMPUTE_UNITS / tiles);
+        least = M <= 256 ? 8 : 4;
+    } else {
+        // Some hundred rows of x: still bound by reading w, and too few tiles to fill the chip without a split. Tiles of 128 x 64 or 128 x 128
+        // and the number of parts by an estimate of the time, against one of the product without a split. (Narrow tiles read x twice as often, which
+        // does not stay in a die's L2 when k is long: 4096 rows of w, k = 14336, 100 rows of x 34.7 us in wide tiles, 40.3 in narrow ones.)
+        const long tiles = (long)((M + 127) / 128) * tiles_n;
+        tile = columns = 128;
+        least = 1;
+        splits = 1;
+        if (tiles <= (M <= 256 ? 2 * XRT_COMPUTE_UNITS : XRT_COMPUTE_UNITS)) {      // (more fill the chip as they are)
+            long best = unsplit_time(M, N, K, mode);
+            for (const PartTime& shape : {NARROW_PARTS, M <= 256 ? WIDE_PARTS : WIDE_PARTS_TWO}) {
+                if (shape.columns == 64 && K >= 8192 && N > 2048) continue;
+                for (int parts = 2; parts <= 16 && parts <= units; ++parts) {
+                    const int per = (units + parts - 1) / parts;
+                    if ((units + per - 1) / per != parts) continue;          // (as many pieces a part with fewer parts)
+                    const long time = parts_time(shape, M, N, per, parts);
+                    if (time < best) { best = time; splits = parts; columns = shape.columns; }
+                }
             }
-            // a gated product with a round of tiles or nearly so does without a split: its tiles apply the epilogue themselves
-            const int target = M <= 128 && columns == 64 ? 2 * XRT_COMPUTE_UNITS : XRT_COMPUTE_UNITS;
-            splits = tiles >= 384 || (mode == MODE_GATED && tiles >= 200) ? 1 : (int)((target + tiles - 1) / tiles);
-            least = columns == 64 ? 16 : 8;
-        } else {
-            // The workgroups run two to a compute unit: as many parts as still fit those 512 places at once, and none where
-            // that is one. A few workgroups over (96 tiles in 6 parts) run a second round for a few; so do parts enough for
-            // two rounds of shorter workgroups, which an estimate by rounds prefers and the clock does not. (The four products
-            // of a layer at 384 rows 295 -> 251 us; q/k/v at 512 rows 54 -> 45 us, at 768 rows 77 -> 65; o at 768 rows 55 -> 47.)
-            splits = (int)(2 * XRT_COMPUTE_UNITS / tiles);
-            least = 4;
         }
     }
     splits = splits < 1 ? 1 : (splits > 16 ? 16 : splits);
