@@ -416,7 +416,10 @@ def test_rmsnorm_done_by_the_products_around_it(ops, m, hidden, k, n, packed):
     assert (again is not None) == (m <= 16)                     # 64 to 127 columns: only the kernel for up to 16 rows writes them
 
 
-@pytest.mark.parametrize("m,hidden,k", [(520, 1032, 4160), (2048, 4096, 4096), (600, 520, 8192), (1024, 8192, 4096)])
+@pytest.mark.parametrize("m,hidden,k", [(520, 1032, 4160), (2048, 4096, 4096), (600, 520, 8192), (1024, 8192, 4096),
+                                        # few rows: smaller tiles, and workgroups of 1024 threads up to 511 rows
+                                        (65, 1024, 512), (100, 2048, 8192), (333, 4096, 14336), (129, 8192, 2048), (200, 264, 3072),
+                                        (511, 1032, 4096), (512, 1032, 4096)])
 @pytest.mark.parametrize("gain_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("packed", [False, True])
 def test_rmsnorm_done_by_the_second_kernel_of_a_product_of_many_rows(ops, m, hidden, k, gain_dtype, packed):
@@ -650,6 +653,40 @@ def test_linear_qkv_in_one_kernel(ops, nh, nkv, hd, rope_dim, k, tokens, packed)
         ops.linear(a, w, want)
         ops.linear(a, plain_w, got)
         assert rel(want.float(), got.float()) < ULP["bfloat16"] * 2
+
+
+@pytest.mark.parametrize("nh,nkv,hd,rope_dim,k,tokens", [(32, 8, 64, 64, 2048, 100), (16, 8, 128, 128, 1024, 65), (32, 8, 128, 128, 4096, 333), (4, 2, 16, 16, 512, 70),
+                                                          (3, 1, 256, 256, 1024, 127), (6, 2, 32, 0, 768, 128), (64, 8, 128, 128, 512, 40),
+                                                          (4, 2, 128, 64, 512, 90), (3, 3, 48, 48, 512, 100)])      # the last two: kernels of their own
+@pytest.mark.parametrize("norm_dtype", [None, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("longest_run", [1, 100])
+@pytest.mark.parametrize("packed", [False, True])
+def test_parts_of_a_qkv_projection_added_by_the_kernel_that_prepares_its_heads(ops, nh, nkv, hd, rope_dim, k, tokens, norm_dtype, longest_run, packed):
+    # against the product and qkv_prepare one after the other: the same sums, roundings and formulas in the same order
+    positions = [0, 63, 64, 5, 1000] + list(range(200, 195 + tokens))
+    slots = [0, 0, 1, -1, 1] + [0] * (tokens - 5)                # one token is padding
+    positions, slots = i32(positions), i32(slots)
+    width = (nh + 2 * nkv) * hd
+    a = rand(tokens, k, dtype=torch.bfloat16, seed=hd)
+    w = rand(width, k, dtype=torch.bfloat16, seed=k, scale=1.0 / math.sqrt(k))
+    w = packed_or_not(ops, w, packed, "rotary", head_dim=hd, rotated_heads=nh + nkv if rope_dim == hd else 0)
+    kv = make_cache(40, nkv, hd, torch.bfloat16, 2, 16)
+    kv.block_table[0, :16] = torch.arange(3, 19, dtype=torch.int32)
+    kv.block_table[1, :16] = torch.arange(39, 23, -1, dtype=torch.int32)
+    theta = (torch.tensor(10000.0) ** (torch.arange(rope_dim // 2) * 2.0 / max(rope_dim, 1))).to(DEV) if rope_dim else None
+    args = dict(rope_theta=theta, rope_dim=rope_dim, rope_scale=0.5, longest_run=longest_run)
+    if norm_dtype is not None:
+        args.update(q_norm=(rand(hd, seed=1) + 1.0).to(norm_dtype), k_norm=(rand(hd, seed=2) + 1.0).to(norm_dtype), norm_eps=1e-4)
+    for with_cache in (True, False):
+        got, want = (torch.full((tokens, width), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        kv_got, kv_want = clone_cache(kv), clone_cache(kv)
+        ops.linear_qkv(a, w, got, nh, nkv, hd, positions, slots, kv=kv_got if with_cache else None, **args)
+        ops.linear(a, w, want)
+        ops.qkv_prepare(want, nh, nkv, hd, positions, slots, kv=kv_want if with_cache else None, **args)
+        # (up to 64 tokens without head norms another kernel's contraction of a multiply-add may differ)
+        same = torch.equal if tokens > 64 or norm_dtype is not None else lambda x, y: rel(x.float(), y.float()) < ULP["bfloat16"]
+        assert same(got, want) and same(kv_got.k, kv_want.k) and torch.equal(kv_got.v, kv_want.v)
+        assert bool((kv_got.v != 0).any()) == with_cache
 
 
 def test_rope_reference_vector_and_pairing(ops):

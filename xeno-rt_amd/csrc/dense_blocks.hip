@@ -59,7 +59,7 @@ struct Step {
         const int takes = then != nullptr && mode == 1 && N % 8 == 0 ? xrt_linear_takes_norm(a.values, w.data, packing, s.dtype, M, N, K, mode) : 0;
         xrt_linear_norm around = {};
         long need = 0;
-        if (takes == 2 && a.squares == nullptr && out_dtype == XRT_F32) {
+        if (takes == 2 && a.squares == nullptr && out_dtype == XRT_F32 && (uintptr_t)out % 16 == 0 && (uintptr_t)then->gain % 16 == 0) {
             around.eps = then->eps;
             around.scaled_out = room->values; around.gain = then->gain; around.gain_dtype = then->dtype;
             *after = Rows{room->values, nullptr, 0, 0.f};

@@ -1281,54 +1281,79 @@ __global__ void __launch_bounds__(256) split_reduce_wide_kernel(const float* __r
 // The second kernel of an accumulating product of many rows that an RMSNorm follows: a workgroup takes a whole row, adds the
 // parts onto the residual and writes the row's norm as well. The norm is the norm kernel's (elementwise.hip) to the bit: the same
 // four columns a thread, the same order of the sum of squares, (x * 1/rms) * gain.
-constexpr int NORM_QUADS = 8;                      // four-column pieces a thread holds: rows of up to 8 * 256 * 4 columns
-template <typename TW>
-__global__ void __launch_bounds__(256) split_reduce_rmsnorm_kernel(const float* __restrict__ parts, int splits, long count, int N,
+constexpr int NORM_THREADS = 256, NORM_QUADS = 8;       // of the norm kernel, and the four-column pieces a thread of it holds: rows of up to 8 * 256 * 4 columns
+// THREADS: 256, or 1024 where the rows are too few to fill the chip with workgroups of 256 (a thread then holds a quarter of the
+// pieces, and 256 threads add up the squares from LDS, in the norm kernel's order).
+// Instead of a kernel that adds the parts and one that norms the rows (3.5 + 3.3 us for 100 rows of 2048, 6.3 + 4.9 for 333 of 4096). With the same for
+// q, k and v (qkv_prepare.hip): logits of 100 tokens at the Llama-3.2-1B sizes 1549 -> 1366 us, 333 tokens on 3001 at the 8B sizes (6 layers) 1706 -> 1623.
+template <typename TW, int THREADS>
+__global__ void __launch_bounds__(THREADS) split_reduce_rmsnorm_kernel(const float* __restrict__ parts, int splits, long count, int N,
                                                                     float* __restrict__ out, const TW* __restrict__ gain, float eps,
                                                                     bf16* __restrict__ normed) {
+    typedef float floatx4 __attribute__((ext_vector_type(4)));
+    constexpr int QUADS = NORM_QUADS * NORM_THREADS / THREADS, AT_ONCE = THREADS == NORM_THREADS ? 1 : 4;     // parts asked for at once
     __shared__ float scratch[32];
+    __shared__ floatx4 row_quads[THREADS == NORM_THREADS ? 1 : NORM_QUADS * NORM_THREADS];
     const long row = (long)blockIdx.x * N;
     const int quads = N / 4;
-    float4 kept[NORM_QUADS];
-    Four<TW> weight[NORM_QUADS];
+    floatx4 kept[QUADS];
+    Four<TW> weight[QUADS];
 #pragma unroll
-    for (int i = 0; i < NORM_QUADS; ++i) {
-        const int q = threadIdx.x + i * 256;
-        kept[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (int i = 0; i < QUADS; ++i) {
+        const int q = threadIdx.x + i * THREADS;
+        kept[i] = floatx4{0.f, 0.f, 0.f, 0.f};
         weight[i] = Four<TW>{};
         if (q < quads) {
             const long index = row + 4L * q;
-            typedef float floatx4 __attribute__((ext_vector_type(4)));
-            const floatx4 first = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(parts + index));     // read once, by nobody else
-            float4 sum = make_float4(first[0], first[1], first[2], first[3]);
-            for (int p = 1; p < splits; ++p) {
-                const floatx4 part = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(parts + p * count + index));
-                sum.x += part[0]; sum.y += part[1]; sum.z += part[2]; sum.w += part[3];
-            }
-            const float4 before = *reinterpret_cast<const float4*>(out + index);
-            kept[i] = make_float4(before.x + sum.x, before.y + sum.y, before.z + sum.z, before.w + sum.w);
-            *reinterpret_cast<float4*>(out + index) = kept[i];
+            const floatx4 before = *reinterpret_cast<const floatx4*>(out + index);
             weight[i] = *reinterpret_cast<const Four<TW>*>(gain + 4 * q);
+            floatx4 sum = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(parts + index));     // read once, by nobody else
+            for (int p0 = 1; p0 < splits; p0 += AT_ONCE) {
+                floatx4 part[AT_ONCE];
+#pragma unroll
+                for (int u = 0; u < AT_ONCE; ++u)
+                    part[u] = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(parts + min(p0 + u, splits - 1) * count + index));
+#pragma unroll
+                for (int u = 0; u < AT_ONCE; ++u)
+                    if (p0 + u < splits) sum += part[u];
+            }
+            kept[i] = before + sum;
+            *reinterpret_cast<floatx4*>(out + index) = kept[i];
         }
     }
     float squares = 0.f;
+    auto add_squares = [&](const floatx4& v) { squares = fmaf(v[0], v[0], fmaf(v[1], v[1], fmaf(v[2], v[2], fmaf(v[3], v[3], squares)))); };
+    if constexpr (THREADS == NORM_THREADS) {
 #pragma unroll
-    for (int i = 0; i < NORM_QUADS; ++i)
-        squares = fmaf(kept[i].x, kept[i].x, fmaf(kept[i].y, kept[i].y, fmaf(kept[i].z, kept[i].z, fmaf(kept[i].w, kept[i].w, squares))));
-    squares = block_sum(squares, scratch);
+        for (int i = 0; i < QUADS; ++i) add_squares(kept[i]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < QUADS; ++i) row_quads[threadIdx.x + i * THREADS] = kept[i];
+        __syncthreads();
+        if (threadIdx.x < NORM_THREADS) {
+#pragma unroll
+            for (int i = 0; i < NORM_QUADS; ++i) add_squares(row_quads[threadIdx.x + i * NORM_THREADS]);
+        }
+    }
+    squares = block_sum(squares, scratch);                     // (wavefronts beyond the norm kernel's four add zeros behind theirs)
     const float inv_rms = 1.0f / sqrtf(squares / (float)N + eps);
 #pragma unroll
-    for (int i = 0; i < NORM_QUADS; ++i) {
-        const int q = threadIdx.x + i * 256;
+    for (int i = 0; i < QUADS; ++i) {
+        const int q = threadIdx.x + i * THREADS;
         if (q < quads) {
             Four<bf16> r;
-            r.e[0] = from_float<bf16>((kept[i].x * inv_rms) * to_float(weight[i].e[0]));
-            r.e[1] = from_float<bf16>((kept[i].y * inv_rms) * to_float(weight[i].e[1]));
-            r.e[2] = from_float<bf16>((kept[i].z * inv_rms) * to_float(weight[i].e[2]));
-            r.e[3] = from_float<bf16>((kept[i].w * inv_rms) * to_float(weight[i].e[3]));
+#pragma unroll
+            for (int e = 0; e < 4; ++e) r.e[e] = from_float<bf16>((kept[i][e] * inv_rms) * to_float(weight[i].e[e]));
             *reinterpret_cast<Four<bf16>*>(normed + row + 4L * q) = r;
         }
     }
+}
+template <typename TW>
+void launch_reduce_rmsnorm(const float* parts, int splits, int M, int N, float* out, const void* gain, float eps, void* normed, hipStream_t s) {
+    if (M < 2 * XRT_COMPUTE_UNITS)
+        split_reduce_rmsnorm_kernel<TW, 1024><<<M, 1024, 0, s>>>(parts, splits, (long)M * N, N, out, (const TW*)gain, eps, (bf16*)normed);
+    else
+        split_reduce_rmsnorm_kernel<TW, NORM_THREADS><<<M, NORM_THREADS, 0, s>>>(parts, splits, (long)M * N, N, out, (const TW*)gain, eps, (bf16*)normed);
 }
 
 // The second kernel of a q/k/v projection split along k (no head norms, the rotation over the whole head):
@@ -1398,6 +1423,20 @@ __global__ void __launch_bounds__(256) split_reduce_qkv_kernel(const float* __re
     }
 }
 
+// The product of all rows of w, ungated, into the workspace: [splits][M][rows_w]
+int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, const Packing& packing, const SplitPlan& plan, hipStream_t s) {
+    const int rows_w = (int)plan.rows_w;
+    if (M <= SPLIT_BM)
+        return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+    if (plan.tile == 256)
+        return launch_large<256, MODE_STORE, float>(a, w, workspace, M, rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split);
+    if (plan.columns == 64)
+        return launch_kernel<128, 64, 2, 2, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+    if (M <= 256)           // (one workgroup to a compute unit anyway: a third stage keeps more of w on its way; with more, two share a unit)
+        return launch_kernel<128, 128, 2, 2, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+    return launch_kernel<128, 128, 2, 2, MODE_STORE, 64, 2, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+}
+
 template <typename TO>
 int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int mode, int activation, const Packing& packing,
                  float* workspace, const xrt_linear_norm* norm, const QkvAfter* after, hipStream_t s) {
@@ -1407,7 +1446,7 @@ int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int
     const bool scaled = norm && norm->squares_in, emits = norm && norm->squares_out;
     XRT_REQUIRE(!norm || M <= SPLIT_BM || whole_norm, "linear (mfma): the halves of a norm around a product take at most %d rows here", SPLIT_BM);
     if (whole_norm)
-        XRT_REQUIRE(M > SPLIT_BM && mode == MODE_ACCUMULATE && sizeof(TO) == 4 && plan.tile == 256 && plan.splits > 1 && N % 4 == 0 &&
+        XRT_REQUIRE(M > SPLIT_BM && mode == MODE_ACCUMULATE && sizeof(TO) == 4 && plan.splits > 1 && N % 4 == 0 &&
                     N <= NORM_QUADS * 256 * 4 && norm->gain && (uintptr_t)out % 16 == 0 && (uintptr_t)norm->scaled_out % 8 == 0,
                     "linear (mfma): M=%d N=%d K=%d is not a product whose second kernel does the norm after it", M, N, K);
     const RowScale scale = scaled ? RowScale{norm->squares_in, norm->tiles_in, norm->width_in, norm->eps, activation}
@@ -1423,21 +1462,7 @@ int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int
         XRT_REQUIRE(false, "linear (mfma): accumulation needs a float32 output");
     }
     XRT_REQUIRE(workspace != nullptr, "linear (mfma): a product split along k needs its workspace");
-    // the product of all rows of w, ungated, into the workspace: [splits][M][rows_w]
-    const int status = M <= SPLIT_BM
-        ? launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, float>(
-              a, w, workspace, M, (int)plan.rows_w, K, packing, s, plan.splits, plan.k_per_split)
-        : plan.tile == 256
-        ? launch_large<256, MODE_STORE, float>(a, w, workspace, M, (int)plan.rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split)
-        : plan.columns == 64
-        ? launch_kernel<128, 64, 2, 2, MODE_STORE, 64, 3, float>(
-              a, w, workspace, M, (int)plan.rows_w, K, packing, s, plan.splits, plan.k_per_split)
-        : M <= 256          // (one workgroup to a compute unit anyway: a third stage keeps more of w on its way; with more, two share a unit)
-        ? launch_kernel<128, 128, 2, 2, MODE_STORE, 64, 3, float>(
-              a, w, workspace, M, (int)plan.rows_w, K, packing, s, plan.splits, plan.k_per_split)
-        : launch_kernel<128, 128, 2, 2, MODE_STORE, 64, 2, float>(
-              a, w, workspace, M, (int)plan.rows_w, K, packing, s, plan.splits, plan.k_per_split);
-    if (status != 0) return status;
+    if (launch_parts(a, w, workspace, M, K, packing, plan, s) != 0) return 1;
     const unsigned blocks = (unsigned)(((long)M * N + 255) / 256);
     const xrt_linear_norm none = {};
     const xrt_linear_norm& around = norm ? *norm : none;
@@ -1453,11 +1478,8 @@ int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int
     }
     if (whole_norm) {
         if constexpr (sizeof(TO) == 4) {
-            const long count = (long)M * N;
-            if (norm->gain_dtype == XRT_F32)
-                split_reduce_rmsnorm_kernel<float><<<M, 256, 0, s>>>(workspace, plan.splits, count, N, out, (const float*)norm->gain, norm->eps, (bf16*)norm->scaled_out);
-            else
-                split_reduce_rmsnorm_kernel<bf16><<<M, 256, 0, s>>>(workspace, plan.splits, count, N, out, (const bf16*)norm->gain, norm->eps, (bf16*)norm->scaled_out);
+            if (norm->gain_dtype == XRT_F32) launch_reduce_rmsnorm<float>(workspace, plan.splits, M, N, out, norm->gain, norm->eps, norm->scaled_out, s);
+            else launch_reduce_rmsnorm<bf16>(workspace, plan.splits, M, N, out, norm->gain, norm->eps, norm->scaled_out, s);
             XRT_LAUNCH_CHECK("linear (split reduce with the norm after it)");
         }
         return 0;
@@ -1539,16 +1561,15 @@ bool xrt_linear_split_takes(const void* a, const void* w, int M, int N, int K, i
     return true;
 }
 
-// Whether an accumulating product of many rows runs as large tiles that split k, so that its second kernel can do the
-// RMSNorm that follows it outright; and the floats of workspace it then needs. (With the smaller tiles' few rows the
-// kernel that takes a row per workgroup has too few workgroups: 5.75 against 5.65 ms a prompt of 128 tokens.)
+// Whether an accumulating product of more than 64 rows runs as tiles that split k, so that its second kernel can do the
+// RMSNorm that follows it outright; and the floats of workspace it then needs.
 bool xrt_linear_split_takes_whole_norm(const void* a, const void* w, int M, int N, int K, int mode, long* workspace_floats) {
     *workspace_floats = 0;
     if (mode != MODE_ACCUMULATE || M <= SPLIT_BM || K % 64 != 0 || N % 4 != 0 || N > NORM_QUADS * 256 * 4 ||
         !xrt_linear_mfma_accepts(a, w, M, N, K, mode))
         return false;
     const SplitPlan plan = split_plan(M, N, K, mode, true);
-    if (plan.tile != 256 || plan.splits < 2 || (long)M * N >= (1L << 31)) return false;
+    if (plan.splits < 2 || (long)M * N >= (1L << 31)) return false;
     *workspace_floats = (long)plan.splits * M * N;
     return true;
 }
@@ -1581,4 +1602,11 @@ bool xrt_linear_split_takes_qkv(const void* a, const void* w, int M, int N, int 
 int xrt_linear_split_qkv(const void* a, const void* w, void* qkv, int M, int N, int K, const Packing& packing, float* workspace,
                          const xrt_linear_norm* norm, const QkvAfter& after, hipStream_t s) {
     return launch_split<bf16>((const bf16*)a, (const bf16*)w, (bf16*)qkv, M, N, K, MODE_STORE, XRT_ACT_SILU, packing, workspace, norm, &after, s);
+}
+
+// The first kernel alone of a bfloat16 product split along k (xrt_linear_split_takes says so and asks for a workspace): the sums of the parts,
+// [parts][M][N], for a kernel that adds them itself. Returns the number of parts, or 0 on failure.
+int xrt_linear_split_parts(const void* a, const void* w, int M, int N, int K, const Packing& packing, float* workspace, hipStream_t s) {
+    const SplitPlan plan = split_plan(M, N, K, MODE_STORE);
+    return launch_parts((const bf16*)a, (const bf16*)w, workspace, M, K, packing, plan, s) == 0 ? plan.splits : 0;
 }

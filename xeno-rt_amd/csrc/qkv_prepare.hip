@@ -7,13 +7,15 @@
 // (i, i + rope_dim/2), d[i] = a cos - b sin, d[i + half] = a sin + b cos; elements beyond
 // rope_dim stay. Norm, angle, sine, cosine and rotation are float32.
 //
-// Three kernels. The vector kernel takes the usual case (the rotation spans the whole head, and
+// Two kernels. The vector kernel takes the usual case (the rotation spans the whole head, and
 // the head size is 16 bytes times a power of two, twice): the lanes of a head each hold 16 bytes
 // of its lower and of its upper half, which are each other's partners in the rotation, so a
 // head is read and written in 16-byte pieces and the norm's sum is a few lane exchanges. When a
-// step brings many tokens, the values go to their transposed cache blocks through a kernel of
-// their own, which turns tiles of 64 tokens in LDS so that writes to the cache are whole lines.
+// step brings many tokens, the values go to their transposed cache blocks through workgroups of
+// their own, which turn tiles of 64 tokens in LDS so that writes to the cache are whole lines.
 // Where a key or a value lies inside its block: cache_layout.h.
+// A projection that was split along k comes as the float32 sums of its parts (PARTS): the vector kernel then adds
+// them, in order, and rounds them to bfloat16 as the kernel that adds them alone does, before it goes on as ever.
 // The general kernel (one wavefront per (token, head), any even head size and rotation width)
 // takes the rest. A token with a negative slot is padding and is not cached. Per head, all
 // kernels use the same formulas in the same order; only the order of the norm's sum differs,
@@ -100,23 +102,128 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) qkv_prepare_kernel(
 
 template <typename T, int N> struct alignas(sizeof(T) * N) Pack { T e[N]; };
 
-// One workgroup per token. LANES lanes per head; head_dim = 2 * LANES * VEC with VEC elements in
+// The parts of a projection split along k: part p of element i at values[p * stride + i]. splits 0: there are none.
+struct QkvParts { const float* values; long stride; int splits; };
+
+// 16 bytes of a row of q/k/v. `at` counts elements from the first row's first.
+template <bool PARTS, typename T>
+__device__ __forceinline__ Pack<T, 16 / (int)sizeof(T)> read_qkv(const T* qkv, const QkvParts& parts, long at) {
+    if constexpr (!PARTS) {
+        return *reinterpret_cast<const Pack<T, 16 / (int)sizeof(T)>*>(qkv + at);
+    } else {
+        static_assert(sizeof(T) == 2, "parts are rounded to bfloat16");
+        constexpr int AT_ONCE = 4;                             // parts asked for at once (those beyond the last: that one again)
+        float4 low = make_float4(0.f, 0.f, 0.f, 0.f), high = low;
+        for (int p0 = 0; p0 < parts.splits; p0 += AT_ONCE) {
+            float4 a[AT_ONCE], b[AT_ONCE];
+#pragma unroll
+            for (int u = 0; u < AT_ONCE; ++u) {
+                const float* from = parts.values + min(p0 + u, parts.splits - 1) * parts.stride + at;
+                a[u] = *reinterpret_cast<const float4*>(from);
+                b[u] = *reinterpret_cast<const float4*>(from + 4);
+            }
+#pragma unroll
+            for (int u = 0; u < AT_ONCE; ++u) {
+                if (p0 + u >= parts.splits) continue;
+                low.x += a[u].x; low.y += a[u].y; low.z += a[u].z; low.w += a[u].w;
+                high.x += b[u].x; high.y += b[u].y; high.z += b[u].z; high.w += b[u].w;
+            }
+        }
+        Pack<T, 8> out;
+        out.e[0] = from_float<T>(low.x); out.e[1] = from_float<T>(low.y); out.e[2] = from_float<T>(low.z); out.e[3] = from_float<T>(low.w);
+        out.e[4] = from_float<T>(high.x); out.e[5] = from_float<T>(high.y); out.e[6] = from_float<T>(high.z); out.e[7] = from_float<T>(high.w);
+        return out;
+    }
+}
+
+// 32 dims of the values of 64 consecutive tokens of a step and one key/value head: read row by row (a piece a thread), turned in
+// LDS, and written so that a store instruction of a wavefront takes 8 tokens of 8 dims: where the
+// tokens follow each other in a sequence these are the eight pieces of one line of the cache block
+// (cache_layout.h). Tokens of different sequences or blocks may share a tile: every token has its
+// own block.
+constexpr int TILE_DIMS = 32;
+// A store step reads 8 tokens (rows) x 8 dims: with rows of 40 elements the 8 rows start at banks 0, 20, 40, .. (bfloat16) or
+// 0, 40, 80, .. (float32) of the 64, and the step's 32 or 64 words lie in as many banks.
+template <typename T> struct ValueTile {
+    T tile[XRT_WAVE][TILE_DIMS + 8];
+    long bases[XRT_WAVE];                                             // of the tile's tokens: their block (-1: none) ...
+    int withins[XRT_WAVE];                                            // ... and their place in it
+};
+template <typename T, bool PARTS>
+__device__ __forceinline__ void write_values(
+    ValueTile<T>& shared, int first, int kv_head, int d0, T* __restrict__ qkv, const QkvParts& parts, int tokens, int n_heads, int n_kv_heads, int head_dim,
+    const int* __restrict__ positions, const int* __restrict__ slots, T* __restrict__ v_cache,
+    const int* __restrict__ block_table, int table_stride, int n_blocks) {
+    const int wave = threadIdx.x / XRT_WAVE, lane = threadIdx.x % XRT_WAVE;
+    const int heads_total = n_heads + 2 * n_kv_heads;
+    if (wave == 0) {
+        const int token = first + lane;
+        long cache_base = -1;
+        int within = 0;
+        if (token < tokens) {
+            const int pos = positions[token];
+            cache_base = cache_block_base(block_table, table_stride, n_blocks, slots[token], pos, n_kv_heads, kv_head, head_dim);
+            within = pos % XRT_BLOCK_TOKENS;
+        }
+        shared.bases[lane] = cache_base;
+        shared.withins[lane] = within;
+    }
+    const long source = (long)(n_heads + n_kv_heads + kv_head) * head_dim;
+    constexpr int VEC = 16 / (int)sizeof(T);                  // the launcher sends only head sizes that are multiples of this
+    const int dims = min(TILE_DIMS, head_dim - d0);
+    const int pieces = dims / VEC;                            // 16-byte pieces per row
+    for (int i = threadIdx.x; i < XRT_WAVE * pieces; i += WAVES * XRT_WAVE) {
+        const int r = i / pieces, d = (i % pieces) * VEC;
+        const long from = min(first + r, tokens - 1);         // rows past the end repeat the last one; nobody writes them to the cache
+        const long at = source + from * heads_total * head_dim + d0 + d;
+        const Pack<T, VEC> piece = read_qkv<PARTS>(qkv, parts, at);
+        if constexpr (PARTS) if (first + r < tokens) *reinterpret_cast<Pack<T, VEC>*>(qkv + at) = piece;
+        *reinterpret_cast<Pack<T, VEC>*>(&shared.tile[r][d]) = piece;
+    }
+    __syncthreads();
+    // a store of a wavefront: tokens 8 g .. 8 g + 7 of the tile (lane % 8), dims 8 h .. 8 h + 7 (lane / 8);
+    // a wavefront keeps its tokens while it walks the dims
+    for (int g = wave; g < XRT_WAVE / 8; g += WAVES) {
+        const int token = g * 8 + lane % 8;
+        const long cache_base = shared.bases[token];
+        const int within = shared.withins[token];
+        if (cache_base < 0) continue;
+#pragma unroll 4
+        for (int d = lane / 8; d < dims; d += 8)
+            v_cache[cache_base + cache_value_offset(d0 + d, within, head_dim)] = shared.tile[token][d];
+    }
+}
+
+// The first value_tiles * n_kv_heads * (pieces of 32 dims) workgroups turn values (none of them: the others write the values themselves); then
+// come `chunks` workgroups per token. LANES lanes per head; head_dim = 2 * LANES * VEC with VEC elements in
 // 16 bytes. Sine and cosine of the token's angles are worked out once, into LDS, and serve all
-// its heads.
-template <typename T, typename TW, int LANES>
+// the workgroup's heads.
+// One launch for both: as kernels of their own, values after heads, they took 11.5 + 6.1 us (2048 tokens, 32 heads of 128 on 8) and 3.3 + 4.1
+// (100 tokens, 32 heads of 64 on 8).
+template <typename T, typename TW, int LANES, bool PARTS>
 __global__ void __launch_bounds__(WAVES * XRT_WAVE) qkv_prepare_vector_kernel(
-    T* __restrict__ qkv, int n_heads, int n_kv_heads,
+    T* __restrict__ qkv, const QkvParts parts, int tokens, int n_heads, int n_kv_heads,
     const int* __restrict__ positions, const int* __restrict__ slots,
     const TW* __restrict__ q_norm, const TW* __restrict__ k_norm, float norm_eps,
     const float* __restrict__ rope_theta, float rope_scale,
     T* __restrict__ k_cache, T* __restrict__ v_cache, const int* __restrict__ block_table,
-    int table_stride, int n_blocks, int write_values) {
+    int table_stride, int n_blocks, int value_tiles, int chunks) {
     constexpr int VEC = 16 / (int)sizeof(T);
     constexpr int HALF = LANES * VEC, HEAD = 2 * HALF;
     constexpr int HEADS_PER_WAVE = XRT_WAVE / LANES;
-    __shared__ float cosines[HALF], sines[HALF];
+    __shared__ __attribute__((aligned(16))) union { struct { float cosines[HALF], sines[HALF]; } angles; ValueTile<T> values; } shared;
+    constexpr int PIECES = (HEAD + TILE_DIMS - 1) / TILE_DIMS;
+    const int value_blocks = value_tiles * n_kv_heads * PIECES;
+    if ((int)blockIdx.x < value_blocks) {
+        write_values<T, PARTS>(shared.values, (int)blockIdx.x / PIECES % value_tiles * XRT_WAVE, (int)blockIdx.x / PIECES / value_tiles,
+                               (int)blockIdx.x % PIECES * TILE_DIMS, qkv, parts, tokens, n_heads, n_kv_heads, HEAD, positions, slots, v_cache, block_table, table_stride, n_blocks);
+        return;
+    }
+    float* cosines = shared.angles.cosines;
+    float* sines = shared.angles.sines;
     const int wave = threadIdx.x / XRT_WAVE, lane = threadIdx.x % XRT_WAVE;
-    const int token = blockIdx.x;
+    const int item = (int)blockIdx.x - value_blocks;
+    const int token = item / chunks, chunk = item % chunks;
     const int pos = positions[token];
     const int slot = slots[token];
     if (rope_theta != nullptr) {
@@ -129,18 +236,23 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) qkv_prepare_vector_kernel(
     const int at = (lane % LANES) * VEC;           // this lane's elements: at.. in the lower half, HALF + at.. in the upper
     const int heads_total = n_heads + 2 * n_kv_heads;
     const int within = pos % XRT_BLOCK_TOKENS;
-    const int heads_here = write_values ? heads_total : n_heads + n_kv_heads;     // value heads come last
-    for (int head = wave * HEADS_PER_WAVE + lane / LANES; head < heads_here; head += WAVES * HEADS_PER_WAVE) {
+    const int heads_here = value_blocks == 0 ? heads_total : n_heads + n_kv_heads;     // value heads come last
+    for (int head = (chunk * WAVES + wave) * HEADS_PER_WAVE + lane / LANES; head < heads_here; head += chunks * WAVES * HEADS_PER_WAVE) {
         // lanes of one head stay together: the exchanges below are within a head
         const bool is_q = head < n_heads, is_v = head >= n_heads + n_kv_heads, is_k = !is_q && !is_v;
-        T* row = qkv + (long)token * heads_total * HEAD + (long)head * HEAD;
-        const Pack<T, VEC> lower = *reinterpret_cast<const Pack<T, VEC>*>(row + at);
-        const Pack<T, VEC> upper = *reinterpret_cast<const Pack<T, VEC>*>(row + HALF + at);
+        const long row_at = (long)token * heads_total * HEAD + (long)head * HEAD;
+        T* row = qkv + row_at;
+        const Pack<T, VEC> lower = read_qkv<PARTS>(qkv, parts, row_at + at);
+        const Pack<T, VEC> upper = read_qkv<PARTS>(qkv, parts, row_at + HALF + at);
         long cache_base = -1;
         if (!is_q && k_cache != nullptr)
             cache_base = cache_block_base(block_table, table_stride, n_blocks, slot, pos, n_kv_heads,
                                           head - n_heads - (is_v ? n_kv_heads : 0), HEAD);
         if (is_v) {
+            if constexpr (PARTS) {
+                *reinterpret_cast<Pack<T, VEC>*>(row + at) = lower;
+                *reinterpret_cast<Pack<T, VEC>*>(row + HALF + at) = upper;
+            }
             if (cache_base >= 0) {
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
@@ -189,63 +301,6 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) qkv_prepare_vector_kernel(
     }
 }
 
-// Values of 64 consecutive tokens of a step and one key/value head: read row by row, turned in
-// LDS, and written so that a store instruction of a wavefront takes 8 tokens of 8 dims: where the
-// tokens follow each other in a sequence these are the eight pieces of one line of the cache block
-// (cache_layout.h). Tokens of different sequences or blocks may share a tile: every token has its
-// own block.
-constexpr int TILE_DIMS = 128;
-template <typename T>
-__global__ void __launch_bounds__(WAVES * XRT_WAVE) value_cache_write_kernel(
-    const T* __restrict__ qkv, int tokens, int n_heads, int n_kv_heads, int head_dim,
-    const int* __restrict__ positions, const int* __restrict__ slots, T* __restrict__ v_cache,
-    const int* __restrict__ block_table, int table_stride, int n_blocks) {
-    // A store step reads 8 tokens (rows) x 8 dims: with rows 8 elements longer than a multiple of 256 bytes the 8 rows
-    // start 4 (bfloat16) or 8 (float32) banks apart, and the step's 32 or 64 words lie in as many banks.
-    __shared__ __attribute__((aligned(16))) T tile[XRT_WAVE][TILE_DIMS + 8];
-    __shared__ long bases[XRT_WAVE];                                  // of the tile's tokens: their block (-1: none) ...
-    __shared__ int withins[XRT_WAVE];                                 // ... and their place in it
-    const int wave = threadIdx.x / XRT_WAVE, lane = threadIdx.x % XRT_WAVE;
-    const int first = blockIdx.x * XRT_WAVE, kv_head = blockIdx.y;
-    const int heads_total = n_heads + 2 * n_kv_heads;
-    if (wave == 0) {
-        const int token = first + lane;
-        long cache_base = -1;
-        int within = 0;
-        if (token < tokens) {
-            const int pos = positions[token];
-            cache_base = cache_block_base(block_table, table_stride, n_blocks, slots[token], pos, n_kv_heads, kv_head, head_dim);
-            within = pos % XRT_BLOCK_TOKENS;
-        }
-        bases[lane] = cache_base;
-        withins[lane] = within;
-    }
-    const T* source = qkv + (long)(n_heads + n_kv_heads + kv_head) * head_dim;
-    constexpr int VEC = 16 / (int)sizeof(T);                  // the launcher sends only head sizes that are multiples of this
-    for (int d0 = 0; d0 < head_dim; d0 += TILE_DIMS) {
-        const int dims = min(TILE_DIMS, head_dim - d0);
-        const int pieces = dims / VEC;                        // 16-byte pieces per row
-        for (int i = threadIdx.x; i < XRT_WAVE * pieces; i += WAVES * XRT_WAVE) {
-            const int r = i / pieces, d = (i % pieces) * VEC;
-            const long from = min(first + r, tokens - 1);     // rows past the end repeat the last one; nobody writes them
-            *reinterpret_cast<Pack<T, VEC>*>(&tile[r][d]) = *reinterpret_cast<const Pack<T, VEC>*>(source + from * heads_total * head_dim + d0 + d);
-        }
-        __syncthreads();
-        // a store of a wavefront: tokens 8 g .. 8 g + 7 of the tile (lane % 8), dims 8 h .. 8 h + 7 (lane / 8);
-        // a wavefront keeps its tokens while it walks the dims
-        for (int g = wave; g < XRT_WAVE / 8; g += WAVES) {
-            const int token = g * 8 + lane % 8;
-            const long cache_base = bases[token];
-            const int within = withins[token];
-            if (cache_base < 0) continue;
-#pragma unroll 4
-            for (int d = lane / 8; d < dims; d += 8)
-                v_cache[cache_base + cache_value_offset(d0 + d, within, head_dim)] = tile[token][d];
-        }
-        __syncthreads();
-    }
-}
-
 __global__ void __launch_bounds__(256) rope_table_kernel(const float* __restrict__ rope_theta, int half, float rope_scale,
                                                          long entries, float2* __restrict__ table) {
     const long index = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -268,11 +323,24 @@ extern "C" int xrt_rope_table(const float* rope_theta, int rope_dim, float rope_
     return 0;
 }
 
-extern "C" int xrt_qkv_prepare(void* qkv, int dtype, int tokens, int n_heads, int n_kv_heads, int head_dim,
-                               const int* positions, const int* slots, const void* q_norm, const void* k_norm,
-                               int norm_dtype, float norm_eps, const float* rope_theta, int rope_dim,
-                               float rope_scale, void* k_cache, void* v_cache, const int* block_table,
-                               int table_stride, int n_blocks, int longest_run, void* stream) {
+// What the vector kernel takes: rotation over the whole head (or none), 16-byte pieces, a power of two of lanes per head.
+static int vector_lanes(const void* qkv, int dtype, int head_dim, const float* rope_theta, int rope_dim, const void* k_cache) {
+    const int vec = dtype == XRT_F32 ? 4 : 8;
+    const int lanes = head_dim % (2 * vec) == 0 ? head_dim / (2 * vec) : 0;
+    return lanes >= 1 && lanes <= XRT_WAVE && (lanes & (lanes - 1)) == 0 && (rope_theta == nullptr || rope_dim == head_dim) &&
+           (uintptr_t)qkv % 16 == 0 && (k_cache == nullptr || (uintptr_t)k_cache % 16 == 0) ? lanes : 0;
+}
+
+// Whether xrt_qkv_prepare_parts takes the sums of a projection's parts (bfloat16 results).
+bool xrt_qkv_prepare_takes_parts(const void* qkv, const float* parts, int head_dim, const float* rope_theta, int rope_dim, const void* k_cache) {
+    return (uintptr_t)parts % 16 == 0 && vector_lanes(qkv, XRT_BF16, head_dim, rope_theta, rope_dim, k_cache) > 0;
+}
+
+static int prepare(void* qkv, const QkvParts& parts, int dtype, int tokens, int n_heads, int n_kv_heads, int head_dim,
+                   const int* positions, const int* slots, const void* q_norm, const void* k_norm,
+                   int norm_dtype, float norm_eps, const float* rope_theta, int rope_dim,
+                   float rope_scale, void* k_cache, void* v_cache, const int* block_table,
+                   int table_stride, int n_blocks, int longest_run, void* stream) {
     XRT_REQUIRE(tokens >= 0 && n_heads > 0 && n_kv_heads > 0, "qkv_prepare: bad head counts %d/%d", n_heads, n_kv_heads);
     XRT_REQUIRE(head_dim > 0 && head_dim % 2 == 0 && head_dim <= MAX_HEAD_DIM,
                 "qkv_prepare: head_dim %d must be even and at most %d", head_dim, MAX_HEAD_DIM);
@@ -287,53 +355,47 @@ extern "C" int xrt_qkv_prepare(void* qkv, int dtype, int tokens, int n_heads, in
     if (tokens == 0) return 0;
     const long items = (long)tokens * (n_heads + 2 * n_kv_heads);
     hipStream_t s = (hipStream_t)stream;
-    // the vector kernel: rotation over the whole head (or none), 16-byte pieces, a power of two of lanes per head
-    const int vec = dtype == XRT_F32 ? 4 : 8;
-    const int lanes = head_dim % (2 * vec) == 0 ? head_dim / (2 * vec) : 0;
-    const bool vector = lanes >= 1 && lanes <= XRT_WAVE && (lanes & (lanes - 1)) == 0 &&
-                        (rope_theta == nullptr || rope_dim == head_dim) && (uintptr_t)qkv % 16 == 0 &&
-                        (k_cache == nullptr || ((uintptr_t)k_cache % 16 == 0));
-    if (vector) {
-        // sequences that bring many tokens: their values go through the transposing kernel;
-        // otherwise element by element from this one
+    const int lanes = vector_lanes(qkv, dtype, head_dim, rope_theta, rope_dim, k_cache);
+    if (lanes > 0) {
+        // sequences that bring many tokens: their values go through the workgroups that turn them;
+        // otherwise element by element from those that do the heads
         const bool values_apart = v_cache != nullptr && longest_run >= XRT_WAVE / 2;
-        const unsigned grid = (unsigned)tokens;
-#define XRT_VEC(T, TW, L)                                                                                  \
-    qkv_prepare_vector_kernel<T, TW, L><<<grid, WAVES * XRT_WAVE, 0, s>>>(                                 \
-        (T*)qkv, n_heads, n_kv_heads, positions, slots, (const TW*)q_norm, (const TW*)k_norm,              \
+        const int value_tiles = values_apart ? (tokens + XRT_WAVE - 1) / XRT_WAVE : 0;
+        // a workgroup per token, which walks the heads; with parts, whose sums have a long way, as many as the heads fill
+        const int heads = n_heads + (values_apart ? 1 : 2) * n_kv_heads, heads_at_once = WAVES * (XRT_WAVE / lanes);
+        const int chunks = parts.splits > 0 ? (heads + heads_at_once - 1) / heads_at_once : 1;
+        const long blocks = (long)value_tiles * n_kv_heads * ((head_dim + TILE_DIMS - 1) / TILE_DIMS) + (long)tokens * chunks;
+        XRT_REQUIRE(blocks < (1L << 31), "qkv_prepare: too many workgroups");
+        const unsigned grid = (unsigned)blocks;
+#define XRT_VEC(T, TW, L, PARTS)                                                                           \
+    qkv_prepare_vector_kernel<T, TW, L, PARTS><<<grid, WAVES * XRT_WAVE, 0, s>>>(                          \
+        (T*)qkv, parts, tokens, n_heads, n_kv_heads, positions, slots, (const TW*)q_norm, (const TW*)k_norm, \
         norm_eps, rope_theta, rope_scale, (T*)k_cache, (T*)v_cache, block_table, table_stride, n_blocks,   \
-        values_apart ? 0 : 1)
-#define XRT_VEC_LANES(T, TW)                                                                               \
+        value_tiles, chunks)
+#define XRT_VEC_LANES(T, TW, PARTS)                                                                        \
     switch (lanes) {                                                                                       \
-        case 1: XRT_VEC(T, TW, 1); break;                                                                  \
-        case 2: XRT_VEC(T, TW, 2); break;                                                                  \
-        case 4: XRT_VEC(T, TW, 4); break;                                                                  \
-        case 8: XRT_VEC(T, TW, 8); break;                                                                  \
-        case 16: XRT_VEC(T, TW, 16); break;                                                                \
-        case 32: XRT_VEC(T, TW, 32); break;                                                                \
-        default: XRT_VEC(T, TW, 64); break;                                                                \
+        case 1: XRT_VEC(T, TW, 1, PARTS); break;                                                           \
+        case 2: XRT_VEC(T, TW, 2, PARTS); break;                                                           \
+        case 4: XRT_VEC(T, TW, 4, PARTS); break;                                                           \
+        case 8: XRT_VEC(T, TW, 8, PARTS); break;                                                           \
+        case 16: XRT_VEC(T, TW, 16, PARTS); break;                                                         \
+        case 32: XRT_VEC(T, TW, 32, PARTS); break;                                                         \
+        default: XRT_VEC(T, TW, 64, PARTS); break;                                                         \
     }
-        if (dtype == XRT_F32 && norm_dtype == XRT_F32) { XRT_VEC_LANES(float, float) }
-        else if (dtype == XRT_F32) { XRT_VEC_LANES(float, bf16) }
-        else if (norm_dtype == XRT_F32) { XRT_VEC_LANES(bf16, float) }
-        else { XRT_VEC_LANES(bf16, bf16) }
+        if (parts.splits > 0) {
+            XRT_REQUIRE(dtype == XRT_BF16, "qkv_prepare: the parts of a projection become bfloat16");
+            if (norm_dtype == XRT_F32) { XRT_VEC_LANES(bf16, float, true) }
+            else { XRT_VEC_LANES(bf16, bf16, true) }
+        } else if (dtype == XRT_F32 && norm_dtype == XRT_F32) { XRT_VEC_LANES(float, float, false) }
+        else if (dtype == XRT_F32) { XRT_VEC_LANES(float, bf16, false) }
+        else if (norm_dtype == XRT_F32) { XRT_VEC_LANES(bf16, float, false) }
+        else { XRT_VEC_LANES(bf16, bf16, false) }
 #undef XRT_VEC_LANES
 #undef XRT_VEC
         XRT_LAUNCH_CHECK("qkv_prepare");
-        if (values_apart) {
-            const dim3 tiles((unsigned)((tokens + XRT_WAVE - 1) / XRT_WAVE), (unsigned)n_kv_heads);
-            if (dtype == XRT_F32)
-                value_cache_write_kernel<float><<<tiles, WAVES * XRT_WAVE, 0, s>>>(
-                    (const float*)qkv, tokens, n_heads, n_kv_heads, head_dim, positions, slots, (float*)v_cache,
-                    block_table, table_stride, n_blocks);
-            else
-                value_cache_write_kernel<bf16><<<tiles, WAVES * XRT_WAVE, 0, s>>>(
-                    (const bf16*)qkv, tokens, n_heads, n_kv_heads, head_dim, positions, slots, (bf16*)v_cache,
-                    block_table, table_stride, n_blocks);
-            XRT_LAUNCH_CHECK("qkv_prepare (values)");
-        }
         return 0;
     }
+    XRT_REQUIRE(parts.splits == 0, "qkv_prepare: heads of %d dims take no parts of a projection", head_dim);
     const unsigned grid = (unsigned)((items + WAVES - 1) / WAVES);
 #define XRT_PREP(T, TW)                                                                                   \
     qkv_prepare_kernel<T, TW><<<grid, WAVES * XRT_WAVE, 0, s>>>(                                          \
@@ -347,4 +409,25 @@ extern "C" int xrt_qkv_prepare(void* qkv, int dtype, int tokens, int n_heads, in
 #undef XRT_PREP
     XRT_LAUNCH_CHECK("qkv_prepare");
     return 0;
+}
+
+extern "C" int xrt_qkv_prepare(void* qkv, int dtype, int tokens, int n_heads, int n_kv_heads, int head_dim,
+                               const int* positions, const int* slots, const void* q_norm, const void* k_norm,
+                               int norm_dtype, float norm_eps, const float* rope_theta, int rope_dim,
+                               float rope_scale, void* k_cache, void* v_cache, const int* block_table,
+                               int table_stride, int n_blocks, int longest_run, void* stream) {
+    return prepare(qkv, QkvParts{nullptr, 0, 0}, dtype, tokens, n_heads, n_kv_heads, head_dim, positions, slots, q_norm, k_norm, norm_dtype, norm_eps,
+                   rope_theta, rope_dim, rope_scale, k_cache, v_cache, block_table, table_stride, n_blocks, longest_run, stream);
+}
+
+// The same for a bfloat16 projection that comes as `splits` parts of tokens x (all heads' dims) float32 sums, one after another.
+int xrt_qkv_prepare_parts(const float* parts, int splits, void* qkv, int tokens, int n_heads, int n_kv_heads, int head_dim,
+                          const int* positions, const int* slots, const void* q_norm, const void* k_norm,
+                          int norm_dtype, float norm_eps, const float* rope_theta, int rope_dim,
+                          float rope_scale, void* k_cache, void* v_cache, const int* block_table,
+                          int table_stride, int n_blocks, int longest_run, void* stream) {
+    XRT_REQUIRE(parts != nullptr && splits > 0, "qkv_prepare: no parts");
+    return prepare(qkv, QkvParts{parts, (long)tokens * (n_heads + 2 * n_kv_heads) * head_dim, splits}, XRT_BF16, tokens, n_heads, n_kv_heads, head_dim,
+                   positions, slots, q_norm, k_norm, norm_dtype, norm_eps, rope_theta, rope_dim, rope_scale, k_cache, v_cache, block_table, table_stride,
+                   n_blocks, longest_run, stream);
 }

@@ -435,8 +435,8 @@ class HipOps:
         # over the n columns it writes, can take it
         emit = None
         takes = int(self.lib.xrt_linear_takes_norm(*packed, m, n, k, mode)) if then_norm is not None and mode == 1 and n % 8 == 0 else 0
-        if takes == 2 and scaled is None and out.dtype == torch.float32:
-            # many rows: the product's second kernel adds its parts and writes the rows' norm outright
+        if takes == 2 and scaled is None and out.dtype == torch.float32 and out.data_ptr() % 16 == 0 and then_norm[0].data_ptr() % 16 == 0:
+            # more than 64 rows: the product's second kernel adds its parts and writes the rows' norm outright
             gain, eps = then_norm
             self._require(gain, "norm gain", None, (n,), a)
             normed = self._empty((m, n), torch.bfloat16, a.device)
