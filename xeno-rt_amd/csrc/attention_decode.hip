@@ -54,17 +54,34 @@ static_assert(cache_key_offset(32 + 8 * 2 + 4 * 1 + 3, 32 * 3 + 8 * 1, 128) == (
 static_assert(cache_key_offset(8 * 3 + 4 * 0 + 1, 32 * 1 + 8 * 3 + 5, 64) == ((0 * 2 + 0) * 2 + 1) * 512 + lane_place(3 * 4 + 1, 3) + 5, "keys of a block");
 static_assert(cache_value_offset(16 * 5 + 9, 32 + 8 * 2 + 6, 128) == (1 * 8 + 5) * 512 + lane_place(9, 2) + 6, "values of a block");
 
-// One head (the dims of this lane: 32 s + 8 c .. + 7) through its RMSNorm (weight `gain`, null: none) and the rotation
-// by the token's position, in float32, and back to bfloat16: what qkv_prepare does to a head.
-// turns: the (cosine, sine) of this position's HD / 2 angles, as xrt_rope_table has worked them out (the same sincosf of the
-// same angles as in qkv_prepare.hip: worked out here, for every workgroup again, they would cost more than the kernel saves);
-// null: no rotation.
+// What finishing a head reads, of this lane's dims 32 s + 8 c .. + 7: the norm's gains (none: gain null), and the (cosine, sine) of
+// this position's HD / 2 angles, as xrt_rope_table has worked them out (the same sincosf of the same angles as in qkv_prepare.hip:
+// worked out here, for every workgroup again, they would cost more than the kernel saves; turns null: no rotation). All of it is asked for
+// ahead of the first keys, whose loads then run while the heads are finished. (Asked for where they are used, and the keys after: one sequence at 334
+// keys, 16 heads on 8, 10.4 us inside a step; now 9.5. A step at the Qwen3-0.6B sizes 911 -> 888 us, three layers of the Qwen3-32B sizes and 32 sequences 1038 -> 1030.)
+template <int HD, typename TW> struct alignas(sizeof(TW) * 8) Gains { TW e[8]; };
 template <int HD, typename TW>
-__device__ __forceinline__ void finish_head(bf16x8 (&x)[HD / 32], const TW* __restrict__ gain, float eps,
-                                            const float2* __restrict__ turns, int c) {
+__device__ __forceinline__ void ask_gains(Gains<HD, TW> (&gains)[HD / 32], const TW* __restrict__ gain, int c) {
+    if (gain == nullptr) return;
+#pragma unroll
+    for (int ks = 0; ks < HD / 32; ++ks) gains[ks] = *reinterpret_cast<const Gains<HD, TW>*>(gain + ks * 32 + c * 8);
+}
+struct alignas(16) Turns { float2 e[8]; };
+template <int HD>
+__device__ __forceinline__ void ask_turns(Turns (&turns)[HD / 64], const float2* __restrict__ from, int c) {
+    if (from == nullptr) return;
+#pragma unroll
+    for (int ks = 0; ks < HD / 64; ++ks) turns[ks] = *reinterpret_cast<const Turns*>(from + ks * 32 + c * 8);
+}
+
+// One head (the dims of this lane) through its RMSNorm and the rotation by the token's position, in float32, and back to
+// bfloat16: what qkv_prepare does to a head.
+template <int HD, typename TW>
+__device__ __forceinline__ void finish_head(bf16x8 (&x)[HD / 32], bool norms, const Gains<HD, TW> (&gains)[HD / 32], float eps,
+                                            bool rotates, const Turns (&turns)[HD / 64]) {
     constexpr int KS = HD / 32;
     float inv_rms = 1.0f;
-    if (gain != nullptr) {
+    if (norms) {
         float squares = 0.f;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
@@ -80,22 +97,17 @@ __device__ __forceinline__ void finish_head(bf16x8 (&x)[HD / 32], const TW* __re
         float lower[8], upper[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) { lower[e] = (float)x[ks][e]; upper[e] = (float)x[ks + KS / 2][e]; }
-        if (gain != nullptr) {
-            struct alignas(sizeof(TW) * 8) Eight { TW e[8]; };
-            const Eight of_lower = *reinterpret_cast<const Eight*>(gain + ks * 32 + c * 8);
-            const Eight of_upper = *reinterpret_cast<const Eight*>(gain + (ks + KS / 2) * 32 + c * 8);
+        if (norms) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                lower[e] = lower[e] * inv_rms * to_float(of_lower.e[e]);
-                upper[e] = upper[e] * inv_rms * to_float(of_upper.e[e]);
+                lower[e] = lower[e] * inv_rms * to_float(gains[ks].e[e]);
+                upper[e] = upper[e] * inv_rms * to_float(gains[ks + KS / 2].e[e]);
             }
         }
-        if (turns != nullptr) {
-            struct alignas(16) Pairs { float2 e[8]; };
-            const Pairs read = *reinterpret_cast<const Pairs*>(turns + ks * 32 + c * 8);
+        if (rotates) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const float cosine = read.e[e].x, sine = read.e[e].y;
+                const float cosine = turns[ks].e[e].x, sine = turns[ks].e[e].y;
                 const float a = lower[e], b = upper[e];
                 lower[e] = a * cosine - b * sine;
                 upper[e] = a * sine + b * cosine;
@@ -107,7 +119,8 @@ __device__ __forceinline__ void finish_head(bf16x8 (&x)[HD / 32], const TW* __re
 }
 
 // FINISH: q, k and v come as the projection left them, and `finish` says what is still to do (see the head of this file).
-template <int HD, bool FINISH, int WAVES>
+// TW: the element type of the head norms' gains.
+template <int HD, bool FINISH, int WAVES, typename TW>
 __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
     const bf16* __restrict__ qkv, int row_width, int n_heads, int n_kv_heads,
     const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache, const int* __restrict__ block_table,
@@ -148,43 +161,12 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
     const float scale2 = scale * LOG2E;                    // scores are kept in units of log2
     float m = -INFINITY, l = 0.f;
     floatx4 o[DT];
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
 
     if (active) {
         bf16x8 q[KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
             q[ks] = *reinterpret_cast<const bf16x8*>(qkv + (long)token * row_width + (long)head * HD + ks * 32 + c * 8);
-        // The sequence's newest token: its block and its place there. What is still to do to q (and, in the wavefront whose
-        // keys end with the newest block, to the new key) is done before the first keys are asked for: behind their loads
-        // it would wait for them, and with a block's keys and values in registers there is no room for it.
-        const int newest_block = (n_keys - 1) / XRT_BLOCK_TOKENS, newest = (n_keys - 1) % XRT_BLOCK_TOKENS;
-        const bool has_newest = FINISH && last_block == newest_block;
-        bf16x8 new_key[KS];
-        bf16 new_value[DT];
-        if constexpr (FINISH) {
-            const int pos = n_keys - 1;
-            const float2* turns = finish.rope_table != nullptr ? finish.rope_table + (long)min(pos, finish.table_positions - 1) * (HD / 2) : nullptr;   // (the host sends only steps that the table covers)
-            if (has_newest) {                          // (the same for all lanes of the wavefront)
-                const bf16* key_row = qkv + (long)token * row_width + (long)(n_heads + kv_head) * HD;
-                const bf16* value_row = key_row + (long)n_kv_heads * HD;
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks) new_key[ks] = *reinterpret_cast<const bf16x8*>(key_row + ks * 32 + c * 8);
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) new_value[dt] = value_row[dt * 16 + r];
-            }
-            if (finish.norm_dtype == XRT_F32)
-                finish_head<HD>(q, (const float*)finish.q_norm, finish.norm_eps, turns, c);
-            else
-                finish_head<HD>(q, (const bf16*)finish.q_norm, finish.norm_eps, turns, c);
-            if (has_newest) {
-                if (finish.norm_dtype == XRT_F32)
-                    finish_head<HD>(new_key, (const float*)finish.k_norm, finish.norm_eps, turns, c);
-                else
-                    finish_head<HD>(new_key, (const bf16*)finish.k_norm, finish.norm_eps, turns, c);
-            }
-        }
         // Loads are always on their way: a block's values are asked for before its scores are computed, and the
         // next block's keys right after, before the softmax and the value product of this one.
         const int* table = block_table + (long)slot * table_stride;
@@ -200,8 +182,41 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
                     for (int ks = 0; ks < KS; ++ks)
                         kreg[g][t][ks] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(kb + ((g * 2 + t) * KS + ks) * 512 + lane * 8));
         };
+        // The sequence's newest token: its block and its place there. What is still to do to q (and, in the wavefront whose
+        // keys end with the newest block, to the new key) is done while the first keys are on their way, with everything that it reads
+        // asked for before them (loads arrive in their order: behind the keys it would wait for those too).
+        const int newest_block = (n_keys - 1) / XRT_BLOCK_TOKENS, newest = (n_keys - 1) % XRT_BLOCK_TOKENS;
+        const bool has_newest = FINISH && last_block == newest_block;
+        bf16x8 new_key[KS];
+        bf16 new_value[DT];
+        Gains<HD, TW> q_gains[KS], k_gains[KS];
+        Turns turns[KS / 2];
+        const float2* turns_from = nullptr;
         int block = block_of(first_block), next_block = block_of(first_block + 1);
+        if constexpr (FINISH) {
+            const int pos = n_keys - 1;
+            if (finish.rope_table != nullptr) turns_from = finish.rope_table + (long)min(pos, finish.table_positions - 1) * (HD / 2);   // (the host sends only steps that the table covers)
+            ask_turns<HD>(turns, turns_from, c);
+            ask_gains<HD, TW>(q_gains, (const TW*)finish.q_norm, c);
+            if (has_newest) {                          // (the same for all lanes of the wavefront)
+                const bf16* key_row = qkv + (long)token * row_width + (long)(n_heads + kv_head) * HD;
+                const bf16* value_row = key_row + (long)n_kv_heads * HD;
+#pragma unroll
+                for (int ks = 0; ks < KS; ++ks) new_key[ks] = *reinterpret_cast<const bf16x8*>(key_row + ks * 32 + c * 8);
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) new_value[dt] = value_row[dt * 16 + r];
+                ask_gains<HD, TW>(k_gains, (const TW*)finish.k_norm, c);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
         ask_keys(block);
+        if constexpr (FINISH) {
+            __builtin_amdgcn_sched_barrier(0);
+            finish_head<HD, TW>(q, finish.q_norm != nullptr, q_gains, finish.norm_eps, turns_from != nullptr, turns);
+            if (has_newest) finish_head<HD, TW>(new_key, finish.k_norm != nullptr, k_gains, finish.norm_eps, turns_from != nullptr, turns);
+        }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
         for (int b = first_block; b <= last_block; ++b) {
             const bf16* vb = v_cache + ((long)block * n_kv_heads + kv_head) * HD * XRT_BLOCK_TOKENS;
             const int valid = min(XRT_BLOCK_TOKENS, n_keys - b * XRT_BLOCK_TOKENS);   // keys of this block that exist
@@ -311,6 +326,9 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
         }
         l += __shfl_xor(l, 16, XRT_WAVE);
         l += __shfl_xor(l, 32, XRT_WAVE);
+    } else {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
 
     // ---- the wavefronts' results become one, in wavefront order
@@ -473,19 +491,24 @@ int launch(const bf16* qkv, int tokens, int n_heads, int n_kv_heads, const bf16*
     XRT_REQUIRE(tokens <= 65535 && n_kv_heads * q_tiles <= 65535, "attention (decode): grid too large");
     const dim3 grid(cut.n_parts, n_kv_heads * q_tiles, tokens);
     const size_t lds = cut.waves * (sizeof(floatx4) * HD / 16 * XRT_WAVE + 2 * 16 * sizeof(float));
-#define XRT_DECODE(FINISH_, WAVES_, HOW)                                                                                            \
+#define XRT_DECODE(FINISH_, WAVES_, TW_, HOW)                                                                                           \
     do {                                                                                                                            \
-        static const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_decode_kernel<HD, FINISH_, WAVES_>),   \
+        static const hipError_t room = hipFuncSetAttribute(reinterpret_cast<const void*>(attention_decode_kernel<HD, FINISH_, WAVES_, TW_>),   \
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                 \
         XRT_REQUIRE(room == hipSuccess, "attention (decode): cannot reserve LDS: %s", hipGetErrorString(room));                    \
-        attention_decode_kernel<HD, FINISH_, WAVES_><<<grid, WAVES_ * XRT_WAVE, lds, s>>>(                                            \
+        attention_decode_kernel<HD, FINISH_, WAVES_, TW_><<<grid, WAVES_ * XRT_WAVE, lds, s>>>(                                            \
             qkv, row_width, n_heads, n_kv_heads, k_cache, v_cache, block_table, table_stride, n_blocks, positions, slots,            \
             scale, cut.chunk_blocks, cut.n_parts, q_tiles, part_o, part_ml, out, HOW);                                              \
     } while (0)
-    if (finish != nullptr && cut.waves == 8) XRT_DECODE(true, 8, *finish);
-    else if (finish != nullptr) XRT_DECODE(true, 4, *finish);
-    else if (cut.waves == 8) XRT_DECODE(false, 8, Finish{});
-    else XRT_DECODE(false, 4, Finish{});
+    const bool float_gains = finish != nullptr && finish->norm_dtype == XRT_F32;
+    if (finish != nullptr && cut.waves == 8) {
+        if (float_gains) XRT_DECODE(true, 8, float, *finish);
+        else XRT_DECODE(true, 8, bf16, *finish);
+    } else if (finish != nullptr) {
+        if (float_gains) XRT_DECODE(true, 4, float, *finish);
+        else XRT_DECODE(true, 4, bf16, *finish);
+    } else if (cut.waves == 8) XRT_DECODE(false, 8, bf16, Finish{});
+    else XRT_DECODE(false, 4, bf16, Finish{});
 #undef XRT_DECODE
     XRT_LAUNCH_CHECK("attention (decode)");
     if (cut.n_parts == 1) return 0;
