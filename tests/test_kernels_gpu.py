@@ -450,6 +450,34 @@ def test_rmsnorm_done_by_the_second_kernel_of_a_product_of_many_rows(ops, m, hid
     assert float(normed[m - 1].abs().max()) == 0.0
 
 
+@pytest.mark.parametrize("m,n,k", [(65, 1024, 768), (128, 1032, 256), (129, 96, 1024), (256, 3072, 1024), (100, 8192, 512),      # gated: one round of 128 x 64
+                                   (65, 9000, 384), (200, 8192, 256), (129, 5000, 512),                                        # of 128 x 128
+                                   (257, 12320, 1024), (333, 12328, 1024), (384, 12320, 1088),                                 # tiles of 192 rows
+                                   (700, 1000, 8192)])
+@pytest.mark.parametrize("mode", ["gated", "store", "add"])
+@pytest.mark.parametrize("packed", [False, True])
+def test_products_of_some_hundred_rows_in_every_tile(ops, m, n, k, mode, packed):
+    """Against float32 products on the GPU: sums of k products of bfloat16 numbers in another order differ by a few 1e-6 of the largest; bfloat16
+    results by half of their last place more."""
+    a = rand(m, k, dtype=torch.bfloat16, seed=1)
+    w = rand(2 * n, k, dtype=torch.bfloat16, seed=2, scale=1.0 / math.sqrt(k))
+    sums = a.float() @ w.float().t()
+    if mode == "gated":
+        out = torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+        ops.linear_glu(a, packed_or_not(ops, w, packed, "gated", gated_n=n), out)
+        want = torch.nn.functional.silu(sums[:, :n]) * sums[:, n:]
+    elif mode == "store":
+        out = torch.empty(m, 2 * n, dtype=torch.bfloat16, device=DEV)
+        ops.linear(a, packed_or_not(ops, w, packed), out)
+        want = sums
+    else:
+        before = rand(m, 2 * n, seed=3)
+        out = before.clone()
+        ops.linear(a, packed_or_not(ops, w, packed), out, accumulate=True)
+        want = before + sums
+    assert rel(out.float(), want) < (1e-5 if mode == "add" else ULP["bfloat16"])
+
+
 def test_rmsnorm_is_left_to_its_own_kernel_where_the_products_cannot_do_it(ops):
     gain = rand(200, seed=4).to(torch.bfloat16)
     for m, dtype in ((17, torch.bfloat16), (300, torch.bfloat16), (4, torch.float32)):

@@ -1,7 +1,7 @@
 // Matrix product for many rows (prefill), bfloat16 operands, float32 accumulation on the
 // matrix cores: out[m, n] = sum_k a[m, k] * w[n, k]; both operands are contiguous along k.
 //
-// The large tiles (256 or 128 rows by 256, eight wavefronts; K a multiple of 64) are gemm_large_tile. In the others
+// The large tiles (256, 192 or 128 rows by 256, eight wavefronts; K a multiple of 64) are gemm_large_tile. In the others
 // a workgroup computes a BM x BN tile of the output with v_mfma_f32_32x32x16_bf16. Tiles of
 // a and w travel through LDS, several steps ahead of the matrix cores, with one barrier per
 // step. When K is a multiple of 64 they are loaded from global memory straight into LDS, in a
@@ -528,7 +528,7 @@ __device__ __forceinline__ void store_four(TO* out, long m, long n, int M, int N
 
 constexpr int LARGE_BN = 256;
 
-// The large tiles: eight wavefronts, two to a SIMD, BM x 256, for K that is a multiple of 64; any split of k and all three epilogues.
+// The large tiles: eight wavefronts, two to a SIMD, BM (256, 192 or 128) x 256, for K that is a multiple of 64; any split of k and all three epilogues.
 //
 // What bounds them is the chip's power: run without a pause on random operands the clock falls to 1.5 GHz, and what counts is
 // the energy of a product, not its cycles. v_mfma_f32_16x16x32_bf16 moves half as many partial sums per product through the
@@ -550,7 +550,8 @@ __device__ __forceinline__ void gemm_large_tile(
     constexpr int BN = LARGE_BN, DK = 64, WAVES_N = 4;
     constexpr int WAVE_M = BM / 2, WAVE_N = BN / WAVES_N;      // the wavefront's part of the tile
     constexpr int TM = WAVE_M / 16, TN = WAVE_N / 16, HM = TM / 2, HN = TN / 2;      // blocks of 16 rows of x and of w: all, and a half
-    constexpr int LOADS_A = BM / 128, LOADS_B = BN / 128;      // load instructions of a wavefront for one half
+    constexpr int BLOCKS_A = BM / 16;                          // kilobytes of one half of x: where they do not divide among the wavefronts, the spare loads fetch the last one again
+    constexpr int LOADS_A = (BLOCKS_A + 7) / 8, LOADS_B = BN / 128;      // load instructions of a wavefront for one half
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
     bf16* stage_a = reinterpret_cast<bf16*>(lds_raw);          // [2][BM][64]: rows of eight 16-byte pieces, swizzled
     bf16* stage_b = stage_a + 2 * BM * DK;                     // [2][256][64]: likewise, or packed tiles as they lie
@@ -579,8 +580,8 @@ __device__ __forceinline__ void gemm_large_tile(
     auto swizzle_of = [](int r) { return r % 8; };
     // The kilobyte of LDS (8 rows of 64, or a packed tile of 16 rows and 32 columns) that load i of half h fills, for a
     // wavefront; rows: a wavefront's rows of the operand in the tile.
-    auto block_of = [&](int h, int i, int rows) {
-        const int p = i * 8 + wave, per = rows / 16;
+    auto block_of = [&](int h, int i, int rows, int blocks) {
+        const int per = rows / 16, p = min(i * 8 + wave, blocks - 1);
         return (p / per * rows + h * (rows / 2)) / 8 + p % per;
     };
     const long row_a = lda > 0 ? lda : K, row_w = ldw > 0 ? ldw : K;
@@ -592,12 +593,12 @@ __device__ __forceinline__ void gemm_large_tile(
     for (int h = 0; h < 2; ++h) {
 #pragma unroll
         for (int i = 0; i < LOADS_A; ++i) {
-            const int r = block_of(h, i, WAVE_M) * 8 + lane / 8;
+            const int r = block_of(h, i, WAVE_M, BLOCKS_A) * 8 + lane / 8;
             off_a[h][i] = (unsigned)(min(m0 + r, (long)M - 1) * row_a + ((lane % 8) ^ swizzle_of(r)) * 8) * 2u;
         }
 #pragma unroll
         for (int i = 0; i < LOADS_B; ++i) {
-            const int block = block_of(h, i, WAVE_N);
+            const int block = block_of(h, i, WAVE_N, BN / 16);
             if (packed_b) {
                 const long group = min(first_packed / 16 + block / 2, last_group);       // groups beyond the matrix: the last one again
                 off_b[h][i] = (unsigned)(((group * (row_w / 32) + block % 2) * 512 + lane * 8) * 2);
@@ -612,12 +613,12 @@ __device__ __forceinline__ void gemm_large_tile(
     auto issue_a = [&](int h, int stage, int k0) {
 #pragma unroll
         for (int i = 0; i < LOADS_A; ++i)
-            load_to_lds(a, off_a[h][i] + (unsigned)k0 * 2u, lds_a0 + (unsigned)(stage * BM * DK * 2 + block_of(h, i, WAVE_M) * 1024));
+            load_to_lds(a, off_a[h][i] + (unsigned)k0 * 2u, lds_a0 + (unsigned)(stage * BM * DK * 2 + block_of(h, i, WAVE_M, BLOCKS_A) * 1024));
     };
     auto issue_b = [&](int h, int stage, int k0) {
 #pragma unroll
         for (int i = 0; i < LOADS_B; ++i)
-            load_to_lds(w, off_b[h][i] + (unsigned)k0 * w_step, lds_b0 + (unsigned)(stage * BN * DK * 2 + block_of(h, i, WAVE_N) * 1024));
+            load_to_lds(w, off_b[h][i] + (unsigned)k0 * w_step, lds_b0 + (unsigned)(stage * BN * DK * 2 + block_of(h, i, WAVE_N, BN / 16) * 1024));
     };
     // where this lane finds its 16 bytes of block 0 of its wavefront, for either 32 columns of the tile
     const bf16* place_a[2];
@@ -792,7 +793,7 @@ __device__ __forceinline__ void gemm_large_tile(
                 return;
             }
         }
-        constexpr int RUN = 4;                                 // blocks of x whose old values are read in one go, before any is written
+        constexpr int RUN = TM % 4 == 0 ? 4 : 3;               // blocks of x whose old values are read in one go, before any is written
 #pragma unroll
         for (int i0 = 0; i0 < TM; i0 += RUN) {
             float before[RUN][TN][4];
@@ -985,11 +986,13 @@ int launch_large(const bf16* a, const bf16* w, TO* out, int M, int N, int K, con
 // first loads and its epilogue. A last round that is partly filled takes `least` percent of a full one and its share of the
 // rest: the chip is bound by its power, and with fewer compute units at work their clock rises. The numbers are fitted to 1985
 // products (layers of seven sizes and sizes drawn at random, k from 64 to 25600, 129 to 8192 rows of x), every tile shape of
-// each of them timed: what the estimate chooses is 0.6 % off the best of them on average, which is within the runs' differences.
+// each of them timed: what the estimate chooses is 0.6 % off the best of them on average, which is within the runs' differences. (The tiles of 192 rows came later,
+// fitted to 90 gated products: 28672 rows of w, k = 4096, 333 rows of x 90 -> 76 us, 1100 rows 234 -> 213; 16384 rows, k = 2048, 540 rows 46 -> 38; 51200
+// rows, k = 5120, 576 rows 317 -> 279.)
 enum { ENDS_BF16 = 0, ENDS_F32 = 1, ENDS_ADDING = 2, ENDS_GATED = 3 };
 struct TileTime { int bm, bn, places, products, ends[4], least; };
 constexpr TileTime LARGE_TILE = {256, 256, XRT_COMPUTE_UNITS, 88, {10, 16, 15, 16}, 55}, HALF_TILE = {128, 256, XRT_COMPUTE_UNITS, 54, {6, 8, 9, 9}, 62},
-                   NARROW_TILE = {256, 192, XRT_COMPUTE_UNITS, 81, {0, 11, 8, 0}, 55}, SMALL_TILE = {128, 128, 2 * XRT_COMPUTE_UNITS, 67, {7, 7, 5, 10}, 41};
+                   MIDDLE_TILE = {192, 256, XRT_COMPUTE_UNITS, 71, {8, 13, 12, 13}, 55}, NARROW_TILE = {256, 192, XRT_COMPUTE_UNITS, 81, {0, 11, 8, 0}, 55}, SMALL_TILE = {128, 128, 2 * XRT_COMPUTE_UNITS, 67, {7, 7, 5, 10}, 41};
 long rounds_cost(long tiles, const TileTime& tile, int K, int kind) {        // in nanoseconds or so
     const long round = tile.products * 1000L * K / 4096 + tile.ends[kind] * 1000L;
     const long whole = tiles / tile.places, rest = tiles % tile.places;
@@ -1008,11 +1011,15 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
         if (large <= small) return launch_kernel<256, 256, 2, 4, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
         return launch_kernel<128, 128, 2, 2, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
     }
-    // Up to 128 rows of a, gated: one round of tiles of 128 x 128 (or nearly), bound by reading w: three stages keep more of
-    // it on its way than the two that the tiles below have (gate/up of 14336 pairs and 128 rows: 76 us split in three
-    // with a second kernel, 49 us so).
-    if constexpr (MODE == MODE_GATED)
-        if (M <= 128) return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+    // Up to 256 rows of a, gated: tiles that fit one round and are bound by reading w, in three or four stages, which keep more of it on
+    // its way than the two that the tiles below have. (Split along k with a second kernel: 3072 pairs, k = 1024, 100 rows 14.6 us, so 9.5, 256 rows
+    // 17.8 -> 9.9; 8192 pairs, k = 2048, 100 rows 24.4 -> 19.9, 200 rows 31.2 -> 24.7; 12288 pairs, k = 4096, 100 rows 59.6 -> 50.9; 5000 pairs,
+    // k = 3072, 65 rows 28.8 -> 21.8. Tiles of 128 x 64 beyond one round lose to one of 128 x 128: 12288 pairs, 100 rows 55.7.)
+    if constexpr (MODE == MODE_GATED) {
+        if (M <= 256 && tiles(128, 64) <= XRT_COMPUTE_UNITS) return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+        if (M <= 128 || (M <= 256 && tiles(128, 128) <= XRT_COMPUTE_UNITS))
+            return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+    }
     // 256 x 256 tiles cost the least energy a product, and tiles of half the height somewhat more (2048 rows of x, 4096 rows of
     // w, k = 4096: 128 tiles of the one 85 us, 256 of the other 58; 6144 rows of w: 82 and 102); tiles of 128 x 128, two to a compute
     // unit, where neither fills the chip, or where k is so short that one's epilogue wants another's products beside it (200 rows of x,
@@ -1025,7 +1032,7 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
     constexpr long NARROW_W = 150L * 1000 * 1000;              // bytes
     constexpr int KIND = MODE == MODE_GATED ? ENDS_GATED : MODE == MODE_ACCUMULATE ? ENDS_ADDING : sizeof(TO) == 4 ? ENDS_F32 : ENDS_BF16;
     auto cost = [&](const TileTime& tile) { return rounds_cost(tiles(tile.bm, tile.bn), tile, K, KIND); };
-    const long large = cost(LARGE_TILE), half = cost(HALF_TILE), small = cost(SMALL_TILE);
+    const long large = cost(LARGE_TILE), middle = cost(MIDDLE_TILE), half = cost(HALF_TILE), small = cost(SMALL_TILE);
     constexpr bool NARROW = MODE != MODE_GATED && sizeof(TO) == 4;
     const long narrow = NARROW && (long)N * K * (long)sizeof(bf16) <= NARROW_W ? cost(NARROW_TILE) : LONG_MAX;
     // Large tiles for as many columns as make whole rounds, and tiles of half the height for the rest, if those then fit
@@ -1037,7 +1044,7 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
     long mixed = LONG_MAX;
     if (whole_columns > 0 && whole_columns < tiles_n && rest_tiles <= XRT_COMPUTE_UNITS)
         mixed = rounds_cost((long)tiles_m * whole_columns, LARGE_TILE, K, KIND) + rounds_cost(rest_tiles, HALF_TILE, K, KIND);
-    if (mixed < large && mixed <= half && mixed <= small && mixed <= narrow) {
+    if (mixed < large && mixed <= middle && mixed <= half && mixed <= small && mixed <= narrow) {
         const int split = whole_columns * (256 / DIV);
         const int small_tiles_m = (M + 127) / 128, small_tiles_n = tiles_n - whole_columns;
         const int large_blocks = (tiles_m * whole_columns + 7) / 8 * 8;      // whole rounds over the XCDs
@@ -1055,7 +1062,8 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
         XRT_LAUNCH_CHECK("linear (mfma, two tile shapes)");
         return 0;
     }
-    if (large <= half && large <= small && large <= narrow) return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+    if (large <= middle && large <= half && large <= small && large <= narrow) return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+    if (middle <= half && middle <= small && middle <= narrow) return launch_large<192, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
     if (half <= small && half <= narrow) return launch_large<128, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
     if constexpr (NARROW)
         if (narrow <= small) return launch_kernel<256, 192, 4, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
@@ -1103,9 +1111,16 @@ long parts_time(const PartTime& shape, int M, long N, int steps, int parts) {
 }
 // The same of the tiles without a split (a fit to the same products: their own estimate counts a warm chip's rounds alone).
 long unsplit_time(int M, int N, int K, int mode) {
-    const int kind = mode == MODE_ACCUMULATE ? ENDS_ADDING : ENDS_BF16;
-    auto cost = [&](const TileTime& tile) { return rounds_cost((long)((M + tile.bm - 1) / tile.bm) * ((N + tile.bn - 1) / tile.bn), tile, K, kind); };
-    return 1000 + min(min(cost(LARGE_TILE), cost(HALF_TILE)), cost(SMALL_TILE)) * 127 / 100;
+    const int kind = mode == MODE_GATED ? ENDS_GATED : mode == MODE_ACCUMULATE ? ENDS_ADDING : ENDS_BF16;
+    const long rows_w = mode == MODE_GATED ? 2L * N : N;
+    auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((rows_w + bn - 1) / bn); };
+    if (mode == MODE_GATED && M <= 256) {                      // one round of tiles in several stages
+        if (tiles(128, 64) <= XRT_COMPUTE_UNITS) return 5000 + (NARROW_PARTS.step + NARROW_PARTS.share * tiles(128, 64) / XRT_COMPUTE_UNITS) * (K / 64);
+        if (tiles(128, 128) <= XRT_COMPUTE_UNITS) return 5000 + (WIDE_PARTS.step + WIDE_PARTS.share * tiles(128, 128) / XRT_COMPUTE_UNITS) * (K / 64);
+    }
+    auto cost = [&](const TileTime& tile) { return rounds_cost(tiles(tile.bm, tile.bn), tile, K, kind); };
+    const long least = min(min(cost(LARGE_TILE), cost(MIDDLE_TILE)), min(cost(HALF_TILE), cost(SMALL_TILE)));
+    return 1000 + (mode == MODE_GATED ? least : least * 127 / 100);
 }
 
 // whole_norm: an RMSNorm follows that the second kernel can do outright, which is worth a split in two where the product alone
@@ -1128,16 +1143,9 @@ SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
         splits = splits > 8 ? 8 : splits;
         least = 24;
         tile = columns = 256;
-    } else if (mode == MODE_GATED) {
-        // Some hundred rows of x, gated: with a round of tiles or nearly so no split, for the tiles then apply the epilogue themselves.
-        // Beyond 256 rows the workgroups run two to a compute unit: as many parts as still fit those 512 places at once.
-        const long tiles = (long)((M + 127) / 128) * tiles_n;
-        tile = columns = 128;
-        splits = M <= 256 ? (tiles >= 200 ? 1 : (int)((XRT_COMPUTE_UNITS + tiles - 1) / tiles)) : (int)(2 * XRT_COMPUTE_UNITS / tiles);
-        least = M <= 256 ? 8 : 4;
     } else {
         // Some hundred rows of x: still bound by reading w, and too few tiles to fill the chip without a split. Tiles of 128 x 64 or 128 x 128
-        // and the number of parts by an estimate of the time, against one of the product without a split. (Narrow tiles read x twice as often, which
+        // and the number of parts by an estimate of the time, against one of the product without a split (which saves a gated product the sums of both halves). (Narrow tiles read x twice as often, which
         // does not stay in a die's L2 when k is long: 4096 rows of w, k = 14336, 100 rows of x 34.7 us in wide tiles, 40.3 in narrow ones.)
         const long tiles = (long)((M + 127) / 128) * tiles_n;
         tile = columns = 128;
@@ -1146,11 +1154,11 @@ SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
         if (tiles <= (M <= 256 ? 2 * XRT_COMPUTE_UNITS : XRT_COMPUTE_UNITS)) {      // (more fill the chip as they are)
             long best = unsplit_time(M, N, K, mode);
             for (const PartTime& shape : {NARROW_PARTS, M <= 256 ? WIDE_PARTS : WIDE_PARTS_TWO}) {
-                if (shape.columns == 64 && K >= 8192 && N > 2048) continue;
+                if (shape.columns == 64 && K >= 8192 && rows_w > 2048) continue;
                 for (int parts = 2; parts <= 16 && parts <= units; ++parts) {
                     const int per = (units + parts - 1) / parts;
                     if ((units + per - 1) / per != parts) continue;          // (as many pieces a part with fewer parts)
-                    const long time = parts_time(shape, M, N, per, parts);
+                    const long time = parts_time(shape, M, rows_w, per, parts);
                     if (time < best) { best = time; splits = parts; columns = shape.columns; }
                 }
             }
