@@ -1315,12 +1315,16 @@ __global__ void __launch_bounds__(THREADS) split_reduce_rmsnorm_kernel(const flo
             const long index = row + 4L * q;
             const floatx4 before = *reinterpret_cast<const floatx4*>(out + index);
             weight[i] = *reinterpret_cast<const Four<TW>*>(gain + 4 * q);
-            floatx4 sum = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(parts + index));     // read once, by nobody else
+            auto part_of = [&](int p) {                        // read once, by nobody else; few rows' parts still lie in the last cache
+                const floatx4* from = reinterpret_cast<const floatx4*>(parts + p * count + index);
+                return THREADS == NORM_THREADS ? __builtin_nontemporal_load(from) : *from;
+            };
+            floatx4 sum = part_of(0);
             for (int p0 = 1; p0 < splits; p0 += AT_ONCE) {
                 floatx4 part[AT_ONCE];
 #pragma unroll
                 for (int u = 0; u < AT_ONCE; ++u)
-                    part[u] = __builtin_nontemporal_load(reinterpret_cast<const floatx4*>(parts + min(p0 + u, splits - 1) * count + index));
+                    part[u] = part_of(min(p0 + u, splits - 1));
 #pragma unroll
                 for (int u = 0; u < AT_ONCE; ++u)
                     if (p0 + u < splits) sum += part[u];
@@ -1438,8 +1442,14 @@ int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, c
         return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
     if (plan.tile == 256)
         return launch_large<256, MODE_STORE, float>(a, w, workspace, M, rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split);
-    if (plan.columns == 64)
+    if (plan.columns == 64) {
+        // a fourth stage where a compute unit has one workgroup anyway (2048 rows of w, k = 8192, 65 / 200 rows of x 16.0 / 22.5 -> 14.7 / 20.5 us with its
+        // second kernel; k = 2048, 3072 rows, 100 rows of x 12.0 -> 11.5)
+        const long groups = (long)((M + 127) / 128) * ((rows_w + 63) / 64) * plan.splits;
+        if (groups <= XRT_COMPUTE_UNITS)
+            return launch_kernel<128, 64, 4, 1, MODE_STORE, 64, 4, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
         return launch_kernel<128, 64, 2, 2, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+    }
     if (M <= 256)           // (one workgroup to a compute unit anyway: a third stage keeps more of w on its way; with more, two share a unit)
         return launch_kernel<128, 128, 2, 2, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
     return launch_kernel<128, 128, 2, 2, MODE_STORE, 64, 2, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
