@@ -419,7 +419,7 @@ def test_rmsnorm_done_by_the_products_around_it(ops, m, hidden, k, n, packed):
 @pytest.mark.parametrize("m,hidden,k", [(520, 1032, 4160), (2048, 4096, 4096), (600, 520, 8192), (1024, 8192, 4096),
                                         # few rows: smaller tiles, and workgroups of 1024 threads up to 511 rows
                                         (65, 1024, 512), (100, 2048, 8192), (333, 4096, 14336), (129, 8192, 2048), (200, 264, 3072),
-                                        (511, 1032, 4096), (512, 1032, 4096)])
+                                        (511, 1032, 4096), (512, 1032, 4096), (333, 4104, 14336)])
 @pytest.mark.parametrize("gain_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("packed", [False, True])
 def test_rmsnorm_done_by_the_second_kernel_of_a_product_of_many_rows(ops, m, hidden, k, gain_dtype, packed):
@@ -453,7 +453,7 @@ def test_rmsnorm_done_by_the_second_kernel_of_a_product_of_many_rows(ops, m, hid
 @pytest.mark.parametrize("m,n,k", [(65, 1024, 768), (128, 1032, 256), (129, 96, 1024), (256, 3072, 1024), (100, 8192, 512),      # gated: one round of 128 x 64
                                    (65, 9000, 384), (200, 8192, 256), (129, 5000, 512),                                        # of 128 x 128
                                    (257, 12320, 1024), (333, 12328, 1024), (384, 12320, 1088),                                 # tiles of 192 rows
-                                   (700, 1000, 8192)])
+                                   (700, 1000, 8192), (150, 5128, 5120), (192, 6000, 4096), (333, 2056, 14336), (193, 2048, 16384)])     # the last four: parts of 192 rows
 @pytest.mark.parametrize("mode", ["gated", "store", "add"])
 @pytest.mark.parametrize("packed", [False, True])
 def test_products_of_some_hundred_rows_in_every_tile(ops, m, n, k, mode, packed):

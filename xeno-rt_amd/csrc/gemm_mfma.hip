@@ -1089,7 +1089,7 @@ int launch_shape(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int
 // few to fill the chip: such products are still bound by reading w.
 constexpr int SPLIT_BM = 64, SPLIT_BN = 128;
 
-struct SplitPlan { int splits, k_per_split; long rows_w; int tile, columns; };      // tile: rows of x per tile (64, 128 or 256), columns: rows of w
+struct SplitPlan { int splits, k_per_split; long rows_w; int tile, columns; };      // tile: rows of x per tile (64, 128, 192 or 256), columns: rows of w
 
 // What a product of some hundred rows of x takes (nanoseconds) in parts along k: tiles of 128 rows of x and `columns` rows of w, `places` of them to a compute
 // unit. A step of 64 along k takes `step`, `share` more for each tile that a compute unit has on average, and `beside` more where some have two; `once` is
@@ -1161,6 +1161,16 @@ SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
                     const long time = parts_time(shape, M, rows_w, per, parts);
                     if (time < best) { best = time; splits = parts; columns = shape.columns; }
                 }
+            }
+            // Large tiles of 192 rows, in parts that make one round: fewer operands read a product, more at the ends (beside the best of the others: 333 rows
+            // of x, 5120 rows of w, k = 25600 129 -> 113 us, 4096 rows, k = 14336 61 -> 58, but k = 4096 30 -> 33; 150 rows of x, 10240 rows of w, k = 5120
+            // 43 -> 34). The figures are of those and 100 more such products.
+            const long large = (long)((M + 191) / 192) * ((rows_w + 255) / 256);
+            for (int parts = 2; M > 128 && parts <= 16 && parts <= units && parts * large <= XRT_COMPUTE_UNITS; ++parts) {
+                const int per = (units + parts - 1) / parts;
+                if ((units + per - 1) / per != parts) continue;
+                const long time = 10000 + 1200L * per + 1400L * parts * (M * rows_w / 1000) / 1000;
+                if (time < best) { best = time; splits = parts; tile = 192; columns = 256; }
             }
         }
     }
@@ -1440,6 +1450,8 @@ int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, c
     const int rows_w = (int)plan.rows_w;
     if (M <= SPLIT_BM)
         return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+    if (plan.tile == 192)
+        return launch_large<192, MODE_STORE, float>(a, w, workspace, M, rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split);
     if (plan.tile == 256)
         return launch_large<256, MODE_STORE, float>(a, w, workspace, M, rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split);
     if (plan.columns == 64) {
