@@ -1166,7 +1166,9 @@ SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
             // of x, 5120 rows of w, k = 25600 129 -> 113 us, 4096 rows, k = 14336 61 -> 58, but k = 4096 30 -> 33; 150 rows of x, 10240 rows of w, k = 5120
             // 43 -> 34). The figures are of those and 100 more such products.
             const long large = (long)((M + 191) / 192) * ((rows_w + 255) / 256);
-            for (int parts = 2; M > 128 && parts <= 16 && parts <= units && parts * large <= XRT_COMPUTE_UNITS; ++parts) {
+            // Not for one row of tiles on a w beyond the caches, which the smaller tiles' three stages stream faster (150 rows, 5120 rows of w, k = 25600 94 against 101 us).
+            const bool suits = M > 192 || (M > 128 && rows_w * K * (long)sizeof(bf16) <= 150L * 1000 * 1000);
+            for (int parts = 2; suits && parts <= 16 && parts <= units && parts * large <= XRT_COMPUTE_UNITS; ++parts) {
                 const int per = (units + parts - 1) / parts;
                 if ((units + per - 1) / per != parts) continue;
                 const long time = 10000 + 1200L * per + 1400L * parts * (M * rows_w / 1000) / 1000;
