@@ -493,7 +493,7 @@ int launch(const bf16* qkv, int tokens, int n_heads, int n_kv_heads, const bf16*
     float* part_o = workspace;
     float* part_ml = workspace + (long)tokens * n_heads * cut.n_parts * HD;
     const int row_width = (n_heads + 2 * n_kv_heads) * HD;
-    XRT_REQUIRE(tokens <= 65535 && n_kv_heads * q_tiles <= 65535, "attention (decode): grid too large");
+    XRT_REQUIRE(tokens <= XRT_GRID_ROWS && n_kv_heads * q_tiles <= XRT_GRID_ROWS, "attention (decode): grid too large");
     const dim3 grid(cut.n_parts, n_kv_heads * q_tiles, tokens);
     const size_t lds = cut.waves * (sizeof(floatx4) * HD / 16 * XRT_WAVE + 2 * 16 * sizeof(float));
 #define XRT_DECODE(FINISH_, WAVES_, TW_, HOW)                                                                                           \

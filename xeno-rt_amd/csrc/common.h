@@ -16,6 +16,8 @@ enum { XRT_F32 = 0, XRT_BF16 = 1 };
 #define XRT_WAVE 64
 // compute units of the chip: what the launchers count in when they deal work out in rounds
 #define XRT_COMPUTE_UNITS 256
+// the most workgroups in a grid's second and third dimension
+#define XRT_GRID_ROWS 65535
 
 // ---- error reporting -------------------------------------------------------
 void xrt_set_error(const char* format, ...);

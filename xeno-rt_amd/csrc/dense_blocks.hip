@@ -9,8 +9,12 @@
 //
 // Memory: one piece, given by the caller, whose size the call itself says beforehand (arena null). A layer's buffers lie where the layer's before lay (the
 // stream's order keeps them apart); what a layer hands to the next lies in two places that take turns.
+#include <algorithm>
+
 #include "common.h"
 #include "xrt_hip.h"
+
+bool xrt_attention_decode_accepts(int head_dim);
 
 namespace {
 
@@ -38,6 +42,27 @@ struct Rows {
 };
 // where a product may put such rows
 struct Room { void* values; float* squares; };
+
+// Whether the attention of a step's `rows` wanted rows alone, as a step in which every row is a sequence with one token, takes less than that of all its tokens.
+// The decode kernel reads a row's keys for that row only, the kernel for prompts shares them among the rows of a tile. In nanoseconds, for keys of the step's
+// average position: a row of the one costs 200 a thousand keys of 8 heads of 128 and somewhat more where they lie beyond the caches, a row of the other 16 a thousand keys of 32 query heads
+// of 128, and 6000 + 2 a key once; every sequence's keys are read once either way. Fitted to 1280 steps (32 heads on 8, 16 on 8 and 64 on 8 of 128 dims, 32 on 8
+// of 64; 17 to 8192 tokens of one sequence or four behind 0 to 16000; a row of 4 to the last alone): 0.6 % off the better of the two on
+// average, where the wanted rows alone at all times are 22 % off. 32 heads of 128 on 8: 2048 of 8192 tokens 2121 us alone, 671 all (behind 16000
+// 14091 and 2581), 256 of them 260 (1609); 41 of 333 behind 4000 46 and 55, 83 of them 91.
+// Whole steps, two layers, before any of this, with the wanted rows alone at all times, and by this rule: 8B sizes, 2048 of 8192 tokens 8151, 8116, 6601 us; 250 of 1000 behind
+// 8000 1555, 2002, 1341; Qwen3-0.6B sizes, 512 of 2048 behind 8000 940, 1903, 879; float32, Llama-3.2-1B sizes, 250 of 1000 behind 4000 13646, 5135, 4232.
+// float32, to the same bits: where the matrix cores take the step, a thousand keys are 240 us to a wavefront of the general kernel that goes through them by itself,
+// which it does with more (token, head) pairs than the kernel of the many takes from; below that it shares them out (2048 tokens, 32 heads of 64 on 8: 428 us all, 64 rows alone 242, 128 482).
+bool wanted_alone(const xrt_dense_step& s, const xrt_dense_layer& l, const void* qkv, int rows) {
+    if (s.dtype == XRT_F32)
+        return (long)rows * l.n_heads <= 8L * XRT_COMPUTE_UNITS ||
+               !xrt_attention_float_prompts_accepts(qkv, s.tokens, l.n_heads, l.n_kv_heads, l.head_dim, l.k_cache, l.v_cache, qkv, s.fewest);
+    if (!xrt_attention_decode_accepts(l.head_dim)) return true;                // (the general kernel, a token at a time either way)
+    if (rows > XRT_GRID_ROWS) return false;
+    const double keys = std::max(1.0, s.max_context - 0.5 * s.max_count), row = (200 + 0.008 * keys) * (l.n_kv_heads * l.head_dim / 1024.0) * keys / 1000;
+    return row * (rows - s.n_seqs) <= 6000 + 2 * keys + 16 * (l.n_heads * l.head_dim / 4096.0) * keys / 1000 * s.tokens;
+}
 
 struct Step {
     const xrt_dense_step& s;
@@ -134,23 +159,31 @@ struct Step {
                                l.writable ? l.n_blocks : 0, s.max_count, workspace, need, s.stream))
                 return 1;
         }
-        void* out;
-        if (wanted == nullptr) {
+        if (wanted != nullptr && wanted->count == 0) return 0;
+        const bool alone = wanted != nullptr && wanted_alone(s, l, qkv, wanted->count);
+        void* out = nullptr;
+        if (!alone) {
             out = arena.take((long)rows * q_width * element);
             if (attention(l, qkv, rows, s.positions, s.slots, s.seq_offsets, s.seq_slots, s.seq_starts, s.n_seqs, s.max_count, s.fewest, finishes ? &finish : nullptr, out))
                 return 1;
-        } else {
-            // the rows that somebody wants go on alone, as a step in which every row is a sequence with one token
-            if (wanted->count == 0) return 0;
+        }
+        if (wanted != nullptr) {
+            // The rows that somebody wants go on alone: with their queries, as a step in which every row is a sequence with one token, or with what
+            // the attention of all rows has made.
             rows = wanted->count;
-            void* q = arena.take((long)rows * width * element);
+            const void* of = alone ? qkv : out;
+            const long of_stride = alone ? width * element : q_width * element;
+            void* taken = arena.take(rows * of_stride);
             int* described = (int*)arena.take((3L * rows + 1) * 4);
             x = wanted->x;
-            if (!arena.plan && xrt_take_rows(qkv, width * element, (int)(q_width * element), q, width * element, s.x, s.hidden * 4, x, s.positions, s.slots,
+            if (!arena.plan && xrt_take_rows(of, of_stride, (int)(q_width * element), taken, of_stride, s.x, s.hidden * 4, x, s.positions, s.slots,
                                              wanted->rows, rows, s.tokens, described, s.stream))
                 return 1;
-            out = arena.take((long)rows * q_width * element);
-            if (attention(l, q, rows, described, described + rows, described + 2 * rows, described + rows, described, rows, 1, 1, nullptr, out)) return 1;
+            out = taken;
+            if (alone) {
+                out = arena.take((long)rows * q_width * element);
+                if (attention(l, taken, rows, described, described + rows, described + 2 * rows, described + rows, described, rows, 1, 1, nullptr, out)) return 1;
+            }
         }
         const Room between = room();
         Rows middle;
@@ -167,6 +200,8 @@ struct Step {
 };
 
 }  // namespace
+
+extern "C" int xrt_dense_wanted_alone(const xrt_dense_layer* layer, const xrt_dense_step* step, int rows) { return wanted_alone(*step, *layer, nullptr, rows); }
 
 extern "C" long xrt_dense_blocks(const xrt_dense_layer* layers, int count, const xrt_dense_step* step, const xrt_dense_wanted* wanted, void* arena, long arena_bytes) {
     const auto refuse = [](const char* what) -> long { xrt_set_error("dense blocks: %s", what); return -1; };

@@ -343,6 +343,8 @@ typedef struct xrt_dense_step {
     int dtype; int tokens; int hidden; int n_seqs; int max_count; int max_context; int fewest;
 } xrt_dense_step;
 typedef struct xrt_dense_wanted { const int* rows; float* x; int count; } xrt_dense_wanted;
+// Whether the wanted rows of such a step go through the last layer's attention alone, as sequences of one token (else with all tokens, and go on alone behind it).
+int xrt_dense_wanted_alone(const xrt_dense_layer* layer, const xrt_dense_step* step, int rows);
 long xrt_dense_blocks(const xrt_dense_layer* layers, int count, const xrt_dense_step* step, const xrt_dense_wanted* wanted, void* arena, long arena_bytes);
 
 // Attention without a softmax: the weight of a visible key is sigmoid(score_h + head_bias[h]), not normalised over the keys;

@@ -323,8 +323,9 @@ class Attention(Mixer):
         return type(self) is Attention and not self.general and self.window is None and (self.position is None or self.position.rotation() is not None) and (
             self.position is None or self.position.score_slopes() is None)
 
-    # Tokens whose results nobody wants need go no further than the cache behind the model's last attention: for the others alone the step
-    # goes on from there with their queries, which costs a kernel that brings them together. Up to 16 rows a product is bound by reading its weights, and where
+    # Tokens whose results nobody wants need go no further than the cache behind the model's last attention: the others alone go on from there,
+    # which costs a kernel that brings them together (csrc/dense_blocks.hip says whether their attention runs alone as well, or with all tokens
+    # because many of them share keys). Up to 16 rows a product is bound by reading its weights, and where
     # the output projection has fewer than WANTED_FROM elements a layer is all launches. Measured with every kernel launched from Python: tiny models 305 -> 330 us
     # a prompt by it, 1024 x 2048 the same up to 200 tokens and 3220 -> 3168 us at 400, 4096 x 4096 (4 layers) 633 -> 618 at 17 tokens, 822 -> 780 at 100,
     # 1304 -> 1171 at 400; a prompt of 2048 tokens through 6 layers 4847 -> 4260, of 8192 through 4 13374 -> 10535. (One layer of a model's: of 32 layers 2 to 3 %.)
