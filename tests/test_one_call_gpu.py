@@ -1,6 +1,7 @@
 """The layers of a plain dense decoder launched by one call (csrc/dense_blocks.hip) at sizes whose products, norms and attention take the
 kernels that the tiny models of test_engine_gpu.py are too small for."""
 import ctypes
+from types import SimpleNamespace
 
 import pytest
 import torch
@@ -101,3 +102,32 @@ def test_more_wanted_rows_than_a_decode_step_has_sequences(monkeypatch):
         want = engine.step([(slot, step[i][1], list(range(257)))])[step[i][2]]
         engine.free_slot(slot)
         assert_logits(got[64 * i:64 * i + 64], want.cpu(), "bfloat16", f"sequence {i}")
+
+
+# ---- what `DecoderModel.forward` is given ------------------------------------------------------------------------------------------------
+
+def forward(engine, slot, ids, wanted, without=(), cache=None, **changes):
+    """The model on a step of one sequence from its first token, its batch without the fields named."""
+    from xeno_rt_amd.engine.batch import build_batch
+    engine.cache.reserve(slot, len(ids))
+    engine.cache.sync()
+    batch = vars(build_batch([slot], [ids], [0], [wanted], "cuda:0"))
+    try:
+        return engine.model.forward(SimpleNamespace(**{**{name: value for name, value in batch.items() if name not in without}, **changes}), cache or engine.cache)
+    finally:
+        engine.cache.cancel(slot)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", ["llama", "qwen3"])
+def test_batches_that_say_less_of_themselves(name, dtype):
+    """What a batch need not say: its counts on the host, how its tokens fall into sequences."""
+    engine = wide_engine(name, dtype)
+    slot, ids = engine.alloc_slot(), token_ids(engine.vocab_size, 150, seed=3)
+    want = forward(engine, slot, ids, [0, 70, 149])
+    sequences = ("sequence_offsets", "sequence_slots", "sequence_starts", "n_sequences", "max_count", "max_context", "is_decode")
+    on_host = ("host_counts", "host_slots", "host_starts")
+    for without, changes in ((on_host, {}), (sequences + on_host, {}), (on_host, {"max_count": 0}), (on_host, {"max_context": 0})):
+        got = forward(engine, slot, ids, [0, 70, 149], without, **changes)
+        assert_logits(got, want.cpu(), dtype, f"{name} without {without} {changes}")
+        assert dtype != "float32" or torch.equal(got, want), (without, changes)

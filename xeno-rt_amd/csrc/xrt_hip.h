@@ -326,7 +326,7 @@ int xrt_attention_float_prompts(const void* qkv, int tokens, int n_heads, int n_
 // The layers of a plain dense decoder from one call (dense_blocks.hip): for each of `count` layers in turn the RMSNorm of the float32 stream x, q/k/v with
 // head norms, rotation and cache write, causal attention, the output projection onto x, the second norm, the gated (silu) product and the one back onto x, with the kernels and operands
 // that the calls above would get one by one. q_norm, k_norm: null without head norms; rope_theta: null without rotation, else float32 [rope_dim / 2]; rope_table: null, or xrt_rope_table's
-// for the first table_positions positions; writable 0: the keys and values are another call's. fewest: the fewest new tokens of a sequence. wanted: null, or the rows of the step that the last
+// for the first table_positions positions; writable 0: the keys and values are another call's. fewest: the fewest new tokens of a sequence (0: unknown). wanted: null, or the rows of the step that the last
 // layer goes on with behind its keys and values (count 0: none): x is then left as the layers before it made it, and those rows, updated, lie in wanted->x.
 // arena null: returns the bytes of memory the call needs (launches nothing); else memory of at least so many, aligned to 256. Returns that number, or -1 (xrt_last_error).
 typedef struct xrt_dense_matrix { const void* data; xrt_packing packing; } xrt_dense_matrix;

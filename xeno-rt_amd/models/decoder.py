@@ -122,6 +122,12 @@ class DecoderModel:
             return ops.dense_blocks(layers, x, batch, self.runtime.dtype, rows=batch.logit_rows), None
         return ops.dense_blocks(layers, x, batch, self.runtime.dtype), batch.logit_rows
 
+    @staticmethod
+    def _says_its_sequences(batch) -> bool:
+        """Whether the batch describes its tokens as sequences, which the call that launches all layers wants to know (the parts by themselves take any batch)."""
+        return (all(getattr(batch, name, None) is not None for name in ("sequence_offsets", "sequence_slots", "sequence_starts"))
+                and 0 < batch.n_sequences <= batch.n_tokens and batch.max_count > 0 and batch.max_context > 0)
+
     def _first_reads_stream(self) -> bool:
         """Whether the first block reads the stream itself in the compute dtype and the embedding can hand it that beside the stream."""
         spec = self.spec
@@ -145,9 +151,10 @@ class DecoderModel:
             x = spec.streams.open(x)
         wanted = batch.logit_rows
         opened = spec.entry.open(x) if spec.entry is not None else None      # (before any layer: the stream still is what the embedding left)
-        if self.one_call:
+        by_one_call = self.one_call and self._says_its_sequences(batch)
+        if by_one_call:
             x, wanted = self._layers_by_one_call(x, batch, cache)
-        for index, call in enumerate(spec.schedule if not self.one_call else ()):
+        for index, call in enumerate(spec.schedule if not by_one_call else ()):
             block = spec.layers[call.layer]
             if call.enters:
                 spec.entry.forward(x, opened)

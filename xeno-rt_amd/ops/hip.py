@@ -394,9 +394,10 @@ class HipOps:
         self._require(batch.sequence_offsets, "sequence offsets", torch.int32, (n_seqs + 1,), x)
         self._require(batch.sequence_slots, "sequence slots", torch.int32, (n_seqs,), x)
         self._require(batch.sequence_starts, "sequence starts", torch.int32, (n_seqs,), x)
+        counts = getattr(batch, "host_counts", None)
         step = _DenseStep(x.data_ptr(), batch.positions.data_ptr(), batch.slots.data_ptr(), batch.sequence_offsets.data_ptr(), batch.sequence_slots.data_ptr(),
                           batch.sequence_starts.data_ptr(), self._stream(x), _CODES[dtype], tokens, hidden, n_seqs, int(batch.max_count), int(batch.max_context),
-                          min(batch.host_counts))
+                          min(counts) if counts else 0)
         wanted, out = None, x
         if rows is not None:
             count = rows.shape[0]
