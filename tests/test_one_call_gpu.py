@@ -131,3 +131,69 @@ def test_batches_that_say_less_of_themselves(name, dtype):
         got = forward(engine, slot, ids, [0, 70, 149], without, **changes)
         assert_logits(got, want.cpu(), dtype, f"{name} without {without} {changes}")
         assert dtype != "float32" or torch.equal(got, want), (without, changes)
+
+
+class OtherCache:
+    """A cache whose last layer's keys and values are not what the model's layers write."""
+
+    def __init__(self, cache, **changes):
+        self.cache, self.changes, self.last = cache, changes, len(cache.needs) - 1
+
+    def layer_cache(self, call):
+        from dataclasses import replace
+        layer = self.cache.layer_cache(call)
+        if call != self.last:
+            return layer
+        return replace(layer, kv=replace(layer.kv, **{name: change(getattr(layer.kv, name)) for name, change in self.changes.items()}))
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_what_a_layer_is_made_of_is_looked_at_before_anything_runs(dtype, monkeypatch):
+    """Caches, weights and norms of another type, size, layout or device are refused, as they are by the parts one by one."""
+    from xeno_rt_amd.ops.hip import KernelError, PackedMatrix
+    engine = wide_engine("qwen3", dtype)
+    slot, ids = engine.alloc_slot(), token_ids(engine.vocab_size, 40, seed=3)
+    other = torch.bfloat16 if dtype == "float32" else torch.float32
+    want = forward(engine, slot, ids, [39])
+    launched = []
+    before = engine.ops.lib.xrt_dense_blocks
+    monkeypatch.setattr(engine.ops.lib, "xrt_dense_blocks", lambda *arguments: (launched.append(1), before(*arguments))[1])
+
+    def spread(t):                                               # the same elements, each row twice as far from the next
+        return torch.stack([t, t], dim=-2).flatten(-3, -2)[..., ::2, :] if t.dim() > 1 else torch.stack([t, t], dim=-1)[..., 0]
+
+    changes = {"another type": lambda t: t.to(torch.float16), "the host": lambda t: t.cpu(), "not contiguous": spread, "fewer rows": lambda t: t[..., :-1].contiguous()}
+    for what, change in changes.items():
+        for name in ("k", "v"):
+            with pytest.raises(KernelError, match="key cache" if name == "k" else "value cache"):
+                forward(engine, slot, ids, [39], cache=OtherCache(engine.cache, **{name: change}))
+    for change in (lambda t: t.to(other), lambda t: t[:, :2].contiguous()):            # the other compute type; fewer heads
+        with pytest.raises(KernelError, match="key cache"):
+            forward(engine, slot, ids, [39], cache=OtherCache(engine.cache, k=change, v=change))
+    with pytest.raises(KernelError, match="value cache"):
+        forward(engine, slot, ids, [39], cache=OtherCache(engine.cache, v=lambda t: t[:-1]))
+    for change in (lambda t: t.long(), lambda t: t.cpu(), lambda t: t.reshape(-1), lambda t: t[:, ::2]):
+        with pytest.raises(KernelError, match="block table"):
+            forward(engine, slot, ids, [39], cache=OtherCache(engine.cache, block_table=change))
+    layer = engine.model.spec.layers[-1]
+    mixer, feed_forward = layer.mixer, layer.feed_forward
+    places = [(mixer, "w_qkv"), (mixer, "w_o"), (feed_forward, "w_gate_up"), (feed_forward, "w_down"), (mixer, "q_norm"), (mixer, "k_norm"),
+              (layer.mixer_norm, "weight"), (layer.feed_forward_norm, "weight"), (mixer.position, "theta"), (mixer.position, "table")]
+    for part, name in places:
+        held = getattr(part, name)
+        if held is None:
+            continue
+        for what, change in changes.items():
+            if isinstance(held, PackedMatrix):
+                if what == "fewer rows":
+                    changed = PackedMatrix(held.data, held.shape[0] - 16, held.shape[1], held.packing)
+                else:
+                    changed = PackedMatrix(change(held.data), *held.shape, held.packing)
+            else:
+                changed = change(held)
+            with monkeypatch.context() as patch:
+                patch.setattr(part, name, changed)
+                with pytest.raises(KernelError):
+                    forward(engine, slot, ids, [39])
+    assert not launched
+    assert torch.equal(forward(engine, slot, ids, [39]), want) and len(launched) == 2

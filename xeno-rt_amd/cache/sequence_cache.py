@@ -152,7 +152,7 @@ class SequenceCache:
 
         max_blocks = blocks_for(self.max_context)
         self.groups: List[KVGroup] = []
-        self._group_of: Dict[int, KVGroup] = {}
+        self._views: Dict[int, KVView] = {}                      # of the calls that keep keys and values
         by_spec: Dict[KVSpec, List[int]] = {}
         for call, need in enumerate(needs):
             if need is not None and need.kv is not None:
@@ -160,8 +160,8 @@ class SequenceCache:
         for spec, calls in by_spec.items():
             group = KVGroup(spec, calls, self.n_blocks, max_slots, max_blocks, dtype, device)
             self.groups.append(group)
-            for call in calls:
-                self._group_of[call] = group
+            for index, call in enumerate(calls):
+                self._views[call] = KVView(spec, group.k[index], group.v[index], group.device_table)
 
         self.states: Dict[int, torch.Tensor] = {}
         self.named_states: Dict[int, Dict[str, torch.Tensor]] = {}
@@ -256,12 +256,7 @@ class SequenceCache:
     # -- views ---------------------------------------------------------------
     def layer_cache(self, call: int) -> LayerCache:
         source = self.reads_from[call]
-        group = self._group_of.get(source)
-        kv = None
-        if group is not None:
-            index = group.calls.index(source)
-            kv = KVView(group.spec, group.k[index], group.v[index], group.device_table)
-        return LayerCache(kv=kv, state=self.states.get(source), writable=(source == call),
+        return LayerCache(kv=self._views.get(source), state=self.states.get(source), writable=(source == call),
                           states=self.named_states.get(source))
 
     # -- accounting ----------------------------------------------------------

@@ -116,8 +116,9 @@ class DecoderModel:
         """(the stream behind the layers, the rows of it that are wanted: None for all). Behind the last attention only the wanted tokens count."""
         spec, ops = self.spec, self.runtime.ops
         layers = (ops.DenseLayer * len(spec.schedule))()
+        hidden, device, seen = x.shape[1], x.get_device(), {}
         for index, call in enumerate(spec.schedule):
-            spec.layers[call.layer].describe(layers[index], cache.layer_cache(index))
+            spec.layers[call.layer].describe(layers[index], cache.layer_cache(index), hidden, device, seen)
         if spec.layers[spec.schedule[-1].layer].mixer.goes_on_with(batch):
             return ops.dense_blocks(layers, x, batch, self.runtime.dtype, rows=batch.logit_rows), None
         return ops.dense_blocks(layers, x, batch, self.runtime.dtype), batch.logit_rows

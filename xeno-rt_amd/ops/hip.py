@@ -136,15 +136,9 @@ class _LinearNorm(ctypes.Structure):
 class _DenseMatrix(ctypes.Structure):
     _fields_ = [("data", ctypes.c_void_p), ("packing", _Packing)]
 
-    def set(self, w) -> None:
-        if isinstance(w, PackedMatrix):
-            self.data, self.packing = w.data.data_ptr(), w.packing
-        else:
-            self.data, self.packing.kind = w.data_ptr(), 0
-
 
 class DenseLayer(ctypes.Structure):
-    """A layer of `dense_blocks`, as its parts describe it (`PreNormBlock.describe`)."""
+    """A layer of `dense_blocks`, as its parts describe it (`PreNormBlock.describe`): addresses, which `dense_address` and `dense_matrix` give out."""
     _fields_ = [("mixer_gain", ctypes.c_void_p), ("ff_gain", ctypes.c_void_p), ("mixer_gain_dtype", ctypes.c_int), ("ff_gain_dtype", ctypes.c_int),
                 ("mixer_eps", ctypes.c_float), ("ff_eps", ctypes.c_float), ("qkv", _DenseMatrix), ("o", _DenseMatrix), ("gate_up", _DenseMatrix),
                 ("down", _DenseMatrix), ("q_norm", ctypes.c_void_p), ("k_norm", ctypes.c_void_p), ("head_norm_dtype", ctypes.c_int),
@@ -380,7 +374,54 @@ class HipOps:
         self._check(self.lib.xrt_replace_rows(_ptr(x), _ptr(base), _ptr(copy), _code(copy), ctypes.c_long(x.numel()), self._stream(x)))
 
     DenseLayer = DenseLayer
-    dtype_codes = _CODES
+
+    # (A step describes all its layers before the first kernel starts: what there is to check of a tensor is looked at in place, and said again only of one that is wrong.)
+    def dense_address(self, tensor, what: str, dtype, shape, device: int) -> int:
+        """The address of a tensor for a DenseLayer: it lies on the GPU `device`, contiguous, with this element type and shape (None: any)."""
+        try:
+            if tensor.dtype is dtype and tensor.get_device() == device and (shape is None or tensor.shape == shape) and tensor.is_contiguous():
+                return tensor.data_ptr()
+        except AttributeError:
+            pass
+        self._require(tensor, what, dtype, shape)
+        raise KernelError(f"{what}: on {tensor.device}, expected cuda:{device}")
+
+    def dense_vector(self, tensor, what: str, size: int, device: int):
+        """(address, element type code) of a norm's gains."""
+        return self.dense_address(tensor, what, getattr(tensor, "dtype", None), (size,), device), _code(tensor)
+
+    def dense_matrix(self, into, w, what: str, dtype, shape, device: int) -> None:
+        """A weight matrix in either form into the record's matrix."""
+        if isinstance(w, PackedMatrix):
+            if w.shape != shape:
+                raise KernelError(f"{what}: shape {tuple(w.shape)}, expected {shape}")
+            into.data, into.packing = self.dense_address(w.data, what, dtype, None, device), w.packing
+        else:
+            into.data, into.packing.kind = self.dense_address(w, what, dtype, shape, device), 0
+
+    def dense_cache(self, record, kv, dtype, device: int, seen: dict) -> None:
+        """The keys and values of the record's layer. seen: what layers before it in the same step have in common with it."""
+        from ..cache import BLOCK_TOKENS
+        k, v, table = kv.k, kv.v, kv.block_table
+        record.n_blocks = n_blocks = k.shape[0]
+        record.k_cache = self.dense_address(k, "key cache", dtype, (n_blocks, record.n_kv_heads, BLOCK_TOKENS, record.head_dim), device)
+        record.v_cache = self.dense_address(v, "value cache", dtype, (n_blocks, record.n_kv_heads, record.head_dim, BLOCK_TOKENS), device)
+        if id(table) not in seen:
+            address = self.dense_address(table, "block table", torch.int32, None, device)
+            if table.dim() != 2:
+                raise KernelError("block table: expected [slots, blocks]")
+            seen[id(table)] = (address, table.shape[1], table)   # (held, so that its id stays its own)
+        record.block_table, record.table_stride, _ = seen[id(table)]
+
+    def dense_rotation(self, rotation, device: int):
+        """(rope_theta, rope_dim, rope_scale, rope_table, table_positions) for a DenseLayer; rotation: a HalfSplitRotation, or None."""
+        if rotation is None:
+            return None, 0, 0.0, None, 0
+        half, table = rotation.rope_dim // 2, rotation.table
+        theta = self.dense_address(rotation.theta, "rope_theta", torch.float32, (half,), device)
+        if table is None:
+            return theta, rotation.rope_dim, rotation.scale, None, 0
+        return theta, rotation.rope_dim, rotation.scale, self.dense_address(table, "rope_table", torch.float32, (table.shape[0], half, 2), device), table.shape[0]
 
     def dense_blocks(self, layers, x, batch, dtype, rows=None):
         """The layers of a plain dense decoder (an array of DenseLayer) on the float32 stream x, all launched by one call. rows: None, or the rows (int32)

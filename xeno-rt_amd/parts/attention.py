@@ -337,23 +337,22 @@ class Attention(Mixer):
         return batch.n_logit_rows == 0 or (batch.n_tokens > 16 and 4 * batch.n_logit_rows <= batch.n_tokens and self.q_width * self.hidden >= self.WANTED_FROM
                                            and self.q_width * size % 16 == 0 and self.kv_width * size % 8 == 0 and self.hidden % 4 == 0)
 
-    def describe(self, record, cache) -> None:
-        """This layer in the record that `ops.dense_blocks` reads."""
-        codes = self.runtime.ops.dtype_codes
-        record.qkv.set(self.w_qkv)
-        record.o.set(self.w_o)
+    def describe(self, record, cache, hidden: int, device: int, seen: dict) -> None:
+        """This layer in the record that `ops.dense_blocks` reads, for a stream of width `hidden`. seen: what the step's layers have in common."""
+        ops, dtype = self.runtime.ops, self.runtime.dtype
+        ops.dense_matrix(record.qkv, self.w_qkv, "q/k/v weight", dtype, (self.q_width + 2 * self.kv_width, hidden), device)
+        ops.dense_matrix(record.o, self.w_o, "output weight", dtype, (hidden, self.q_width), device)
         if self.qk_norm:
-            record.q_norm, record.k_norm = self.q_norm.data_ptr(), self.k_norm.data_ptr()
-            record.head_norm_dtype, record.head_norm_eps = codes[self.q_norm.dtype], self.qk_norm_eps
+            record.q_norm, record.head_norm_dtype = ops.dense_vector(self.q_norm, "q_norm", self.head_dim, device)
+            record.k_norm = ops.dense_address(self.k_norm, "k_norm", self.q_norm.dtype, (self.head_dim,), device)
+            record.head_norm_eps = self.qk_norm_eps
         record.n_heads, record.n_kv_heads, record.head_dim, record.scale = self.n_heads, self.n_kv_heads, self.head_dim, self.scale
-        rotation = None if self.position is None else self.position.rotation()
-        if rotation is not None:
-            record.rope_theta, record.rope_dim, record.rope_scale = rotation.theta.data_ptr(), rotation.rope_dim, rotation.scale
-            if rotation.table is not None:
-                record.rope_table, record.table_positions = rotation.table.data_ptr(), rotation.table.shape[0]
-        k, v, table = cache.kv.k, cache.kv.v, cache.kv.block_table
-        record.k_cache, record.v_cache, record.block_table = k.data_ptr(), v.data_ptr(), table.data_ptr()
-        record.table_stride, record.n_blocks, record.writable = table.shape[1], k.shape[0], cache.writable
+        position = self.position
+        if id(position) not in seen:                             # (one encoding may serve many layers)
+            seen[id(position)] = ops.dense_rotation(None if position is None else position.rotation(), device)
+        record.rope_theta, record.rope_dim, record.rope_scale, record.rope_table, record.table_positions = seen[id(position)]
+        ops.dense_cache(record, cache.kv, dtype, device, seen)
+        record.writable = cache.writable
 
     def _project(self, h, batch, cache):
         """q, k and v of the step's tokens, rotated, keys and values in the cache: the projection, then in one pass (in the same kernel, where a

@@ -99,15 +99,16 @@ class PreNormBlock(Block):
         return (type(self) is PreNormBlock and self.passes_norms and getattr(self.mixer, "one_call", False) and getattr(self.feed_forward, "one_call", False)
                 and self.mixer_norm.row_scale() is not None and self.feed_forward_norm.row_scale() is not None)
 
-    def describe(self, record, cache) -> None:
-        """This block in the record that `ops.dense_blocks` reads, with the cache of the call under way."""
-        codes = self.runtime.ops.dtype_codes
+    def describe(self, record, cache, hidden: int, device: int, seen: dict) -> None:
+        """This block in the record that `ops.dense_blocks` reads, with the cache of the call under way, for a stream of width `hidden` on the GPU
+        `device`. seen: a dict for the step, in which its layers note what they have in common."""
+        ops = self.runtime.ops
         gain, record.mixer_eps = self.mixer_norm.row_scale()
-        record.mixer_gain, record.mixer_gain_dtype = gain.data_ptr(), codes[gain.dtype]
+        record.mixer_gain, record.mixer_gain_dtype = ops.dense_vector(gain, "norm gain", hidden, device)
         gain, record.ff_eps = self.feed_forward_norm.row_scale()
-        record.ff_gain, record.ff_gain_dtype = gain.data_ptr(), codes[gain.dtype]
-        self.mixer.describe(record, cache)
-        self.feed_forward.describe(record)
+        record.ff_gain, record.ff_gain_dtype = ops.dense_vector(gain, "norm gain", hidden, device)
+        self.mixer.describe(record, cache, hidden, device, seen)
+        self.feed_forward.describe(record, hidden, device)
 
 
 class SandwichBlock(Block):

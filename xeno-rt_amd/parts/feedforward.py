@@ -51,10 +51,11 @@ class GatedMLP(FeedForward):
         """Whether `describe` says all there is to say of this feed-forward."""
         return type(self) is GatedMLP and self.activation == "silu"
 
-    def describe(self, record) -> None:
-        """This feed-forward in the record that `ops.dense_blocks` reads."""
-        record.gate_up.set(self.w_gate_up)
-        record.down.set(self.w_down)
+    def describe(self, record, hidden: int, device: int) -> None:
+        """This feed-forward in the record that `ops.dense_blocks` reads, for a stream of width `hidden`."""
+        ops, dtype = self.runtime.ops, self.runtime.dtype
+        ops.dense_matrix(record.gate_up, self.w_gate_up, "gate and up weight", dtype, (2 * self.intermediate, hidden), device)
+        ops.dense_matrix(record.down, self.w_down, "down weight", dtype, (hidden, self.intermediate), device)
         record.intermediate = self.intermediate
 
     def forward_into(self, h, batch, out: torch.Tensor) -> None:
