@@ -782,10 +782,10 @@ def test_attention(ops, dtype, nh, nkv, hd):
         assert rel(out[t:t + 1].cpu(), want) < (2e-5 if dtype == "float32" else 1e-2), (t, slot, pos)
 
 
-@pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 64), (5, 5, 64), (6, 2, 128), (16, 2, 64), (32, 1, 128)])
+@pytest.mark.parametrize("nh,nkv,hd", [(8, 2, 64), (5, 5, 64), (6, 2, 128), (16, 2, 64), (32, 1, 128), (10, 2, 64), (14, 2, 128)])
 def test_float32_attention_of_many_tokens_gives_the_bits_of_few(ops, nh, nkv, hd):
-    """A step of many tokens takes the matrix cores in tiles of 16 tokens, four of them a workgroup (groups of 4, 1, 3, 8 and 32 heads
-    here); the same tokens as a step that nothing describes take the general kernel. Runs of a sequence that begin and end inside tiles, padding
+    """A step of many tokens takes the matrix cores in tiles of 16 tokens, four of them a workgroup (groups of 4, 1, 3, 8, 32, 5 and 7
+    heads here); the same tokens as a step that nothing describes take the general kernel. Runs of a sequence that begin and end inside tiles, padding
     behind them, queries at the edges of blocks and of chunks of 512 keys; infinite and NaN keys and values, which only those who see them may feel."""
     lengths = [700, 130, 1, 64, 1100]          # (one, two and three chunks of 512 keys)
     kv, keys, values = filled_cache(nkv, hd, torch.float32, lengths, seed=hd + nh)
@@ -823,6 +823,20 @@ def test_float32_attention_of_many_tokens_gives_the_bits_of_few(ops, nh, nkv, hd
     many, few = attend(list(range(len(where))), True), attend(list(range(len(where))), False)
     assert bool(torch.isnan(few).any()) and bool(torch.isinf(few).any())
     assert torch.equal(torch.nan_to_num(many, nan=7.0), torch.nan_to_num(few, nan=7.0))
+
+
+def test_float32_prompts_take_the_matrix_cores_where_that_takes_less(ops):
+    """(heads, key/value heads, dims, sequences, tokens each, tokens held before): whether the step does; measured times in us there and in the general kernel."""
+    steps = [(14, 2, 64, 30, 9, 60, False), (10, 2, 64, 40, 8, 300, False), (9, 1, 64, 40, 8, 2000, False), (16, 8, 64, 30, 9, 60, False),     # 54 and 17, 105 and 51, 617 and 266, 55 and 18
+             (28, 4, 128, 11, 8, 0, False), (12, 12, 64, 40, 8, 300, False),                                                           # 52 and 10, 204 and 53
+             (32, 8, 64, 40, 8, 2000, True), (28, 4, 64, 20, 16, 2000, True), (40, 4, 64, 100, 8, 1000, True), (32, 8, 64, 1, 777, 0, True),   # 319 and 1165, 313 and 734, 409 and 745, 94 and 412
+             (32, 8, 128, 1, 777, 0, True), (12, 12, 64, 1, 300, 3000, True), (14, 2, 64, 1, 150, 0, True),                          # 189 and 763, 231 and 397, 20 and 20
+             (32, 8, 64, 100, 7, 2000, False), (32, 8, 64, 1, 64, 0, False)]                                    # fewer than eight tokens a sequence; as few pairs as the general kernel shares out
+    aligned = ctypes.c_void_p(256)
+    for nh, nkv, hd, seqs, count, held, there in steps:
+        got = ops.lib.xrt_attention_float_prompts_accepts(aligned, seqs * count, nh, nkv, hd, aligned, aligned, aligned, count, held + count)
+        assert bool(got) == there, (nh, nkv, hd, seqs, count, held)
+    assert not ops.lib.xrt_attention_float_prompts_accepts(ctypes.c_void_p(264), 777, 32, 8, 64, aligned, aligned, aligned, 777, 777)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

@@ -8,14 +8,16 @@
 // Here a block of 64 keys of 64 dims takes a workgroup 5 us, of which the matrix cores need 2 (one wavefront a SIMD, whose
 // products, softmax and waits come one after the other), and the latest tokens' blocks set the time: 777 tokens, 32 heads of 64 on 8
 // 412 -> 94 us, 100 tokens 30 -> 15, 1500 tokens 1299 -> 231; 32 heads of 128 on 8, 777 tokens 763 -> 189; 14 heads of 64 on 2, 150 tokens
-// 20 -> 20, the least that a step reaching this kernel gains. Tiles of 32 tokens (v_mfma_f32_32x32x2_f32) took 107, 22 and 279 us.
+// 20 -> 20. Tiles of 32 tokens (v_mfma_f32_32x32x2_f32) took 107, 22 and 279 us.
 //
-// A wavefront takes 16 tokens of one head, a workgroup four such tiles of one key/value head: where groups are of four heads or more
+// A wavefront takes 16 tokens of one head, a workgroup four such tiles of one key/value head: where groups are multiples of four heads
 // they are heads of the same tokens. The workgroup's tokens may be of several sequences: they are taken run by run. Scores:
 // S[key][token] with keys as rows; a lane (token = lane % 16) then holds of every 16 keys four neighbouring ones, and an
 // exchange among the quarters of the wavefront (v_permlane32_swap, v_permlane16_swap) makes them the operand of the product with the
 // values, O[dim][token]. Keys and values of the next block are on their way into registers while this block is worked on; in LDS, in
 // two stages, the elements that a quarter of a wavefront takes of 16 lie together, so that a lane reads four steps at once.
+#include <algorithm>
+
 #include "cache_layout.h"
 #include "xrt_hip.h"
 
@@ -381,31 +383,39 @@ int launch(const float* q, int row_width, int tokens, int n_heads, int n_kv_head
 
 }  // namespace
 
-// Takes steps that bring every sequence `fewest` tokens at least: the sequences whose tokens share a workgroup are passes over their keys
-// one after the other, and there must be few of them. A workgroup of 16 tokens (groups of four heads and more) is at most three passes where
-// every sequence has eight: 40 of 8 tokens at 2000, 32 heads of 64 on 8, 1164 -> 323 us, 30 of 9 at 60 36 -> 25. Smaller groups give
-// a workgroup 32 or 64 tokens and a pass fewer wavefronts (12 heads of 64, 40 of 8 at 300: 52 -> 206 us): from two tiles' tokens each on (4 of
-// 100 at 300 67 -> 51, 1 of 300 at 3000 397 -> 231). Steps of few (token, head) pairs stay with the general kernel, which shares their
-// chunks of keys out.
-static int fewest_served(int group) {
-    const int tiles = (WAVES + group - 1) / group;
-    return tiles == 1 ? TILE / 2 : tiles * TILE;
+// Whether a step of more (token, head) pairs than the general kernel shares the keys of (8 to a compute unit) takes less here than there, where one wavefront goes
+// through all keys of up to four heads of a token. In microseconds: here 4.5 a block of 64 keys of 64 dims and 2 besides, for every pass of a workgroup over
+// a sequence's keys, and as often as there are workgroups for a compute unit; there 0.04 a thousand (pair, key) of 64 dims, and no less than 0.15 a key. A workgroup's tokens
+// (16, where the heads of a tile are whole workgroups; 64 for groups of one head; else 32, of which some workgroups take parts of two tiles) may be of
+// several sequences, which are passes one after the other. Of 586 steps drawn at random (8 to 200 tokens a sequence, 1 to 148 sequences, behind 0 to 2000
+// tokens, groups of 1 to 16 heads, 64 and 128 dims) the choice is 5 % off the better of the two on average and never more than 1.5 times; by tokens a
+// sequence alone (8, or 32 and 64 where groups are smaller than four heads) it was 30 % off, up to 5 times: 30 sequences of 9 tokens at 60, 14 heads on 2, 17 us there and
+// 54 here, 40 of 8 at 300, 10 on 2, 51 and 105. What is served: 40 of 8 at 2000, 32 on 8, 1165 -> 319; 20 of 16 at 2000, 28 on 4, 734 -> 313; 1 of 300 at 3000, 12 on 12, 397 -> 231.
+static bool takes_less(int tokens, int n_heads, int n_kv_heads, int head_dim, int fewest, int max_context) {
+    const int group = n_heads / n_kv_heads, span = group % WAVES == 0 ? TILE : group == 1 ? SPAN : 2 * TILE;
+    const int passes = tokens < 2L * fewest ? 1 : 1 + (span - 2 + fewest) / fewest;
+    const double wide = head_dim / 64.0, keys = max_context, pairs = (double)tokens * n_heads;
+    const double workgroups = (tokens + TILE - 1) / TILE * (double)n_heads / WAVES;
+    const double here = 5 + passes * (4.5 * wide * ((max_context + XRT_BLOCK_TOKENS - 1) / XRT_BLOCK_TOKENS) + 2) * std::max(1.0, workgroups / XRT_COMPUTE_UNITS);
+    const double there = 9 + wide * std::max(0.15 * keys, 0.04 * pairs * (keys - 0.5 * fewest) / 1000);
+    return here <= there;
 }
 
 extern "C" int xrt_attention_float_prompts_accepts(const void* qkv, int tokens, int n_heads, int n_kv_heads, int head_dim, const void* k_cache,
-                                                   const void* v_cache, const void* out, int fewest) {
-    return (head_dim == 64 || head_dim == 128) && n_heads > 0 && n_kv_heads > 0 && n_heads % n_kv_heads == 0 && n_kv_heads <= 65535 &&
-           fewest >= fewest_served(n_heads / n_kv_heads) && (long)tokens * n_heads > 8L * XRT_COMPUTE_UNITS &&
+                                                   const void* v_cache, const void* out, int fewest, int max_context) {
+    return (head_dim == 64 || head_dim == 128) && n_heads > 0 && n_kv_heads > 0 && n_heads % n_kv_heads == 0 && n_kv_heads <= XRT_GRID_ROWS &&
+           fewest >= TILE / 2 && (long)tokens * n_heads > 8L * XRT_COMPUTE_UNITS && max_context > 0 &&
+           takes_less(tokens, n_heads, n_kv_heads, head_dim, fewest, max_context) &&
            (uintptr_t)qkv % 16 == 0 && (uintptr_t)out % 16 == 0 && (uintptr_t)k_cache % 32 == 0 && (uintptr_t)v_cache % 32 == 0;
 }
 
 extern "C" int xrt_attention_float_prompts(const void* qkv, int tokens, int n_heads, int n_kv_heads, int head_dim, const void* k_cache,
                                            const void* v_cache, const int* block_table, int table_stride, int n_blocks, const int* positions,
-                                           const int* slots, void* out, float scale, int fewest, void* stream) {
+                                           const int* slots, void* out, float scale, int fewest, int max_context, void* stream) {
     XRT_REQUIRE(qkv && k_cache && v_cache && block_table && positions && slots && out, "attention (float32 prompts): null operand");
     XRT_REQUIRE(table_stride > 0 && n_blocks > 0, "attention (float32 prompts): empty cache");
-    XRT_REQUIRE(xrt_attention_float_prompts_accepts(qkv, tokens, n_heads, n_kv_heads, head_dim, k_cache, v_cache, out, fewest),
-                "attention (float32 prompts): %d tokens, %d at least a sequence, %d/%d heads of %d dims are not served", tokens, fewest, n_heads, n_kv_heads, head_dim);
+    XRT_REQUIRE(xrt_attention_float_prompts_accepts(qkv, tokens, n_heads, n_kv_heads, head_dim, k_cache, v_cache, out, fewest, max_context),
+                "attention (float32 prompts): %d tokens, %d at least a sequence, up to %d keys, %d/%d heads of %d dims are not served", tokens, fewest, max_context, n_heads, n_kv_heads, head_dim);
     const int row_width = (n_heads + 2 * n_kv_heads) * head_dim;
     hipStream_t s = (hipStream_t)stream;
     if (head_dim == 64)

@@ -57,7 +57,7 @@ struct Room { void* values; float* squares; };
 bool wanted_alone(const xrt_dense_step& s, const xrt_dense_layer& l, const void* qkv, int rows) {
     if (s.dtype == XRT_F32)
         return (long)rows * l.n_heads <= 8L * XRT_COMPUTE_UNITS ||
-               !xrt_attention_float_prompts_accepts(qkv, s.tokens, l.n_heads, l.n_kv_heads, l.head_dim, l.k_cache, l.v_cache, qkv, s.fewest);
+               !xrt_attention_float_prompts_accepts(qkv, s.tokens, l.n_heads, l.n_kv_heads, l.head_dim, l.k_cache, l.v_cache, qkv, s.fewest, s.max_context);
     if (!xrt_attention_decode_accepts(l.head_dim)) return true;                // (the general kernel, a token at a time either way)
     if (rows > XRT_GRID_ROWS) return false;
     const double keys = std::max(1.0, s.max_context - 0.5 * s.max_count), row = (200 + 0.008 * keys) * (l.n_kv_heads * l.head_dim / 1024.0) * keys / 1000;
@@ -110,10 +110,10 @@ struct Step {
     // attention over the cache for `rows` queries in rows of `qkv`
     int attention(const xrt_dense_layer& l, const void* qkv, int rows, const int* positions, const int* slots, const int* offsets, const int* seq_slots,
                   const int* starts, int n_seqs, int max_count, int fewest, const xrt_qkv_finish* finish, void* out) {
-        if (s.dtype == XRT_F32 && xrt_attention_float_prompts_accepts(qkv, rows, l.n_heads, l.n_kv_heads, l.head_dim, l.k_cache, l.v_cache, out, fewest)) {
+        if (s.dtype == XRT_F32 && xrt_attention_float_prompts_accepts(qkv, rows, l.n_heads, l.n_kv_heads, l.head_dim, l.k_cache, l.v_cache, out, fewest, s.max_context)) {
             if (arena.plan) return 0;
             return xrt_attention_float_prompts(qkv, rows, l.n_heads, l.n_kv_heads, l.head_dim, l.k_cache, l.v_cache, l.block_table, l.table_stride, l.n_blocks,
-                                               positions, slots, out, l.scale, fewest, s.stream);
+                                               positions, slots, out, l.scale, fewest, s.max_context, s.stream);
         }
         const long need = xrt_attention_workspace(s.dtype, rows, l.n_heads, l.n_kv_heads, l.head_dim, 0, max_count, s.max_context);
         const long before = arena.at;

@@ -314,14 +314,14 @@ int xrt_attention_stretches(const void* q, long q_stride, int dtype, int tokens,
                             const int* seq_offsets, const int* seq_slots, const int* seq_starts, int n_seqs, void* out,
                             float scale, int chunk, const float* distance_bias, int bias_span, const float* sink_scores, void* stream);
 
-// Plain causal attention of a float32 step that brings every sequence `fewest` tokens at least, on the matrix cores, to the bits of
-// xrt_attention (rows of qkv as there). `accepts` says which steps: heads of 64 or 128 dims, more (token, head) pairs than a
-// decode step has, aligned operands.
+// Plain causal attention of a float32 step that brings every sequence `fewest` tokens at least and the longest to `max_context`, on the matrix cores, to the
+// bits of xrt_attention (rows of qkv as there). `accepts` says which steps: heads of 64 or 128 dims, eight tokens a sequence or more, more (token, head)
+// pairs than a decode step has and so many that it takes less time here, aligned operands.
 int xrt_attention_float_prompts_accepts(const void* qkv, int tokens, int n_heads, int n_kv_heads, int head_dim, const void* k_cache,
-                                        const void* v_cache, const void* out, int fewest);
+                                        const void* v_cache, const void* out, int fewest, int max_context);
 int xrt_attention_float_prompts(const void* qkv, int tokens, int n_heads, int n_kv_heads, int head_dim, const void* k_cache,
                                 const void* v_cache, const int* block_table, int table_stride, int n_blocks, const int* positions,
-                                const int* slots, void* out, float scale, int fewest, void* stream);
+                                const int* slots, void* out, float scale, int fewest, int max_context, void* stream);
 
 // The layers of a plain dense decoder from one call (dense_blocks.hip): for each of `count` layers in turn the RMSNorm of the float32 stream x, q/k/v with
 // head norms, rotation and cache write, causal attention, the output projection onto x, the second norm, the gated (silu) product and the one back onto x, with the kernels and operands

@@ -688,10 +688,10 @@ class HipOps:
             if qkv.dtype == torch.float32 and not window and distance_slopes is None and counts:
                 # float32 prompts: the matrix cores, to the bits of the general kernel
                 fewest, k_at, v_at, q_at, out_at = min(counts), _ptr(k_cache), _ptr(v_cache), _ptr(qkv), _ptr(out)
-                if self.lib.xrt_attention_float_prompts_accepts(q_at, tokens, n_heads, n_kv_heads, head_dim, k_at, v_at, out_at, fewest):
+                if self.lib.xrt_attention_float_prompts_accepts(q_at, tokens, n_heads, n_kv_heads, head_dim, k_at, v_at, out_at, fewest, max_context):
                     self._check(self.lib.xrt_attention_float_prompts(
                         q_at, tokens, n_heads, n_kv_heads, head_dim, k_at, v_at, _ptr(table), stride, n_blocks, _ptr(batch.positions), _ptr(batch.slots),
-                        out_at, ctypes.c_float(scale), fewest, self._stream(qkv)))
+                        out_at, ctypes.c_float(scale), fewest, max_context, self._stream(qkv)))
                     return None
             if distance_slopes is None:                         # (the general kernel, which serves those, needs none)
                 workspace_floats = int(self.lib.xrt_attention_workspace(_code(qkv), tokens, n_heads, n_kv_heads, head_dim,
