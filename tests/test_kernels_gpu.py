@@ -450,15 +450,41 @@ def test_rmsnorm_done_by_the_second_kernel_of_a_product_of_many_rows(ops, m, hid
     assert float(normed[m - 1].abs().max()) == 0.0
 
 
+def parts_of(ops, m, n, k, mode, whole_norm=False):
+    """(a tile's rows of x, its rows of w, the parts along k) of a product."""
+    rows, columns = ctypes.c_int(), ctypes.c_int()
+    parts = ops.lib.xrt_linear_parts(m, n, k, {"store": 0, "add": 1, "gated": 2}[mode], int(whole_norm), ctypes.byref(rows), ctypes.byref(columns))
+    return rows.value, columns.value, parts
+
+
+@pytest.mark.parametrize("mode", ["gated", "store", "add"])
+def test_parts_along_k_make_one_round_on_every_die(ops, mode):
+    """Tiles are dealt to the eight dies in equal runs, the same in every part: what counts against a die's 32 compute units is its run times the parts. (With the
+    workgroups' number alone counted, 298 rows of x and 5328 of w went into six parts: 36 workgroups on seven dies, none on the eighth.)"""
+    taken = 0
+    for m in (150, 193, 224, 298, 333, 385, 409, 465, 500, 777):
+        for rows_w in (1744, 2192, 4096, 5120, 5328, 6800, 7040, 9736, 10240, 10720):
+            for k in (2048, 4672, 8192, 9664, 17280, 25600):
+                rows, columns, parts = parts_of(ops, m, rows_w // 2 if mode == "gated" else rows_w, k, mode)
+                if rows == 192:
+                    taken += 1
+                    run = -(-(-(-m // rows) * -(-rows_w // columns)) // 8)
+                    assert parts * run <= 32, (m, rows_w, k, parts)
+    assert taken > 50
+
+
 @pytest.mark.parametrize("m,n,k", [(65, 1024, 768), (128, 1032, 256), (129, 96, 1024), (256, 3072, 1024), (100, 8192, 512),      # gated: one round of 128 x 64
                                    (65, 9000, 384), (200, 8192, 256), (129, 5000, 512),                                        # of 128 x 128
                                    (257, 12320, 1024), (333, 12328, 1024), (384, 12320, 1088),                                 # tiles of 192 rows
-                                   (700, 1000, 8192), (150, 5128, 5120), (192, 6000, 4096), (333, 2056, 14336), (193, 2048, 16384)])     # the last four: parts of 192 rows
+                                   (700, 1000, 8192), (193, 2048, 16384),
+                                   (150, 5128, 5120), (192, 6000, 4096), (333, 2056, 14336), (193, 4872, 6144)])              # parts of 192 rows
 @pytest.mark.parametrize("mode", ["gated", "store", "add"])
 @pytest.mark.parametrize("packed", [False, True])
 def test_products_of_some_hundred_rows_in_every_tile(ops, m, n, k, mode, packed):
     """Against float32 products on the GPU: sums of k products of bfloat16 numbers in another order differ by a few 1e-6 of the largest; bfloat16
     results by half of their last place more."""
+    if (m, n) in ((150, 5128), (192, 6000), (333, 2056), (193, 4872)):
+        assert parts_of(ops, m, n if mode == "gated" else 2 * n, k, mode)[:2] == (192, 256)
     a = rand(m, k, dtype=torch.bfloat16, seed=1)
     w = rand(2 * n, k, dtype=torch.bfloat16, seed=2, scale=1.0 / math.sqrt(k))
     sums = a.float() @ w.float().t()

@@ -1099,11 +1099,17 @@ struct SplitPlan { int splits, k_per_split; long rows_w; int tile, columns; };  
 // products drawn at random afterwards ran 1.34 times as fast up to 128 rows, 1.17 up to 256, 1.13 up to 512, 1.1 beyond (worst: 0.84, two
 // more below 0.92): 4096 rows of w, k = 1024, 100 rows of x 14.5 -> 10.6 us, 1024 rows, k = 3072, 333 rows of x 18.1 -> 13.3, 2048 rows, k = 8192, 100 rows
 // of x 20.8 -> 18.3, 5120 rows, k = 25600, 100 rows of x 85.9 -> 61.6; those of the 8B models stay within 4 % of what they were.
+// Workgroups are counted as the fullest die has them: counting their number alone put two rounds on seven of the eight dies where the tiles are no multiple of
+// eight (298 rows of x, 5328 rows of w in pairs, k = 9664: 77 us, 55 by the rule before this estimate; 140 rows, 5120 rows, k = 25600 96, now 70). Of 1086 more products drawn
+// at random, 65 to 1800 rows of x, k up to 26000, 46 took over 5 % longer by it than by that rule, up to 1.42 times; counted so 7 do, up to 1.18, and the average of all is 0.875.
 struct PartTime { int columns, places, once, step, share, beside, part, sums; };
+constexpr int DIES = 8;
+// Tiles are dealt to the dies in equal runs (tile_place): what the largest run comes to on all of them.
+long dealt(long tiles) { return (tiles + DIES - 1) / DIES * DIES; }
 constexpr PartTime NARROW_PARTS = {64, 2, 5950, 256, 166, 95, 250, 1540}, WIDE_PARTS = {128, 1, 6630, 445, 200, 0, 251, 1720},
                    WIDE_PARTS_TWO = {128, 2, 7190, 592, 237, 0, 268, 1050};          // (two stages instead of three: two to a compute unit, beyond 256 rows)
 long parts_time(const PartTime& shape, int M, long N, int steps, int parts) {
-    const long groups = (long)((M + 127) / 128) * ((N + shape.columns - 1) / shape.columns) * parts, places = (long)shape.places * XRT_COMPUTE_UNITS;
+    const long groups = dealt((long)((M + 127) / 128) * ((N + shape.columns - 1) / shape.columns)) * parts, places = (long)shape.places * XRT_COMPUTE_UNITS;
     const long whole = groups / places, rest = groups % places;
     const long full = shape.step + shape.share * shape.places + shape.beside;
     const long last = rest == 0 ? 0 : shape.step + shape.share * rest / XRT_COMPUTE_UNITS + (rest > XRT_COMPUTE_UNITS ? shape.beside : 0);
@@ -1165,10 +1171,8 @@ SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
             // Large tiles of 192 rows, in parts that make one round: fewer operands read a product, more at the ends (beside the best of the others: 333 rows
             // of x, 5120 rows of w, k = 25600 129 -> 113 us, 4096 rows, k = 14336 61 -> 58, but k = 4096 30 -> 33; 150 rows of x, 10240 rows of w, k = 5120
             // 43 -> 34). The figures are of those and 100 more such products.
-            const long large = (long)((M + 191) / 192) * ((rows_w + 255) / 256);
-            // Not for one row of tiles on a w beyond the caches, which the smaller tiles' three stages stream faster (150 rows, 5120 rows of w, k = 25600 94 against 101 us).
-            const bool suits = M > 192 || (M > 128 && rows_w * K * (long)sizeof(bf16) <= 150L * 1000 * 1000);
-            for (int parts = 2; suits && parts <= 16 && parts <= units && parts * large <= XRT_COMPUTE_UNITS; ++parts) {
+            const long large = dealt((long)((M + 191) / 192) * ((rows_w + 255) / 256));
+            for (int parts = 2; M > 128 && parts <= 16 && parts <= units && parts * large <= XRT_COMPUTE_UNITS; ++parts) {
                 const int per = (units + parts - 1) / parts;
                 if ((units + per - 1) / per != parts) continue;
                 const long time = 10000 + 1200L * per + 1400L * parts * (M * rows_w / 1000) / 1000;
@@ -1459,8 +1463,7 @@ int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, c
     if (plan.columns == 64) {
         // a fourth stage where a compute unit has one workgroup anyway (2048 rows of w, k = 8192, 65 / 200 rows of x 16.0 / 22.5 -> 14.7 / 20.5 us with its
         // second kernel; k = 2048, 3072 rows, 100 rows of x 12.0 -> 11.5)
-        const long groups = (long)((M + 127) / 128) * ((rows_w + 63) / 64) * plan.splits;
-        if (groups <= XRT_COMPUTE_UNITS)
+        if (dealt((long)((M + 127) / 128) * ((rows_w + 63) / 64)) * plan.splits <= XRT_COMPUTE_UNITS)
             return launch_kernel<128, 64, 4, 1, MODE_STORE, 64, 4, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
         return launch_kernel<128, 64, 2, 2, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
     }
@@ -1634,6 +1637,14 @@ bool xrt_linear_split_takes_qkv(const void* a, const void* w, int M, int N, int 
 int xrt_linear_split_qkv(const void* a, const void* w, void* qkv, int M, int N, int K, const Packing& packing, float* workspace,
                          const xrt_linear_norm* norm, const QkvAfter& after, hipStream_t s) {
     return launch_split<bf16>((const bf16*)a, (const bf16*)w, (bf16*)qkv, M, N, K, MODE_STORE, XRT_ACT_SILU, packing, workspace, norm, &after, s);
+}
+
+// How a product is cut that runs through the tiles of this section: the number of parts along k (1: not cut, another kernel's if M > 64), a tile's rows of x and of w.
+extern "C" int xrt_linear_parts(int M, int N, int K, int mode, int whole_norm, int* rows, int* columns) {
+    const SplitPlan plan = split_plan(M, N, K, mode, whole_norm != 0);
+    *rows = plan.tile;
+    *columns = plan.columns;
+    return plan.splits;
 }
 
 // The first kernel alone of a bfloat16 product split along k (xrt_linear_split_takes says so and asks for a workspace): the sums of the parts,

@@ -126,6 +126,9 @@ typedef struct xrt_linear_norm {
 int xrt_linear_takes_norm(const void* a, const void* w, const xrt_packing* packing, int dtype, int M, int N, int K, int mode);
 int xrt_linear_norm_tiles(const void* a, const void* w, const xrt_packing* packing, int dtype, int M, int N, int K);   // rows of the table at squares_out
 long xrt_linear_whole_norm_workspace(const void* a, const void* w, int dtype, int M, int N, int K, int mode);
+// How a bfloat16 product of more than 16 rows and whole steps of 64 along k is cut along k: returns the number of parts (1: it is not), and a tile's rows
+// of x and of w. whole_norm: as one whose second kernel does the norm after it.
+int xrt_linear_parts(int M, int N, int K, int mode, int whole_norm, int* rows, int* columns);
 int xrt_linear_normed(const void* a, const void* w, const xrt_packing* packing, int dtype, void* out, int out_dtype, int M, int N,
                       int K, int mode, const xrt_linear_norm* norm, float* workspace, long workspace_floats, void* stream);
 
