@@ -1086,7 +1086,7 @@ def test_attention_decode_that_finishes_q_k_and_v_itself(ops, nh, nkv, hd, rotat
     assert float(same.float().mean()) > 0.999               # only the newest keys can differ at all, by a rounding
 
 
-@pytest.mark.parametrize("longest", [64, 65, 256, 257, 512, 513, 960, 961, 1100])      # (961: eight wavefronts of two blocks each for more than 256 pairs)
+@pytest.mark.parametrize("longest", [64, 65, 256, 257, 512, 513, 960, 961, 1100])
 @pytest.mark.parametrize("nh,nkv,hd,tokens", [(8, 4, 128, 2), (8, 4, 128, 65), (12, 4, 64, 64), (20, 1, 64, 3)])
 def test_attention_decode_of_short_contexts(ops, nh, nkv, hd, tokens, longest):
     """The longest sequence at the edges of four and eight blocks of keys: workgroups of four wavefronts, of eight (a block each, up to 256 pairs of
