@@ -711,6 +711,7 @@ def test_linear_qkv_in_one_kernel(ops, nh, nkv, hd, rope_dim, k, tokens, packed)
 
 @pytest.mark.parametrize("nh,nkv,hd,rope_dim,k,tokens", [(32, 8, 64, 64, 2048, 100), (16, 8, 128, 128, 1024, 65), (32, 8, 128, 128, 4096, 333), (4, 2, 16, 16, 512, 70),
                                                           (3, 1, 256, 256, 1024, 127), (6, 2, 32, 0, 768, 128), (64, 8, 128, 128, 512, 40),
+                                                          (8, 4, 64, 64, 2048, 40),      # sixteen parts: added by it where the values are written apart
                                                           (4, 2, 128, 64, 512, 90), (3, 3, 48, 48, 512, 100)])      # the last two: kernels of their own
 @pytest.mark.parametrize("norm_dtype", [None, torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("longest_run", [1, 100])

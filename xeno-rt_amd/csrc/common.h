@@ -18,6 +18,8 @@ enum { XRT_F32 = 0, XRT_BF16 = 1 };
 #define XRT_COMPUTE_UNITS 256
 // the most workgroups in a grid's second and third dimension
 #define XRT_GRID_ROWS 65535
+// new tokens of some sequence from which a step's values go to the cache through workgroups that turn them (qkv_prepare.hip)
+#define XRT_QKV_VALUES_APART 32
 
 // ---- error reporting -------------------------------------------------------
 void xrt_set_error(const char* format, ...);

@@ -359,7 +359,7 @@ static int prepare(void* qkv, const QkvParts& parts, int dtype, int tokens, int 
     if (lanes > 0) {
         // sequences that bring many tokens: their values go through the workgroups that turn them;
         // otherwise element by element from those that do the heads
-        const bool values_apart = v_cache != nullptr && longest_run >= XRT_WAVE / 2;
+        const bool values_apart = v_cache != nullptr && longest_run >= XRT_QKV_VALUES_APART;
         const int value_tiles = values_apart ? (tokens + XRT_WAVE - 1) / XRT_WAVE : 0;
         // a workgroup per token, which walks the heads; with parts, whose sums have a long way, as many as the heads fill
         const int heads = n_heads + (values_apart ? 1 : 2) * n_kv_heads, heads_at_once = WAVES * (XRT_WAVE / lanes);
