@@ -222,8 +222,8 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) qkv_prepare_vector_kernel(
     float* cosines = shared.angles.cosines;
     float* sines = shared.angles.sines;
     const int wave = threadIdx.x / XRT_WAVE, lane = threadIdx.x % XRT_WAVE;
-    const int item = (int)blockIdx.x - value_blocks;
-    const int token = item / chunks, chunk = item % chunks;
+    const int item = (int)blockIdx.x - value_blocks, chunks_here = PARTS ? chunks : 1;      // (a division less where it is known)
+    const int token = item / chunks_here, chunk = item % chunks_here;
     const int pos = positions[token];
     const int slot = slots[token];
     if (rope_theta != nullptr) {
@@ -237,7 +237,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) qkv_prepare_vector_kernel(
     const int heads_total = n_heads + 2 * n_kv_heads;
     const int within = pos % XRT_BLOCK_TOKENS;
     const int heads_here = value_blocks == 0 ? heads_total : n_heads + n_kv_heads;     // value heads come last
-    for (int head = (chunk * WAVES + wave) * HEADS_PER_WAVE + lane / LANES; head < heads_here; head += chunks * WAVES * HEADS_PER_WAVE) {
+    for (int head = (chunk * WAVES + wave) * HEADS_PER_WAVE + lane / LANES; head < heads_here; head += chunks_here * WAVES * HEADS_PER_WAVE) {
         // lanes of one head stay together: the exchanges below are within a head
         const bool is_q = head < n_heads, is_v = head >= n_heads + n_kv_heads, is_k = !is_q && !is_v;
         const long row_at = (long)token * heads_total * HEAD + (long)head * HEAD;
