@@ -163,17 +163,41 @@ def test_linear_float32_has_the_same_bits_with_few_rows_and_with_many(ops, m, n,
             assert torch.equal(torch.nan_to_num(got, nan=7.0), torch.nan_to_num(want, nan=7.0))
 
 
-# The tiles of eight wavefronts (256 and 128 rows by 256) and those of 256 x 192 at the edges of tiles, with one, two and three steps along
-# k and more, columns that do and do not allow 16 bytes a store. By the rule of the launcher the last six are half, half, large, large, mixed
-# and mixed for every kind of result; (520, 16128, 320), (393, 16400, 64) and (2816, 3070, 512) are large for bfloat16 results and the tiles of 256 x 192
-# for float32 ones; of the others the bfloat16 results are large or mixed, the float32 ones tiles of 128 x 128.
+MODES = {"store": 0, "add": 1, "gated": 2}
+TILES = ["256", "192", "128", "256 and 128", "256 x 192", "128 x 128", "128 x 128, three stages", "128 x 64, four stages", "256, ragged", "128, ragged"]
+
+
+def parts_of(ops, m, n, k, mode, whole_norm=False):
+    """(a tile's rows of x, its rows of w, the parts along k) of a product."""
+    rows, columns = ctypes.c_int(), ctypes.c_int()
+    parts = ops.lib.xrt_linear_parts(m, n, k, MODES[mode], int(whole_norm), ctypes.byref(rows), ctypes.byref(columns))
+    return rows.value, columns.value, parts
+
+
+def tiles_of(ops, dtype, m, n, k, mode):
+    """The tiles of a product of more than 64 rows (rows of x by 256 of w, where there is one number), or that it is cut along k."""
+    if k >= 128 and k % 64 == 0 and parts_of(ops, m, n, k, mode)[2] > 1:
+        return "parts"
+    return TILES[ops.lib.xrt_linear_tiles(0 if dtype == torch.float32 else 1, m, n, k, MODES[mode])]
+
+
+# The tiles of eight wavefronts (256, 192 and 128 rows by 256) and those of 256 x 192 at the edges of tiles, with one, two and three steps along
+# k and more, columns that do and do not allow 16 bytes a store; by the rule of the launcher: for a bfloat16 result, adding, for a float32 result.
+LARGE = {(250, 61001, 64): ("256", "128 x 128", "128 x 128"), (257, 47104, 128): ("192", "128 x 128", "128 x 128"), (130, 61440, 192): ("192", "192", "192"),
+         (520, 16128, 320): ("192", "256 x 192", "192"), (1100, 16000, 128): ("192", "128 x 128", "128 x 128"), (2048, 11008, 64): ("256 and 128", "128 x 128", "128 x 128"),
+         (393, 16400, 64): ("192", "256 x 192", "256 x 192"), (2816, 3070, 512): ("192", "256 x 192", "256 x 192"), (270, 16890, 2496): ("128", "128", "128"),
+         (1900, 4090, 2496): ("128", "128", "128"), (531, 16561, 1984): ("192", "192", "192"), (520, 16640, 1984): ("192", "192", "192"),
+         (778, 18840, 3008): ("192", "192", "192"), (1030, 19712, 1984): ("192", "192", "192"), (778, 13061, 1984): ("256", "256", "256"),
+         (778, 13312, 1984): ("256", "256", "256"), (2000, 8215, 1984): ("256 and 128", "256 and 128", "256 and 128"),
+         (1000, 16640, 1984): ("256 and 128", "256 and 128", "256 and 128")}
+
+
 @pytest.mark.parametrize("kind", ["plain", "packed", "rotary"])
-@pytest.mark.parametrize("m,n,k", [(250, 61001, 64), (257, 47104, 128), (130, 61440, 192), (520, 16128, 320), (1100, 16000, 128), (2048, 11008, 64),
-                                   (393, 16400, 64), (2816, 3070, 512),
-                                   (270, 16890, 2496), (1900, 4090, 2496), (531, 16561, 1984), (520, 16640, 1984), (778, 18840, 3008), (1030, 19712, 1984)])
+@pytest.mark.parametrize("m,n,k", list(LARGE))
 def test_linear_large_tiles(ops, m, n, k, kind):
     if kind == "rotary" and n % 256 != 0:
         pytest.skip("whole heads")
+    assert (tiles_of(ops, torch.bfloat16, m, n, k, "store"), tiles_of(ops, torch.float32, m, n, k, "add"), tiles_of(ops, torch.float32, m, n, k, "store")) == LARGE[(m, n, k)]
     a = rand(m, k, dtype=torch.bfloat16, seed=m)
     w = rand(n, k, dtype=torch.bfloat16, seed=n, scale=0.1)
     want = (a.double() @ w.double().t()).cpu()
@@ -190,11 +214,15 @@ def test_linear_large_tiles(ops, m, n, k, kind):
     assert rel(out32.cpu(), want) < 1e-5
 
 
-# (large, mixed, large, large, mixed; then half, half, mixed)
+LARGE_GATED = {(250, 30504, 64): "256", (257, 24000, 128): "192", (140, 31000, 192): "192", (520, 8200, 320): "192", (2048, 5504, 64): "256 and 128",
+               (140, 8032, 704): "128 x 128, three stages", (2040, 2040, 64): "128", (790, 9352, 64): "256 and 128", (778, 6536, 320): "256", (778, 6544, 1984): "256",
+               (778, 9352, 320): "256 and 128", (2000, 4144, 1984): "256 and 128", (257, 5320, 320): "128", (270, 8440, 2496): "128"}
+
+
 @pytest.mark.parametrize("packed", [False, True])
-@pytest.mark.parametrize("m,n,k", [(250, 30504, 64), (257, 24000, 128), (140, 31000, 192), (520, 8200, 320), (2048, 5504, 64),
-                                   (140, 8032, 704), (2040, 2040, 64), (790, 9352, 64)])
+@pytest.mark.parametrize("m,n,k", list(LARGE_GATED))
 def test_linear_glu_large_tiles(ops, m, n, k, packed):
+    assert {tiles_of(ops, dtype, m, n, k, "gated") for dtype in (torch.bfloat16, torch.float32)} == {LARGE_GATED[(m, n, k)]}
     a = rand(m, k, dtype=torch.bfloat16, seed=m)
     w = rand(2 * n, k, dtype=torch.bfloat16, seed=n, scale=0.3)
     both = a.double() @ w.double().t()
@@ -206,12 +234,17 @@ def test_linear_glu_large_tiles(ops, m, n, k, packed):
         assert rel(out.cpu(), want) < (ULP["bfloat16"] * 2 if dtype == torch.bfloat16 else 1e-5)
 
 
-# Results that do not begin at a multiple of 16 bytes go out in single elements: the same bits (large tiles, both shapes in a launch, half
-# tiles, by kind of result; the padding around the result stays).
-@pytest.mark.parametrize("m,n,k,kind", [(520, 16640, 1984, "store"), (1030, 19712, 1984, "store"), (270, 16888, 2496, "store"), (520, 8200, 320, "gated"),
-                                        (790, 9352, 64, "gated"), (140, 8032, 704, "gated"), (531, 16560, 1984, "add"), (1900, 4096, 2496, "add")])
+# Results that do not begin at a multiple of 16 bytes go out in single elements: the same bits (every kind of tile, by kind of result; the
+# padding around the result stays).
+@pytest.mark.parametrize("m,n,k,kind,tiles", [(520, 16640, 1984, "store", "192"), (1030, 19712, 1984, "store", "192"), (270, 16888, 2496, "store", "128"),
+                                              (778, 13312, 1984, "store", "256"), (1000, 16640, 1984, "store", "256 and 128"),
+                                              (520, 8200, 320, "gated", "192"), (790, 9352, 64, "gated", "256 and 128"), (140, 8032, 704, "gated", "128 x 128, three stages"),
+                                              (778, 6536, 320, "gated", "256"), (257, 5320, 320, "gated", "128"),
+                                              (531, 16560, 1984, "add", "192"), (1900, 4096, 2496, "add", "128"), (778, 13312, 1984, "add", "256"),
+                                              (1000, 16640, 1984, "add", "256 and 128")])
 @pytest.mark.parametrize("packed", [False, True])
-def test_large_tiles_into_a_result_that_is_not_aligned(ops, m, n, k, kind, packed):
+def test_large_tiles_into_a_result_that_is_not_aligned(ops, m, n, k, kind, tiles, packed):
+    assert tiles_of(ops, torch.float32 if kind == "add" else torch.bfloat16, m, n, k, kind) == tiles
     a, w = rand(m, k, dtype=torch.bfloat16, seed=m), rand(2 * n if kind == "gated" else n, k, dtype=torch.bfloat16, seed=n, scale=0.1)
     w = packed_or_not(ops, w, packed, "gated" if kind == "gated" else "tiles", **({"gated_n": n} if kind == "gated" else {}))
     dtype = torch.float32 if kind == "add" else torch.bfloat16
@@ -450,13 +483,6 @@ def test_rmsnorm_done_by_the_second_kernel_of_a_product_of_many_rows(ops, m, hid
     assert float(normed[m - 1].abs().max()) == 0.0
 
 
-def parts_of(ops, m, n, k, mode, whole_norm=False):
-    """(a tile's rows of x, its rows of w, the parts along k) of a product."""
-    rows, columns = ctypes.c_int(), ctypes.c_int()
-    parts = ops.lib.xrt_linear_parts(m, n, k, {"store": 0, "add": 1, "gated": 2}[mode], int(whole_norm), ctypes.byref(rows), ctypes.byref(columns))
-    return rows.value, columns.value, parts
-
-
 @pytest.mark.parametrize("mode", ["gated", "store", "add"])
 def test_parts_along_k_make_one_round_on_every_die(ops, mode):
     """Tiles are dealt to the eight dies in equal runs, the same in every part: what counts against a die's 32 compute units is its run times the parts. (With the
@@ -473,17 +499,22 @@ def test_parts_along_k_make_one_round_on_every_die(ops, mode):
     assert taken > 50
 
 
-@pytest.mark.parametrize("m,n,k", [(65, 1024, 768), (128, 1032, 256), (129, 96, 1024), (256, 3072, 1024), (100, 8192, 512),      # gated: one round of 128 x 64
-                                   (65, 9000, 384), (200, 8192, 256), (129, 5000, 512),                                        # of 128 x 128
-                                   (257, 12320, 1024), (333, 12328, 1024), (384, 12320, 1088),                                 # tiles of 192 rows
-                                   (700, 1000, 8192), (193, 2048, 16384),
-                                   (150, 5128, 5120), (192, 6000, 4096), (333, 2056, 14336), (193, 4872, 6144)])              # parts of 192 rows
+# what the gated products take; "parts of 192": cut along k into tiles of that many rows, as the others of the size are
+SOME_HUNDRED = {(65, 1024, 768): "128 x 64, four stages", (128, 1032, 256): "128 x 64, four stages", (129, 96, 1024): "parts", (256, 3072, 1024): "128 x 64, four stages",
+                (100, 8192, 512): "128 x 64, four stages", (65, 9000, 384): "128 x 128, three stages", (200, 8192, 256): "128 x 128, three stages",
+                (129, 5000, 512): "128 x 128, three stages", (257, 12320, 1024): "192", (333, 12328, 1024): "192", (384, 12320, 1088): "192", (700, 1000, 8192): "parts",
+                (193, 2048, 16384): "parts", (150, 5128, 5120): "parts of 192", (192, 6000, 4096): "parts of 192", (333, 2056, 14336): "parts of 192",
+                (193, 4872, 6144): "parts of 192"}
+
+
+@pytest.mark.parametrize("m,n,k", list(SOME_HUNDRED))
 @pytest.mark.parametrize("mode", ["gated", "store", "add"])
 @pytest.mark.parametrize("packed", [False, True])
 def test_products_of_some_hundred_rows_in_every_tile(ops, m, n, k, mode, packed):
     """Against float32 products on the GPU: sums of k products of bfloat16 numbers in another order differ by a few 1e-6 of the largest; bfloat16
     results by half of their last place more."""
-    if (m, n) in ((150, 5128), (192, 6000), (333, 2056), (193, 4872)):
+    assert SOME_HUNDRED[(m, n, k)].startswith(tiles_of(ops, torch.bfloat16, m, n, k, "gated"))
+    if SOME_HUNDRED[(m, n, k)] == "parts of 192":
         assert parts_of(ops, m, n if mode == "gated" else 2 * n, k, mode)[:2] == (192, 256)
     a = rand(m, k, dtype=torch.bfloat16, seed=1)
     w = rand(2 * n, k, dtype=torch.bfloat16, seed=2, scale=1.0 / math.sqrt(k))

@@ -999,26 +999,27 @@ long rounds_cost(long tiles, const TileTime& tile, int K, int kind) {        // 
     return whole * round + (rest == 0 ? 0 : (tile.least * (long)tile.places + (100 - tile.least) * rest) * round / (100L * tile.places));
 }
 
+// The tiles of a product without a split along k: rows of a by rows of w, and beside them the stages where there is more than one choice.
+enum TileShape { TILES_256, TILES_192, TILES_128, TILES_256_AND_128, TILES_256_BY_192, TILES_128_BY_128, TILES_128_BY_128_THREE_STAGES, TILES_128_BY_64_FOUR_STAGES,
+                 TILES_RAGGED_256, TILES_RAGGED_128 };
+// whole_columns: of TILES_256_AND_128, the tiles along the columns that are 256 rows high.
 template <int MODE, typename TO>
-int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, const Packing& packing, int activation, hipStream_t s) {
+TileShape tile_shape(int M, int N, int K, int* whole_columns) {
     // output columns per tile are half the tile's w rows in the gated mode
     constexpr int DIV = MODE == MODE_GATED ? 2 : 1;
-    const RowScale plain = {nullptr, 0, 0, 0.f, activation};
     auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn / DIV - 1) / (bn / DIV)); };
     if (K % 64 != 0) {                 // a ragged last tile along k: the path through registers
         const long large = ((tiles(256, 256) + XRT_COMPUTE_UNITS - 1) / XRT_COMPUTE_UNITS) * 100;
         const long small = ((tiles(128, 128) + 2 * XRT_COMPUTE_UNITS - 1) / (2 * XRT_COMPUTE_UNITS)) * 59;
-        if (large <= small) return launch_kernel<256, 256, 2, 4, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
-        return launch_kernel<128, 128, 2, 2, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+        return large <= small ? TILES_RAGGED_256 : TILES_RAGGED_128;
     }
     // Up to 256 rows of a, gated: tiles that fit one round and are bound by reading w, in three or four stages, which keep more of it on
     // its way than the two that the tiles below have. (Split along k with a second kernel: 3072 pairs, k = 1024, 100 rows 14.6 us, so 9.5, 256 rows
     // 17.8 -> 9.9; 8192 pairs, k = 2048, 100 rows 24.4 -> 19.9, 200 rows 31.2 -> 24.7; 12288 pairs, k = 4096, 100 rows 59.6 -> 50.9; 5000 pairs,
     // k = 3072, 65 rows 28.8 -> 21.8. Tiles of 128 x 64 beyond one round lose to one of 128 x 128: 12288 pairs, 100 rows 55.7.)
     if constexpr (MODE == MODE_GATED) {
-        if (M <= 256 && tiles(128, 64) <= XRT_COMPUTE_UNITS) return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
-        if (M <= 128 || (M <= 256 && tiles(128, 128) <= XRT_COMPUTE_UNITS))
-            return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+        if (M <= 256 && tiles(128, 64) <= XRT_COMPUTE_UNITS) return TILES_128_BY_64_FOUR_STAGES;
+        if (M <= 128 || (M <= 256 && tiles(128, 128) <= XRT_COMPUTE_UNITS)) return TILES_128_BY_128_THREE_STAGES;
     }
     // 256 x 256 tiles cost the least energy a product, and tiles of half the height somewhat more (2048 rows of x, 4096 rows of
     // w, k = 4096: 128 tiles of the one 85 us, 256 of the other 58; 6144 rows of w: 82 and 102); tiles of 128 x 128, two to a compute
@@ -1039,36 +1040,59 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
     // one round: the last round is full of half-sized work instead of half empty (28672 rows of w, k = 4096, 2048 rows of x:
     // 366 against 372 us).
     const int tiles_m = (M + 255) / 256, tiles_n = (N + 256 / DIV - 1) / (256 / DIV);
-    const int whole_columns = (int)((long)tiles_m * tiles_n / XRT_COMPUTE_UNITS * XRT_COMPUTE_UNITS / tiles_m);     // n-tiles that run in full rounds
-    const long rest_tiles = (long)((M + 127) / 128) * (tiles_n - whole_columns);
+    *whole_columns = (int)((long)tiles_m * tiles_n / XRT_COMPUTE_UNITS * XRT_COMPUTE_UNITS / tiles_m);     // n-tiles that run in full rounds
+    const long rest_tiles = (long)((M + 127) / 128) * (tiles_n - *whole_columns);
     long mixed = LONG_MAX;
-    if (whole_columns > 0 && whole_columns < tiles_n && rest_tiles <= XRT_COMPUTE_UNITS)
-        mixed = rounds_cost((long)tiles_m * whole_columns, LARGE_TILE, K, KIND) + rounds_cost(rest_tiles, HALF_TILE, K, KIND);
-    if (mixed < large && mixed <= middle && mixed <= half && mixed <= small && mixed <= narrow) {
-        const int split = whole_columns * (256 / DIV);
-        const int small_tiles_m = (M + 127) / 128, small_tiles_n = tiles_n - whole_columns;
-        const int large_blocks = (tiles_m * whole_columns + 7) / 8 * 8;      // whole rounds over the XCDs
-        const int small_blocks = (small_tiles_m * small_tiles_n + 7) / 8 * 8;
-        constexpr size_t lds = (size_t)2 * (256 + 256) * 64 * sizeof(bf16);
-        auto kernel = gemm_mfma_mixed_kernel<MODE, TO>;
-        static bool configured = false;      // per instantiation
-        if (!configured) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-            XRT_REQUIRE(e == hipSuccess, "linear (mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
-            configured = true;
-        }
-        kernel<<<large_blocks + small_blocks, 8 * XRT_WAVE, lds, s>>>(a, w, out, M, N, K, large_blocks, tiles_m, whole_columns,
-                                                                      split, small_tiles_m, small_tiles_n, packing, activation);
-        XRT_LAUNCH_CHECK("linear (mfma, two tile shapes)");
-        return 0;
+    if (*whole_columns > 0 && *whole_columns < tiles_n && rest_tiles <= XRT_COMPUTE_UNITS)
+        mixed = rounds_cost((long)tiles_m * *whole_columns, LARGE_TILE, K, KIND) + rounds_cost(rest_tiles, HALF_TILE, K, KIND);
+    if (mixed < large && mixed <= middle && mixed <= half && mixed <= small && mixed <= narrow) return TILES_256_AND_128;
+    if (large <= middle && large <= half && large <= small && large <= narrow) return TILES_256;
+    if (middle <= half && middle <= small && middle <= narrow) return TILES_192;
+    if (half <= small && half <= narrow) return TILES_128;
+    if (NARROW && narrow <= small) return TILES_256_BY_192;
+    return TILES_128_BY_128;           // (four stages of 32 keep a load in flight for longer but meet at twice as many barriers, and measured slower)
+}
+
+template <int MODE, typename TO>
+int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, const Packing& packing, int activation, hipStream_t s) {
+    constexpr int DIV = MODE == MODE_GATED ? 2 : 1;
+    const RowScale plain = {nullptr, 0, 0, 0.f, activation};
+    int whole_columns = 0;
+    switch (tile_shape<MODE, TO>(M, N, K, &whole_columns)) {
+        case TILES_RAGGED_256: return launch_kernel<256, 256, 2, 4, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+        case TILES_RAGGED_128: return launch_kernel<128, 128, 2, 2, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+        case TILES_128_BY_64_FOUR_STAGES:
+            if constexpr (MODE == MODE_GATED) return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+            break;
+        case TILES_128_BY_128_THREE_STAGES:
+            if constexpr (MODE == MODE_GATED) return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+            break;
+        case TILES_256: return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+        case TILES_192: return launch_large<192, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+        case TILES_128: return launch_large<128, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
+        case TILES_256_BY_192:
+            if constexpr (MODE != MODE_GATED && sizeof(TO) == 4) return launch_kernel<256, 192, 4, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+            break;
+        case TILES_128_BY_128: return launch_kernel<128, 128, 2, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+        case TILES_256_AND_128: break;
     }
-    if (large <= middle && large <= half && large <= small && large <= narrow) return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
-    if (middle <= half && middle <= small && middle <= narrow) return launch_large<192, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
-    if (half <= small && half <= narrow) return launch_large<128, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
-    if constexpr (NARROW)
-        if (narrow <= small) return launch_kernel<256, 192, 4, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
-    // (four stages of 32 keep a load in flight for longer but meet at twice as many barriers, and measured slower)
-    return launch_kernel<128, 128, 2, 2, MODE, 64, 2, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+    const int tiles_m = (M + 255) / 256, tiles_n = (N + 256 / DIV - 1) / (256 / DIV);
+    const int split = whole_columns * (256 / DIV);
+    const int small_tiles_m = (M + 127) / 128, small_tiles_n = tiles_n - whole_columns;
+    const int large_blocks = (tiles_m * whole_columns + 7) / 8 * 8;      // whole rounds over the XCDs
+    const int small_blocks = (small_tiles_m * small_tiles_n + 7) / 8 * 8;
+    constexpr size_t lds = (size_t)2 * (256 + 256) * 64 * sizeof(bf16);
+    auto kernel = gemm_mfma_mixed_kernel<MODE, TO>;
+    static bool configured = false;      // per instantiation
+    if (!configured) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        XRT_REQUIRE(e == hipSuccess, "linear (mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
+        configured = true;
+    }
+    kernel<<<large_blocks + small_blocks, 8 * XRT_WAVE, lds, s>>>(a, w, out, M, N, K, large_blocks, tiles_m, whole_columns,
+                                                                  split, small_tiles_m, small_tiles_n, packing, activation);
+    XRT_LAUNCH_CHECK("linear (mfma, two tile shapes)");
+    return 0;
 }
 
 template <typename TO>
@@ -1637,6 +1661,14 @@ bool xrt_linear_split_takes_qkv(const void* a, const void* w, int M, int N, int 
 int xrt_linear_split_qkv(const void* a, const void* w, void* qkv, int M, int N, int K, const Packing& packing, float* workspace,
                          const xrt_linear_norm* norm, const QkvAfter& after, hipStream_t s) {
     return launch_split<bf16>((const bf16*)a, (const bf16*)w, (bf16*)qkv, M, N, K, MODE_STORE, XRT_ACT_SILU, packing, workspace, norm, &after, s);
+}
+
+// The tiles of a product that is not cut along k, more than 64 rows of x.
+extern "C" int xrt_linear_tiles(int out_dtype, int M, int N, int K, int mode) {
+    int unused = 0;
+    if (mode == MODE_GATED) return out_dtype == XRT_F32 ? tile_shape<MODE_GATED, float>(M, N, K, &unused) : tile_shape<MODE_GATED, bf16>(M, N, K, &unused);
+    if (mode == MODE_ACCUMULATE) return tile_shape<MODE_ACCUMULATE, float>(M, N, K, &unused);
+    return out_dtype == XRT_F32 ? tile_shape<MODE_STORE, float>(M, N, K, &unused) : tile_shape<MODE_STORE, bf16>(M, N, K, &unused);
 }
 
 // How a product is cut that runs through the tiles of this section: the number of parts along k (1: not cut, another kernel's if M > 64), a tile's rows of x and of w.
