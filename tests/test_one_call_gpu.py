@@ -36,6 +36,39 @@ def one_by_one(engine, step):
     return logits
 
 
+# ---- one call against part by part ---------------------------------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("pack", ["always", False])
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("name", ["llama", "qwen3"])
+def test_layers_of_real_widths_launched_by_one_call(name, dtype, pack, monkeypatch):
+    """All logits of a step, to the bits: products cut along k whose second kernel does the norm, or the heads of q, k and v; attention of prompts, cut by keys and
+    not, of float32 prompts, of decode steps with a merge, without, and finishing q and k itself. Every kernel of a step lays its workspace behind what is still
+    read of the step's memory."""
+    engine = wide_engine(name, dtype, pack_weights=pack)
+    if dtype == "bfloat16":
+        from test_kernels_gpu import parts_of
+        assert parts_of(engine.ops, 100, 1024, 3072, "add", True)[2] > 1 and parts_of(engine.ops, 333, 2048, 1024, "store")[2] > 1
+        assert bool(engine.ops.lib.xrt_attention_finishes_qkv(1, 8, 4, 128, 0, 1, 128, 4096, 1100))
+    ids = token_ids(engine.vocab_size, 2200, seed=3)
+    slots = [engine.alloc_slot() for _ in range(4)]
+    one_call, taken = engine.ops.dense_blocks, []
+    monkeypatch.setattr(engine.ops, "dense_blocks", lambda *arguments, **more: (taken.append(1), one_call(*arguments, **more))[1])
+    held = [0] * 4
+
+    def check(counts):
+        step = [(slot, ids[at:at + count], list(range(count))) for slot, at, count in zip(slots, held, counts) if count]
+        want, before = one_by_one(engine, step), len(taken)
+        got = engine.step(step)
+        assert len(taken) == before + 1 and torch.isfinite(got).all() and torch.equal(got, want), counts
+        held[:] = [at + count for at, count in zip(held, counts)]
+
+    for counts in ([40, 0, 0, 0], [60, 0, 0, 0], [0, 333, 0, 0], [0, 0, 700, 0], [1, 1, 1, 0], [17, 1, 64, 300], [1, 1, 1, 1], [0, 0, 1200, 0], [100, 0, 40, 0], [1, 1, 1, 1],
+                   [0, 0, 1, 0]):
+        check(counts)
+    engine.cache.check()
+
+
 # ---- the rows that somebody wants, behind the last attention ---------------------------------------------------------------------------
 
 # (heads, key/value heads, dims, tokens, sequences, tokens held before, wanted rows, whether their attention runs alone); measured: the comment at the rule
