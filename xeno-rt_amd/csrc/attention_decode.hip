@@ -58,7 +58,8 @@ static_assert(cache_value_offset(16 * 5 + 9, 32 + 8 * 2 + 6, 128) == (1 * 8 + 5)
 // this position's HD / 2 angles, as xrt_rope_table has worked them out (the same sincosf of the same angles as in qkv_prepare.hip:
 // worked out here, for every workgroup again, they would cost more than the kernel saves; turns null: no rotation). All of it is asked for
 // ahead of the first keys, whose loads then run while the heads are finished. (Asked for where they are used, and the keys after: one sequence at 334
-// keys, 16 heads on 8, 10.4 us inside a step; now 9.5. A step at the Qwen3-0.6B sizes 911 -> 888 us, three layers of the Qwen3-32B sizes and 32 sequences 1038 -> 1030.)
+// keys, 16 heads on 8, 10.4 us inside a step; now 9.5. A step at the Qwen3-0.6B sizes 911 -> 888 us; 223 steps drawn at random, 90 to 800 pairs of
+// sequence and key/value head at 1000 to 9000 keys, 0.97 of what they took. Three layers of the Qwen3-32B sizes and 32 sequences 1042 -> 1032, with the products around.)
 template <int HD, typename TW> struct alignas(sizeof(TW) * 8) Gains { TW e[8]; };
 template <int HD, typename TW>
 __device__ __forceinline__ void ask_gains(Gains<HD, TW> (&gains)[HD / 32], const TW* __restrict__ gain, int c) {
@@ -448,7 +449,8 @@ Cut cut_for(int tokens, int n_kv_heads, int q_tiles, int max_context, int head_d
     // Up to eight blocks: one workgroup sees all keys, and nothing is left to merge. From five blocks on it has eight wavefronts, a block
     // each, where every pair finds a compute unit of its own, and four of two blocks beyond (16 heads of 128 on 8, 334 keys: 1 sequence 7.4 us in two
     // parts and their merge, 6.0 with four wavefronts, 5.8 with eight; 16 sequences 9.1, 8.4, 7.9; 48 sequences 18.0, 14.4, 15.9; heads of 64 gain
-    // 0.2 to 1 us by the eight). Nine blocks and more: two blocks one after the other cost more than the merge.
+    // 0.2 to 1 us by the eight). Nine blocks and more: two blocks one after the other cost more than the merge. (max_context is what the caller says of the step:
+    // a recorded decode step says the engine's limit or the next 1024 tokens, whichever is less, so that it comes here in engines for up to 512 tokens.)
     if (max_blocks <= 8) {
         const int waves = max_blocks > 4 && pairs <= XRT_COMPUTE_UNITS ? 8 : 4;
         return Cut{(max_blocks + waves - 1) / waves, 1, waves};
