@@ -201,7 +201,9 @@ struct Step {
 
 }  // namespace
 
-extern "C" int xrt_dense_wanted_alone(const xrt_dense_layer* layer, const xrt_dense_step* step, int rows) { return wanted_alone(*step, *layer, nullptr, rows); }
+extern "C" int xrt_dense_wanted_alone(const xrt_dense_layer* layer, const xrt_dense_step* step, int rows) {
+    return layer == nullptr || step == nullptr || rows <= 0 ? -1 : wanted_alone(*step, *layer, nullptr, rows);
+}
 
 extern "C" long xrt_dense_blocks(const xrt_dense_layer* layers, int count, const xrt_dense_step* step, const xrt_dense_wanted* wanted, void* arena, long arena_bytes) {
     const auto refuse = [](const char* what) -> long { xrt_set_error("dense blocks: %s", what); return -1; };

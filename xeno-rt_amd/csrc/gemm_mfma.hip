@@ -1667,6 +1667,7 @@ int xrt_linear_split_qkv(const void* a, const void* w, void* qkv, int M, int N, 
 // The tiles of a product that is not cut along k, more than 64 rows of x.
 extern "C" int xrt_linear_tiles(int out_dtype, int M, int N, int K, int mode) {
     int unused = 0;
+    if (M <= 0 || N <= 0 || K <= 0 || mode < MODE_STORE || mode > MODE_GATED) return -1;
     if (mode == MODE_GATED) return out_dtype == XRT_F32 ? tile_shape<MODE_GATED, float>(M, N, K, &unused) : tile_shape<MODE_GATED, bf16>(M, N, K, &unused);
     if (mode == MODE_ACCUMULATE) return tile_shape<MODE_ACCUMULATE, float>(M, N, K, &unused);
     return out_dtype == XRT_F32 ? tile_shape<MODE_STORE, float>(M, N, K, &unused) : tile_shape<MODE_STORE, bf16>(M, N, K, &unused);
@@ -1674,6 +1675,7 @@ extern "C" int xrt_linear_tiles(int out_dtype, int M, int N, int K, int mode) {
 
 // How a product is cut that runs through the tiles of this section: the number of parts along k (1: not cut, another kernel's if M > 64), a tile's rows of x and of w.
 extern "C" int xrt_linear_parts(int M, int N, int K, int mode, int whole_norm, int* rows, int* columns) {
+    if (M <= 16 || N <= 0 || K < 64 || K % 64 != 0 || mode < MODE_STORE || mode > MODE_GATED || !rows || !columns) return -1;
     const SplitPlan plan = split_plan(M, N, K, mode, whole_norm != 0);
     *rows = plan.tile;
     *columns = plan.columns;

@@ -214,7 +214,7 @@ extern "C" int xrt_linear_qkv(const void* a, const void* w, const xrt_packing* p
     // more tokens, or head norms, the product split along k: the kernel that prepares the heads adds the partial sums itself (as two
     // kernels, the sums and the heads: with the values' kernel 2.9 + 3.3 + 4.1 us for 100 tokens of 32 heads of 64 on 8). Not for up to 64 tokens in more
     // than seven parts whose values it writes one by one: a token's workgroup then goes through all parts by itself, and the sums in a kernel of their own, with a thread an
-    // output, and the heads after it take less (176 products drawn at random: two to four parts 0.9 of that, seven 0.99, nine 1.05, sixteen 1.2 times: 40 tokens of 512
+    // output, and the heads after it take less (162 products drawn at random: two to four parts 0.9 of that, seven 0.99, nine 1.05, sixteen 1.2 times: 40 tokens of 512
     // outputs, k = 2944, 12.4 against 15.8 us). Where the values are written apart it pays up to sixteen (0.95).
     if (dtype == XRT_BF16 && a && w && qkv && M > 0 && K > 0 && !norm && xrt_linear_split_takes(a, w, M, N, K, 0, &need) && need > 0 &&
         (M > 64 || (v_cache != nullptr && longest_run >= XRT_QKV_VALUES_APART) || need <= 7L * M * N) && workspace != nullptr && workspace_floats >= need && xrt_qkv_prepare_takes_parts(qkv, workspace, head_dim, rope_theta, rope_dim, k_cache)) {
