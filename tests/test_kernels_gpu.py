@@ -163,6 +163,32 @@ def test_linear_float32_has_the_same_bits_with_few_rows_and_with_many(ops, m, n,
             assert torch.equal(torch.nan_to_num(got, nan=7.0), torch.nan_to_num(want, nan=7.0))
 
 
+# The tiles of that product (rows of a, 16 columns shared by all wavefronts or 16 of each), by the rule of the launcher, with one step along k, as many as there are
+# stages in LDS and more, a last step that is whole, partial or a single piece, results that do and do not allow 16 bytes a store.
+FLOAT_TILES = {(777, 2052, 2048): "112", (777, 2050, 2020): "112", (129, 8190, 576): "80", (692, 3070, 772): "80", (777, 2048, 52): "32", (1023, 1021, 1988): "32", (690, 3070, 36): "32",
+               (100, 2048, 1024): "16", (70, 2046, 484): "16", (33, 500, 1028): "16 shared", (17, 64, 100): "16 shared", (18, 68, 384): "16 shared",
+               (100, 1023, 3084): "32 shared", (40, 2048, 644): "32 shared", (64, 2048, 512): "32 shared"}
+
+
+@pytest.mark.parametrize("m,n,k", FLOAT_TILES)
+def test_linear_float32_has_the_same_bits_in_every_tile(ops, m, n, k):
+    a, w, base = rand(m, k, seed=m), rand(2 * n, k, seed=n, scale=0.3), rand(m, n, seed=5)
+    a[m - 2] *= 1e-36
+    a[m // 2, k - 1] = float("inf")
+    rows, together = ctypes.c_int(), ctypes.c_int()
+    for mode in ("store", "add", "gated"):
+        assert ops.lib.xrt_linear_float_tile(m, n, k, MODES[mode], ctypes.byref(rows), ctypes.byref(together)) == 0
+        assert f"{rows.value}{' shared' if together.value else ''}" == FLOAT_TILES[m, n, k], mode
+        many, few = base.clone(), base.clone()
+        for out, step in ((many, m), (few, 16)):
+            for at in range(0, m, step):
+                if mode == "gated":
+                    ops.linear_glu(a[at:at + step], w, out[at:at + step])
+                else:
+                    ops.linear(a[at:at + step], w[:n], out[at:at + step], accumulate=mode == "add")
+        assert torch.equal(torch.nan_to_num(many, nan=7.0), torch.nan_to_num(few, nan=7.0)), mode
+
+
 MODES = {"store": 0, "add": 1, "gated": 2}
 TILES = ["256", "192", "128", "256 and 128", "256 x 192", "128 x 128", "128 x 128, three stages", "128 x 64, four stages", "256, ragged", "128, ragged"]
 

@@ -10,10 +10,12 @@
 // the error grows with the square root of k / 16 + 16 instead of k). Semantics of the reference's
 // row-major matvec (crates/xrt-kernels/src/cpu/matmul.rs:153-167, 269-288): w is
 // [out][in], no bias.
-#include <type_traits>
 #include "common.h"
 #include "xrt_hip.h"
 #include "activation.h"
+
+bool xrt_linear_float_accepts(const void* a, const void* w, int M, int K);
+int xrt_linear_float(const float* a, const float* w, float* out, int M, int N, int K, int mode, int activation, hipStream_t s);
 
 namespace {
 
@@ -299,163 +301,6 @@ int launch_stream(const float* a, const float* w, float* out, int M, int N, int 
     return 0;
 }
 
-// ---- many rows of a, float32, on the matrix cores: v_mfma_f32_32x32x2_f32 adds its two products to the sum one after the
-// other, fmaf by fmaf, denormals and infinities included, so eight of them from zero make the sum of 16 consecutive k to the
-// bit as the kernel above makes it, and the sums of 16 are added up on the vector ALU in the same order: an output has the
-// same bits whichever of the three kernels made it.
-//
-// Bound by the matrix cores (155 TFLOP/s with the operands in registers; the vector ALUs reach half of that). A workgroup's
-// tile is small, 64 x 64, four wavefronts of 32 x 32: the rate is so low that the operands' way through LDS costs little, several
-// workgroups share a compute unit, and a prompt of some hundred rows still fills the rounds. Against the kernel above: 777 rows, 2048
-// columns and k = 8192 876 -> 323 us, gated 16384 rows of w and k = 2048 783 -> 546 us, 33 rows 892 -> 187 and 219 -> 55 us, 2048 rows
-// 1084 -> 631 and 1689 -> 1242 us (111 TFLOP/s). Tiles travel global -> registers -> LDS (32 along k, two stages in either), so
-// that k need only be a multiple of 4: what lies beyond is zero. Two steps in registers instead of one are worth a tenth where a
-// compute unit has one workgroup; three workgroups a unit, for with the registers of four the sums spill.
-//
-// The instruction's A operand is w, its B operand a: a lane then holds four neighbouring columns of one row of the output.
-// It takes k = 2s from its lower lanes and 2s + 1 from its upper ones: of 16 consecutive k the even ones lie in LDS before the
-// odd ones, and a lane reads its eight with two 16-byte reads. Gated: of 32 rows of w in the tile 16 are gate rows and 16 the up rows
-// of the same outputs, which meet in one lane.
-typedef float mfma_sums __attribute__((ext_vector_type(16)));
-constexpr int CORE_TILE = 64, CORE_BK = 32, CORE_PLACES = 3;      // (PLACES: workgroups of a compute unit; with a bound the sums stay out of the AGPRs)
-
-template <int MODE>
-__global__ void __launch_bounds__(256, CORE_PLACES) gemm_float_mfma_kernel(const float* __restrict__ a, const float* __restrict__ w, float* __restrict__ out,
-                                                              int M, int N, int K, int tiles_m, int activation) {
-    __shared__ __attribute__((aligned(16))) float tile_a[2][CORE_TILE][CORE_BK];
-    __shared__ __attribute__((aligned(16))) float tile_w[2][CORE_TILE][CORE_BK];
-    constexpr int OUTPUTS = MODE == MODE_GATED ? CORE_TILE / 2 : CORE_TILE;
-    const int tid = threadIdx.x, lane = tid % XRT_WAVE, wave = tid / XRT_WAVE, wave_m = wave / 2, wave_n = wave % 2;
-    // neighbouring workgroups go to different XCDs: every XCD takes a run of tiles of its own, down the rows first, so that
-    // the tiles that run there together share their w
-    const int total = gridDim.x, per = total / 8;
-    const int id = blockIdx.x < per * 8 ? blockIdx.x % 8 * per + blockIdx.x / 8 : blockIdx.x;
-    const long m0 = (long)(id % tiles_m) * CORE_TILE, n0 = (long)(id / tiles_m) * OUTPUTS;
-    auto w_row = [&](int r) -> long {                        // row of w behind row r of the tile, clamped into the matrix
-        if constexpr (MODE == MODE_GATED) return min(n0 + r / 32 * 16 + r % 16, (long)N - 1) + (long)(r / 16 % 2) * N;
-        return min(n0 + r, (long)N - 1);
-    };
-    // pieces of 16 bytes of a row change places so that the lanes which a read serves at once find them in different banks
-    auto place_of = [](int r, int piece) { return (piece ^ (r % 8) ^ (r / 8 % 2)) * 4; };
-
-    // a thread moves two pieces of four columns of either operand
-    const int row[2] = {tid / 8, 32 + tid / 8}, column = tid % 8 * 4;
-    const float* from_a[2];
-    const float* from_w[2];
-    int to[2][2];                                            // where the even and the odd two of its four columns go
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        from_a[i] = a + min(m0 + row[i], (long)M - 1) * K + column;
-        from_w[i] = w + w_row(row[i]) * K + column;
-#pragma unroll
-        for (int odd = 0; odd < 2; ++odd)                    // of each 16 columns: two pieces of even ones, two of odd ones
-            to[i][odd] = place_of(row[i], column / 16 * 4 + odd * 2 + column % 16 / 8) + column % 8 / 2;
-    }
-    float4 next_a[2][2], next_w[2][2];                       // two steps on their way: [step of two][piece]
-    auto fetch = [&](auto set, int k0) {                     // columns beyond K: something inside the row, zeroed on its way into LDS
-        const int k = min(k0, K - 4 - column);               // (K is a multiple of 4: a piece lies inside it or beyond it)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            next_a[set][i] = *reinterpret_cast<const float4*>(from_a[i] + k);
-            next_w[set][i] = *reinterpret_cast<const float4*>(from_w[i] + k);
-        }
-    };
-    auto stash = [&](auto set, int k0) {                     // into the stage of the same number
-        if (k0 + CORE_BK > K && k0 + column >= K) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i) next_a[set][i] = next_w[set][i] = make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const float4 from = next_a[set][i], of_w = next_w[set][i];
-            *reinterpret_cast<float2*>(&tile_a[set][row[i]][to[i][0]]) = make_float2(from.x, from.z);
-            *reinterpret_cast<float2*>(&tile_a[set][row[i]][to[i][1]]) = make_float2(from.y, from.w);
-            *reinterpret_cast<float2*>(&tile_w[set][row[i]][to[i][0]]) = make_float2(of_w.x, of_w.z);
-            *reinterpret_cast<float2*>(&tile_w[set][row[i]][to[i][1]]) = make_float2(of_w.y, of_w.w);
-        }
-    };
-    mfma_sums acc = {};
-    const int steps = (K + CORE_BK - 1) / CORE_BK;
-    const int row_a = wave_m * 32 + lane % 32, row_w = wave_n * 32 + lane % 32;
-    auto step = [&](auto stage, auto other, int t) {
-        __syncthreads();                                     // this stage is written, the other one has been read
-        fetch(stage, (t + 2) * CORE_BK);                     // (beyond the last step: zeros in a stage that nobody reads)
-        __builtin_amdgcn_sched_barrier(0);                   // asked for now, not when the products are half done
-        mfma_sums part[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {                        // the first and the last eight of each 16 columns
-            float4 of_a[2], of_w[2];
-#pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                of_a[c] = *reinterpret_cast<const float4*>(&tile_a[stage][row_a][place_of(row_a, c * 4 + lane / 32 * 2 + q)]);
-                of_w[c] = *reinterpret_cast<const float4*>(&tile_w[stage][row_w][place_of(row_w, c * 4 + lane / 32 * 2 + q)]);
-            }
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int c = 0; c < 2; ++c)
-                    part[c] = __builtin_amdgcn_mfma_f32_32x32x2f32((&of_w[c].x)[s], (&of_a[c].x)[s], q + s == 0 ? mfma_sums{} : part[c], 0, 0, 0);
-        }
-        stash(other, (t + 1) * CORE_BK);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            acc[e] += part[0][e];
-            acc[e] += part[1][e];                            // (columns beyond K are zeros, and so is their sum: adding it changes nothing)
-        }
-    };
-    const std::integral_constant<int, 0> even;
-    const std::integral_constant<int, 1> odd;
-    fetch(even, 0);
-    fetch(odd, CORE_BK);
-    stash(even, 0);
-    int t = 0;
-    for (; t + 1 < steps; t += 2) {
-        step(even, odd, t);
-        step(odd, even, t + 1);
-    }
-    if (t < steps) step(even, odd, t);
-    // ---- epilogue: element e is row e / 4 * 8 + lane / 32 * 4 + e % 4 of w's 32 rows, row lane % 32 of a's
-    const long m = m0 + wave_m * 32 + lane % 32;
-    if (m >= M) return;
-    const bool wide = N % 4 == 0 && (uintptr_t)out % 16 == 0;
-    constexpr int QUADS = MODE == MODE_GATED ? 2 : 4;
-#pragma unroll
-    for (int q = 0; q < QUADS; ++q) {
-        const long n = n0 + wave_n * (MODE == MODE_GATED ? 16 : 32) + q * 8 + lane / 32 * 4;
-        if (n >= N) continue;
-        float* dst = out + m * (long)N + n;
-        float made[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if constexpr (MODE == MODE_GATED) made[e] = gate_activation(acc[q * 4 + e], activation) * acc[(q + 2) * 4 + e];
-            else made[e] = acc[q * 4 + e];
-        }
-        if (wide) {
-            if constexpr (MODE == MODE_ACCUMULATE) {
-                const float4 before = *reinterpret_cast<const float4*>(dst);
-                made[0] = before.x + made[0]; made[1] = before.y + made[1]; made[2] = before.z + made[2]; made[3] = before.w + made[3];
-            }
-            *reinterpret_cast<float4*>(dst) = make_float4(made[0], made[1], made[2], made[3]);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (n + e < N) dst[e] = MODE == MODE_ACCUMULATE ? dst[e] + made[e] : made[e];
-        }
-    }
-}
-
-int launch_float_mfma(const float* a, const float* w, float* out, int M, int N, int K, int mode, int activation, hipStream_t s) {
-    const int outputs = mode == MODE_GATED ? CORE_TILE / 2 : CORE_TILE;
-    const int tiles_m = (M + CORE_TILE - 1) / CORE_TILE;
-    const long tiles = (long)tiles_m * ((N + outputs - 1) / outputs);
-    XRT_REQUIRE(tiles < (1L << 31), "linear (plain): %ld tiles", tiles);
-    if (mode == MODE_STORE) gemm_float_mfma_kernel<MODE_STORE><<<(unsigned)tiles, 256, 0, s>>>(a, w, out, M, N, K, tiles_m, activation);
-    else if (mode == MODE_ACCUMULATE) gemm_float_mfma_kernel<MODE_ACCUMULATE><<<(unsigned)tiles, 256, 0, s>>>(a, w, out, M, N, K, tiles_m, activation);
-    else gemm_float_mfma_kernel<MODE_GATED><<<(unsigned)tiles, 256, 0, s>>>(a, w, out, M, N, K, tiles_m, activation);
-    XRT_LAUNCH_CHECK("linear (plain, matrix cores)");
-    return 0;
-}
-
 template <typename TI, typename TO, int RM>
 void launch_rows(const void* a, const void* w, void* out, int M, int N, int K, int mode, int activation, hipStream_t s) {
     constexpr int BM = 16 * RM;
@@ -484,8 +329,8 @@ int xrt_linear_plain(const void* a, const void* w, int dtype, void* out, int out
     if (dtype == XRT_F32 && out_dtype == XRT_F32 && stream_takes(a, w, M, K))
         return launch_stream((const float*)a, (const float*)w, (float*)out, M, N, K, mode, activation, s);
     // more rows than that, in whole pieces of 16 bytes: the matrix cores (any other k: the tiles on the vector ALUs)
-    if (dtype == XRT_F32 && out_dtype == XRT_F32 && M > 2 * STREAM_HALF && K % 4 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0)
-        return launch_float_mfma((const float*)a, (const float*)w, (float*)out, M, N, K, mode, activation, s);
+    if (dtype == XRT_F32 && out_dtype == XRT_F32 && xrt_linear_float_accepts(a, w, M, K))
+        return xrt_linear_float((const float*)a, (const float*)w, (float*)out, M, N, K, mode, activation, s);
     if (dtype == XRT_F32 && out_dtype == XRT_F32) return launch<float, float>(a, w, out, M, N, K, mode, activation, s);
     if (dtype == XRT_BF16 && out_dtype == XRT_F32) return launch<bf16, float>(a, w, out, M, N, K, mode, activation, s);
     if (dtype == XRT_BF16 && out_dtype == XRT_BF16) return launch<bf16, bf16>(a, w, out, M, N, K, mode, activation, s);
