@@ -189,6 +189,42 @@ def test_linear_float32_has_the_same_bits_in_every_tile(ops, m, n, k):
         assert torch.equal(torch.nan_to_num(many, nan=7.0), torch.nan_to_num(few, nan=7.0)), mode
 
 
+# Gated products of 17 to 64 rows: one round of tiles of 64 rows of w without a split, its last full tile and one more (then wider tiles, or parts), rows of x without
+# their RMSNorm's division over more tiles of columns than the threads ask for at once, and the tiles of 65 to 128 rows and beyond at the edge of w past the caches.
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("m,n,k", [(17, 40, 128), (33, 8192, 192), (64, 8200, 192), (64, 1000, 5248), (48, 72, 256), (65, 8192, 256), (128, 8200, 192), (129, 8192, 192)])
+def test_gated_products_of_few_rows_in_one_round_of_narrow_tiles(ops, m, n, k, packed):
+    from xeno_rt_amd.ops.hip import Prescaled
+    a, w = rand(m, k, dtype=torch.bfloat16, seed=m), rand(2 * n, k, dtype=torch.bfloat16, seed=n, scale=0.1)
+    if m <= 64:
+        rows, columns = ctypes.c_int(), ctypes.c_int()
+        parts = ops.lib.xrt_linear_parts(m, n, k, 2, 0, ctypes.byref(rows), ctypes.byref(columns))
+        assert (parts == 1 and columns.value == 64) == (n <= 8192)
+    squares = torch.rand(k // 16, 64, device=DEV) * 16
+    want = a.double().cpu() @ w.double().cpu().t()
+    rms = (squares[:, :m].double().cpu().sum(0) / k + 1e-5).sqrt()[:, None] if m <= 64 else 1.0
+    w = packed_or_not(ops, w, packed, "gated", gated_n=n)
+    plain, divided = torch.empty(m, n, dtype=torch.bfloat16, device=DEV), torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    ops.linear_glu(a, w, plain)
+    ops.linear_glu(Prescaled(a, squares, 1e-5) if m <= 64 else a, w, divided)
+    assert rel(plain.cpu(), P.swiglu(want[:, :n], want[:, n:])) < ULP["bfloat16"] * 2
+    assert rel(divided.cpu(), P.swiglu(want[:, :n] / rms, want[:, n:] / rms)) < ULP["bfloat16"] * 2
+
+
+# Parts along k in eight wavefronts: 17 to 64 rows, w past the caches and not, its last tile of 128 rows not full; 65 rows and more of a short k and of one at its edge.
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("m,n,k", [(20, 256, 16448), (64, 1030, 3136), (40, 3072, 1024), (17, 3080, 1024), (33, 130, 384), (100, 2000, 2048), (70, 520, 4032), (70, 520, 4096)])
+def test_products_in_parts_of_eight_wavefronts(ops, m, n, k, packed):
+    a, w, base = rand(m, k, dtype=torch.bfloat16, seed=m), rand(n, k, dtype=torch.bfloat16, seed=n, scale=0.1), rand(m, n, seed=5)
+    assert int(ops.lib.xrt_linear_workspace(ctypes.c_void_p(a.data_ptr()), ctypes.c_void_p(w.data_ptr()), 1, m, n, k, 1)) >= 2 * m * n      # (two parts or more)
+    want = a.double().cpu() @ w.double().cpu().t()
+    w = packed_or_not(ops, w, packed)
+    stored, added = torch.empty(m, n, device=DEV), base.clone()
+    ops.linear(a, w, stored)
+    ops.linear(a, w, added, accumulate=True)
+    assert rel(stored.cpu(), want) < 1e-5 and rel(added.cpu(), base.double().cpu() + want) < 1e-5
+
+
 MODES = {"store": 0, "add": 1, "gated": 2}
 TILES = ["256", "192", "128", "256 and 128", "256 x 192", "128 x 128", "128 x 128, three stages", "128 x 64, four stages", "256, ragged", "128, ragged"]
 

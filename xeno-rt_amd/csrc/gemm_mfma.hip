@@ -97,18 +97,19 @@ __device__ __forceinline__ void gemm_tile(
         }
     };
     // 1 / rms of the tile's rows, if the rows of a come without it. The sums of squares are asked for now,
-    // all at once (a thread takes four neighbouring rows of every sixteenth tile, 16 bytes a load), and added
+    // all at once (a thread takes four neighbouring rows of every sixteenth tile, or eighth where there are 128 threads, 16 bytes a load), and added
     // up after the main loop, when they have long arrived.
-    constexpr int SQUARE_LOADS = 16;                           // tiles of 16 columns per thread: rows of up to 16 * 16 * 16 columns
+    constexpr int SUMMERS = THREADS < 256 ? THREADS / 16 : 16; // threads that add up the sums of a row
+    constexpr int SQUARE_LOADS = 256 / SUMMERS;                // tiles of 16 columns per thread: rows of up to 256 * 16 columns
     __shared__ float row_scale[BM <= 64 ? 64 : 1];
-    __shared__ float row_parts[BM <= 64 ? 16 : 1][64];
+    __shared__ float row_parts[BM <= 64 ? SUMMERS : 1][64];
     float4 early_squares[BM <= 64 ? SQUARE_LOADS : 1];
     const bool scaled = BM <= 64 && scale.squares != nullptr;
     if constexpr (BM <= 64) {
         if (scaled && tid < 256) {
 #pragma unroll
             for (int u = 0; u < SQUARE_LOADS; ++u) {
-                const int t = tid / 16 + 16 * u;
+                const int t = tid / 16 + SUMMERS * u;
                 early_squares[u] = t < scale.tiles
                     ? *reinterpret_cast<const float4*>(scale.squares + (long)t * XRT_SQUARES_STRIDE + (tid % 16) * 4)
                     : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -368,7 +369,7 @@ __device__ __forceinline__ void gemm_tile(
                     sum.x += early_squares[u].x; sum.y += early_squares[u].y; sum.z += early_squares[u].z; sum.w += early_squares[u].w;
                 }
                 // rows of more than 4096 columns: the tiles beyond, one after the other
-                for (int t = tid / 16 + 16 * SQUARE_LOADS; t < scale.tiles; t += 16) {
+                for (int t = tid / 16 + SUMMERS * SQUARE_LOADS; t < scale.tiles; t += SUMMERS) {
                     const float4 more = *reinterpret_cast<const float4*>(scale.squares + (long)t * XRT_SQUARES_STRIDE + (tid % 16) * 4);
                     sum.x += more.x; sum.y += more.y; sum.z += more.z; sum.w += more.w;
                 }
@@ -378,7 +379,7 @@ __device__ __forceinline__ void gemm_tile(
             if (tid < 64) {
                 float total = 0.f;
 #pragma unroll
-                for (int part = 0; part < 16; ++part) total += row_parts[part][tid];
+                for (int part = 0; part < SUMMERS; ++part) total += row_parts[part][tid];
                 row_scale[tid] = 1.0f / sqrtf(total / (float)scale.width + scale.eps);
             }
             __syncthreads();
@@ -1063,10 +1064,17 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
         case TILES_RAGGED_256: return launch_kernel<256, 256, 2, 4, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
         case TILES_RAGGED_128: return launch_kernel<128, 128, 2, 2, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
         case TILES_128_BY_64_FOUR_STAGES:
-            if constexpr (MODE == MODE_GATED) return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+            // (one row of tiles: w past the caches; 8192 pairs, k = 2048, 72 / 100 / 128 rows 17.7 / 18.6 / 19.6 -> 16.1 / 17.7 / 18.0 us. With two rows of
+            // tiles the second reads it from there: 3072 pairs, k = 1024, 160 rows 8.9 us as it is, 9.8 past them)
+            if constexpr (MODE == MODE_GATED) {
+                if (M <= 128) return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO, true>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+                return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+            }
             break;
         case TILES_128_BY_128_THREE_STAGES:
-            if constexpr (MODE == MODE_GATED) return launch_kernel<128, 128, 2, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+            // (eight wavefronts, w past the caches: 14336 pairs, k = 4096, 72 / 100 / 128 rows 45.4 / 46.9 / 48.8 -> 43.4 / 45.7 / 47.0 us; 25600 pairs, k = 5120
+            // 110 / 114 / 121 -> 107 / 112 / 118; 8192 pairs, k = 2048, 160 / 256 rows 24.9 / 26.0 -> 22.7 / 24.4)
+            if constexpr (MODE == MODE_GATED) return launch_kernel<128, 128, 4, 2, MODE, 64, 3, TO, true>(a, w, out, M, N, K, packing, s, 1, 0, plain);
             break;
         case TILES_256: return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
         case TILES_192: return launch_large<192, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
@@ -1165,6 +1173,10 @@ SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
     if (M <= SPLIT_BM) {
         splits = (int)(XRT_COMPUTE_UNITS / tiles_n);                         // one workgroup per compute unit, or fewer
         least = 1;
+        // gated, and one round of tiles of half the width: those, without a second kernel. 6144 rows of w, k = 1024 10.3 -> 8.9 us (17 rows of x), 13.5 -> 9.6
+        // (64 rows); 16384 rows, k = 2048 19.3 -> 15.1 and 21.4 -> 16.5; 10240 rows, k = 3072 18.7 -> 18.0 and 21.2 -> 19.9. (Beyond one round they read x too
+        // often: 28672 rows, k = 4096, 64 rows of x 43 us in tiles of 128, 47 in these.)
+        if (mode == MODE_GATED && (rows_w + 63) / 64 <= XRT_COMPUTE_UNITS) { splits = 1; columns = 64; }
     } else if (large_tiles <= 128 && M >= 512 && mode != MODE_GATED && units >= (whole_norm ? 64 : 128)) {
         // Many rows and a very long k, but so few columns that the largest tiles would leave half of the compute
         // units idle (the projection back from the feed-forward's width): the large tiles split k between them.
@@ -1479,8 +1491,15 @@ __global__ void __launch_bounds__(256) split_reduce_qkv_kernel(const float* __re
 // The product of all rows of w, ungated, into the workspace: [splits][M][rows_w]
 int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, const Packing& packing, const SplitPlan& plan, hipStream_t s) {
     const int rows_w = (int)plan.rows_w;
-    if (M <= SPLIT_BM)
-        return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+    if (M <= SPLIT_BM) {
+        // Eight wavefronts, two to a SIMD: one reads its operands while the other multiplies (with four: 3 to 6 % longer, the second kernel included; 1024 rows of w,
+        // k = 2048, 24 rows of x 8.8 -> 8.2 us, 10240 rows, k = 5120 26.7 -> 26.3). w past the caches where w has few rows but is not tiny, or k is very long
+        // (24 / 64 rows of x: 2048 rows of w, k = 2048 8.9 / 10.2 -> 8.1 / 9.6 us, k = 8192 13.7 / 15.7 -> 12.2 / 13.4; 5120 rows, k = 25600 49.5 / 53 -> 46 / 50); not
+        // elsewhere (4096 rows, k = 4096 13.7 / 15.9 us as it is, 13.9 / 17.7 past them; 1024 rows, k = 2048 8.2 / 9.7 and 8.4 / 10.1).
+        const bool past = K >= 16384 || (rows_w <= 3072 && (long)rows_w * K >= 3000000L);
+        if (past) return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 4, MODE_STORE, 64, 3, float, true>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+        return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 4, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+    }
     if (plan.tile == 192)
         return launch_large<192, MODE_STORE, float>(a, w, workspace, M, rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split);
     if (plan.tile == 256)
@@ -1489,7 +1508,12 @@ int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, c
         // a fourth stage where a compute unit has one workgroup anyway (2048 rows of w, k = 8192, 65 / 200 rows of x 16.0 / 22.5 -> 14.7 / 20.5 us with its
         // second kernel; k = 2048, 3072 rows, 100 rows of x 12.0 -> 11.5)
         if (dealt((long)((M + 127) / 128) * ((rows_w + 63) / 64)) * plan.splits <= XRT_COMPUTE_UNITS)
+        {
+            // eight wavefronts where k is short (2048 rows of w, k = 2048, 72 / 160 rows of x 11.1 / 13.0 -> 10.6 / 12.7 us with its second kernel, 3072 rows 12.9 / 14.9 -> 12.4 / 14.4;
+            // 4096 rows, k = 4096, 72 / 100 rows 16.6 / 17.6 in four, 17.3 / 18.6 in eight)
+            if (K < 4096) return launch_kernel<128, 64, 4, 2, MODE_STORE, 64, 4, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
             return launch_kernel<128, 64, 4, 1, MODE_STORE, 64, 4, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
+        }
         return launch_kernel<128, 64, 2, 2, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
     }
     if (M <= 256)           // (one workgroup to a compute unit anyway: a third stage keeps more of w on its way; with more, two share a unit)
@@ -1516,6 +1540,7 @@ int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int
     if (M <= SPLIT_BM && plan.splits == 1) {                   // tiles enough: each applies the epilogue itself
         XRT_REQUIRE(!emits, "linear (mfma): only a product split along k writes what the norm after it needs");
         if (mode == MODE_STORE) return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
+        if (mode == MODE_GATED && plan.columns == 64) return launch_kernel<SPLIT_BM, 64, 2, 1, MODE_GATED, 64, 4, TO, true>(a, w, out, M, N, K, packing, s, 1, 0, scale);
         if (mode == MODE_GATED) return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 2, MODE_GATED, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
         if constexpr (sizeof(TO) == 4)
             return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_ACCUMULATE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
