@@ -1206,6 +1206,40 @@ def test_attention_decode_of_short_contexts(ops, nh, nkv, hd, tokens, longest):
     assert torch.equal(out, finished)                       # (nothing to norm or rotate: the same operands, the same sums)
 
 
+@pytest.mark.parametrize("norm_dtype", [None, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("nh,nkv,hd", [(2, 2, 128), (24, 2, 128), (13, 1, 128), (16, 1, 64), (17, 1, 128), (12, 1, 64)])
+def test_attention_decode_that_finishes_the_newest_token_at_every_place_of_a_block(ops, nh, nkv, hd, norm_dtype):
+    """Sequences that end at every place of their first block and, some, of their second and sixth: the place decides which lane and which half of a register the
+    new value goes to, and which scores the new key's take the place of. The heads of a key head leave columns of the products empty for the new key (up to 12), or
+    do not, or need two tiles. Against qkv_prepare and the attention after it: the same bits where there is nothing to norm or rotate; with norms and rotation each sequence
+    to the rounding of q and k (a mean square of 64 or 128 terms and one rounding to bfloat16: the same in both but for the order of the sum)."""
+    from xeno_rt_amd.ops.hip import QkvFinish
+    lengths = list(range(1, 65)) + [65, 96, 97, 128, 321, 352, 353, 384]
+    kv, _, _ = filled_cache(nkv, hd, torch.bfloat16, lengths, seed=hd + nh)
+    positions = [n - 1 for n in lengths]
+    batch = described(list(range(len(lengths))), [1] * len(lengths), positions)
+    raw = rand(len(lengths), (nh + 2 * nkv) * hd, dtype=torch.bfloat16, seed=5)
+    norms = norm_dtype is not None
+    qn, kn = ((rand(hd, seed=1) + 1.0).to(norm_dtype), (rand(hd, seed=2) + 2.0).to(norm_dtype)) if norms else (None, None)
+    theta = (torch.tensor(10000.0) ** (torch.arange(hd // 2) * 2.0 / hd)).to(DEV) if norms else None
+    table = ops.rope_table(theta, hd, 1.0, max(lengths)) if norms else None
+    two, qkv_two = clone_cache(kv), raw.clone()
+    ops.qkv_prepare(qkv_two, nh, nkv, hd, batch.positions, batch.slots, kv=two, q_norm=qn, k_norm=kn, norm_eps=1e-5, rope_theta=theta, rope_dim=hd if norms else 0, rope_scale=1.0)
+    want, got = (torch.full((len(lengths), nh * hd), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.attention(qkv_two, nh, nkv, hd, two, batch, want, scale=1.0 / math.sqrt(hd))
+    ops.attention(raw, nh, nkv, hd, kv, batch, got, scale=1.0 / math.sqrt(hd), finish=QkvFinish(qn, kn, 1e-5, table))
+    assert torch.equal(torch.nan_to_num(kv.v.float(), nan=123.0), torch.nan_to_num(two.v.float(), nan=123.0))
+    if not norms:
+        assert torch.equal(got, want)
+        assert torch.equal(torch.nan_to_num(kv.k.float(), nan=123.0), torch.nan_to_num(two.k.float(), nan=123.0))
+    assert torch.isfinite(got).all()
+    for row in range(len(lengths)):
+        assert rel(got[row].float(), want[row].float()) < 2e-2, lengths[row]
+    plain_one, plain_two = cache_order.plain_keys(kv.k).float(), cache_order.plain_keys(two.k).float()
+    same = torch.nan_to_num(plain_one, nan=123.0) == torch.nan_to_num(plain_two, nan=123.0)
+    assert bool((same | ((plain_one - plain_two).abs() <= ULP["bfloat16"] * plain_two.abs().clamp(min=1e-3) * 2)).all())
+
+
 @pytest.mark.parametrize("nh,nkv,hd", [(32, 8, 128), (24, 8, 64)])
 def test_attention_decode_of_many_sequences(ops, nh, nkv, hd):
     """Seventy sequences: with so many (sequence, key/value head) pairs a workgroup takes all keys of its pair

@@ -26,11 +26,23 @@
 // qkv_prepare.hip (crates/xrt-models/src/llama.rs:1025-1040, crates/xrt-kernels/src/cpu/rope.rs:59-89). A lane holds
 // the dims 32 s + 8 c .. + 7 (s = 0 .. HD/32 - 1) of its query head, so the two dims of a rotation's pair (d and
 // d + HD/2) lie in one lane, and the norm's sum over a head is an exchange among four lanes. The new key and
-// value are worked out by the wavefront whose keys end with the sequence's newest block: it puts them into the
-// registers in which the block came from the cache (where the place of the newest token still holds what was
-// there before) and writes them to the cache for the steps to come.
+// value are the work of the wavefront whose keys end with the sequence's newest block: its registers hold the block as it came
+// from the cache, where the place of the newest token still holds what was there before. The new key's scores are a product of
+// their own and take the place of that row's; the new value takes its place in the registers where the block's tail is masked
+// anyway; and both are written to the cache for the steps to come.
+//
+// What bounds short contexts is not memory but one wavefront's chain of instructions and waits: the slot and the position (asked for together), the
+// block table, the first keys and values (all on their way before anything is waited for), the heads' finish, scores, values, merge. So what was in that chain and
+// need not be there is out of it. The four lanes of a head exchange by row swaps in the vector registers, not through LDS. A lane asks for two gains and one (cosine, sine)
+// instead of 32 and 16, and has the others from the 15 lanes beside it as the multiplications run (in full they were 16 loads of a kilobyte a wavefront, and 64 registers, so that
+// the first values had to wait until the heads were finished). Up to 12 heads to a key head leave columns of the products empty: the new key is in one of them and
+// is finished with the heads, in one pass (with a pass of its own 0.45 us more at 1 to 8 sequences). The tail of a block is masked by whole registers. In us before and now, heads of 128:
+// 16 on 8, 1 sequence, 20 keys 6.9, 5.7; 334 keys 8.2, 7.2; 1000 keys 10.9, 9.5; 8 sequences of 334 keys 10.2, 8.7; 32 of 334 14.0, 12.1; 64 on 8, 8 of 1500 15.8, 14.0; 32 on 2, 1 of 334 9.5, 8.6.
+// Without a finish 16 on 8, 1 of 334 5.7, 5.0; 8 of 334 7.6, 7.3; 32 of 3000 (the bandwidth of memory) 62.9, 63.3. A step at the Qwen3-0.6B sizes 889 -> 852 us.
 #include "cache_layout.h"
 #include "xrt_hip.h"
+
+#include <utility>
 
 namespace {
 
@@ -54,32 +66,53 @@ static_assert(cache_key_offset(32 + 8 * 2 + 4 * 1 + 3, 32 * 3 + 8 * 1, 128) == (
 static_assert(cache_key_offset(8 * 3 + 4 * 0 + 1, 32 * 1 + 8 * 3 + 5, 64) == ((0 * 2 + 0) * 2 + 1) * 512 + lane_place(3 * 4 + 1, 3) + 5, "keys of a block");
 static_assert(cache_value_offset(16 * 5 + 9, 32 + 8 * 2 + 6, 128) == (1 * 8 + 5) * 512 + lane_place(9, 2) + 6, "values of a block");
 
-// What finishing a head reads, of this lane's dims 32 s + 8 c .. + 7: the norm's gains (none: gain null), and the (cosine, sine) of
-// this position's HD / 2 angles, as xrt_rope_table has worked them out (the same sincosf of the same angles as in qkv_prepare.hip:
-// worked out here, for every workgroup again, they would cost more than the kernel saves; turns null: no rotation). All of it is asked for
-// ahead of the first keys, whose loads then run while the heads are finished. (Asked for where they are used, and the keys after: one sequence at 334
-// keys, 16 heads on 8, 10.4 us inside a step; now 9.5. A step at the Qwen3-0.6B sizes 911 -> 888 us; 223 steps drawn at random, 90 to 800 pairs of
-// sequence and key/value head at 1000 to 9000 keys, 0.97 of what they took. Three layers of the Qwen3-32B sizes and 32 sequences 1042 -> 1032, with the products around.)
-template <int HD, typename TW> struct alignas(sizeof(TW) * 8) Gains { TW e[8]; };
+// What finishing a head reads: the norm's gains (none: gain null), and the (cosine, sine) of this position's HD / 2 angles, as
+// xrt_rope_table has worked them out (the same sincosf of the same angles as in qkv_prepare.hip: worked out here, for every workgroup again, they would
+// cost more than the kernel saves; from null: no rotation). All of it is asked for ahead of the first keys, whose loads then run while the heads are finished.
+// The 16 lanes (0 .. 15, c) need the same ones, of the dims 32 s + 8 c + e: of gain s * 8 + e the lane 4 s + e / 2 asks for (two neighbours), of angle s * 8 + e the lane of that number.
+template <typename TW> struct alignas(sizeof(TW) * 2) GainPair { TW e[2]; };
 template <int HD, typename TW>
-__device__ __forceinline__ void ask_gains(Gains<HD, TW> (&gains)[HD / 32], const TW* __restrict__ gain, int c) {
-    if (gain == nullptr) return;
-#pragma unroll
-    for (int ks = 0; ks < HD / 32; ++ks) gains[ks] = *reinterpret_cast<const Gains<HD, TW>*>(gain + ks * 32 + c * 8);
+__device__ __forceinline__ GainPair<TW> ask_gains(const TW* __restrict__ gain, int r, int c) {
+    if (gain == nullptr) return GainPair<TW>{};
+    return *reinterpret_cast<const GainPair<TW>*>(gain + r / 4 % (HD / 32) * 32 + c * 8 + r % 4 * 2);
 }
-struct alignas(16) Turns { float2 e[8]; };
 template <int HD>
-__device__ __forceinline__ void ask_turns(Turns (&turns)[HD / 64], const float2* __restrict__ from, int c) {
-    if (from == nullptr) return;
-#pragma unroll
-    for (int ks = 0; ks < HD / 64; ++ks) turns[ks] = *reinterpret_cast<const Turns*>(from + ks * 32 + c * 8);
+__device__ __forceinline__ float2 ask_turns(const float2* __restrict__ from, int r, int c) {
+    return from == nullptr ? make_float2(1.f, 0.f) : from[r / 8 % (HD / 64) * 32 + c * 8 + r % 8];
 }
+// Maximum and sum over the four lanes (r, 0 .. 3), and what the lane (r, C) holds, in all four: rows of 16 lanes exchanged within the vector registers
+// (through LDS, as a shuffle goes, each step waits several times as long).
+__device__ __forceinline__ uint2 exchange_rows(unsigned v) { const auto both = __builtin_amdgcn_permlane16_swap(v, v, false, false); return make_uint2(both[0], both[1]); }      // rows 0 0 2 2, and 1 1 3 3
+__device__ __forceinline__ uint2 exchange_halves(unsigned v) { const auto both = __builtin_amdgcn_permlane32_swap(v, v, false, false); return make_uint2(both[0], both[1]); }    // rows 0 1 0 1, and 2 3 2 3
+__device__ __forceinline__ unsigned as_word(float v) { return __builtin_bit_cast(unsigned, v); }
+__device__ __forceinline__ float as_value(unsigned v) { return __builtin_bit_cast(float, v); }
+__device__ __forceinline__ float max_of_four(float v) {
+    const uint2 rows = exchange_rows(as_word(v));
+    const uint2 halves = exchange_halves(as_word(fmaxf(as_value(rows.x), as_value(rows.y))));
+    return fmaxf(as_value(halves.x), as_value(halves.y));
+}
+__device__ __forceinline__ float sum_of_four(float v) {
+    const uint2 rows = exchange_rows(as_word(v));
+    const uint2 halves = exchange_halves(as_word(as_value(rows.x) + as_value(rows.y)));
+    return as_value(halves.x) + as_value(halves.y);
+}
+template <int C> __device__ __forceinline__ unsigned of_row(unsigned v) {
+    const uint2 halves = exchange_halves(v);
+    const uint2 rows = exchange_rows(C < 2 ? halves.x : halves.y);
+    return C % 2 == 0 ? rows.x : rows.y;
+}
+template <int LANE> __device__ __forceinline__ float of_lane(float v) {          // what the lane (LANE, c) holds, in all lanes (r, c)
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x150 + LANE, 0xF, 0xF, true));      // row_newbcast
+}
+template <int LANE> __device__ __forceinline__ float of_lane(float v, float last) {          // the same of `last` in the lanes (12 .. 15, c)
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, of_lane<LANE>(v)), __builtin_bit_cast(int, last), 0x150 + LANE, 0xF, 0x8, false));
+}
+template <typename F, int... I> __device__ __forceinline__ void each(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
 
 // One head (the dims of this lane) through its RMSNorm and the rotation by the token's position, in float32, and back to
-// bfloat16: what qkv_prepare does to a head.
-template <int HD, typename TW>
-__device__ __forceinline__ void finish_head(bf16x8 (&x)[HD / 32], bool norms, const Gains<HD, TW> (&gains)[HD / 32], float eps,
-                                            bool rotates, const Turns (&turns)[HD / 64]) {
+// bfloat16: what qkv_prepare does to a head. BOTH: the lanes (12 .. 15, c) hold another kind of head, whose gains are last_gains.
+template <int HD, bool BOTH, typename TW>
+__device__ __forceinline__ void finish_head(bf16x8 (&x)[HD / 32], bool norms, GainPair<TW> gains, GainPair<TW> last_gains, float eps, bool rotates, float2 turns) {
     constexpr int KS = HD / 32;
     float inv_rms = 1.0f;
     if (norms) {
@@ -88,42 +121,49 @@ __device__ __forceinline__ void finish_head(bf16x8 (&x)[HD / 32], bool norms, co
         for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
             for (int e = 0; e < 8; ++e) squares = fmaf((float)x[ks][e], (float)x[ks][e], squares);
-        squares += __shfl_xor(squares, 16, XRT_WAVE);          // the four lanes (r, 0 .. 3) hold the head between them
-        squares += __shfl_xor(squares, 32, XRT_WAVE);
+        squares = sum_of_four(squares);                        // the four lanes (r, 0 .. 3) hold the head between them
         inv_rms = 1.0f / sqrtf(squares / (float)HD + eps);
     }
-    // a pair of the rotation at a time (dims d and d + HD / 2 lie in x[ks] and x[ks + KS / 2]): few registers at once
-#pragma unroll
-    for (int ks = 0; ks < KS / 2; ++ks) {
+    // a pair of the rotation at a time (dims d and d + HD / 2 lie in x[ks] and x[ks + KS / 2])
+    each([&](auto number) {
+        constexpr int ks = number, upper_ks = ks + KS / 2;
         float lower[8], upper[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { lower[e] = (float)x[ks][e]; upper[e] = (float)x[ks + KS / 2][e]; }
+        for (int e = 0; e < 8; ++e) { lower[e] = (float)x[ks][e]; upper[e] = (float)x[upper_ks][e]; }
         if (norms) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                lower[e] = lower[e] * inv_rms * to_float(gains[ks].e[e]);
-                upper[e] = upper[e] * inv_rms * to_float(gains[ks + KS / 2].e[e]);
-            }
+            each([&](auto element) {
+                constexpr int e = element;
+                const float mine = to_float(gains.e[e % 2]), last = to_float(last_gains.e[e % 2]);
+                if constexpr (BOTH) {
+                    lower[e] = lower[e] * inv_rms * of_lane<ks * 4 + e / 2>(mine, last);
+                    upper[e] = upper[e] * inv_rms * of_lane<upper_ks * 4 + e / 2>(mine, last);
+                } else {
+                    lower[e] = lower[e] * inv_rms * of_lane<ks * 4 + e / 2>(mine);
+                    upper[e] = upper[e] * inv_rms * of_lane<upper_ks * 4 + e / 2>(mine);
+                }
+            }, std::make_integer_sequence<int, 8>{});
         }
         if (rotates) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float cosine = turns[ks].e[e].x, sine = turns[ks].e[e].y;
+            each([&](auto element) {
+                constexpr int e = element;
+                const float cosine = of_lane<ks * 8 + e>(turns.x), sine = of_lane<ks * 8 + e>(turns.y);
                 const float a = lower[e], b = upper[e];
                 lower[e] = a * cosine - b * sine;
                 upper[e] = a * sine + b * cosine;
-            }
+            }, std::make_integer_sequence<int, 8>{});
         }
 #pragma unroll
-        for (int e = 0; e < 8; ++e) { x[ks][e] = (bf16)lower[e]; x[ks + KS / 2][e] = (bf16)upper[e]; }
-    }
+        for (int e = 0; e < 8; ++e) { x[ks][e] = (bf16)lower[e]; x[upper_ks][e] = (bf16)upper[e]; }
+    }, std::make_integer_sequence<int, KS / 2>{});
 }
+
+enum { FINISH_NONE, FINISH_APART, FINISH_FOLDED };       // nothing to finish; the new key in registers of its own; the new key in the columns 12 .. 15 of the query heads' products
 
 // FINISH: q, k and v come as the projection left them, and `finish` says what is still to do (see the head of this file).
 // TW: the element type of the head norms' gains.
-template <int HD, bool FINISH, int WAVES, typename TW>
+template <int HD, int FINISH, int WAVES, typename TW>
 __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
-    const bf16* __restrict__ qkv, int row_width, int n_heads, int n_kv_heads,
+    const bf16* __restrict__ qkv, int row_width, int group, int n_kv_heads,
     const bf16* __restrict__ k_cache, const bf16* __restrict__ v_cache, const int* __restrict__ block_table,
     int table_stride, int n_blocks, const int* __restrict__ positions, const int* __restrict__ slots,
     float scale, int chunk_blocks, int n_parts, int q_tiles,
@@ -138,10 +178,12 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
     const int r = lane % 16, c = lane / 16;
     const int part = blockIdx.x;                   // this workgroup's chunks become one partial result
     const int chunk = part * WAVES + wave;
-    const int kv_head = blockIdx.y / q_tiles, q_tile = blockIdx.y % q_tiles;
+    const int n_heads = group * n_kv_heads;
+    int kv_head = blockIdx.y, q_tile = 0;
+    if (q_tiles > 1) { kv_head = blockIdx.y / q_tiles; q_tile = blockIdx.y % q_tiles; }
     const int token = blockIdx.z;
-    const int slot = slots[token];
-    const int group = n_heads / n_kv_heads;
+    int slot = slots[token], pos = positions[token];
+    asm volatile("" : "+s"(slot), "+s"(pos));      // both are there before the branch (left alone, the compiler asks for the position behind it)
     if (slot < 0) {                                // padding: the whole workgroup leaves
         // (with one partial result per head there is no merge kernel after this one to write the zeros)
         if (n_parts == 1 && wave == 0 && q_tile * 16 + r < group) {
@@ -150,7 +192,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
         }
         return;
     }
-    const int n_keys = positions[token] + 1;
+    const int n_keys = pos + 1;
     if (part * WAVES * chunk_blocks * XRT_BLOCK_TOKENS >= n_keys) return;      // nothing here for any wavefront
     const int first_block = chunk * chunk_blocks;
     const bool active = first_block * XRT_BLOCK_TOKENS < n_keys;
@@ -165,9 +207,11 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
 
     if (active) {
         bf16x8 q[KS];
+        const bool key_lane = FINISH == FINISH_FOLDED && r >= 12;
+        const int row_head = key_lane ? n_heads + kv_head : head;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-            q[ks] = *reinterpret_cast<const bf16x8*>(qkv + (long)token * row_width + (long)head * HD + ks * 32 + c * 8);
+            q[ks] = *reinterpret_cast<const bf16x8*>(qkv + (long)token * row_width + (long)row_head * HD + ks * 32 + c * 8);
         // Loads are always on their way: a block's values are asked for before its scores are computed, and the
         // next block's keys right after, before the softmax and the value product of this one.
         const int* table = block_table + (long)slot * table_stride;
@@ -183,87 +227,84 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
                     for (int ks = 0; ks < KS; ++ks)
                         kreg[g][t][ks] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(kb + ((g * 2 + t) * KS + ks) * 512 + lane * 8));
         };
-        // The sequence's newest token: its block and its place there. What is still to do to q (and, in the wavefront whose
-        // keys end with the newest block, to the new key) is done while the first keys are on their way, with everything that it reads
-        // asked for before them (loads arrive in their order: behind the keys it would wait for those too).
-        const int newest_block = (n_keys - 1) / XRT_BLOCK_TOKENS, newest = (n_keys - 1) % XRT_BLOCK_TOKENS;
-        const bool has_newest = FINISH && last_block == newest_block;
-        bf16x8 new_key[KS];
-        bf16 new_value[DT];
-        Gains<HD, TW> q_gains[KS], k_gains[KS];
-        Turns turns[KS / 2];
-        const float2* turns_from = nullptr;
-        int block = block_of(first_block), next_block = block_of(first_block + 1);
-        if constexpr (FINISH) {
-            const int pos = n_keys - 1;
-            if (finish.rope_table != nullptr) turns_from = finish.rope_table + (long)min(pos, finish.table_positions - 1) * (HD / 2);   // (the host sends only steps that the table covers)
-            ask_turns<HD>(turns, turns_from, c);
-            ask_gains<HD, TW>(q_gains, (const TW*)finish.q_norm, c);
-            if (has_newest) {                          // (the same for all lanes of the wavefront)
-                const bf16* key_row = qkv + (long)token * row_width + (long)(n_heads + kv_head) * HD;
-                const bf16* value_row = key_row + (long)n_kv_heads * HD;
-#pragma unroll
-                for (int ks = 0; ks < KS; ++ks) new_key[ks] = *reinterpret_cast<const bf16x8*>(key_row + ks * 32 + c * 8);
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) new_value[dt] = value_row[dt * 16 + r];
-                ask_gains<HD, TW>(k_gains, (const TW*)finish.k_norm, c);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        ask_keys(block);
-        if constexpr (FINISH) {
-            __builtin_amdgcn_sched_barrier(0);
-            finish_head<HD, TW>(q, finish.q_norm != nullptr, q_gains, finish.norm_eps, turns_from != nullptr, turns);
-            if (has_newest) finish_head<HD, TW>(new_key, finish.k_norm != nullptr, k_gains, finish.norm_eps, turns_from != nullptr, turns);
-        }
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
-        for (int b = first_block; b <= last_block; ++b) {
+        auto ask_values = [&](int block) {
             const bf16* vb = v_cache + ((long)block * n_kv_heads + kv_head) * HD * XRT_BLOCK_TOKENS;
-            const int valid = min(XRT_BLOCK_TOKENS, n_keys - b * XRT_BLOCK_TOKENS);   // keys of this block that exist
 #pragma unroll
             for (int g = 0; g < 2; ++g)
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
                     vreg[g][dt] = __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(vb + (g * DT + dt) * 512 + lane * 8));
-
-            if constexpr (FINISH) {
-                if (has_newest && b == newest_block) {
-                    // The newest key and value take their places in the registers that hold the block (key 32 g + 8 (r / 4) +
-                    // 4 t + r % 4 lies in lane r of kreg[g][t], token 32 g + 8 c + e in element e of vreg[g] of the lanes c),
-                    // and in the cache (one of the workgroups that share the key/value head writes: q_tile 0).
-                    const int g_new = newest / 32, within = newest % 32;
-                    const int t_new = within % 8 / 4, r_new = within / 8 * 4 + within % 4, c_new = within / 8, e_new = newest % 8;
+        };
+        // The sequence's newest token: its block and its place there. What is still to do to q and to the new key
+        // is done while the first keys and values are on their way, with everything that it reads
+        // asked for before them (loads arrive in their order: behind the keys it would wait for those too).
+        const int newest_block = (unsigned)pos / XRT_BLOCK_TOKENS;
+        const unsigned newest = (unsigned)pos % XRT_BLOCK_TOKENS;
+        const bool has_newest = FINISH != FINISH_NONE && last_block == newest_block;
+        bf16x8 new_key[KS];                            // (FINISH_APART)
+        unsigned short new_value[DT / 4];              // dims 16 (4 i + c) + r
+        GainPair<TW> q_gains, k_gains;
+        float2 turns;
+        const float2* turns_from = nullptr;
+        int block = block_of(first_block), next_block = block_of(first_block + 1);
+        const int newest_place = FINISH == FINISH_NONE ? 0 : block_of(newest_block);
+        if constexpr (FINISH != FINISH_NONE) {
+            if (finish.rope_table != nullptr) turns_from = finish.rope_table + (long)min(pos, finish.table_positions - 1) * (HD / 2);   // (the host sends only steps that the table covers)
+            q_gains = ask_gains<HD, TW>((const TW*)finish.q_norm, r, c);
+            turns = ask_turns<HD>(turns_from, r, c);
+            if (has_newest) {                          // (the same for all lanes of the wavefront)
+                const bf16* key_row = qkv + (long)token * row_width + (long)(n_heads + kv_head) * HD;
+                const unsigned short* value_row = reinterpret_cast<const unsigned short*>(key_row + (long)n_kv_heads * HD);
 #pragma unroll
-                    for (int g = 0; g < 2; ++g) {
-                        if (g != g_new) continue;
+                for (int i = 0; i < DT / 4; ++i) new_value[i] = value_row[(4 * i + c) * 16 + r];
+                if constexpr (FINISH == FINISH_APART) {
 #pragma unroll
-                        for (int t = 0; t < 2; ++t)
-                            if (t == t_new && r == r_new) {
-#pragma unroll
-                                for (int ks = 0; ks < KS; ++ks) kreg[g][t][ks] = new_key[ks];
-                            }
-#pragma unroll
-                        for (int e = 0; e < 8; ++e)
-                            if (e == e_new && c == c_new) {
-#pragma unroll
-                                for (int dt = 0; dt < DT; ++dt) vreg[g][dt][e] = new_value[dt];
-                            }
-                    }
-                    if (q_tile == 0) {
-                        const long base = ((long)block * n_kv_heads + kv_head) * XRT_BLOCK_TOKENS * HD;
-                        if (r == 0) {
-#pragma unroll
-                            for (int ks = 0; ks < KS; ++ks)
-                                *reinterpret_cast<bf16x8*>(finish.k_cache + base + cache_key_offset(newest, ks * 32 + c * 8, HD)) = new_key[ks];
-                        }
-                        if (c == 0) {
-#pragma unroll
-                            for (int dt = 0; dt < DT; ++dt) finish.v_cache[base + cache_value_offset(dt * 16 + r, newest, HD)] = new_value[dt];
-                        }
-                    }
+                    for (int ks = 0; ks < KS; ++ks) new_key[ks] = *reinterpret_cast<const bf16x8*>(key_row + ks * 32 + c * 8);
+                }
+                k_gains = ask_gains<HD, TW>((const TW*)finish.k_norm, r, c);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        ask_keys(block);
+        ask_values(block);
+        if constexpr (FINISH != FINISH_NONE) {
+            __builtin_amdgcn_sched_barrier(0);
+            const bool norms = finish.q_norm != nullptr, rotates = turns_from != nullptr;
+            if (FINISH == FINISH_FOLDED && has_newest) {
+                finish_head<HD, true>(q, norms, q_gains, k_gains, finish.norm_eps, rotates, turns);
+            } else {
+                finish_head<HD, false>(q, norms, q_gains, q_gains, finish.norm_eps, rotates, turns);
+                if constexpr (FINISH == FINISH_APART) {
+                    if (has_newest) finish_head<HD, false>(new_key, norms, k_gains, k_gains, finish.norm_eps, rotates, turns);
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // The newest key against the query heads: in every row of the product (FINISH_APART), or in the rows 12 .. 15 (FINISH_FOLDED)
+        float new_score = 0.f;
+        if (has_newest) {
+            floatx4 product = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks)
+                product = __builtin_amdgcn_mfma_f32_16x16x32_bf16(FINISH == FINISH_FOLDED ? q[ks] : new_key[ks], q[ks], product, 0, 0, 0);
+            new_score = FINISH == FINISH_FOLDED ? as_value(of_row<3>(as_word(product[0]))) : product[0];
+            if (q_tile == 0) {                             // one of the workgroups that share the key/value head writes to the cache
+                const long base = ((long)newest_place * n_kv_heads + kv_head) * XRT_BLOCK_TOKENS * HD;
+#pragma unroll
+                for (int i = 0; i < DT / 4; ++i)
+                    reinterpret_cast<unsigned short*>(finish.v_cache)[base + cache_value_offset((4 * i + c) * 16 + r, newest, HD)] = new_value[i];
+                if (r == 15) {
+#pragma unroll
+                    for (int ks = 0; ks < KS; ++ks)
+                        *reinterpret_cast<bf16x8*>(finish.k_cache + base + cache_key_offset(newest, ks * 32 + c * 8, HD)) = FINISH == FINISH_FOLDED ? q[ks] : new_key[ks];
+                }
+            }
+        }
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int b = first_block; b <= last_block; ++b) {
+            const int valid = min(XRT_BLOCK_TOKENS, n_keys - b * XRT_BLOCK_TOKENS);   // keys of this block that exist
+            const bool newest_here = has_newest && b == newest_block;
             // ---- scores of 64 keys: two groups of 32, two tiles of 16 rows each
             floatx4 s[2][2];
 #pragma unroll
@@ -278,6 +319,17 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
             block = next_block;
             next_block = block_of(b + 2);
             if (b < last_block) ask_keys(block);
+            if constexpr (FINISH != FINISH_NONE) {
+                if (newest_here) {                     // its score takes the place of what the old key there gave
+#pragma unroll
+                    for (int g = 0; g < 2; ++g)
+#pragma unroll
+                        for (int t = 0; t < 2; ++t)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                s[g][t][i] = g * 32 + c * 8 + t * 4 + i == (int)newest ? new_score : s[g][t][i];
+                }
+            }
             // register i of s[g][t] is key g*32 + c*8 + t*4 + i, for query head r
             float block_max = -INFINITY;
 #pragma unroll
@@ -291,8 +343,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
                         s[g][t][i] = v;
                         block_max = fmaxf(block_max, v);
                     }
-            block_max = fmaxf(block_max, __shfl_xor(block_max, 16, XRT_WAVE));
-            block_max = fmaxf(block_max, __shfl_xor(block_max, 32, XRT_WAVE));
+            block_max = max_of_four(block_max);
             const float m_new = fmaxf(m, block_max);           // finite: key 0 of the block exists
             const float correction = __builtin_amdgcn_exp2f(m - m_new);
             m = m_new;
@@ -312,21 +363,35 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) attention_decode_kernel(
                         l += e;
                         p[t * 4 + i] = (bf16)e;
                     }
+                // What lies behind the keys that exist belongs to nobody and must not meet the zeros of p; the newest value takes its place
+                const int kept = (newest_here ? valid - 1 : valid) - g * 32;      // of these 32 tokens
+                if (kept < 32) {
+                    const int mine = kept - c * 8;                 // of the eight of this lane
+                    unsigned keep[4], put[4];
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt) {
-                    bf16x8 v = vreg[g][dt];
-                    if (valid < XRT_BLOCK_TOKENS) {
-                        // the block's tail belongs to nobody: whatever it holds must not meet the zeros of p
-#pragma unroll
-                        for (int e = 0; e < 8; ++e)
-                            if (g * 32 + c * 8 + e >= valid) v[e] = (bf16)0.f;
+                    for (int i = 0; i < 4; ++i) {
+                        keep[i] = mine >= 2 * i + 2 ? ~0u : (mine == 2 * i + 1 ? 0xFFFFu : 0u);
+                        if constexpr (FINISH != FINISH_NONE) put[i] = !newest_here ? 0u : (mine == 2 * i ? 0xFFFFu : (mine == 2 * i + 1 ? 0xFFFF0000u : 0u));
                     }
-                    o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, p, o[dt], 0, 0, 0);
+                    each([&](auto tile) {
+                        constexpr int dt = tile;
+                        union { bf16x8 v; unsigned words[4]; } piece{vreg[g][dt]};
+                        unsigned value = 0;
+                        if constexpr (FINISH != FINISH_NONE) value = of_row<dt % 4>(new_value[dt / 4]) * 0x10001u;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            piece.words[i] &= keep[i];
+                            if constexpr (FINISH != FINISH_NONE) piece.words[i] |= value & put[i];
+                        }
+                        vreg[g][dt] = piece.v;
+                    }, std::make_integer_sequence<int, DT>{});
                 }
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vreg[g][dt], p, o[dt], 0, 0, 0);
             }
+            if (b < last_block) ask_values(block);
         }
-        l += __shfl_xor(l, 16, XRT_WAVE);
-        l += __shfl_xor(l, 32, XRT_WAVE);
+        l = sum_of_four(l);
     } else {
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -501,18 +566,23 @@ int launch(const bf16* qkv, int tokens, int n_heads, int n_kv_heads, const bf16*
                                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);                 \
         XRT_REQUIRE(room == hipSuccess, "attention (decode): cannot reserve LDS: %s", hipGetErrorString(room));                    \
         attention_decode_kernel<HD, FINISH_, WAVES_, TW_><<<grid, WAVES_ * XRT_WAVE, lds, s>>>(                                            \
-            qkv, row_width, n_heads, n_kv_heads, k_cache, v_cache, block_table, table_stride, n_blocks, positions, slots,            \
+            qkv, row_width, group, n_kv_heads, k_cache, v_cache, block_table, table_stride, n_blocks, positions, slots,              \
             scale, cut.chunk_blocks, cut.n_parts, q_tiles, part_o, part_ml, out, HOW);                                              \
     } while (0)
     const bool float_gains = finish != nullptr && finish->norm_dtype == XRT_F32;
-    if (finish != nullptr && cut.waves == 8) {
-        if (float_gains) XRT_DECODE(true, 8, float, *finish);
-        else XRT_DECODE(true, 8, bf16, *finish);
-    } else if (finish != nullptr) {
-        if (float_gains) XRT_DECODE(true, 4, float, *finish);
-        else XRT_DECODE(true, 4, bf16, *finish);
-    } else if (cut.waves == 8) XRT_DECODE(false, 8, bf16, Finish{});
-    else XRT_DECODE(false, 4, bf16, Finish{});
+#define XRT_DECODE_FINISHING(FINISH_)                                                          \
+    do {                                                                                       \
+        if (cut.waves == 8 && float_gains) XRT_DECODE(FINISH_, 8, float, *finish);             \
+        else if (cut.waves == 8) XRT_DECODE(FINISH_, 8, bf16, *finish);                        \
+        else if (float_gains) XRT_DECODE(FINISH_, 4, float, *finish);                          \
+        else XRT_DECODE(FINISH_, 4, bf16, *finish);                                            \
+    } while (0)
+    // (up to 12 heads the columns 12 .. 15 are empty: see the head of this file)
+    if (finish != nullptr && group <= 12) XRT_DECODE_FINISHING(FINISH_FOLDED);
+    else if (finish != nullptr) XRT_DECODE_FINISHING(FINISH_APART);
+    else if (cut.waves == 8) XRT_DECODE(FINISH_NONE, 8, bf16, Finish{});
+    else XRT_DECODE(FINISH_NONE, 4, bf16, Finish{});
+#undef XRT_DECODE_FINISHING
 #undef XRT_DECODE
     XRT_LAUNCH_CHECK("attention (decode)");
     if (cut.n_parts == 1) return 0;
