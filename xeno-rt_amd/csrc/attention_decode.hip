@@ -80,27 +80,6 @@ template <int HD>
 __device__ __forceinline__ float2 ask_turns(const float2* __restrict__ from, int r, int c) {
     return from == nullptr ? make_float2(1.f, 0.f) : from[r / 8 % (HD / 64) * 32 + c * 8 + r % 8];
 }
-// Maximum and sum over the four lanes (r, 0 .. 3), and what the lane (r, C) holds, in all four: rows of 16 lanes exchanged within the vector registers
-// (through LDS, as a shuffle goes, each step waits several times as long).
-__device__ __forceinline__ uint2 exchange_rows(unsigned v) { const auto both = __builtin_amdgcn_permlane16_swap(v, v, false, false); return make_uint2(both[0], both[1]); }      // rows 0 0 2 2, and 1 1 3 3
-__device__ __forceinline__ uint2 exchange_halves(unsigned v) { const auto both = __builtin_amdgcn_permlane32_swap(v, v, false, false); return make_uint2(both[0], both[1]); }    // rows 0 1 0 1, and 2 3 2 3
-__device__ __forceinline__ unsigned as_word(float v) { return __builtin_bit_cast(unsigned, v); }
-__device__ __forceinline__ float as_value(unsigned v) { return __builtin_bit_cast(float, v); }
-__device__ __forceinline__ float max_of_four(float v) {
-    const uint2 rows = exchange_rows(as_word(v));
-    const uint2 halves = exchange_halves(as_word(fmaxf(as_value(rows.x), as_value(rows.y))));
-    return fmaxf(as_value(halves.x), as_value(halves.y));
-}
-__device__ __forceinline__ float sum_of_four(float v) {
-    const uint2 rows = exchange_rows(as_word(v));
-    const uint2 halves = exchange_halves(as_word(as_value(rows.x) + as_value(rows.y)));
-    return as_value(halves.x) + as_value(halves.y);
-}
-template <int C> __device__ __forceinline__ unsigned of_row(unsigned v) {
-    const uint2 halves = exchange_halves(v);
-    const uint2 rows = exchange_rows(C < 2 ? halves.x : halves.y);
-    return C % 2 == 0 ? rows.x : rows.y;
-}
 template <int LANE> __device__ __forceinline__ float of_lane(float v) {          // what the lane (LANE, c) holds, in all lanes (r, c)
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x150 + LANE, 0xF, 0xF, true));      // row_newbcast
 }

@@ -55,6 +55,34 @@ __device__ __forceinline__ float from_eight_lanes_away(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128 /* row_ror:8 */, 0xf, 0xf, false));
 }
 
+// ---- rows of 16 lanes exchanged within the vector registers (every lane of the wavefront takes part) ----
+// Through LDS, as a shuffle goes, each step waits several times as long. Over the four lanes (r, 0 .. 3) that hold column r of a matrix product's result: their maximum and
+// sum (partners as of shuffles over 16 lanes, then 32: the same bits), and what the lane (r, C) holds, in all four; and what the lane 32 away holds.
+// (The ends of the skinny products, four to a layer of a decode step, with them: 0.02 to 0.1 us a product, a step at the Qwen3-0.6B sizes 852 -> 849 us.)
+__device__ __forceinline__ uint2 exchange_rows(unsigned v) { const auto both = __builtin_amdgcn_permlane16_swap(v, v, false, false); return make_uint2(both[0], both[1]); }      // rows 0 0 2 2, and 1 1 3 3
+__device__ __forceinline__ uint2 exchange_halves(unsigned v) { const auto both = __builtin_amdgcn_permlane32_swap(v, v, false, false); return make_uint2(both[0], both[1]); }    // rows 0 1 0 1, and 2 3 2 3
+__device__ __forceinline__ unsigned as_word(float v) { return __builtin_bit_cast(unsigned, v); }
+__device__ __forceinline__ float as_value(unsigned v) { return __builtin_bit_cast(float, v); }
+__device__ __forceinline__ float max_of_four(float v) {
+    const uint2 rows = exchange_rows(as_word(v));
+    const uint2 halves = exchange_halves(as_word(fmaxf(as_value(rows.x), as_value(rows.y))));
+    return fmaxf(as_value(halves.x), as_value(halves.y));
+}
+__device__ __forceinline__ float sum_of_four(float v) {
+    const uint2 rows = exchange_rows(as_word(v));
+    const uint2 halves = exchange_halves(as_word(as_value(rows.x) + as_value(rows.y)));
+    return as_value(halves.x) + as_value(halves.y);
+}
+template <int C> __device__ __forceinline__ unsigned of_row(unsigned v) {
+    const uint2 halves = exchange_halves(v);
+    const uint2 rows = exchange_rows(C < 2 ? halves.x : halves.y);
+    return C % 2 == 0 ? rows.x : rows.y;
+}
+__device__ __forceinline__ float of_other_half(float v) {
+    const uint2 halves = exchange_halves(as_word(v));
+    return as_value(threadIdx.x % XRT_WAVE < XRT_WAVE / 2 ? halves.y : halves.x);
+}
+
 // ---- wave reductions (fixed butterfly order: results do not depend on the launch) ----
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -196,8 +196,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, (MT == 1 ? 4 : 2)) gemm_pack
                 for (int i = 0; i < SQUARES_AHEAD; ++i) sum += early_squares[i];
                 for (int t = begin + 4 * SQUARES_AHEAD; t < end; t += 4)
                     sum += norm.squares_in[(long)t * XRT_SQUARES_STRIDE + row];
-                sum += __shfl_xor(sum, 16);
-                sum += __shfl_xor(sum, 32);
+                sum = sum_of_four(sum);
                 if (thread % XRT_WAVE < 16) squares[thread / XRT_WAVE][thread % 16] = sum;   // read after the barrier of the first tile below
             }
         }
@@ -282,7 +281,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, (MT == 1 ? 4 : 2)) gemm_pack
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 mine[i] = to_float(from_float<bf16>(g[i]));
-                other[i] = __shfl_xor(mine[i], 32);
+                other[i] = of_other_half(mine[i]);
             }
             struct alignas(8) Four { bf16 e[4]; } packed;
 #pragma unroll
@@ -315,7 +314,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, (MT == 1 ? 4 : 2)) gemm_pack
             // lanes c = 0, 1 hold the gate sums of outputs first / 2 + c * 4 + i, lanes c = 2, 3 the up sums of the same
             float u[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) u[i] = __shfl_xor(g[i], 32);
+            for (int i = 0; i < 4; ++i) u[i] = of_other_half(g[i]);
             const long nn = first / 2 + c * 4;
             if (c < 2 && mm < M) {
 #pragma unroll
@@ -351,8 +350,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, (MT == 1 ? 4 : 2)) gemm_pack
         if constexpr (AROUND && MODE == MODE_ACCUMULATE) {
             if (norm.squares_out) {
                 float sum = fmaf(fresh[3], fresh[3], fmaf(fresh[2], fresh[2], fmaf(fresh[1], fresh[1], fresh[0] * fresh[0])));
-                sum += __shfl_xor(sum, 16);
-                sum += __shfl_xor(sum, 32);
+                sum = sum_of_four(sum);
                 if (mm < M) {
                     if (c == 0) norm.squares_out[(long)blockIdx.x * XRT_SQUARES_STRIDE + mm] = sum;
                     if (nn + 3 < N) {                           // N is a multiple of 8: all four or none
@@ -462,7 +460,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, 2) gemm_packed_resident_kern
         if constexpr (MODE == MODE_GATED) {
             float u[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) u[i] = __shfl_xor(g[i], 32);
+            for (int i = 0; i < 4; ++i) u[i] = of_other_half(g[i]);
             const long nn = group * 8 + c * 4;                  // lanes c = 0, 1 hold the gate sums, c = 2, 3 the up sums of the same outputs
             if (c < 2 && r < M) {
 #pragma unroll

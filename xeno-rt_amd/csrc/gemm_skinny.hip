@@ -252,8 +252,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, (MT == 1 ? 4 : 2)) gemm_skin
                 for (int i = 0; i < SQUARES_AHEAD; ++i) sum += early_squares[i];
                 for (int t = first + 4 * SQUARES_AHEAD; t < end; t += 4)
                     sum += norm.squares_in[(long)t * XRT_SQUARES_STRIDE + row];
-                sum += __shfl_xor(sum, 16);
-                sum += __shfl_xor(sum, 32);
+                sum = sum_of_four(sum);
                 if (thread % XRT_WAVE < 16) squares[thread / XRT_WAVE][thread % 16] = sum;   // read after the barrier of the first tile below
             }
         }
@@ -363,7 +362,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, (MT == 1 ? 4 : 2)) gemm_skin
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     mine[i] = to_float(from_float<bf16>(g[i]));
-                    other[i] = __shfl_xor(mine[i], 32);
+                    other[i] = of_other_half(mine[i]);
                 }
                 struct alignas(8) Four { bf16 e[4]; } packed;
 #pragma unroll
@@ -419,8 +418,7 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE, (MT == 1 ? 4 : 2)) gemm_skin
             if constexpr (AROUND && MODE == MODE_ACCUMULATE) {
                 if (norm.squares_out) {
                     float sum = fmaf(fresh[3], fresh[3], fmaf(fresh[2], fresh[2], fmaf(fresh[1], fresh[1], fresh[0] * fresh[0])));
-                    sum += __shfl_xor(sum, 16);
-                    sum += __shfl_xor(sum, 32);
+                    sum = sum_of_four(sum);
                     if (mm < M) {
                         if (c == 0) norm.squares_out[(long)blockIdx.x * XRT_SQUARES_STRIDE + mm] = sum;
                         if (nn < N && c * 4 < rows) {           // N is a multiple of 8 and rows one of 4: all four or none
