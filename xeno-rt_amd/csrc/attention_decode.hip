@@ -450,7 +450,7 @@ __global__ void __launch_bounds__(HD) attention_decode_merge_kernel(
     const int parts = min(n_parts, (n_keys + part_keys - 1) / part_keys);
     float m = d < parts ? early_ml.x : -INFINITY;
     for (int k = d + HD; k < parts; k += HD) m = fmaxf(m, part_ml[(base + k) * 2]);
-    m = wave_max(m);
+    m = whole_wave_max(m);
     if (lane == 0) reduce[wave][0] = m;
     __syncthreads();
     m = reduce[0][0];
@@ -467,7 +467,7 @@ __global__ void __launch_bounds__(HD) attention_decode_merge_kernel(
         weights[k] = weight;
         l = fmaf(weight, part_ml[(base + k) * 2 + 1], l);
     }
-    l = wave_sum(l);
+    l = whole_wave_sum(l);
     if (lane == 0) reduce[wave][1] = l;
     __syncthreads();
     l = reduce[0][1];

@@ -96,6 +96,30 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
+// The same sums and maxima (the same partners in the same order) without LDS, for kernels in which every lane of the wavefront takes part: rows exchanged
+// as above, then rotations of the row, in which lane l meets l ^ 8, and what stands for l ^ 4, l ^ 2, l ^ 1 (by then the values repeat every 8, 4, 2 lanes).
+// (A block's sum, the reduction of split products and the merge of a decode step's parts with them, us before and now: 16 heads on 8, 334 keys of up to 1024, 8.7, 8.4;
+// 32 on 8, 4096 keys 9.5, 9.3; logits of 100 tokens at the Llama-3.2-1B sizes 1228, 1218.)
+template <int BY> __device__ __forceinline__ float of_turned_row(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x120 + BY /* row_ror:BY */, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float whole_wave_sum(float v) {
+    const uint2 halves = exchange_halves(as_word(v));
+    const uint2 rows = exchange_rows(as_word(as_value(halves.x) + as_value(halves.y)));
+    v = as_value(rows.x) + as_value(rows.y);
+    v += of_turned_row<8>(v);
+    v += of_turned_row<4>(v);
+    v += of_turned_row<2>(v);
+    return v + of_turned_row<1>(v);
+}
+__device__ __forceinline__ float whole_wave_max(float v) {
+    v = max_of_four(v);
+    v = fmaxf(v, of_turned_row<8>(v));
+    v = fmaxf(v, of_turned_row<4>(v));
+    v = fmaxf(v, of_turned_row<2>(v));
+    return fmaxf(v, of_turned_row<1>(v));
+}
+
 // Orders the LDS accesses of the lanes of one wavefront: what any lane wrote before is
 // seen by every lane after. (A wavefront's LDS operations execute in order; the fences keep
 // the compiler from moving accesses across.)
@@ -109,7 +133,7 @@ __device__ __forceinline__ void wave_sync() {
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
     const int lane = threadIdx.x % XRT_WAVE, wave = threadIdx.x / XRT_WAVE;
     const int waves = (blockDim.x + XRT_WAVE - 1) / XRT_WAVE;
-    v = wave_sum(v);
+    v = whole_wave_sum(v);                          // (all of a block's threads come here, and blocks are whole wavefronts)
     __syncthreads();
     if (lane == 0) scratch[wave] = v;
     __syncthreads();

@@ -1283,7 +1283,7 @@ __global__ void __launch_bounds__(256) split_reduce_kernel(const float* __restri
     if constexpr (NORM == 1) {
         float total = mine;
         if (N % 256 == 0) {
-            mine = wave_sum(mine);
+            mine = whole_wave_sum(mine);
             if (threadIdx.x % XRT_WAVE == 0) wave_sums[threadIdx.x / XRT_WAVE] = mine;
             __syncthreads();
             total = 0.f;
@@ -1455,7 +1455,7 @@ __global__ void __launch_bounds__(256) split_reduce_qkv_kernel(const float* __re
     if constexpr (NORM == 1) {
         float total = mine;
         if (per_token % 256 == 0) {
-            mine = wave_sum(mine);
+            mine = whole_wave_sum(mine);
             if (threadIdx.x % XRT_WAVE == 0) wave_sums[threadIdx.x / XRT_WAVE] = mine;
             __syncthreads();
             total = 0.f;
