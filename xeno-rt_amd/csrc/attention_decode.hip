@@ -493,7 +493,9 @@ Cut cut_for(int tokens, int n_kv_heads, int q_tiles, int max_context, int head_d
     // Up to eight blocks: one workgroup sees all keys, and nothing is left to merge. From five blocks on it has eight wavefronts, a block
     // each, where every pair finds a compute unit of its own, and four of two blocks beyond (16 heads of 128 on 8, 334 keys: 1 sequence 7.4 us in two
     // parts and their merge, 6.0 with four wavefronts, 5.8 with eight; 16 sequences 9.1, 8.4, 7.9; 48 sequences 18.0, 14.4, 15.9; heads of 64 gain
-    // 0.2 to 1 us by the eight). Nine blocks and more: two blocks one after the other cost more than the merge. (max_context is what the caller says of the step:
+    // 0.2 to 1 us by the eight; all before the chain was as short as it is: 5.0 and 7.3 for 1 and 8 sequences now). Nine blocks and more: two blocks one after the other in
+    // eight wavefronts cost less than parts and their merge where the sequences are much shorter than max_context and more where they are not (1 sequence, with the finish, 334 keys of up to 1024
+    // 6.6 against 8.4, 600 keys 8.5 and 8.5, 1000 keys 11.5 against 9.0: a compute unit takes its half megabyte at 50 bytes a cycle). (max_context is what the caller says of the step:
     // a recorded decode step says the engine's limit or the next 1024 tokens, whichever is less, so that it comes here in engines for up to 512 tokens.)
     if (max_blocks <= 8) {
         const int waves = max_blocks > 4 && pairs <= XRT_COMPUTE_UNITS ? 8 : 4;
