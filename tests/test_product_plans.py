@@ -1,0 +1,24 @@
+"""Which kernel a product takes, by the rules of the launchers: they look at sizes alone, so they are asked here without a GPU."""
+import ctypes
+
+import pytest
+
+MODES = {"store": 0, "add": 1, "gated": 2}
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from xeno_rt_amd.ops import build
+    return ctypes.CDLL(build.find_library() or build.build())
+
+
+# w goes past the caches only where it cannot stay in the last one (256 MB) until the next step: a gated matrix of more than two thirds of that, the matrix back from a
+# feed-forward of 16384 or wider of more than a third; and only where one row of tiles reads it.
+@pytest.mark.parametrize("m,n,k,mode,past", [
+    (17, 3072, 1024, "gated", 0), (64, 8192, 2048, "gated", 0), (40, 14336, 4096, "gated", 1), (64, 10922, 4096, "gated", 0), (64, 10928, 4096, "gated", 1),
+    (72, 8192, 2048, "gated", 0), (128, 3072, 1024, "gated", 0), (100, 14336, 4096, "gated", 1), (128, 8192, 2048, "gated", 0),
+    (129, 14336, 4096, "gated", 0), (200, 8192, 2048, "gated", 0), (256, 6144, 8192, "gated", 0),
+    (24, 2048, 2048, "add", 0), (64, 2048, 8192, "add", 0), (20, 256, 16448, "add", 0), (32, 5120, 25600, "add", 1), (64, 2048, 25600, "add", 1), (64, 1024, 25600, "add", 0),
+    (40, 4096, 14336, "add", 0), (65, 5120, 25600, "add", 0), (64, 131072, 2048, "store", 1), (64, 32000, 2048, "store", 0)])
+def test_w_goes_past_the_caches_only_where_it_cannot_stay_there(lib, m, n, k, mode, past):
+    assert lib.xrt_linear_past_caches(m, n, k, MODES[mode]) == past

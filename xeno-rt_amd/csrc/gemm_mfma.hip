@@ -921,23 +921,26 @@ int launch_grouped_of(const bf16* x, const bf16* m, long w_stride, void* out, in
     return launch_grouped<BM, MODE_STORE, bf16>(x, m, w_stride, (bf16*)out, tiles_m, N, K, lda, ldw, tile_group, packing, activation, splits, s);
 }
 
-// Up to 64 rows of a, k not split: every byte of w is read by one workgroup, in one long run, and is asked for past the caches
+// One row of tiles, k not split: every byte of w is read by one workgroup, in one long run, and is asked for past the caches
 // where it cannot stay in the last one (256 MB) until the next step. (Among other matrices, 64 rows: gate/up of 28672 rows
 // of w and k = 4096 46.6 -> 44.1 us, an output head of 128256 rows and k = 2048 105.0 -> 98.5. A w that does stay is read faster from
 // there: 17408 rows and k = 1024, 214 MB of such matrices in turn, 11.3 us as it is, 12.8 past the caches.) A gated matrix counts one
 // and a half times: a model has the one back from that width too. Split along k the runs are short, and so marked they are
 // read more slowly (4096 x 4096 in eight parts 16.3 -> 18.1 us).
-template <int BM, int MODE>
-bool reads_past_caches(int N, int K, int splits) {
-    constexpr long LAST_CACHE = 256L << 20;
-    return BM <= 64 && splits == 1 && (MODE == MODE_GATED ? 3L * N : (long)N) * K * (long)sizeof(bf16) > LAST_CACHE;
+// The gated tiles of up to 256 rows of a in several stages the same (700 products drawn at random, past the caches against through them: a w too large to stay
+// 0.95 to 0.99 with one row of tiles; matrices of 60 MB in turn 1.02 to 1.08 in tiles of 64 x 64, 1.09 to 1.25 in the others, up to 1.5; with two rows of
+// tiles, the second of which reads what the first has brought, 1.03 to 1.2 whatever w).
+constexpr long LAST_CACHE = 256L << 20;
+bool cannot_stay(long rows_w, int K, int halves) { return rows_w * K * (long)sizeof(bf16) / 2 * halves > LAST_CACHE; }      // halves: what it counts, in half matrices
+bool reads_past_caches(int rows_of_tile, int M, int N, int K, int mode) {
+    return M <= rows_of_tile && (mode == MODE_GATED ? cannot_stay(2L * N, K, 3) : cannot_stay(N, K, 2));
 }
 
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES = false>
 int launch_kernel(const bf16* a, const bf16* w, TO* out, int M, int N, int K, const Packing& packing,
                   hipStream_t s, int splits = 1, int k_per_split = 0, const RowScale scale = RowScale{}) {
-    if constexpr (BM <= 64 && !PAST_CACHES)
-        if (reads_past_caches<BM, MODE>(N, K, splits))
+    if constexpr ((BM <= 64 || (MODE == MODE_GATED && STAGES > 2)) && !PAST_CACHES)
+        if (splits == 1 && reads_past_caches(BM, M, N, K, MODE))
             return launch_kernel<BM, BN, WM, WN, MODE, DK, STAGES, TO, true>(a, w, out, M, N, K, packing, s, splits, k_per_split, scale);
     constexpr int BN_OUT = MODE == MODE_GATED ? BN / 2 : BN;
     constexpr int THREADS = WM * WN * XRT_WAVE;
@@ -1064,17 +1067,12 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
         case TILES_RAGGED_256: return launch_kernel<256, 256, 2, 4, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
         case TILES_RAGGED_128: return launch_kernel<128, 128, 2, 2, MODE, 0, 0, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
         case TILES_128_BY_64_FOUR_STAGES:
-            // (one row of tiles: w past the caches; 8192 pairs, k = 2048, 72 / 100 / 128 rows 17.7 / 18.6 / 19.6 -> 16.1 / 17.7 / 18.0 us. With two rows of
-            // tiles the second reads it from there: 3072 pairs, k = 1024, 160 rows 8.9 us as it is, 9.8 past them)
-            if constexpr (MODE == MODE_GATED) {
-                if (M <= 128) return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO, true>(a, w, out, M, N, K, packing, s, 1, 0, plain);
-                return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
-            }
+            if constexpr (MODE == MODE_GATED) return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
             break;
         case TILES_128_BY_128_THREE_STAGES:
-            // (eight wavefronts, w past the caches: 14336 pairs, k = 4096, 72 / 100 / 128 rows 45.4 / 46.9 / 48.8 -> 43.4 / 45.7 / 47.0 us; 25600 pairs, k = 5120
-            // 110 / 114 / 121 -> 107 / 112 / 118; 8192 pairs, k = 2048, 160 / 256 rows 24.9 / 26.0 -> 22.7 / 24.4)
-            if constexpr (MODE == MODE_GATED) return launch_kernel<128, 128, 4, 2, MODE, 64, 3, TO, true>(a, w, out, M, N, K, packing, s, 1, 0, plain);
+            // (eight wavefronts: 66 such products drawn at random take 0.92 of what they take in four, the slowest 1.02; 14336 pairs, k = 4096, 100 rows 51.6 -> 50.1 us, 25600 pairs,
+            // k = 5120 121 -> 118)
+            if constexpr (MODE == MODE_GATED) return launch_kernel<128, 128, 4, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
             break;
         case TILES_256: return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
         case TILES_192: return launch_large<192, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
@@ -1488,15 +1486,19 @@ __global__ void __launch_bounds__(256) split_reduce_qkv_kernel(const float* __re
     }
 }
 
+// Parts of up to 64 rows of x: w past the caches where it cannot stay in them and k is long, which makes the runs of the parts long again. So long a k is a feed-forward's
+// width, and the matrix back from it counts three times: the gated one of twice its size stands beside it. (700 products drawn at random, past the caches against through them:
+// such a w 0.97, 5120 rows, k = 25600, 32 rows of x 48.6 against 52.9 us; as large and k of 4096 to 16384 0.99, up to 1.08 with more than 48 rows of x; smaller and among
+// more than the caches hold 0.97 to 1.04, 60 MB of them in turn 1.03 to 1.25.)
+bool parts_read_past_caches(long rows_w, int K) { return K >= 16384 && cannot_stay(rows_w, K, 6); }
+
 // The product of all rows of w, ungated, into the workspace: [splits][M][rows_w]
 int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, const Packing& packing, const SplitPlan& plan, hipStream_t s) {
     const int rows_w = (int)plan.rows_w;
     if (M <= SPLIT_BM) {
         // Eight wavefronts, two to a SIMD: one reads its operands while the other multiplies (with four: 3 to 6 % longer, the second kernel included; 1024 rows of w,
-        // k = 2048, 24 rows of x 8.8 -> 8.2 us, 10240 rows, k = 5120 26.7 -> 26.3). w past the caches where w has few rows but is not tiny, or k is very long
-        // (24 / 64 rows of x: 2048 rows of w, k = 2048 8.9 / 10.2 -> 8.1 / 9.6 us, k = 8192 13.7 / 15.7 -> 12.2 / 13.4; 5120 rows, k = 25600 49.5 / 53 -> 46 / 50); not
-        // elsewhere (4096 rows, k = 4096 13.7 / 15.9 us as it is, 13.9 / 17.7 past them; 1024 rows, k = 2048 8.2 / 9.7 and 8.4 / 10.1).
-        const bool past = K >= 16384 || (rows_w <= 3072 && (long)rows_w * K >= 3000000L);
+        // k = 2048, 24 rows of x 8.8 -> 8.2 us, 10240 rows, k = 5120 26.7 -> 26.3).
+        const bool past = parts_read_past_caches(plan.rows_w, K);
         if (past) return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 4, MODE_STORE, 64, 3, float, true>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
         return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 4, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
     }
@@ -1540,7 +1542,7 @@ int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int
     if (M <= SPLIT_BM && plan.splits == 1) {                   // tiles enough: each applies the epilogue itself
         XRT_REQUIRE(!emits, "linear (mfma): only a product split along k writes what the norm after it needs");
         if (mode == MODE_STORE) return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_STORE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
-        if (mode == MODE_GATED && plan.columns == 64) return launch_kernel<SPLIT_BM, 64, 2, 1, MODE_GATED, 64, 4, TO, true>(a, w, out, M, N, K, packing, s, 1, 0, scale);
+        if (mode == MODE_GATED && plan.columns == 64) return launch_kernel<SPLIT_BM, 64, 2, 1, MODE_GATED, 64, 4, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
         if (mode == MODE_GATED) return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 2, MODE_GATED, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
         if constexpr (sizeof(TO) == 4)
             return launch_kernel<SPLIT_BM, SPLIT_BN, 1, 4, MODE_ACCUMULATE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, scale);
@@ -1705,6 +1707,18 @@ extern "C" int xrt_linear_parts(int M, int N, int K, int mode, int whole_norm, i
     *rows = plan.tile;
     *columns = plan.columns;
     return plan.splits;
+}
+
+// Whether a product of 17 to 256 rows of x asks for w past the caches (k a multiple of 64).
+extern "C" int xrt_linear_past_caches(int M, int N, int K, int mode) {
+    if (M <= 16 || M > 256 || N <= 0 || K < (M <= SPLIT_BM ? 128 : 64) || K % 64 != 0 || mode < MODE_STORE || mode > MODE_GATED) return -1;
+    const SplitPlan plan = split_plan(M, N, K, mode);
+    if (plan.splits > 1) return M <= SPLIT_BM && parts_read_past_caches(plan.rows_w, K);
+    if (M > SPLIT_BM) {
+        const int shape = xrt_linear_tiles(XRT_BF16, M, N, K, mode);
+        if (shape != TILES_128_BY_64_FOUR_STAGES && shape != TILES_128_BY_128_THREE_STAGES) return 0;
+    }
+    return reads_past_caches(M <= SPLIT_BM ? SPLIT_BM : 128, M, N, K, mode);
 }
 
 // The first kernel alone of a bfloat16 product split along k (xrt_linear_split_takes says so and asks for a workspace): the sums of the parts,
