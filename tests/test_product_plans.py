@@ -18,7 +18,18 @@ def lib():
     (17, 3072, 1024, "gated", 0), (64, 8192, 2048, "gated", 0), (40, 14336, 4096, "gated", 1), (64, 10922, 4096, "gated", 0), (64, 10928, 4096, "gated", 1),
     (72, 8192, 2048, "gated", 0), (128, 3072, 1024, "gated", 0), (100, 14336, 4096, "gated", 1), (128, 8192, 2048, "gated", 0),
     (129, 14336, 4096, "gated", 0), (200, 8192, 2048, "gated", 0), (256, 6144, 8192, "gated", 0),
-    (24, 2048, 2048, "add", 0), (64, 2048, 8192, "add", 0), (20, 256, 16448, "add", 0), (32, 5120, 25600, "add", 1), (64, 2048, 25600, "add", 1), (64, 1024, 25600, "add", 0),
+    (24, 2048, 2048, "add", 0), (64, 2048, 8192, "add", 0), (20, 256, 16448, "add", 0), (32, 5120, 25600, "add", 1), (64, 2048, 25600, "add", 1), (64, 1024, 25600, "add", 0), 
     (40, 4096, 14336, "add", 0), (65, 5120, 25600, "add", 0), (64, 131072, 2048, "store", 1), (64, 32000, 2048, "store", 0)])
 def test_w_goes_past_the_caches_only_where_it_cannot_stay_there(lib, m, n, k, mode, past):
     assert lib.xrt_linear_past_caches(m, n, k, MODES[mode]) == past
+
+
+# Gated products of 17 to 64 rows: in one round of tiles of 64 rows of w, unsplit, where k is short for the number of tiles; in parts along k where a few workgroups would
+# walk all of a long k alone.
+@pytest.mark.parametrize("m,n,k,unsplit", [
+    (17, 40, 128, True), (33, 8192, 192, True), (24, 3072, 1024, True), (64, 8192, 2048, True), (64, 8192, 4160, True), (64, 32, 512, True), (17, 512, 768, True),
+    (64, 5120, 3072, False), (64, 704, 4096, False), (64, 1000, 5248, False), (30, 1408, 2048, False), (25, 688, 16320, False), (48, 72, 2048, False), (17, 64, 6400, False), (64, 2816, 4096, False)])
+def test_gated_products_of_few_rows_walk_a_long_k_in_parts(lib, m, n, k, unsplit):
+    rows, columns = ctypes.c_int(), ctypes.c_int()
+    parts = lib.xrt_linear_parts(m, n, k, MODES["gated"], 0, ctypes.byref(rows), ctypes.byref(columns))
+    assert (parts, columns.value) == (1, 64) if unsplit else parts >= 3 and columns.value == 128

@@ -1160,6 +1160,20 @@ long unsplit_time(int M, int N, int K, int mode) {
     return 1000 + (mode == MODE_GATED ? least : least * 127 / 100);
 }
 
+// Gated products of 17 to 64 rows of x (nanoseconds): unsplit in one round of tiles of 64 x 64, every workgroup all of k, or in parts of 64 x 128 as many as the compute units
+// take, and a second kernel. A step of 64 along k takes its time however few the tiles, so a long k with few of them wants parts (64 rows of x, 1408 rows of w, k = 4096 20.4 us unsplit,
+// 13.2 in parts; 512 rows, k = 8192 36.4, 12.4; 10240 rows, k = 3072 21.2, 20.1) and a short one none (6144 rows of w, k = 1024, 24 rows of x 8.4 us, 10.1 in parts; 16384 rows, k = 2048, 64 rows
+// 17.7, 21.0). Fitted to 3841 products drawn at random (128 to 16384 rows of w, k of 128 to 16384, 17 to 64 rows of x, a third of them of widths that are multiples of 256): what the
+// estimates choose is 0.1 % off the better of the two on average and takes 0.91 of what parts alone do, 34 above 1.03, up to 1.17.
+long narrow_gated_time(int M, long rows_w, int units) {
+    const long share = dealt((rows_w + 63) / 64);              // (of the compute units; at most all of them)
+    return 3970 + units * (243 + (77 * 64 + 33 * M) * share / (64 * XRT_COMPUTE_UNITS)) + 2510 * (M * rows_w / 1000) / 1000;
+}
+long few_rows_parts_time(int M, long rows_w, int per, int parts) {
+    const long groups = dealt((rows_w + SPLIT_BN - 1) / SPLIT_BN) * parts;
+    return 5330 + 94 * parts + per * (328 + 318 * groups / XRT_COMPUTE_UNITS + (groups > XRT_COMPUTE_UNITS ? 250 : 0)) + 2490 * parts * (M * rows_w / 1000) / 1000;
+}
+
 // whole_norm: an RMSNorm follows that the second kernel can do outright, which is worth a split in two where the product alone
 // would do as well without (k from 4096 on instead of from 8192 on).
 SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
@@ -1171,10 +1185,11 @@ SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
     if (M <= SPLIT_BM) {
         splits = (int)(XRT_COMPUTE_UNITS / tiles_n);                         // one workgroup per compute unit, or fewer
         least = 1;
-        // gated, and one round of tiles of half the width: those, without a second kernel. 6144 rows of w, k = 1024 10.3 -> 8.9 us (17 rows of x), 13.5 -> 9.6
-        // (64 rows); 16384 rows, k = 2048 19.3 -> 15.1 and 21.4 -> 16.5; 10240 rows, k = 3072 18.7 -> 18.0 and 21.2 -> 19.9. (Beyond one round they read x too
-        // often: 28672 rows, k = 4096, 64 rows of x 43 us in tiles of 128, 47 in these.)
-        if (mode == MODE_GATED && (rows_w + 63) / 64 <= XRT_COMPUTE_UNITS) { splits = 1; columns = 64; }
+        if (mode == MODE_GATED && (rows_w + 63) / 64 <= XRT_COMPUTE_UNITS) {
+            // one round of tiles of half the width is there for the taking, without a second kernel: by the estimates of both
+            const int parts = max(1, min(min(splits, 16), units)), per = (units + parts - 1) / parts;
+            if (parts == 1 || narrow_gated_time(M, rows_w, units) < few_rows_parts_time(M, rows_w, per, (units + per - 1) / per)) { splits = 1; columns = 64; }
+        }
     } else if (large_tiles <= 128 && M >= 512 && mode != MODE_GATED && units >= (whole_norm ? 64 : 128)) {
         // Many rows and a very long k, but so few columns that the largest tiles would leave half of the compute
         // units idle (the projection back from the feed-forward's width): the large tiles split k between them.
