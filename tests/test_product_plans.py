@@ -18,7 +18,7 @@ def lib():
     (17, 3072, 1024, "gated", 0), (64, 8192, 2048, "gated", 0), (40, 14336, 4096, "gated", 1), (64, 10922, 4096, "gated", 0), (64, 10928, 4096, "gated", 1),
     (72, 8192, 2048, "gated", 0), (128, 3072, 1024, "gated", 0), (100, 14336, 4096, "gated", 1), (128, 8192, 2048, "gated", 0),
     (129, 14336, 4096, "gated", 0), (200, 8192, 2048, "gated", 0), (256, 6144, 8192, "gated", 0),
-    (24, 2048, 2048, "add", 0), (64, 2048, 8192, "add", 0), (20, 256, 16448, "add", 0), (32, 5120, 25600, "add", 1), (64, 2048, 25600, "add", 1), (64, 1024, 25600, "add", 0), 
+    (24, 2048, 2048, "add", 0), (64, 2048, 8192, "add", 0), (20, 256, 16448, "add", 0), (32, 5120, 25600, "add", 1), (64, 2048, 25600, "add", 1), (64, 1024, 25600, "add", 0), (45, 1792, 16384, "gated", 0), (45, 2816, 16384, "gated", 1),
     (40, 4096, 14336, "add", 0), (65, 5120, 25600, "add", 0), (64, 131072, 2048, "store", 1), (64, 32000, 2048, "store", 0)])
 def test_w_goes_past_the_caches_only_where_it_cannot_stay_there(lib, m, n, k, mode, past):
     assert lib.xrt_linear_past_caches(m, n, k, MODES[mode]) == past

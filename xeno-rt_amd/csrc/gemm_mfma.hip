@@ -1501,19 +1501,19 @@ __global__ void __launch_bounds__(256) split_reduce_qkv_kernel(const float* __re
     }
 }
 
-// Parts of up to 64 rows of x: w past the caches where it cannot stay in them and k is long, which makes the runs of the parts long again. So long a k is a feed-forward's
+// Parts of up to 64 rows of x: w past the caches where it cannot stay in them and k is long, which makes the runs of the parts long again. Ungated, so long a k is a feed-forward's
 // width, and the matrix back from it counts three times: the gated one of twice its size stands beside it. (700 products drawn at random, past the caches against through them:
 // such a w 0.97, 5120 rows, k = 25600, 32 rows of x 48.6 against 52.9 us; as large and k of 4096 to 16384 0.99, up to 1.08 with more than 48 rows of x; smaller and among
 // more than the caches hold 0.97 to 1.04, 60 MB of them in turn 1.03 to 1.25.)
-bool parts_read_past_caches(long rows_w, int K) { return K >= 16384 && cannot_stay(rows_w, K, 6); }
+bool parts_read_past_caches(long rows_w, int K, bool gated) { return K >= 16384 && cannot_stay(rows_w, K, gated ? 3 : 6); }
 
 // The product of all rows of w, ungated, into the workspace: [splits][M][rows_w]
-int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, const Packing& packing, const SplitPlan& plan, hipStream_t s) {
+int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, bool gated, const Packing& packing, const SplitPlan& plan, hipStream_t s) {
     const int rows_w = (int)plan.rows_w;
     if (M <= SPLIT_BM) {
         // Eight wavefronts, two to a SIMD: one reads its operands while the other multiplies (with four: 3 to 6 % longer, the second kernel included; 1024 rows of w,
         // k = 2048, 24 rows of x 8.8 -> 8.2 us, 10240 rows, k = 5120 26.7 -> 26.3).
-        const bool past = parts_read_past_caches(plan.rows_w, K);
+        const bool past = parts_read_past_caches(plan.rows_w, K, gated);
         if (past) return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 4, MODE_STORE, 64, 3, float, true>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
         return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 4, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
     }
@@ -1564,7 +1564,7 @@ int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int
         XRT_REQUIRE(false, "linear (mfma): accumulation needs a float32 output");
     }
     XRT_REQUIRE(workspace != nullptr, "linear (mfma): a product split along k needs its workspace");
-    if (launch_parts(a, w, workspace, M, K, packing, plan, s) != 0) return 1;
+    if (launch_parts(a, w, workspace, M, K, mode == MODE_GATED, packing, plan, s) != 0) return 1;
     const unsigned blocks = (unsigned)(((long)M * N + 255) / 256);
     const xrt_linear_norm none = {};
     const xrt_linear_norm& around = norm ? *norm : none;
@@ -1728,7 +1728,7 @@ extern "C" int xrt_linear_parts(int M, int N, int K, int mode, int whole_norm, i
 extern "C" int xrt_linear_past_caches(int M, int N, int K, int mode) {
     if (M <= 16 || M > 256 || N <= 0 || K < (M <= SPLIT_BM ? 128 : 64) || K % 64 != 0 || mode < MODE_STORE || mode > MODE_GATED) return -1;
     const SplitPlan plan = split_plan(M, N, K, mode);
-    if (plan.splits > 1) return M <= SPLIT_BM && parts_read_past_caches(plan.rows_w, K);
+    if (plan.splits > 1) return M <= SPLIT_BM && parts_read_past_caches(plan.rows_w, K, mode == MODE_GATED);
     if (M > SPLIT_BM) {
         const int shape = xrt_linear_tiles(XRT_BF16, M, N, K, mode);
         if (shape != TILES_128_BY_64_FOUR_STAGES && shape != TILES_128_BY_128_THREE_STAGES) return 0;
@@ -1740,5 +1740,5 @@ extern "C" int xrt_linear_past_caches(int M, int N, int K, int mode) {
 // [parts][M][N], for a kernel that adds them itself. Returns the number of parts, or 0 on failure.
 int xrt_linear_split_parts(const void* a, const void* w, int M, int N, int K, const Packing& packing, float* workspace, hipStream_t s) {
     const SplitPlan plan = split_plan(M, N, K, MODE_STORE);
-    return launch_parts((const bf16*)a, (const bf16*)w, workspace, M, K, packing, plan, s) == 0 ? plan.splits : 0;
+    return launch_parts((const bf16*)a, (const bf16*)w, workspace, M, K, false, packing, plan, s) == 0 ? plan.splits : 0;
 }
