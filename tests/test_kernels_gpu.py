@@ -163,11 +163,28 @@ def test_linear_float32_has_the_same_bits_with_few_rows_and_with_many(ops, m, n,
             assert torch.equal(torch.nan_to_num(got, nan=7.0), torch.nan_to_num(want, nan=7.0))
 
 
-# The tiles of that product (rows of a, 16 columns shared by all wavefronts or 16 of each), by the rule of the launcher, with one step along k, as many as there are
-# stages in LDS and more, a last step that is whole, partial or a single piece, results that do and do not allow 16 bytes a store.
-FLOAT_TILES = {(777, 2052, 2048): "112", (777, 2050, 2020): "112", (129, 8190, 576): "80", (692, 3070, 772): "80", (777, 2048, 52): "32", (1023, 1021, 1988): "32", (690, 3070, 36): "32",
+# The tiles of that product (rows of a, 16 columns shared by all wavefronts or 16 of each), by the rule of the launcher, of many steps along k but for a few, with a
+# last step that is whole, partial or a single piece, results that do and do not allow 16 bytes a store.
+FLOAT_TILES = {(777, 2052, 2048): "112", (777, 2050, 2020): "112", (129, 8190, 576): "80", (692, 3070, 772): "80", (777, 2048, 52): "112", (1023, 1021, 1988): "32", (1420, 130, 36): "32",
                (100, 2048, 1024): "16", (70, 2046, 484): "16", (33, 500, 1028): "16 shared", (17, 64, 100): "16 shared", (18, 68, 384): "16 shared",
                (100, 1023, 3084): "32 shared", (40, 2048, 644): "32 shared", (64, 2048, 512): "32 shared"}
+
+
+def float_tile(ops, m, n, k, mode):
+    rows, together = ctypes.c_int(), ctypes.c_int()
+    assert ops.lib.xrt_linear_float_tile(m, n, k, MODES[mode], ctypes.byref(rows), ctypes.byref(together)) == 0
+    return f"{rows.value}{' shared' if together.value else ''}"
+
+
+def same_bits_as_few_rows_at_a_time(ops, a, w, base, mode):
+    n, many, few = base.shape[1], base.clone(), base.clone()
+    for out, step in ((many, a.shape[0]), (few, 16)):
+        for at in range(0, a.shape[0], step):
+            if mode == "gated":
+                ops.linear_glu(a[at:at + step], w, out[at:at + step])
+            else:
+                ops.linear(a[at:at + step], w[:n], out[at:at + step], accumulate=mode == "add")
+    return torch.equal(torch.nan_to_num(many, nan=7.0), torch.nan_to_num(few, nan=7.0))
 
 
 @pytest.mark.parametrize("m,n,k", FLOAT_TILES)
@@ -175,18 +192,28 @@ def test_linear_float32_has_the_same_bits_in_every_tile(ops, m, n, k):
     a, w, base = rand(m, k, seed=m), rand(2 * n, k, seed=n, scale=0.3), rand(m, n, seed=5)
     a[m - 2] *= 1e-36
     a[m // 2, k - 1] = float("inf")
-    rows, together = ctypes.c_int(), ctypes.c_int()
     for mode in ("store", "add", "gated"):
-        assert ops.lib.xrt_linear_float_tile(m, n, k, MODES[mode], ctypes.byref(rows), ctypes.byref(together)) == 0
-        assert f"{rows.value}{' shared' if together.value else ''}" == FLOAT_TILES[m, n, k], mode
-        many, few = base.clone(), base.clone()
-        for out, step in ((many, m), (few, 16)):
-            for at in range(0, m, step):
-                if mode == "gated":
-                    ops.linear_glu(a[at:at + step], w, out[at:at + step])
-                else:
-                    ops.linear(a[at:at + step], w[:n], out[at:at + step], accumulate=mode == "add")
-        assert torch.equal(torch.nan_to_num(many, nan=7.0), torch.nan_to_num(few, nan=7.0)), mode
+        assert float_tile(ops, m, n, k, mode) == FLOAT_TILES[m, n, k], mode
+        assert same_bits_as_few_rows_at_a_time(ops, a, w, base, mode), mode
+
+
+# Every tile with one step along k (32 columns, 64 where the wavefronts share their columns), one less than there are stages in LDS, as many, one and two more, and the last numbers without and the
+# first with steps whose loads go out between the products; the last step whole and partial. A size takes the tile named, by the launcher's rule: the first of these that does.
+FLOAT_SIZES = [(17, 5), (17, 64), (17, 2050), (17, 3000), (17, 4100), (17, 8), (52, 4100), (1420, 130), (2091, 66), (261, 4100), (322, 3000), (322, 4100), (749, 2050), (1664, 260), (1542, 1024)]
+
+
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 11, 12, 13])
+@pytest.mark.parametrize("tile", ["16", "32", "80", "96", "112", "16 shared", "32 shared"])
+def test_linear_float32_has_the_same_bits_at_the_edges_of_its_stages(ops, tile, steps):
+    step = 64 if "shared" in tile else 32
+    for mode in ("store", "add", "gated"):
+        if tile == "96" and mode != "gated":
+            continue
+        for k in (steps * step, steps * step - 4 * (1 + steps * 5 % (step // 4 - 1))):
+            m, n = next((m, n) for m, n in FLOAT_SIZES if float_tile(ops, m, n, k, mode) == tile)
+            a, w, base = rand(m, k, seed=m), rand(2 * n if mode == "gated" else n, k, seed=n, scale=0.3), rand(m, n, seed=5)
+            a[m - 2] *= 1e-36
+            assert same_bits_as_few_rows_at_a_time(ops, a, w, base, mode), (m, n, k, mode)
 
 
 # Gated products of 17 to 64 rows: one round of tiles of 64 rows of w without a split, its last full tile and one more (then wider tiles), a long k (then parts), rows of x without

@@ -33,3 +33,14 @@ def test_gated_products_of_few_rows_walk_a_long_k_in_parts(lib, m, n, k, unsplit
     rows, columns = ctypes.c_int(), ctypes.c_int()
     parts = lib.xrt_linear_parts(m, n, k, MODES["gated"], 0, ctypes.byref(rows), ctypes.byref(columns))
     assert (parts, columns.value) == (1, 64) if unsplit else parts >= 3 and columns.value == 128
+
+
+# Float32 products of a short k, which are little but a tile's start and end: not in many small tiles, nor in large ones where results leave one by one; six blocks where five make two
+# rounds and seven leave compute units without work.
+@pytest.mark.parametrize("m,n,k,mode,tile", [
+    (358, 3536, 8, "gated", 96), (1479, 844, 8, "gated", 96), (223, 5756, 40, "gated", 112), (551, 2484, 192, "gated", 96), (354, 3272, 348, "gated", 96), (886, 948, 16, "gated", 32),
+    (281, 1890, 60, "add", 16), (1149, 478, 4, "add", 16), (1699, 1328, 4, "gated", 80), (17, 64, 100, "store", 16), (777, 2048, 2048, "add", 112)])
+def test_float32_products_of_a_short_k_take_the_tile_that_ends_soonest(lib, m, n, k, mode, tile):
+    rows, together = ctypes.c_int(), ctypes.c_int()
+    assert lib.xrt_linear_float_tile(m, n, k, MODES[mode], ctypes.byref(rows), ctypes.byref(together)) == 0
+    assert rows.value == tile

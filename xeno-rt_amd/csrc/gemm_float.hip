@@ -371,23 +371,32 @@ int launch(const float* a, const float* w, float* out, int M, int N, int K, int 
     return 0;
 }
 
-// The tiles that there are, and what a product takes in them, in us: fixed + chunks of k * max(alone, share * tiles of the fullest compute unit). Alone: a chunk of
-// a tile that has a compute unit to itself; share: what each tile adds where several run there. Fitted to 400 products drawn at random (17 to 2000 rows of a, 64 to
-// 8192 columns, k of 64 to 8192), of which every tile was timed: what it chooses is 3 % off the best of these six (5 % off the best of fifteen: blocks of
-// 1 to 8, six stages), and takes 0.56 of what the kernel before took. The slowest against that kernel: 41 rows, 684 columns, k = 68, 5.8 -> 7.0 us.
-struct Tile { int rows; bool together; struct { double fixed, alone, share; } plain, gated; };
+// The tiles that there are, and what a product takes in them, in us: fixed + ends * n + chunks of k * max(alone, share * n), n being the tiles of the fullest compute unit. Alone: a chunk of
+// a tile that has a compute unit to itself; share: what each tile adds where several run there; ends: a tile's first loads and its epilogue, of each of the kinds below. Fitted to 2994 products
+// drawn at random (17 to 2500 rows of a, 8 to 9000 columns, k of 4 to 8192), of which every tile was timed: what it chooses is 1.5 % off the best of nine (blocks of 1 to 7, of 1 and 2 shared), takes
+// 0.544 of what the kernel before these took, and 55 of them more than 1.03 of that, 14 more than 1.1 (gated, k up to 350 and few rounds of tiles, or k of 4 to 16 and nothing but
+// ends: 49 x 5136, k = 44 5.3 -> 6.2 us, 2414 x 8504, k = 12 61 -> 75, the most; of 1494 more 32 and 7, 1040 x 452, k = 140 8.6 -> 12.5). Without the ends, which a short k consists of, 90 were above 1.03 and 49 above 1.1, up to 1.45 (358 x 3536 gated, k = 8
+// 7.4 -> 10.6, now 7.9). Six blocks gated close the gap between five and seven, where as many tiles make two rounds and one (551 x 2484, k = 192 19.5 -> 17.2, 18.3 before).
+enum { STORES_WIDE, STORES_NARROW, ADDS_WIDE, ADDS_NARROW };       // results in pieces of 16 bytes, or one by one; gated ones are stores
+struct Takes { double fixed, alone, share, ends[4]; };
+struct Tile { int rows; bool together; Takes plain, gated; };
+constexpr Takes NEVER = {1e9, 0, 0, {}};
 constexpr Tile TILES[] = {
-    {1, false, {6.4, 0.080, 0.0875}, {6.3, 0.160, 0.168}}, {2, false, {6.0, 0.161, 0.145}, {6.6, 0.270, 0.275}}, {5, false, {6.5, 0.325, 0.337}, {7.3, 0.600, 0.674}},
-    {7, false, {6.5, 0.476, 0.478}, {8.6, 0.916, 0.941}}, {1, true, {6.5, 0.041, 0.034}, {6.7, 0.060, 0.061}}, {2, true, {6.5, 0.056, 0.056}, {6.4, 0.098, 0.110}}};
+    {1, false, {3.2, 0.115, 0.089, {0.5, 0.7, 0.5, 1.1}}, {2.9, 0.195, 0.168, {1.2, 1.3}}}, {2, false, {2.9, 0.178, 0.143, {0.8, 1.3, 1.0, 2.1}}, {2.8, 0.304, 0.270, {1.7, 1.9}}},
+    {5, false, {2.5, 0.278, 0.338, {1.8, 3.2, 2.4, 5.6}}, {2.1, 0.277, 0.665, {4.5, 5.3}}}, {7, false, {1.1, 0.470, 0.456, {3.9, 6.0, 5.2, 10.1}}, {1.9, 0.126, 0.931, {5.5, 6.6}}},
+    {1, true, {3.4, 0.047, 0.037, {0.3, 0.3, 0.4, 0.5}}, {3.2, 0.029, 0.063, {0.6, 0.6}}}, {2, true, {3.3, 0.016, 0.060, {0.5, 0.6, 0.7, 1.0}}, {2.2, 0.014, 0.109, {2.0, 2.0}}},
+    {6, false, NEVER, {1.9, 0.127, 0.777, {4.9, 6.0}}}};
 
 int tile_for(int M, int N, int K, int mode) {
+    const int kind = (N % 4 == 0 ? STORES_WIDE : STORES_NARROW) + (mode == MODE_ACCUMULATE ? ADDS_WIDE : 0);
     int best = 0;
     double least = 0;
     for (int i = 0; i < (int)(sizeof(TILES) / sizeof(TILES[0])); ++i) {
         const Tile& t = TILES[i];
-        const auto& takes = mode == MODE_GATED ? t.gated : t.plain;
+        const Takes& takes = mode == MODE_GATED ? t.gated : t.plain;
         const long tiles = (((long)M + 16 * t.rows - 1) / (16 * t.rows)) * ((N + (t.together ? 15 : 63L)) / (t.together ? 16 : 64));
-        const double us = takes.fixed + (K + 15L) / 16 * std::fmax(takes.alone, takes.share * ((tiles + XRT_COMPUTE_UNITS - 1) / XRT_COMPUTE_UNITS));
+        const long fullest = (tiles + XRT_COMPUTE_UNITS - 1) / XRT_COMPUTE_UNITS;
+        const double us = takes.fixed + takes.ends[kind] * fullest + (K + 15L) / 16 * std::fmax(takes.alone, takes.share * fullest);
         if (i == 0 || us < least) { best = i; least = us; }
     }
     return best;
@@ -401,8 +410,11 @@ int launch_mode(const float* a, const float* w, float* out, int M, int N, int K,
         case 2: return launch<MODE, 5, false>(a, w, out, M, N, K, activation, s);
         case 3: return launch<MODE, 7, false>(a, w, out, M, N, K, activation, s);
         case 4: return launch<MODE, 1, true>(a, w, out, M, N, K, activation, s);
-        default: return launch<MODE, 2, true>(a, w, out, M, N, K, activation, s);
+        case 5: return launch<MODE, 2, true>(a, w, out, M, N, K, activation, s);
+        default: break;
     }
+    if constexpr (MODE == MODE_GATED) return launch<MODE, 6, false>(a, w, out, M, N, K, activation, s);
+    XRT_REQUIRE(false, "linear (float32): no tile for such a product");
 }
 
 }  // namespace
