@@ -129,11 +129,15 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// sum over a block of up to 1024 threads; every thread gets the result. `scratch` holds 32 floats.
+// The threads of a block for `threads` pieces of work: whole wavefronts, as block_sum wants them.
+inline int whole_wavefronts(int threads) { return (threads + XRT_WAVE - 1) / XRT_WAVE * XRT_WAVE; }
+
+// sum over a block of up to 1024 threads, whole wavefronts of them (row exchanges want every lane there); every
+// thread comes here and gets the result. `scratch` holds 32 floats.
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
     const int lane = threadIdx.x % XRT_WAVE, wave = threadIdx.x / XRT_WAVE;
-    const int waves = (blockDim.x + XRT_WAVE - 1) / XRT_WAVE;
-    v = whole_wave_sum(v);                          // (all of a block's threads come here, and blocks are whole wavefronts)
+    const int waves = blockDim.x / XRT_WAVE;
+    v = whole_wave_sum(v);
     __syncthreads();
     if (lane == 0) scratch[wave] = v;
     __syncthreads();

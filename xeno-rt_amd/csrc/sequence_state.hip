@@ -768,7 +768,7 @@ extern "C" int xrt_add_normed(float* residual, const float* x0, const void* gain
     if (rows == 0) return 0;
     const int quads = width / 4;
     if (x1 == nullptr && width % 4 == 0 && quads <= 1024 * ADD_NORMED_OWNED && ((uintptr_t)residual | (uintptr_t)x0 | (uintptr_t)copy) % 16 == 0) {
-        const int threads = min(1024, (quads + XRT_WAVE - 1) / XRT_WAVE * XRT_WAVE);
+        const int threads = min(1024, whole_wavefronts(quads));
         add_normed_row_kernel<<<(unsigned)rows, threads, 0, (hipStream_t)stream>>>(residual, x0, gain0, gain_dtype, width, eps, scale, copy, copy_dtype);
         XRT_LAUNCH_CHECK("add_normed");
         return 0;

@@ -309,7 +309,7 @@ extern "C" int xrt_embed_normed(const void* table, const void* positions_table, 
     XRT_REQUIRE(tokens >= 0 && tokens < (1L << 31) && width > 0 && (positions_table == nullptr || (positions && position_rows > 0)), "embed_normed: bad sizes");
     if (tokens == 0) return 0;
     if (dtype == XRT_BF16 && width % 8 == 0 && width <= 8192 && ((uintptr_t)table | (uintptr_t)positions_table | (uintptr_t)out | (uintptr_t)copy) % 16 == 0) {
-        const int threads = (width / 8 + XRT_WAVE - 1) / XRT_WAVE * XRT_WAVE;
+        const int threads = whole_wavefronts(width / 8);
         embed_normed_row_kernel<<<(unsigned)tokens, threads, 0, (hipStream_t)stream>>>((const bf16*)table, (const bf16*)positions_table, ids, positions,
                                                                                      position_rows, gain, gain_dtype, eps, width, out, copy, copy_dtype);
         XRT_LAUNCH_CHECK("embed_normed");
