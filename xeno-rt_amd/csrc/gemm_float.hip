@@ -17,18 +17,20 @@
 //             in the order of k, two steps behind the products. Four times as many tiles, for products that have few.
 // Rows of a come in blocks of 16, so that a tile of 5 or 7 blocks divides what is left over: 777 rows, 2048 columns are 224 tiles of 7 blocks by
 // 64, one round; in blocks of 64 by 64, as it was before, 416 tiles for 256 compute units. Before (32x32x2, operands through registers) and now,
-// us, k = 2048 unless said:
+// us, k = 2048 unless said, four matrices in turn:
 //   rows of a                         17 .. 20      64           100          200          400          777
-//   2048 columns                      49 -> 10      49 -> 12     49 -> 18     50 -> 24     51 -> 39     84 -> 64
-//   3072 columns                      49 -> 12      50 -> 18     50 -> 24     51 -> 33     84 -> 49     120 -> 83
-//   8192 gated                        54 -> 31      53 -> 41     89 -> 70     168 -> 131   279 -> 228   498 -> 416
-//   2048 columns, k = 8192            184 -> 34     184 -> 41    184 -> 60    186 -> 88    188 -> 135   319 -> 233
-// The last column is 81 to 87 % of what the matrix cores do (157 TFLOP/s), counted with the rows and columns that fill tiles up; the additions alone take 11 %.
+//   2048 columns                      50 -> 10      50 -> 12     50 -> 18     51 -> 26     53 -> 41     88 -> 67
+//   3072 columns                      49 -> 12      50 -> 18     51 -> 25     53 -> 33     86 -> 49     121 -> 86
+//   8192 gated                        50 -> 30      51 -> 40     86 -> 70     161 -> 123   271 -> 242   499 -> 427
+//   2048 columns, k = 8192            184 -> 37     186 -> 44    187 -> 80    187 -> 91    189 -> 141   320 -> 232
+// The last column is 63, 75, 80 and 72 % of what the matrix cores do (157 TFLOP/s), counted with the rows and columns that fill tiles up; of the compute units that have a
+// tile in the last round 72, 80, 80 and 82 %. The additions alone take 11 %.
 #include <type_traits>
 #include <utility>
 #include <cmath>
 #include "common.h"
 #include "xrt_hip.h"
+#include "gemm_float.h"
 #include "activation.h"
 
 namespace {
@@ -419,7 +421,6 @@ int launch_mode(const float* a, const float* w, float* out, int M, int N, int K,
 
 }  // namespace
 
-// Whole pieces of 16 bytes, and offsets inside a tile that 32 bits hold.
 bool xrt_linear_float_accepts(const void* a, const void* w, int M, int K) {
     return M > 16 && K % 4 == 0 && K <= (1 << 22) && (uintptr_t)a % 16 == 0 && (uintptr_t)w % 16 == 0;
 }

@@ -1133,6 +1133,9 @@ struct SplitPlan { int splits, k_per_split; long rows_w; int tile, columns; };  
 // Workgroups are counted as the fullest die has them: counting their number alone put two rounds on seven of the eight dies where the tiles are no multiple of
 // eight (298 rows of x, 5328 rows of w in pairs, k = 9664: 77 us, 55 by the rule before this estimate; 140 rows, 5120 rows, k = 25600 96, now 70). Of 1086 more products drawn
 // at random, 65 to 1800 rows of x, k up to 26000, 46 took over 5 % longer by it than by that rule, up to 1.42 times; counted so 7 do, up to 1.18, and the average of all is 0.875.
+// (The times are of kernels of four wavefronts; those of 128 x 64 with k < 4096 and the gated ones of 128 x 128 have eight now, and are 3 to 8 % faster. With the kernels as they
+// are, of 1444 gated products of 65 to 256 rows of x drawn at random the choice is 0.7 % off the better of parts and none, 24 of them over 1.1; of 587 others from k = 1024 on 0.3 %. Below that
+// the tiles without a split are taken for faster than they are: 58 adding ones of k < 512 and fewer than 2000 rows of w would be 1.4 times as fast in parts.)
 struct PartTime { int columns, places, once, step, share, beside, part, sums; };
 constexpr int DIES = 8;
 // Tiles are dealt to the dies in equal runs (tile_place): what the largest run comes to on all of them.

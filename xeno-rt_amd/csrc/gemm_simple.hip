@@ -12,10 +12,8 @@
 // [out][in], no bias.
 #include "common.h"
 #include "xrt_hip.h"
+#include "gemm_float.h"
 #include "activation.h"
-
-bool xrt_linear_float_accepts(const void* a, const void* w, int M, int K);
-int xrt_linear_float(const float* a, const float* w, float* out, int M, int N, int K, int mode, int activation, hipStream_t s);
 
 namespace {
 
