@@ -350,6 +350,23 @@ def test_large_tiles_into_a_result_that_is_not_aligned(ops, m, n, k, kind, tiles
     assert torch.equal(results[0], results[1]) and not bool((results[0] == 7.0).all())
 
 
+# The other kernels that ask for w past the caches: gated tiles of 64 x 64, 128 x 64 and 128 x 128, and parts along k.
+@pytest.mark.parametrize("packed", [True, False])
+@pytest.mark.parametrize("m,n,k,mode", [(64, 8190, 5504, "gated"), (128, 7680, 5888, "gated"), (100, 24000, 2048, "gated"), (33, 2044, 25600, "add"), (64, 2800, 16384, "gated")])
+def test_products_of_a_w_beyond_the_caches_in_tiles_and_in_parts(ops, m, n, k, mode, packed):
+    n = n // 8 * 8 if mode == "gated" and packed else n
+    assert ops.lib.xrt_linear_past_caches(m, n, k, MODES[mode]) == 1
+    a, w, base = rand(m, k, dtype=torch.bfloat16, seed=m), rand(2 * n if mode == "gated" else n, k, dtype=torch.bfloat16, seed=n, scale=0.1), rand(m, n, seed=5)
+    both = a.double() @ w.double().t()
+    if mode == "gated":
+        out, want, limit = torch.empty(m, n, dtype=torch.bfloat16, device=DEV), P.swiglu(both[:, :n].cpu(), both[:, n:].cpu()), ULP["bfloat16"] * 2
+        ops.linear_glu(a, packed_or_not(ops, w, packed, "gated", gated_n=n), out)
+    else:
+        out, want, limit = base.clone(), (base.double() + both).cpu(), 1e-5
+        ops.linear(a, packed_or_not(ops, w, packed), out, accumulate=True)
+    assert rel(out.cpu(), want) < limit
+
+
 # 17 to 64 rows: a w that the last cache cannot keep passes the caches by; the halves of it, which do not, give the same bits.
 @pytest.mark.parametrize("m", [17, 64])
 def test_linear_of_a_w_beyond_the_caches(ops, m):
