@@ -377,7 +377,7 @@ int launch(const float* a, const float* w, float* out, int M, int N, int K, int 
 // a tile that has a compute unit to itself; share: what each tile adds where several run there; ends: a tile's first loads and its epilogue, of each of the kinds below. Fitted to 2994 products
 // drawn at random (17 to 2500 rows of a, 8 to 9000 columns, k of 4 to 8192), of which every tile was timed: what it chooses is 1.5 % off the best of nine (blocks of 1 to 7, of 1 and 2 shared), takes
 // 0.544 of what the kernel before these took, and 55 of them more than 1.03 of that, 14 more than 1.1 (gated, k up to 350 and few rounds of tiles, or k of 4 to 16 and nothing but
-// ends: 49 x 5136, k = 44 5.3 -> 6.2 us, 2414 x 8504, k = 12 61 -> 75, the most; of 1494 more 32 and 7, 1040 x 452, k = 140 8.6 -> 12.5). Without the ends, which a short k consists of, 90 were above 1.03 and 49 above 1.1, up to 1.45 (358 x 3536 gated, k = 8
+// ends: 49 x 5136, k = 44 5.3 -> 6.2 us, 2414 x 8504, k = 12 61 -> 75, the most; of 1494 more 32 and 7, 1040 x 452, k = 140 8.6 -> 12.5: 255 tiles of 64 x 32 then, 264 of 32 x 64 now). Without the ends, which a short k consists of, 90 were above 1.03 and 49 above 1.1, up to 1.45 (358 x 3536 gated, k = 8
 // 7.4 -> 10.6, now 7.9). Six blocks gated close the gap between five and seven, where as many tiles make two rounds and one (551 x 2484, k = 192 19.5 -> 17.2, 18.3 before).
 enum { STORES_WIDE, STORES_NARROW, ADDS_WIDE, ADDS_NARROW };       // results in pieces of 16 bytes, or one by one; gated ones are stores
 struct Takes { double fixed, alone, share, ends[4]; };
