@@ -105,36 +105,72 @@ template <typename T, int N> struct alignas(sizeof(T) * N) Pack { T e[N]; };
 // The parts of a projection split along k: part p of element i at values[p * stride + i]. splits 0: there are none.
 struct QkvParts { const float* values; long stride; int splits; };
 
-// 16 bytes of a row of q/k/v. `at` counts elements from the first row's first.
-template <bool PARTS, typename T>
-__device__ __forceinline__ Pack<T, 16 / (int)sizeof(T)> read_qkv(const T* qkv, const QkvParts& parts, long at) {
-    if constexpr (!PARTS) {
-        return *reinterpret_cast<const Pack<T, 16 / (int)sizeof(T)>*>(qkv + at);
-    } else {
-        static_assert(sizeof(T) == 2, "parts are rounded to bfloat16");
-        constexpr int AT_ONCE = 4;                             // parts asked for at once (those beyond the last: that one again)
-        float4 low = make_float4(0.f, 0.f, 0.f, 0.f), high = low;
-        for (int p0 = 0; p0 < parts.splits; p0 += AT_ONCE) {
-            float4 a[AT_ONCE], b[AT_ONCE];
+// PIECES pieces of 16 bytes of a row of q/k/v, `apart` elements from one another; `at` counts elements from the first row's first. Asked for
+// with ask, which waits for nothing, and there with take: the parts' sums, four parts at a time (those beyond the last: that one again,
+// not added) for all pieces at once. (Piece by piece, with a branch around every part's addition, each waited for the one before it.)
+template <bool PARTS, int PIECES, typename T>
+struct QkvPieces {
+    static constexpr int VEC = 16 / (int)sizeof(T), AT_ONCE = 4, QUADS = VEC / 4;
+    Pack<T, VEC> pieces[PARTS ? 1 : PIECES];
+    float4 asked[PARTS ? AT_ONCE : 1][PIECES][QUADS];
+    const float* first;
+    long apart;
+    __device__ __forceinline__ void ask_parts(const QkvParts& parts, int p0) {
 #pragma unroll
-            for (int u = 0; u < AT_ONCE; ++u) {
-                const float* from = parts.values + min(p0 + u, parts.splits - 1) * parts.stride + at;
-                a[u] = *reinterpret_cast<const float4*>(from);
-                b[u] = *reinterpret_cast<const float4*>(from + 4);
-            }
+        for (int u = 0; u < AT_ONCE; ++u) {
+            const float* from = first + min(p0 + u, parts.splits - 1) * parts.stride;
 #pragma unroll
-            for (int u = 0; u < AT_ONCE; ++u) {
-                if (p0 + u >= parts.splits) continue;
-                low.x += a[u].x; low.y += a[u].y; low.z += a[u].z; low.w += a[u].w;
-                high.x += b[u].x; high.y += b[u].y; high.z += b[u].z; high.w += b[u].w;
-            }
+            for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+                for (int q = 0; q < QUADS; ++q) asked[u][i][q] = *reinterpret_cast<const float4*>(from + i * apart + 4 * q);
         }
-        Pack<T, 8> out;
-        out.e[0] = from_float<T>(low.x); out.e[1] = from_float<T>(low.y); out.e[2] = from_float<T>(low.z); out.e[3] = from_float<T>(low.w);
-        out.e[4] = from_float<T>(high.x); out.e[5] = from_float<T>(high.y); out.e[6] = from_float<T>(high.z); out.e[7] = from_float<T>(high.w);
-        return out;
     }
-}
+    __device__ __forceinline__ void ask(const T* qkv, const QkvParts& parts, long at, long pieces_apart) {
+        if constexpr (!PARTS) {
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) pieces[i] = *reinterpret_cast<const Pack<T, VEC>*>(qkv + at + i * pieces_apart);
+        } else {
+            static_assert(sizeof(T) == 2, "parts are rounded to bfloat16");
+            first = parts.values + at;
+            apart = pieces_apart;
+            ask_parts(parts, 0);
+        }
+    }
+    __device__ __forceinline__ void take(const QkvParts& parts, Pack<T, VEC> (&out)[PIECES]) {
+        if constexpr (!PARTS) {
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) out[i] = pieces[i];
+        } else {
+            float sum[PIECES][VEC] = {};
+            for (int p0 = 0;;) {
+#pragma unroll
+                for (int u = 0; u < AT_ONCE; ++u) {
+                    const bool there = p0 + u < parts.splits;
+#pragma unroll
+                    for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+                        for (int q = 0; q < QUADS; ++q) {
+                            const float4 part = asked[u][i][q];
+                            float (&of)[VEC] = sum[i];
+                            of[4 * q] = there ? of[4 * q] + part.x : of[4 * q];
+                            of[4 * q + 1] = there ? of[4 * q + 1] + part.y : of[4 * q + 1];
+                            of[4 * q + 2] = there ? of[4 * q + 2] + part.z : of[4 * q + 2];
+                            of[4 * q + 3] = there ? of[4 * q + 3] + part.w : of[4 * q + 3];
+                        }
+                }
+                p0 += AT_ONCE;
+                if (p0 >= parts.splits) break;
+                __builtin_amdgcn_sched_barrier(0);             // (into the registers of the parts before)
+                ask_parts(parts, p0);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) out[i].e[e] = from_float<T>(sum[i][e]);
+        }
+    }
+};
 
 // 32 dims of the values of 64 consecutive tokens of a step and one key/value head: read row by row (a piece a thread), turned in
 // LDS, and written so that a store instruction of a wavefront takes 8 tokens of 8 dims: where the
@@ -176,9 +212,12 @@ __device__ __forceinline__ void write_values(
         const int r = i / pieces, d = (i % pieces) * VEC;
         const long from = min(first + r, tokens - 1);         // rows past the end repeat the last one; nobody writes them to the cache
         const long at = source + from * heads_total * head_dim + d0 + d;
-        const Pack<T, VEC> piece = read_qkv<PARTS>(qkv, parts, at);
-        if constexpr (PARTS) if (first + r < tokens) *reinterpret_cast<Pack<T, VEC>*>(qkv + at) = piece;
-        *reinterpret_cast<Pack<T, VEC>*>(&shared.tile[r][d]) = piece;
+        QkvPieces<PARTS, 1, T> source_piece;
+        Pack<T, VEC> piece[1];
+        source_piece.ask(qkv, parts, at, 0);
+        source_piece.take(parts, piece);
+        if constexpr (PARTS) if (first + r < tokens) *reinterpret_cast<Pack<T, VEC>*>(qkv + at) = piece[0];
+        *reinterpret_cast<Pack<T, VEC>*>(&shared.tile[r][d]) = piece[0];
     }
     __syncthreads();
     // a store of a wavefront: tokens 8 g .. 8 g + 7 of the tile (lane % 8), dims 8 h .. 8 h + 7 (lane / 8);
@@ -224,26 +263,36 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) qkv_prepare_vector_kernel(
     const int wave = threadIdx.x / XRT_WAVE, lane = threadIdx.x % XRT_WAVE;
     const int item = (int)blockIdx.x - value_blocks, chunks_here = PARTS ? chunks : 1;      // (a division less where it is known)
     const int token = item / chunks_here, chunk = item % chunks_here;
+    const int at = (lane % LANES) * VEC;           // this lane's elements: at.. in the lower half, HALF + at.. in the upper
+    const int heads_total = n_heads + 2 * n_kv_heads;
+    const int heads_here = value_blocks == 0 ? heads_total : n_heads + n_kv_heads;     // value heads come last
+    const int first_head = (chunk * WAVES + wave) * HEADS_PER_WAVE + lane / LANES;
+    // the parts of the first head are asked for before the angles are worked out, behind what those are made of
     const int pos = positions[token];
     const int slot = slots[token];
+    const float theta = rope_theta != nullptr ? rope_theta[min((int)threadIdx.x, HALF - 1)] : 1.f;
+    __builtin_amdgcn_sched_barrier(0);
+    QkvPieces<PARTS, 2, T> halves;
+    auto ask = [&](int head) { halves.ask(qkv, parts, ((long)token * heads_total + min(head, heads_total - 1)) * HEAD + at, HALF); };
+    if constexpr (PARTS) ask(first_head);
     if (rope_theta != nullptr) {
         for (int i = threadIdx.x; i < HALF; i += WAVES * XRT_WAVE) {
-            const float angle = (float)pos * rope_scale / rope_theta[i];
+            const float angle = (float)pos * rope_scale / (i < WAVES * XRT_WAVE ? theta : rope_theta[i]);
             sincosf(angle, &sines[i], &cosines[i]);
         }
     }
-    __syncthreads();
-    const int at = (lane % LANES) * VEC;           // this lane's elements: at.. in the lower half, HALF + at.. in the upper
-    const int heads_total = n_heads + 2 * n_kv_heads;
+    // (not __syncthreads, which would wait for the head that is on its way)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const int within = pos % XRT_BLOCK_TOKENS;
-    const int heads_here = value_blocks == 0 ? heads_total : n_heads + n_kv_heads;     // value heads come last
-    for (int head = (chunk * WAVES + wave) * HEADS_PER_WAVE + lane / LANES; head < heads_here; head += chunks_here * WAVES * HEADS_PER_WAVE) {
+    const int step = chunks_here * WAVES * HEADS_PER_WAVE;
+    for (int head = first_head; head < heads_here; head = PARTS ? heads_here : head + step) {      // (with parts the chunks are as many as leave no workgroup a second round)
         // lanes of one head stay together: the exchanges below are within a head
         const bool is_q = head < n_heads, is_v = head >= n_heads + n_kv_heads, is_k = !is_q && !is_v;
-        const long row_at = (long)token * heads_total * HEAD + (long)head * HEAD;
-        T* row = qkv + row_at;
-        const Pack<T, VEC> lower = read_qkv<PARTS>(qkv, parts, row_at + at);
-        const Pack<T, VEC> upper = read_qkv<PARTS>(qkv, parts, row_at + HALF + at);
+        T* row = qkv + ((long)token * heads_total + head) * HEAD;
+        if constexpr (!PARTS) ask(head);
+        Pack<T, VEC> both[2];
+        halves.take(parts, both);
+        const Pack<T, VEC> lower = both[0], upper = both[1];
         long cache_base = -1;
         if (!is_q && k_cache != nullptr)
             cache_base = cache_block_base(block_table, table_stride, n_blocks, slot, pos, n_kv_heads,
