@@ -46,23 +46,40 @@ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, int tiles_n
     const int xcds = 8;
     id = (id % xcds) * ((total + xcds - 1) / xcds) + id / xcds;
     if (id >= total) return TilePlace{-1, 0};
+    if (tiles_m <= 4) return TilePlace{id % tiles_m, id / tiles_m};     // (a panel's tiles of one n would often lie on two XCDs, which then both read their w)
     constexpr int PANEL = 8;
     const int panel = id / (PANEL * tiles_m), in_panel = id % (PANEL * tiles_m);
     const int panel_width = min(PANEL, tiles_n - panel * PANEL);
     return TilePlace{in_panel / panel_width, panel * PANEL + in_panel % panel_width};
 }
 
+// The same of a product whose k is split into parts, in one of two orders. By columns: an XCD gets a run of tiles and all parts of them, a grid row each. By parts
+// (by_parts: their number): it gets a run of tiles and parts, part after part, so that it reads some slices of k of a, which its L2
+// holds, instead of all of a, and no XCD has more to do for a number of tiles that does not divide.
+struct PartPlace { TilePlace tile; int part; };
+__device__ __forceinline__ PartPlace part_place(int id, int tiles_m, int tiles_n, int by_parts) {
+    if (by_parts == 0) return PartPlace{tile_place(id, tiles_m, tiles_n), (int)blockIdx.y};
+    constexpr int XCDS = 8;
+    const int tiles = tiles_m * tiles_n, total = tiles * by_parts;
+    id = (id % XCDS) * ((total + XCDS - 1) / XCDS) + id / XCDS;
+    if (id >= total) return PartPlace{TilePlace{-1, 0}, 0};
+    const int tile = id % tiles;
+    return PartPlace{TilePlace{tile % tiles_m, tile / tiles_m}, id / tiles};
+}
+// Workgroups that such a product's launch has, places that no tile is dealt to among them.
+inline long part_ids(long tiles, int parts, bool by_parts) { return by_parts ? (tiles * parts + 7) / 8 * 8 : (tiles + 7) / 8 * 8 * parts; }
+
 // The rows of a that come without their RMSNorm's division (see xrt_linear_norm in xrt_hip.h): the sums of
 // squares per tile of 16 columns, from which a tile of up to 64 rows works out 1 / rms of its rows and
 // multiplies its sums by it before the epilogue. squares null: nothing of the kind.
 struct RowScale { const float* squares; int tiles; int width; float eps; int activation; };     // (activation: of a gated epilogue)
 
-// One tile of the product, by one workgroup: `id` is the workgroup's number among the tiles_m x tiles_n tiles.
+// One tile of the product, or of one part of its k, by one workgroup: `id` is the workgroup's number among them.
 // PAST_CACHES: w is asked for past the caches.
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES = false>
 __device__ __forceinline__ void gemm_tile(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
-    int id, int tiles_m, int tiles_n, int k_per_split, const Packing packing, const RowScale scale) {
+    int id, int tiles_m, int tiles_n, int by_parts, int k_per_split, const Packing packing, const RowScale scale) {
     constexpr int THREADS = WM * WN * XRT_WAVE;
     constexpr int WAVE_M = BM / WM, WAVE_N = BN / WN;        // part of the tile owned by one wavefront
     constexpr int TM = WAVE_M / 32, TN = WAVE_N / 32;        // 32x32 accumulator tiles of a wavefront
@@ -73,11 +90,14 @@ __device__ __forceinline__ void gemm_tile(
     bf16* lds_a = reinterpret_cast<bf16*>(lds_raw);                    // [2][BM][PITCH]; laid out differently on the direct path
     bf16* lds_b = lds_a + 2 * BM * PITCH;                              // [2][BN][PITCH]
 
-    const TilePlace place = tile_place(id, tiles_m, tiles_n);
+    // (a float32 store may be of a part; of the others none is, and their way to the first loads is shorter)
+    const PartPlace of_part = MODE == MODE_STORE && sizeof(TO) == 4 ? part_place(id, tiles_m, tiles_n, by_parts) : PartPlace{tile_place(id, tiles_m, tiles_n), 0};
+    const TilePlace place = of_part.tile;
     if (place.m < 0) return;
-    const long m0 = (long)place.m * BM;
+    // (rows, columns and byte offsets fit 32 bits: the launcher checks)
+    const int m0 = place.m * BM;
     constexpr int BN_OUT = MODE == MODE_GATED ? BN / 2 : BN;          // output columns of a tile
-    const long n0 = (long)place.n * BN_OUT;
+    const int n0 = place.n * BN_OUT;
 
     const int tid = threadIdx.x, lane = tid % XRT_WAVE, wave = tid / XRT_WAVE;
     const int wave_m = wave / WN, wave_n = wave % WN;
@@ -87,13 +107,13 @@ __device__ __forceinline__ void gemm_tile(
     // pair meets in that wavefront's registers. Rows beyond the operands are clamped to the last
     // row: loads then need no guard, and what such a row contributes lands in outputs that are
     // not written.
-    auto w_row = [&](int r) -> long {
+    auto w_row = [&](int r) -> int {
         if constexpr (MODE == MODE_GATED) {
             constexpr int HALF = WAVE_N / 2;
             const int within = r % WAVE_N;
-            return min(n0 + (r / WAVE_N) * HALF + within % HALF, (long)N - 1) + (long)(within / HALF) * N;
+            return min(n0 + (r / WAVE_N) * HALF + within % HALF, N - 1) + (within / HALF) * N;
         } else {
-            return min(n0 + r, (long)N - 1);
+            return min(n0 + r, N - 1);
         }
     };
     // 1 / rms of the tile's rows, if the rows of a come without it. The sums of squares are asked for now,
@@ -153,7 +173,7 @@ __device__ __forceinline__ void gemm_tile(
 #pragma unroll
         for (int i = 0; i < LOADS_A; ++i) {
             const int r = min(i * WAVES + wave, BLOCKS_A - 1) * ROWS + sub;
-            off_a[i] = (unsigned)(min(m0 + r, (long)M - 1) * K + chunk_of(r)) * 2u;
+            off_a[i] = ((unsigned)min(m0 + r, M - 1) * (unsigned)K + (unsigned)chunk_of(r)) * 2u;
         }
         // A packed w is copied as it lies: an instruction takes one whole tile of the packing (16 packed rows x 32
         // columns, a contiguous kilobyte, lane by lane), and the stage holds the tile's groups of 16 packed rows
@@ -162,17 +182,20 @@ __device__ __forceinline__ void gemm_tile(
         // rows contiguous along k, every four lanes would touch four cache lines: a fifth slower, measured.)
         // The tile's rows are then packed rows first_packed .. + BN, and the epilogue finds the outputs they make.
         const bool packed_b = is_packed(packing);
-        const long first_packed = MODE == MODE_GATED ? 2 * n0 : n0;
-        const long last_group = ((MODE == MODE_GATED ? 2L * N : (long)N) + 15) / 16 - 1;
+        const int first_packed = MODE == MODE_GATED ? 2 * n0 : n0;
+        const int last_group = ((MODE == MODE_GATED ? 2 * N : N) + 15) / 16 - 1;
+        if (packed_b) {
 #pragma unroll
-        for (int i = 0; i < LOADS_B; ++i) {
-            const int block = min(i * WAVES + wave, BLOCKS_B - 1);
-            if (packed_b) {
-                const long group = min(first_packed / 16 + block / 2, last_group);       // groups beyond the matrix: the last one again
-                off_b[i] = (unsigned)(((group * (K / 32) + block % 2) * 512 + lane * 8) * 2);
-            } else {
-                const int r = block * ROWS + sub;
-                off_b[i] = (unsigned)(w_row(r) * K + chunk_of(r)) * 2u;
+            for (int i = 0; i < LOADS_B; ++i) {
+                const int block = min(i * WAVES + wave, BLOCKS_B - 1);
+                const int group = min(first_packed / 16 + block / 2, last_group);        // groups beyond the matrix: the last one again
+                off_b[i] = ((unsigned)group * (unsigned)(K / 32) + (unsigned)(block % 2)) * 1024u + (unsigned)lane * 16u;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < LOADS_B; ++i) {
+                const int r = min(i * WAVES + wave, BLOCKS_B - 1) * ROWS + sub;
+                off_b[i] = ((unsigned)w_row(r) * (unsigned)K + (unsigned)chunk_of(r)) * 2u;
             }
         }
         // a step of k0 columns along k moves a row contiguous along k by k0 elements, a packed one by k0 / 32 tiles
@@ -226,12 +249,12 @@ __device__ __forceinline__ void gemm_tile(
         // after the barrier, under the products of the last slice of this one.
         constexpr int AHEAD = STAGES - 1;
         constexpr int IN_FLIGHT = (AHEAD - 1) * (LOADS_A + LOADS_B);   // loads that may be outstanding when the next tile is needed
-        // a launch with several grid rows splits k among them: row y takes k_per_split from
-        // y * k_per_split on (less at the end) and writes its sums to the y-th copy of out
-        const int k_begin = blockIdx.y * k_per_split;
+        // part p of a product split along k takes k_per_split from p * k_per_split on (less at the
+        // end) and writes its sums to the p-th copy of out
+        const int k_begin = of_part.part * k_per_split;
         const int steps = min(k_per_split, K - k_begin) / DK;
         const int last_k = k_begin + (steps - 1) * DK;
-        out += (long)blockIdx.y * M * N;
+        out += (long)of_part.part * M * N;
 #pragma unroll
         for (int i = 0; i < AHEAD; ++i) issue(i, min(k_begin + i * DK, last_k));
         wait_loads_and_barrier<IN_FLIGHT>();                      // tile 0 is in LDS
@@ -258,7 +281,7 @@ __device__ __forceinline__ void gemm_tile(
     #pragma unroll
         for (int i = 0; i < CHUNKS_A; ++i) {
             const int chunk = tid + i * THREADS;
-            off_a[i] = (unsigned)(min(m0 + chunk / 8, (long)M - 1) * K + (chunk % 8) * 8);
+            off_a[i] = (unsigned)min(m0 + chunk / 8, M - 1) * (unsigned)K + (unsigned)(chunk % 8) * 8u;
         }
     #pragma unroll
         for (int i = 0; i < CHUNKS_B; ++i) {
@@ -544,10 +567,16 @@ constexpr int LARGE_BN = 256;
 // A half is loaded into the place of the same half two tiles ago as soon as both groups have read that, seven quarters before
 // it is needed, and the waits leave the newer six quarters' loads in flight. So the matrix cores are busy in 98 % of the
 // loop's cycles (2084 a step of 64 for 2048 of products; with one barrier a step and every wavefront doing both at once: 61 %).
+//
+// height: the rows of a that a tile stands for, a multiple of 16 up to BM. The rows of a product are dealt to its tiles evenly (even_height), so that none has
+// more than it must: the first four wavefronts take half of the blocks of 16, or one more than the others, and a wavefront runs the loop that is made for its
+// number of blocks (all, one or two fewer). The chip's power bounds the loop, so that products left out are time: 333 rows in two tiles of 176 instead of 192 and 141, 28672 rows
+// of w in pairs, k = 4096 77.6 -> 73.9 us, 51200, k = 5120 194 -> 179; 400 rows (208 each) 221 -> 196.
 template <int BM, int MODE, typename TO>
 __device__ __forceinline__ void gemm_large_tile(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
-    const TilePlace place, int n_first, int k_per_split, const Packing packing, const int activation, const int lda = 0, const int ldw = 0) {
+    const TilePlace place, int n_first, int part, int k_per_split, const Packing packing, const int activation, const int height = BM, const int lda = 0,
+    const int ldw = 0) {
     constexpr int BN = LARGE_BN, DK = 64, WAVES_N = 4;
     constexpr int WAVE_M = BM / 2, WAVE_N = BN / WAVES_N;      // the wavefront's part of the tile
     constexpr int TM = WAVE_M / 16, TN = WAVE_N / 16, HM = TM / 2, HN = TN / 2;      // blocks of 16 rows of x and of w: all, and a half
@@ -557,22 +586,26 @@ __device__ __forceinline__ void gemm_large_tile(
     bf16* stage_a = reinterpret_cast<bf16*>(lds_raw);          // [2][BM][64]: rows of eight 16-byte pieces, swizzled
     bf16* stage_b = stage_a + 2 * BM * DK;                     // [2][256][64]: likewise, or packed tiles as they lie
 
-    const long m0 = (long)place.m * BM;
+    // (rows, columns and byte offsets fit 32 bits: the launchers check; a short way to the first loads counts in every launch)
+    const int m0 = place.m * height;
     constexpr int BN_OUT = MODE == MODE_GATED ? BN / 2 : BN;   // output columns of a tile
-    const long n0 = n_first + (long)place.n * BN_OUT;
+    const int n0 = n_first + place.n * BN_OUT;
     const int lane = threadIdx.x % XRT_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / XRT_WAVE);
     const int wave_m = wave / WAVES_N, wave_n = wave % WAVES_N;
     const int quad = lane / 16;                                // which four rows of a 16 x 16 block of sums this lane holds
+    const int upper_blocks = (height / 16 + 1) / 2;            // of 16 rows, of the wavefronts 0 to 3
+    const int blocks = wave_m == 0 ? upper_blocks : height / 16 - upper_blocks;
+    const int wave_row = m0 + wave_m * upper_blocks * 16, tile_end = min(m0 + height, M);
 
     // Row of w behind row r of the tile (w not packed). Gated: a wavefront's rows are half gate rows and half the up rows of
     // the same outputs. Rows beyond the operands are clamped to the last one: what they make is not written.
-    auto w_row = [&](int r) -> long {
+    auto w_row = [&](int r) -> int {
         if constexpr (MODE == MODE_GATED) {
             constexpr int HALF = WAVE_N / 2;
             const int within = r % WAVE_N;
-            return min(n0 + (r / WAVE_N) * HALF + within % HALF, (long)N - 1) + (long)(within / HALF) * N;
+            return min(n0 + (r / WAVE_N) * HALF + within % HALF, N - 1) + (within / HALF) * N;
         } else {
-            return min(n0 + r, (long)N - 1);
+            return min(n0 + r, N - 1);
         }
     };
     // Piece c (16 bytes) of row r of 64 lies at place c ^ (r % 8) of the row. The sixteen lanes that a 16-byte read serves at
@@ -585,29 +618,39 @@ __device__ __forceinline__ void gemm_large_tile(
         const int per = rows / 16, p = min(i * 8 + wave, blocks - 1);
         return (p / per * rows + h * (rows / 2)) / 8 + p % per;
     };
-    const long row_a = lda > 0 ? lda : K, row_w = ldw > 0 ? ldw : K;
+    const int row_a = lda > 0 ? lda : K, row_w = ldw > 0 ? ldw : K;
     const bool packed_b = is_packed(packing);
-    const long first_packed = MODE == MODE_GATED ? 2 * n0 : n0;
-    const long last_group = ((MODE == MODE_GATED ? 2L * N : (long)N) + 15) / 16 - 1;
+    const int first_packed = MODE == MODE_GATED ? 2 * n0 : n0;
+    const int last_group = ((MODE == MODE_GATED ? 2 * N : N) + 15) / 16 - 1;
     unsigned off_a[2][LOADS_A], off_b[2][LOADS_B];             // bytes
+    // (rows of the tile that no wavefront has: the last one again, not multiplied)
+    const int missing = WAVE_M - upper_blocks * 16;
+    const unsigned piece_of_lane = (unsigned)((lane % 8) ^ swizzle_of(lane / 8)) * 16u;        // (rows of further loads differ by multiples of 8)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int i = 0; i < LOADS_A; ++i) {
-            const int r = block_of(h, i, WAVE_M, BLOCKS_A) * 8 + lane / 8;
-            off_a[h][i] = (unsigned)(min(m0 + r, (long)M - 1) * row_a + ((lane % 8) ^ swizzle_of(r)) * 8) * 2u;
+            const int block = block_of(h, i, WAVE_M, BLOCKS_A), r = block * 8 + lane / 8;
+            const int row = min(m0 + r - (block * 8 >= WAVE_M ? missing : 0), tile_end - 1);
+            off_a[h][i] = (unsigned)row * (unsigned)row_a * 2u + piece_of_lane;
         }
+    if (packed_b) {
 #pragma unroll
-        for (int i = 0; i < LOADS_B; ++i) {
-            const int block = block_of(h, i, WAVE_N, BN / 16);
-            if (packed_b) {
-                const long group = min(first_packed / 16 + block / 2, last_group);       // groups beyond the matrix: the last one again
-                off_b[h][i] = (unsigned)(((group * (row_w / 32) + block % 2) * 512 + lane * 8) * 2);
-            } else {
-                const int r = block * 8 + lane / 8;
-                off_b[h][i] = (unsigned)(w_row(r) * row_w + ((lane % 8) ^ swizzle_of(r)) * 8) * 2u;
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < LOADS_B; ++i) {
+                const int block = block_of(h, i, WAVE_N, BN / 16);
+                const int group = min(first_packed / 16 + block / 2, last_group);          // groups beyond the matrix: the last one again
+                off_b[h][i] = ((unsigned)group * (unsigned)(row_w / 32) + (unsigned)(block % 2)) * 1024u + (unsigned)lane * 16u;
             }
-        }
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int i = 0; i < LOADS_B; ++i) {
+                const int r = block_of(h, i, WAVE_N, BN / 16) * 8 + lane / 8;
+                off_b[h][i] = (unsigned)w_row(r) * (unsigned)row_w * 2u + piece_of_lane;
+            }
     }
     const unsigned w_step = packed_b ? 32u : 2u;               // bytes per column of k
     const unsigned lds_a0 = lds_address(stage_a), lds_b0 = lds_address(stage_b);
@@ -631,12 +674,14 @@ __device__ __forceinline__ void gemm_large_tile(
         place_b[ks] = stage_b + wave_n * WAVE_N * DK + (packed_b ? ks * 512 + lane * 8 : lane % 16 * DK + piece);
     }
     bf16x8 xa[2][2][HM], wb[2][2][HN];                         // [half][32 columns][block]
-    auto read_a = [&](int h, int stage) {
+    // (T: the blocks of the wavefront, TM or somewhat fewer; they are missing from the second half)
+    auto read_a = [&](auto t, int h, int stage) {
+        constexpr int T = decltype(t)::value;
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int i = 0; i < HM; ++i)
-                xa[h][ks][i] = *reinterpret_cast<const bf16x8*>(place_a[ks] + stage * BM * DK + (h * HM + i) * 16 * DK);
+                if (h * HM + i < T) xa[h][ks][i] = *reinterpret_cast<const bf16x8*>(place_a[ks] + stage * BM * DK + (h * HM + i) * 16 * DK);
     };
     auto read_b = [&](int h, int stage) {
 #pragma unroll
@@ -650,21 +695,23 @@ __device__ __forceinline__ void gemm_large_tile(
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](int h, int g) {
+    auto multiply = [&](auto t, int h, int g) {
+        constexpr int T = decltype(t)::value;
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
             for (int i = 0; i < HM; ++i)
 #pragma unroll
                 for (int j = 0; j < HN; ++j)
-                    acc[h * HM + i][g * HN + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[g][ks][j], xa[h][ks][i], acc[h * HM + i][g * HN + j], 0, 0, 0);
+                    if (h * HM + i < T)
+                        acc[h * HM + i][g * HN + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[g][ks][j], xa[h][ks][i], acc[h * HM + i][g * HN + j], 0, 0, 0);
     };
-    // a launch with several grid rows splits k among them: row y takes k_per_split from y * k_per_split on (less at the
-    // end) and writes its sums to the y-th copy of out
-    const int k_begin = blockIdx.y * k_per_split;
+    // part p of a product split along k takes k_per_split from p * k_per_split on (less at the end) and writes its sums to
+    // the p-th copy of out
+    const int k_begin = part * k_per_split;
     const int steps = min(k_per_split, K - k_begin) / DK;
     const int last_k = k_begin + (steps - 1) * DK;
-    out += (long)blockIdx.y * M * N;
+    out += (long)part * M * N;
     auto k_of = [&](int t) { return min(k_begin + t * DK, last_k); };    // (tiles beyond the end: the last one again, into a place nobody reads)
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -675,42 +722,49 @@ __device__ __forceinline__ void gemm_large_tile(
     }
     // Loads that may stay in flight behind a quarter's reads: those of the six quarters after the next one.
     constexpr int ALL = 2 * (LOADS_A + LOADS_B);
-    wait_loads_and_barrier<ALL + LOADS_A + LOADS_B>();         // x0 and w0 of tile 0 are in LDS
-    read_a(0, 0);
-    wait_loads_and_barrier<ALL + LOADS_A + LOADS_B>();         // and x0 is read by all: the first turn fills its place again
     auto barrier = [] {
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_barrier" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto turn = [&](auto in_flight, int h, int g) {
-        __builtin_amdgcn_sched_barrier(0);
-        wait_loads_and_barrier<decltype(in_flight)::value>();  // this wavefront's reads are done: what it read may be overwritten
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(h, g);
-        barrier();
+    auto walk = [&](auto t_blocks) {
+        wait_loads_and_barrier<ALL + LOADS_A + LOADS_B>();     // x0 and w0 of tile 0 are in LDS
+        read_a(t_blocks, 0, 0);
+        wait_loads_and_barrier<ALL + LOADS_A + LOADS_B>();     // and x0 is read by all: the first turn fills its place again
+        auto turn = [&](auto in_flight, int h, int g) {
+            __builtin_amdgcn_sched_barrier(0);
+            wait_loads_and_barrier<decltype(in_flight)::value>();  // this wavefront's reads are done: what it read may be overwritten
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(t_blocks, h, g);
+            barrier();
+        };
+        if (wave >= 4) barrier();
+        for (int t = 0; t < steps; ++t) {
+            const int now = t % 2, k_next = k_of(t + 2);
+            read_b(0, now);
+            issue_a(0, now, k_next);
+            turn(std::integral_constant<int, ALL + 2 * LOADS_A>{}, 0, 0);           // in flight: x1 x0 w0 w1 x1 x0
+            read_b(1, now);
+            issue_b(0, now, k_next);
+            turn(std::integral_constant<int, ALL + LOADS_A + LOADS_B>{}, 0, 1);     // x0 w0 w1 x1 x0 w0
+            read_a(t_blocks, 1, now);
+            issue_b(1, now, k_next);
+            turn(std::integral_constant<int, ALL + 2 * LOADS_B>{}, 1, 1);           // w0 w1 x1 x0 w0 w1
+            read_a(t_blocks, 0, now ^ 1);
+            issue_a(1, now, k_next);
+            turn(std::integral_constant<int, ALL + LOADS_A + LOADS_B>{}, 1, 0);     // w1 x1 x0 w0 w1 x1
+        }
     };
-    if (wave >= 4) barrier();
-    for (int t = 0; t < steps; ++t) {
-        const int now = t % 2, k_next = k_of(t + 2);
-        read_b(0, now);
-        issue_a(0, now, k_next);
-        turn(std::integral_constant<int, ALL + 2 * LOADS_A>{}, 0, 0);           // in flight: x1 x0 w0 w1 x1 x0
-        read_b(1, now);
-        issue_b(0, now, k_next);
-        turn(std::integral_constant<int, ALL + LOADS_A + LOADS_B>{}, 0, 1);     // x0 w0 w1 x1 x0 w0
-        read_a(1, now);
-        issue_b(1, now, k_next);
-        turn(std::integral_constant<int, ALL + 2 * LOADS_B>{}, 1, 1);           // w0 w1 x1 x0 w0 w1
-        read_a(0, now ^ 1);
-        issue_a(1, now, k_next);
-        turn(std::integral_constant<int, ALL + LOADS_A + LOADS_B>{}, 1, 0);     // w1 x1 x0 w0 w1 x1
-    }
+    // (tiles of up to 128 rows always run the whole loop: the way round the others, cold code, took 0.3 us of 17, and fewer products gained none)
+    if (BM == 128 || blocks == TM) walk(std::integral_constant<int, TM>{});
+    else if (blocks == TM - 1) walk(std::integral_constant<int, TM - 1>{});
+    else walk(std::integral_constant<int, TM - 2>{});          // (fewer than that: some products that nobody writes)
     if (wave < 4) barrier();
     wait_loads_and_barrier<0>();                               // nothing lands in LDS after this
 
     // ---- epilogue: element e of acc[i][j] is row i * 16 + lane % 16 of x and row j * 16 + quad * 4 + e of w
-    const long row0 = m0 + wave_m * WAVE_M + lane % 16;
+    const int row0 = wave_row + lane % 16;
+    const int row_end = min(wave_row + blocks * 16, tile_end);           // of the wavefront's rows
     if (MODE == MODE_GATED && packed_b) {
         // A group of 16 packed rows holds the gate rows of 8 outputs, then their up rows: the lane with an output's up sum
         // is 32 lanes away. One exchange of half a register between the sums of two blocks of x leaves gate and up of
@@ -736,13 +790,13 @@ __device__ __forceinline__ void gemm_large_tile(
                     if (wide) {
                         uint4v piece = join_rows<TO>(made[0], made[1]);
                         const long n = n_wave + (j + quad % 2) * 8;
-                        if (m < M && n < N) *reinterpret_cast<uint4v*>(out + m * (long)N + n) = piece;
+                        if (m < row_end && n < N) *reinterpret_cast<uint4v*>(out + m * (long)N + n) = piece;
                         continue;
                     }
                 }
 #pragma unroll
                 for (int u = 0; u < 2; ++u)
-                    store_four<TO>(out, m, n_wave + (j + u) * 8 + quad % 2 * 4, M, N, made[u], wide);
+                    store_four<TO>(out, m, n_wave + (j + u) * 8 + quad % 2 * 4, row_end, N, made[u], wide);
             }
         }
     } else if constexpr (MODE == MODE_GATED) {
@@ -754,7 +808,7 @@ __device__ __forceinline__ void gemm_large_tile(
                 float made[4];
 #pragma unroll
                 for (int e = 0; e < 4; ++e) made[e] = gate_activation<sizeof(TO) == 2>(acc[i][j][e], activation) * acc[i][j + HN][e];
-                store_four<TO>(out, row0 + i * 16, n0 + wave_n * (WAVE_N / 2) + j * 16 + quad * 4, M, N, made, wide);
+                store_four<TO>(out, row0 + i * 16, n0 + wave_n * (WAVE_N / 2) + j * 16 + quad * 4, row_end, N, made, wide);
             }
     } else {
         const bool wide = N % 8 == 0 && (uintptr_t)out % 16 == 0;
@@ -763,7 +817,7 @@ __device__ __forceinline__ void gemm_large_tile(
         // Two neighbouring blocks of columns change eight lanes with each other, so that an instruction takes eight rows of
         // 128 bytes, whole cache lines, instead of sixteen of 64 (adding onto a float32 residual of 8192 x 4096: 54 instead of 17
         // microseconds a round of tiles without it).
-        const long row8 = m0 + wave_m * WAVE_M + lane % 8;
+        const long row8 = wave_row + lane % 8;
         const int upper = lane % 16 / 8;
         if constexpr (MODE == MODE_STORE && sizeof(TO) == 2) {
             if (wide) {
@@ -788,7 +842,7 @@ __device__ __forceinline__ void gemm_large_tile(
 #pragma unroll
                     for (int u = 0; u < 2; ++u) {
                         const long m = row8 + i * 16 + u * 8;
-                        if (m < M && q < N) *reinterpret_cast<uint4v*>(out + m * (long)N + n) = piece[u];
+                        if (m < row_end && q < N) *reinterpret_cast<uint4v*>(out + m * (long)N + n) = piece[u];
                     }
                 }
                 return;
@@ -804,7 +858,7 @@ __device__ __forceinline__ void gemm_large_tile(
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
                         load_four<TO>(out, row8 + (i0 + i) * 16 + j % 2 * 8, column_of(n0 + wave_n * WAVE_N + (j / 2 * 2 + upper) * 16 + quad * 4),
-                                      M, N, before[i][j], wide);
+                                      row_end, N, before[i][j], wide);
             }
 #pragma unroll
             for (int i = 0; i < RUN; ++i)
@@ -824,28 +878,29 @@ __device__ __forceinline__ void gemm_large_tile(
                     const long q = n0 + wave_n * WAVE_N + (j + upper) * 16 + quad * 4;
                     if (q < N) {
                         const long n = column_of(q);
-                        store_four<TO>(out, row8 + (i0 + i) * 16, n, M, N, made[0], wide);
-                        store_four<TO>(out, row8 + (i0 + i) * 16 + 8, n, M, N, made[1], wide);
+                        store_four<TO>(out, row8 + (i0 + i) * 16, n, row_end, N, made[0], wide);
+                        store_four<TO>(out, row8 + (i0 + i) * 16 + 8, n, row_end, N, made[1], wide);
                     }
                 }
         }
     }
 }
 
-template <int BM, int MODE, typename TO>
+// PARTS: k may be split (without it the way to the first loads is shorter).
+template <int BM, int MODE, typename TO, bool PARTS>
 __global__ void __launch_bounds__(8 * XRT_WAVE) gemm_large_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
-    int tiles_m, int tiles_n, int k_per_split, const Packing packing, int activation) {
-    const TilePlace place = tile_place(blockIdx.x, tiles_m, tiles_n);
-    if (place.m < 0) return;
-    gemm_large_tile<BM, MODE, TO>(a, w, out, M, N, K, place, 0, k_per_split, packing, activation);
+    int tiles_m, int tiles_n, int by_parts, int k_per_split, const Packing packing, int activation, int height) {
+    const PartPlace place = PARTS ? part_place(blockIdx.x, tiles_m, tiles_n, by_parts) : PartPlace{tile_place(blockIdx.x, tiles_m, tiles_n), 0};
+    if (place.tile.m < 0) return;
+    gemm_large_tile<BM, MODE, TO>(a, w, out, M, N, K, place.tile, 0, place.part, k_per_split, packing, activation, height);
 }
 
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES>
 __global__ void __launch_bounds__(WM * WN * XRT_WAVE) gemm_mfma_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
-    int tiles_m, int tiles_n, int k_per_split, const Packing packing, const RowScale scale) {
-    gemm_tile<BM, BN, WM, WN, MODE, DK, STAGES, TO, PAST_CACHES>(a, w, out, M, N, K, blockIdx.x, tiles_m, tiles_n, k_per_split, packing, scale);
+    int tiles_m, int tiles_n, int by_parts, int k_per_split, const Packing packing, const RowScale scale) {
+    gemm_tile<BM, BN, WM, WN, MODE, DK, STAGES, TO, PAST_CACHES>(a, w, out, M, N, K, blockIdx.x, tiles_m, tiles_n, by_parts, k_per_split, packing, scale);
 }
 
 // Two tile shapes in one launch: the first `large_blocks` workgroups take 256 x 256 tiles of the
@@ -857,13 +912,13 @@ template <int MODE, typename TO>
 __global__ void __launch_bounds__(8 * XRT_WAVE) gemm_mfma_mixed_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
     int large_blocks, int large_tiles_m, int large_tiles_n, int split, int small_tiles_m, int small_tiles_n,
-    const Packing packing, int activation) {
+    const Packing packing, int activation, int large_height, int small_height) {
     if ((int)blockIdx.x < large_blocks) {
         const TilePlace place = tile_place(blockIdx.x, large_tiles_m, large_tiles_n);
-        if (place.m >= 0) gemm_large_tile<256, MODE, TO>(a, w, out, M, N, K, place, 0, K, packing, activation);
+        if (place.m >= 0) gemm_large_tile<256, MODE, TO>(a, w, out, M, N, K, place, 0, 0, K, packing, activation, large_height);
     } else {
         const TilePlace place = tile_place(blockIdx.x - large_blocks, small_tiles_m, small_tiles_n);
-        if (place.m >= 0) gemm_large_tile<128, MODE, TO>(a, w, out, M, N, K, place, split, K, packing, activation);
+        if (place.m >= 0) gemm_large_tile<128, MODE, TO>(a, w, out, M, N, K, place, split, 0, K, packing, activation, small_height);
     }
 }
 
@@ -886,7 +941,7 @@ __global__ void __launch_bounds__(8 * XRT_WAVE) gemm_grouped_kernel(
     const TilePlace place = tile_place(blockIdx.x, 1, tiles_n);
     if (place.m < 0) return;
     gemm_large_tile<BM, MODE, TO>(a + (long)tile * BM * lda, w + (long)group * w_stride, out + (long)tile * gridDim.y * BM * N, BM, N, K, place,
-                                  0, K / (int)gridDim.y, packing, activation, lda, ldw);
+                                  0, (int)blockIdx.y, K / (int)gridDim.y, packing, activation, BM, lda, ldw);
 }
 
 template <int BM, int MODE, typename TO>
@@ -936,6 +991,15 @@ bool reads_past_caches(int rows_of_tile, int M, int N, int K, int mode) {
     return M <= rows_of_tile && (mode == MODE_GATED ? cannot_stay(2L * N, K, 3) : cannot_stay(N, K, 2));
 }
 
+// Whether the tiles and parts of a product are dealt by parts (part_place): where k is so long that reading all of a on every XCD costs (tiles of 256 rows
+// of w read it less often, and gain from k = 3072 on: 0.95 of the time by columns beyond k = 6144, 0.97 to 0.98 below; narrower ones 0.97 beyond k = 6144, and 1.01
+// below, where an XCD's parts touch the pages of all of w for little), and where it makes a round less (0.79 to 0.94 up to 64 rows of x).
+bool deals_by_parts(int columns, long tiles, int K, int parts) {
+    if (parts < 2) return false;
+    auto rounds = [](long groups) { return (groups + XRT_COMPUTE_UNITS - 1) / XRT_COMPUTE_UNITS; };
+    return K > (columns >= 256 ? 2048 : 6144) || rounds(part_ids(tiles, parts, false)) > rounds(part_ids(tiles, parts, true));
+}
+
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES = false>
 int launch_kernel(const bf16* a, const bf16* w, TO* out, int M, int N, int K, const Packing& packing,
                   hipStream_t s, int splits = 1, int k_per_split = 0, const RowScale scale = RowScale{}) {
@@ -955,33 +1019,43 @@ int launch_kernel(const bf16* a, const bf16* w, TO* out, int M, int N, int K, co
         configured = true;
     }
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;
-    const int total = tiles_m * tiles_n;
-    const unsigned grid = (unsigned)(((total + 7) / 8) * 8);           // a whole number of rounds over the XCDs
+    const bool by_parts = deals_by_parts(BN, (long)tiles_m * tiles_n, K, splits);
+    const long ids = part_ids((long)tiles_m * tiles_n, by_parts ? splits : 1, by_parts);         // a whole number of rounds over the XCDs
+    XRT_REQUIRE(ids < (1L << 31), "linear (mfma): %ld tiles", ids);
     XRT_REQUIRE(splits == 1 || DK != 0, "linear (mfma): only whole tiles along k can be split");
     XRT_REQUIRE(scale.squares == nullptr || (BM <= 64 && splits == 1), "linear (mfma): rows are scaled by tiles of up to 64 rows that see all of k");
-    kernel<<<dim3(grid, splits), THREADS, lds, s>>>(a, w, out, M, N, K, tiles_m, tiles_n,
-                                                    splits == 1 ? K : k_per_split, packing, scale);
+    kernel<<<dim3((unsigned)ids, by_parts ? 1 : splits), THREADS, lds, s>>>(a, w, out, M, N, K, tiles_m, tiles_n, by_parts ? splits : 0, splits == 1 ? K : k_per_split,
+                                                                            packing, scale);
     XRT_LAUNCH_CHECK("linear (mfma)");
     return 0;
 }
 
+// The rows of a of each tile, where tiles of up to `most` rows (a multiple of 16) share M.
+int even_height(int M, int most) {
+    const int tiles = (M + most - 1) / most;
+    return ((M + tiles - 1) / tiles + 15) / 16 * 16;
+}
+
 // The large tiles over all of w; splits > 1: k dealt out among grid rows, each with its copy of out.
-template <int BM, int MODE, typename TO>
+template <int BM, int MODE, typename TO, bool PARTS = false>
 int launch_large(const bf16* a, const bf16* w, TO* out, int M, int N, int K, const Packing& packing, int activation, hipStream_t s,
                  int splits = 1, int k_per_split = 0) {
     constexpr int BN_OUT = MODE == MODE_GATED ? LARGE_BN / 2 : LARGE_BN;
     constexpr size_t lds = (size_t)2 * (BM + LARGE_BN) * 64 * sizeof(bf16);
-    auto kernel = gemm_large_kernel<BM, MODE, TO>;
+    auto kernel = gemm_large_kernel<BM, MODE, TO, PARTS>;
     static bool configured = false;          // per instantiation
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         XRT_REQUIRE(e == hipSuccess, "linear (mfma): cannot reserve %zu bytes of LDS: %s", lds, hipGetErrorString(e));
         configured = true;
     }
-    XRT_REQUIRE(K % 64 == 0 && (splits == 1 || k_per_split % 64 == 0), "linear (mfma): the large tiles take whole steps of 64 along k (K=%d)", K);
+    XRT_REQUIRE(K % 64 == 0 && (splits == 1 || (PARTS && k_per_split % 64 == 0)), "linear (mfma): the large tiles take whole steps of 64 along k (K=%d)", K);
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;
-    const unsigned grid = (unsigned)((tiles_m * tiles_n + 7) / 8 * 8);               // a whole number of rounds over the XCDs
-    kernel<<<dim3(grid, splits), 8 * XRT_WAVE, lds, s>>>(a, w, out, M, N, K, tiles_m, tiles_n, splits == 1 ? K : k_per_split, packing, activation);
+    const bool by_parts = deals_by_parts(LARGE_BN, (long)tiles_m * tiles_n, K, splits);
+    const long ids = part_ids((long)tiles_m * tiles_n, by_parts ? splits : 1, by_parts);         // a whole number of rounds over the XCDs
+    XRT_REQUIRE(ids < (1L << 31), "linear (mfma): %ld tiles", ids);
+    kernel<<<dim3((unsigned)ids, by_parts ? 1 : splits), 8 * XRT_WAVE, lds, s>>>(a, w, out, M, N, K, tiles_m, tiles_n, by_parts ? splits : 0, splits == 1 ? K : k_per_split,
+                                                                                 packing, activation, even_height(M, BM));
     XRT_LAUNCH_CHECK("linear (mfma, large tiles)");
     return 0;
 }
@@ -1097,7 +1171,7 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
         configured = true;
     }
     kernel<<<large_blocks + small_blocks, 8 * XRT_WAVE, lds, s>>>(a, w, out, M, N, K, large_blocks, tiles_m, whole_columns,
-                                                                  split, small_tiles_m, small_tiles_n, packing, activation);
+                                                                  split, small_tiles_m, small_tiles_n, packing, activation, even_height(M, 256), even_height(M, 128));
     XRT_LAUNCH_CHECK("linear (mfma, two tile shapes)");
     return 0;
 }
@@ -1122,37 +1196,28 @@ constexpr int SPLIT_BM = 64, SPLIT_BN = 128;
 
 struct SplitPlan { int splits, k_per_split; long rows_w; int tile, columns; };      // tile: rows of x per tile (64, 128, 192 or 256), columns: rows of w
 
-// What a product of some hundred rows of x takes (nanoseconds) in parts along k: tiles of 128 rows of x and `columns` rows of w, `places` of them to a compute
+// What a product of some hundred rows of x takes (nanoseconds) in parts along k, if it is gated (of others: what the fixed array of xrt_linear_static is asked for): tiles of 128 rows of x and `columns` rows of w, `places` of them to a compute
 // unit. A step of 64 along k takes `step`, `share` more for each tile that a compute unit has on average, and `beside` more where some have two; `once` is
-// start, end and the second kernel's start, `part` what a further part costs it, `sums` what a million partial sums cost to write and to read again. Fitted to
-// 10800 products (512 to 8192 rows of w, k from 512 to 14336, 65 to 1700 rows of x, 2 to 16 parts): what the estimate chooses is 1 % off the best on average,
-// where a rule made at the sizes of the 8B models was 19 % off up to 128 rows, 16 % up to 256, 21 % up to 512 and 13 % beyond. 150
-// products drawn at random afterwards ran 1.34 times as fast up to 128 rows, 1.17 up to 256, 1.13 up to 512, 1.1 beyond (worst: 0.84, two
-// more below 0.92): 4096 rows of w, k = 1024, 100 rows of x 14.5 -> 10.6 us, 1024 rows, k = 3072, 333 rows of x 18.1 -> 13.3, 2048 rows, k = 8192, 100 rows
-// of x 20.8 -> 18.3, 5120 rows, k = 25600, 100 rows of x 85.9 -> 61.6; those of the 8B models stay within 4 % of what they were.
+// start, end and the second kernel's start, `part` what a further part costs it, `sums` what a million partial sums cost to write and to read again. (Fitted to products of
+// every kind, 512 to 8192 rows of w, k from 512 to 14336, 65 to 1700 rows of x; of 2686 gated products drawn at random afterwards what it chooses is 0.9 % off the best of 27 on average.)
 // Workgroups are counted as the fullest die has them: counting their number alone put two rounds on seven of the eight dies where the tiles are no multiple of
-// eight (298 rows of x, 5328 rows of w in pairs, k = 9664: 77 us, 55 by the rule before this estimate; 140 rows, 5120 rows, k = 25600 96, now 70). Of 1086 more products drawn
-// at random, 65 to 1800 rows of x, k up to 26000, 46 took over 5 % longer by it than by that rule, up to 1.42 times; counted so 7 do, up to 1.18, and the average of all is 0.875.
-// (The times are of kernels of four wavefronts; those of 128 x 64 with k < 4096 and the gated ones of 128 x 128 have eight now, and are 3 to 8 % faster. With the kernels as they
-// are, of 1444 gated products of 65 to 256 rows of x drawn at random the choice is 0.7 % off the better of parts and none, 24 of them over 1.1; of 587 others from k = 1024 on 0.3 %. Below that
-// the tiles without a split are taken for faster than they are: 58 adding ones of k < 512 and fewer than 2000 rows of w would be 1.4 times as fast in parts.)
+// eight (298 rows of x, 5328 rows of w in pairs, k = 9664: 77 us, 55 by the rule before this estimate).
 struct PartTime { int columns, places, once, step, share, beside, part, sums; };
 constexpr int DIES = 8;
 // Tiles are dealt to the dies in equal runs (tile_place): what the largest run comes to on all of them.
 long dealt(long tiles) { return (tiles + DIES - 1) / DIES * DIES; }
 constexpr PartTime NARROW_PARTS = {64, 2, 5950, 256, 166, 95, 250, 1540}, WIDE_PARTS = {128, 1, 6630, 445, 200, 0, 251, 1720},
                    WIDE_PARTS_TWO = {128, 2, 7190, 592, 237, 0, 268, 1050};          // (two stages instead of three: two to a compute unit, beyond 256 rows)
-long parts_time(const PartTime& shape, int M, long N, int steps, int parts) {
-    const long groups = dealt((long)((M + 127) / 128) * ((N + shape.columns - 1) / shape.columns)) * parts, places = (long)shape.places * XRT_COMPUTE_UNITS;
+long parts_time(const PartTime& shape, int M, long rows_w, int steps, int parts) {
+    const long groups = dealt((long)((M + 127) / 128) * ((rows_w + shape.columns - 1) / shape.columns)) * parts, places = (long)shape.places * XRT_COMPUTE_UNITS;
     const long whole = groups / places, rest = groups % places;
     const long full = shape.step + shape.share * shape.places + shape.beside;
     const long last = rest == 0 ? 0 : shape.step + shape.share * rest / XRT_COMPUTE_UNITS + (rest > XRT_COMPUTE_UNITS ? shape.beside : 0);
-    return shape.once + shape.part * parts + steps * (whole * full + last) + shape.sums * parts * ((long)M * N / 1000) / 1000;
+    return shape.once + shape.part * parts + steps * (whole * full + last) + shape.sums * parts * ((long)M * rows_w / 1000) / 1000;
 }
 // The same of the tiles without a split (a fit to the same products: their own estimate counts a warm chip's rounds alone).
-long unsplit_time(int M, int N, int K, int mode) {
+long unsplit_time(int M, long rows_w, int K, int mode) {
     const int kind = mode == MODE_GATED ? ENDS_GATED : mode == MODE_ACCUMULATE ? ENDS_ADDING : ENDS_BF16;
-    const long rows_w = mode == MODE_GATED ? 2L * N : N;
     auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((rows_w + bn - 1) / bn); };
     if (mode == MODE_GATED && M <= 256) {                      // one round of tiles in several stages
         if (tiles(128, 64) <= XRT_COMPUTE_UNITS) return 5000 + (NARROW_PARTS.step + NARROW_PARTS.share * tiles(128, 64) / XRT_COMPUTE_UNITS) * (K / 64);
@@ -1161,6 +1226,73 @@ long unsplit_time(int M, int N, int K, int mode) {
     auto cost = [&](const TileTime& tile) { return rounds_cost(tiles(tile.bm, tile.bn), tile, K, kind); };
     const long least = min(min(cost(LARGE_TILE), cost(MIDDLE_TILE)), min(cost(HALF_TILE), cost(SMALL_TILE)));
     return 1000 + (mode == MODE_GATED ? least : least * 127 / 100);
+}
+struct Cut { int splits, tile, columns; };
+// Tiles of 128 x 64 or 128 x 128 and the number of parts by the estimates, against the product without a split, which saves a gated one the sums of both halves. (Narrow tiles read x
+// twice as often, which does not stay in a die's L2 when k is long: 4096 rows of w, k = 14336, 100 rows of x 34.7 us in wide tiles, 40.3 in narrow ones.)
+Cut cut_by_parts_time(int M, long rows_w, int K, int mode, bool whole_norm = false) {
+    const int units = K / 64;
+    auto per_part = [&](int parts) { return (units + parts - 1) / parts; };
+    auto some = [&](int parts) { return parts <= units && (units + per_part(parts) - 1) / per_part(parts) == parts; };     // (otherwise: as many pieces a part with fewer parts)
+    Cut cut{1, 128, 128};
+    const long large_tiles = (long)((M + 255) / 256) * ((rows_w + 255) / 256);
+    if (large_tiles <= 128 && M >= 512 && mode != MODE_GATED && units >= (whole_norm ? 64 : 128)) return Cut{max(1, min(min((int)(XRT_COMPUTE_UNITS / large_tiles), 8), units / 24)), 256, 256};
+    if ((long)((M + 127) / 128) * ((rows_w + SPLIT_BN - 1) / SPLIT_BN) > (M <= 256 ? 2 * XRT_COMPUTE_UNITS : XRT_COMPUTE_UNITS)) return cut;      // (they fill the chip as they are)
+    long best = unsplit_time(M, rows_w, K, mode);
+    for (const PartTime& shape : {NARROW_PARTS, M <= 256 ? WIDE_PARTS : WIDE_PARTS_TWO}) {
+        if (shape.columns == 64 && K >= 8192 && rows_w > 2048) continue;
+        for (int parts = 2; parts <= 16; ++parts) {
+            if (!some(parts)) continue;
+            const long time = parts_time(shape, M, rows_w, per_part(parts), parts);
+            if (time < best) { best = time; cut = Cut{parts, 128, shape.columns}; }
+        }
+    }
+    // Large tiles of 192 rows, in parts that make one round: fewer operands read a product, more at the ends (150 rows of x, 10240 rows of w, k = 5120
+    // 43 -> 34 us beside the best of the others).
+    const long large = dealt((long)((M + 191) / 192) * ((rows_w + 255) / 256));
+    for (int parts = 2; M > 128 && parts <= 16 && parts * large <= XRT_COMPUTE_UNITS; ++parts) {
+        if (!some(parts)) continue;
+        const long time = 10000 + 1200L * per_part(parts) + 1400L * parts * (M * rows_w / 1000) / 1000;
+        if (time < best) { best = time; cut = Cut{parts, 192, 256}; }
+    }
+    return cut;
+}
+
+// What every other product of more than 64 rows of x takes, in microseconds, cut or not. A step of 64 along k takes `step`, `share` more for each workgroup that a compute unit has
+// on average (up to `places` of them side by side), and `beside` where some have two; reading w, and `again` of what is read of x on all dies (on one, where
+// the parts are dealt so), takes `bytes` a megabyte; the larger of the two counts, smoothly. `part` and `sums` are what a part and a million partial sums cost the second kernel and the first;
+// once and outs (a million results) go by what the product does: store, add with the norm behind it (cut: in the second kernel; not cut: a kernel of its own), add.
+// Fitted to 8000 products (65 to 2100 rows of x, 256 to 16384 rows of w, k from 256 to 25600, half of them of widths that models have), every tile with every number of parts
+// from 2 to 16 of each timed, 150000 times in all: of 2400 others what it chooses is 1.5 % off the best of all on average, where the estimates above, which know the tiles of 128
+// and, for k from 4096 on and 512 rows, of 256 rows, and of 192 as a rule of thumb, were 4.5 % off: 520 rows of x, 4096 rows of w, k = 14336 84 -> 67 us, 2048 rows, k = 8192 45 -> 34, 200 rows, 5120 rows, k = 25600
+// 97 -> 72, 1100 rows, 4096 rows, k = 4096 63 -> 51.
+enum { KIND_STORE, KIND_NORMED, KIND_ADD };
+struct TileCost { double step, share, beside, part, bytes, again, sums, once[3], outs[3]; };
+struct CutShape { int rows, columns, places; TileCost cost; };
+constexpr CutShape CUT_128_BY_64 = {128, 64, 2, {0.295, 0.101, 0.149, 0.174, 0.203, 0.075, 1.385, {6.003, 6.308, 6.525}, {0.075, 1.864, 0.000}}},
+                   // (at most one to a compute unit: four stages; of a short k eight wavefronts)
+                   CUT_128_BY_64_ALONE = {128, 64, 2, {0.329, 0.000, 0.000, 0.219, 0.198, 0.185, 1.762, {5.174, 5.018, 5.524}, {0.169, 3.266, 0.312}}},
+                   CUT_128_BY_64_SHORT = {128, 64, 2, {0.242, 0.039, 0.000, 0.161, 0.165, 0.389, 1.681, {5.474, 5.756, 5.851}, {0.632, 2.781, 0.367}}},
+                   CUT_128_BY_128 = {128, 128, 2, {0.706, 0.122, 0.003, 0.147, 0.314, 0.105, 1.035, {6.869, 7.672, 6.806}, {0.169, 1.672, 0.754}}},
+                   CUT_128_BY_128_THREE_STAGES = {128, 128, 1, {0.543, 0.000, 0.000, 0.204, 0.162, 0.161, 1.942, {5.855, 6.164, 5.901}, {0.694, 0.947, 0.788}}},
+                   CUT_192 = {192, 256, 1, {0.759, 0.209, 0.000, 0.093, 0.165, 0.646, 0.850, {12.673, 13.490, 12.186}, {0.052, 1.386, 0.922}}},
+                   CUT_256 = {256, 256, 1, {0.778, 0.441, 0.000, 0.069, 0.181, 0.632, 0.698, {15.312, 16.178, 14.564}, {0.247, 1.626, 1.237}}},
+                   WHOLE[] = {{256, 256, 1, {0.842, 0.410, 0.000, 0.000, 0.001, 0.196, 0.000, {7.279, 26.096, 21.168}, {0.429, 1.205, 0.632}}},
+                              {192, 256, 1, {0.763, 0.224, 0.000, 0.000, 0.372, 0.000, 0.000, {5.708, 18.654, 14.700}, {0.527, 1.509, 0.977}}},
+                              {128, 256, 1, {0.676, 0.106, 0.000, 0.000, 0.377, 0.000, 0.000, {4.336, 13.687, 9.568}, {0.572, 1.724, 1.275}}},
+                              {128, 128, 2, {0.712, 0.100, 0.039, 0.000, 0.434, 0.106, 0.000, {7.934, 9.724, 8.980}, {0.000, 1.506, 0.346}}}};
+double cut_time(const CutShape& shape, int M, int N, int K, int steps, int parts, int kind) {
+    const TileCost& c = shape.cost;
+    const long tiles = (long)((M + shape.rows - 1) / shape.rows) * ((N + shape.columns - 1) / shape.columns);
+    const bool by_parts = deals_by_parts(shape.columns, tiles, K, parts);
+    const long groups = part_ids(tiles, parts, by_parts), places = (long)shape.places * XRT_COMPUTE_UNITS;
+    const long whole = groups / places, rest = groups % places;
+    const double full = c.step + c.share * shape.places + c.beside;
+    const double last = rest == 0 ? 0. : c.step + c.share * rest / XRT_COMPUTE_UNITS + (rest > XRT_COMPUTE_UNITS ? c.beside : 0.);
+    const double loop = steps * (whole * full + last), results = 1e-6 * M * N;
+    const double memory = c.bytes * 2e-6 * K * (N + c.again * M * (by_parts ? 1 : DIES));
+    const double loop2 = loop * loop, memory2 = memory * memory;
+    return c.once[kind] + c.part * parts + sqrt(sqrt(loop2 * loop2 + memory2 * memory2)) + (parts > 1 ? c.sums * parts * results : 0.) + c.outs[kind] * results;
 }
 
 // Gated products of 17 to 64 rows of x (nanoseconds): unsplit in one round of tiles of 64 x 64, every workgroup all of k, or in parts of 64 x 128 as many as the compute units
@@ -1177,67 +1309,98 @@ long few_rows_parts_time(int M, long rows_w, int per, int parts) {
     return 5330 + 94 * parts + per * (328 + 318 * groups / XRT_COMPUTE_UNITS + (groups > XRT_COMPUTE_UNITS ? 250 : 0)) + 2490 * parts * (M * rows_w / 1000) / 1000;
 }
 
-// whole_norm: an RMSNorm follows that the second kernel can do outright, which is worth a split in two where the product alone
-// would do as well without (k from 4096 on instead of from 8192 on).
-SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false) {
+// Products of 17 to 64 rows of x that are not gated, in tiles of 64 x 128 and `parts` parts: microseconds, as above. Fitted to 6500 products (256 to 16384 rows of w, k from 256 to 20000); of 2700 others
+// the choice by it is 0.9 % off the best number of parts and takes 0.977 of as many parts as leave every compute unit one workgroup (61 rows, 4096 rows of w, k = 1024
+// 12.2 -> 10.4 us, 3072 rows, k = 2048 12.2 -> 11.9; 34 of them more than 1.04, up to 1.11).
+double few_rows_cut_time(int M, int N, int K, int steps, int parts) {
+    const long tiles = (N + SPLIT_BN - 1) / SPLIT_BN;
+    const long groups = part_ids(tiles, parts, deals_by_parts(SPLIT_BN, tiles, K, parts));
+    constexpr double STEP = 0.367, SHARE = 0.292, BESIDE = 0.313;
+    const long whole = groups / XRT_COMPUTE_UNITS, rest = groups % XRT_COMPUTE_UNITS;
+    const double share = SHARE * rest / XRT_COMPUTE_UNITS;
+    double step = whole * (STEP + SHARE) + (rest > 0 ? STEP + share : 0.);
+    if (whole == 1 && rest > 0) step = STEP + SHARE + BESIDE + share;      // two side by side
+    const double loop = steps * step, memory = 0.051 * 2e-6 * K * N, loop2 = loop * loop, memory2 = memory * memory;
+    return 5.287 + 0.051 * parts + sqrt(sqrt(loop2 * loop2 + memory2 * memory2)) + 2.444e-6 * parts * M * N;
+}
+
+// fixed: for xrt_linear_static, whose array holds the sums of so many parts and not of any number of them.
+SplitPlan plan_of(int M, int N, int K, int mode, bool whole_norm, bool fixed) {
     const long rows_w = mode == MODE_GATED ? 2L * N : N;
     const long tiles_n = (rows_w + SPLIT_BN - 1) / SPLIT_BN;
     const int units = K / 64;                                  // k is dealt out in pieces of 64
-    int splits, least, tile = SPLIT_BM, columns = SPLIT_BN;    // least: pieces of k that a part should have
-    const long large_tiles = (long)((M + 255) / 256) * ((rows_w + 255) / 256);
-    if (M <= SPLIT_BM) {
+    int splits = 1, tile = SPLIT_BM, columns = SPLIT_BN;
+    double best = 0;
+    auto per_part = [&](int parts) { return (units + parts - 1) / parts; };
+    auto some = [&](int parts) { return parts <= units && (units + per_part(parts) - 1) / per_part(parts) == parts; };     // (otherwise: as many pieces a part with fewer parts)
+    if (M <= SPLIT_BM && mode == MODE_GATED) {
         splits = (int)(XRT_COMPUTE_UNITS / tiles_n);                         // one workgroup per compute unit, or fewer
-        least = 1;
-        if (mode == MODE_GATED && (rows_w + 63) / 64 <= XRT_COMPUTE_UNITS) {
+        if ((rows_w + 63) / 64 <= XRT_COMPUTE_UNITS) {
             // one round of tiles of half the width is there for the taking, without a second kernel: by the estimates of both
-            const int parts = max(1, min(min(splits, 16), units)), per = (units + parts - 1) / parts;
+            const int parts = max(1, min(min(splits, 16), units)), per = per_part(parts);
             if (parts == 1 || narrow_gated_time(M, rows_w, units) < few_rows_parts_time(M, rows_w, per, (units + per - 1) / per)) { splits = 1; columns = 64; }
         }
-    } else if (large_tiles <= 128 && M >= 512 && mode != MODE_GATED && units >= (whole_norm ? 64 : 128)) {
-        // Many rows and a very long k, but so few columns that the largest tiles would leave half of the compute
-        // units idle (the projection back from the feed-forward's width): the large tiles split k between them.
-        // The tiles of 128 x 128, which fill the chip without a second kernel, read their operands from LDS
-        // more often for the same products and take longer here.
-        splits = (int)(XRT_COMPUTE_UNITS / large_tiles);
-        splits = splits > 8 ? 8 : splits;
-        least = 24;
-        tile = columns = 256;
+    } else if (M <= SPLIT_BM) {
+        // As many parts as leave every compute unit one workgroup, or a number that is a twentieth better by the estimate. A product whose tiles leave no room for
+        // two parts is not cut, and what the parts sum up fits the fixed array of xrt_linear_static.
+        splits = min((int)(XRT_COMPUTE_UNITS / tiles_n), min(16, units));
+        if (splits > 1) {
+            splits = (units + per_part(splits) - 1) / per_part(splits);
+            best = 0.95 * few_rows_cut_time(M, N, K, per_part(splits), splits);
+        }
+        for (int parts = 2; splits > 1 && parts <= 16; ++parts) {
+            if (!some(parts) || parts * tiles_n > 2 * XRT_COMPUTE_UNITS || (long)parts * M * N > XRT_LINEAR_STATIC_FLOATS) continue;
+            const double time = few_rows_cut_time(M, N, K, per_part(parts), parts);
+            if (time < best) { best = time; splits = parts; }
+        }
+    } else if (mode == MODE_GATED || fixed) {
+        const Cut cut = cut_by_parts_time(M, rows_w, K, mode);
+        splits = cut.splits;
+        tile = cut.tile;
+        columns = cut.columns;
     } else {
-        // Some hundred rows of x: still bound by reading w, and too few tiles to fill the chip without a split. Tiles of 128 x 64 or 128 x 128
-        // and the number of parts by an estimate of the time, against one of the product without a split (which saves a gated product the sums of both halves). (Narrow tiles read x twice as often, which
-        // does not stay in a die's L2 when k is long: 4096 rows of w, k = 14336, 100 rows of x 34.7 us in wide tiles, 40.3 in narrow ones.)
-        const long tiles = (long)((M + 127) / 128) * tiles_n;
-        tile = columns = 128;
-        least = 1;
-        splits = 1;
-        if (tiles <= (M <= 256 ? 2 * XRT_COMPUTE_UNITS : XRT_COMPUTE_UNITS)) {      // (more fill the chip as they are)
-            long best = unsplit_time(M, N, K, mode);
-            for (const PartTime& shape : {NARROW_PARTS, M <= 256 ? WIDE_PARTS : WIDE_PARTS_TWO}) {
-                if (shape.columns == 64 && K >= 8192 && rows_w > 2048) continue;
-                for (int parts = 2; parts <= 16 && parts <= units; ++parts) {
-                    const int per = (units + parts - 1) / parts;
-                    if ((units + per - 1) / per != parts) continue;          // (as many pieces a part with fewer parts)
-                    const long time = parts_time(shape, M, rows_w, per, parts);
-                    if (time < best) { best = time; splits = parts; columns = shape.columns; }
-                }
-            }
-            // Large tiles of 192 rows, in parts that make one round: fewer operands read a product, more at the ends (beside the best of the others: 333 rows
-            // of x, 5120 rows of w, k = 25600 129 -> 113 us, 4096 rows, k = 14336 61 -> 58, but k = 4096 30 -> 33; 150 rows of x, 10240 rows of w, k = 5120
-            // 43 -> 34). The figures are of those and 100 more such products.
-            const long large = dealt((long)((M + 191) / 192) * ((rows_w + 255) / 256));
-            for (int parts = 2; M > 128 && parts <= 16 && parts <= units && parts * large <= XRT_COMPUTE_UNITS; ++parts) {
-                const int per = (units + parts - 1) / parts;
-                if ((units + per - 1) / per != parts) continue;
-                const long time = 10000 + 1200L * per + 1400L * parts * (M * rows_w / 1000) / 1000;
-                if (time < best) { best = time; splits = parts; tile = 192; columns = 256; }
+        // The best of all cuts by the estimate, where it is a twentieth less than what the two older estimates choose (what it finds below that is as often slower as
+        // faster: of 2400 products 157 take more than 1.05 of their time without this, 20 with it, and all of them 0.97 either way).
+        const int kind = mode == MODE_STORE ? KIND_STORE : whole_norm ? KIND_NORMED : KIND_ADD;
+        auto time_of = [&](int rows, int wide, int parts) {
+            const CutShape& shape = rows == 256 ? CUT_256 : rows == 192 ? CUT_192 : wide == 128 ? (M <= 256 ? CUT_128_BY_128_THREE_STAGES : CUT_128_BY_128)
+                : dealt((long)((M + 127) / 128) * ((N + 63) / 64)) * parts > XRT_COMPUTE_UNITS ? CUT_128_BY_64 : K < 4096 ? CUT_128_BY_64_SHORT : CUT_128_BY_64_ALONE;
+            return cut_time(shape, M, N, K, per_part(parts), parts, kind);
+        };
+        double whole = 1e30;
+        for (const CutShape& shape : WHOLE) whole = fmin(whole, cut_time(shape, M, N, K, units, 1, kind));
+        const Cut cut = cut_by_parts_time(M, rows_w, K, mode, whole_norm);
+        splits = cut.splits;
+        tile = cut.tile;
+        columns = cut.columns;
+        best = 0.95 * (splits == 1 ? whole : time_of(tile, columns, splits));
+        if (splits > 1 && whole < best) { best = whole; splits = 1; tile = columns = 128; }
+        for (const Cut& shape : {Cut{0, 128, 64}, Cut{0, 128, 128}, Cut{0, 192, 256}, Cut{0, 256, 256}}) {
+            // (tiles that are mostly empty, and more than a round of the large ones or about two of the others, were not timed)
+            if ((shape.tile == 192 && M <= 96) || (shape.tile == 256 && M < 200)) continue;
+            const long tiles = (long)((M + shape.tile - 1) / shape.tile) * ((N + shape.columns - 1) / shape.columns);
+            for (int parts = 2; parts <= 16 && (shape.columns == 256 ? parts * dealt(tiles) <= XRT_COMPUTE_UNITS : parts * tiles <= 600); ++parts) {
+                if (!some(parts)) continue;
+                const double time = time_of(shape.tile, shape.columns, parts);
+                if (time < best) { best = time; splits = parts; tile = shape.tile; columns = shape.columns; }
             }
         }
     }
-    splits = splits < 1 ? 1 : (splits > 16 ? 16 : splits);
-    splits = splits > units / least ? (units / least < 1 ? 1 : units / least) : splits;
-    const int per = (units + splits - 1) / splits;
+    splits = max(1, min(min(splits, 16), units));
+    const int per = per_part(splits);
     splits = (units + per - 1) / per;                          // no empty part
     return SplitPlan{splits, per * 64, rows_w, tile, columns};
+}
+// whole_norm: an RMSNorm follows that the second kernel can do outright.
+// A step asks for the same plans again and again, several times a product (what it takes, its workspace, its launch): each thread keeps the last ones it has worked out.
+SplitPlan split_plan(int M, int N, int K, int mode, bool whole_norm = false, bool fixed = false) {
+    struct Kept { int M, N, K, kind; SplitPlan plan; };
+    constexpr int PLANS = 64;
+    static thread_local Kept kept[PLANS] = {};                 // (M = 0: none)
+    const int kind = mode * 4 + whole_norm * 2 + fixed;
+    Kept& k = kept[((unsigned)M * 2654435761u ^ (unsigned)N * 2246822519u ^ (unsigned)K * 3266489917u ^ (unsigned)kind * 668265263u) >> 26];
+    if (k.M != M || k.N != N || k.K != K || k.kind != kind) k = Kept{M, N, K, kind, plan_of(M, N, K, mode, whole_norm, fixed)};
+    return k.plan;
 }
 
 // The sums over the parts, in order, of one output, or (BOTH) of it and the one `apart` columns behind; part p lies p * stride floats
@@ -1521,9 +1684,9 @@ int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, b
         return launch_kernel<SPLIT_BM, SPLIT_BN, 2, 4, MODE_STORE, 64, 3, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
     }
     if (plan.tile == 192)
-        return launch_large<192, MODE_STORE, float>(a, w, workspace, M, rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split);
+        return launch_large<192, MODE_STORE, float, true>(a, w, workspace, M, rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split);
     if (plan.tile == 256)
-        return launch_large<256, MODE_STORE, float>(a, w, workspace, M, rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split);
+        return launch_large<256, MODE_STORE, float, true>(a, w, workspace, M, rows_w, K, packing, XRT_ACT_SILU, s, plan.splits, plan.k_per_split);
     if (plan.columns == 64) {
         // a fourth stage where a compute unit has one workgroup anyway (2048 rows of w, k = 8192, 65 / 200 rows of x 16.0 / 22.5 -> 14.7 / 20.5 us with its
         // second kernel; k = 2048, 3072 rows, 100 rows of x 12.0 -> 11.5)
@@ -1543,10 +1706,10 @@ int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, b
 
 template <typename TO>
 int launch_split(const bf16* a, const bf16* w, TO* out, int M, int N, int K, int mode, int activation, const Packing& packing,
-                 float* workspace, const xrt_linear_norm* norm, const QkvAfter* after, hipStream_t s) {
+                 float* workspace, const xrt_linear_norm* norm, const QkvAfter* after, hipStream_t s, bool fixed = false) {
     // the whole norm after an accumulating product of many rows: normed rows asked for, and no sums of squares
     const bool whole_norm = norm && norm->scaled_out && !norm->squares_out && !norm->squares_in;
-    const SplitPlan plan = split_plan(M, N, K, mode, whole_norm);
+    const SplitPlan plan = split_plan(M, N, K, mode, whole_norm, fixed);
     const bool scaled = norm && norm->squares_in, emits = norm && norm->squares_out;
     XRT_REQUIRE(!norm || M <= SPLIT_BM || whole_norm, "linear (mfma): the halves of a norm around a product take at most %d rows here", SPLIT_BM);
     if (whole_norm)
@@ -1652,6 +1815,18 @@ int xrt_linear_groups_mfma(const void* a, int lda, const void* w, long w_stride,
                                       activation, splits, s);
     return launch_grouped_of<128>((const bf16*)a, (const bf16*)w, w_stride, out, out_dtype, tiles_m, N, K, lda, ldw, tile_group, packing, mode,
                                   activation, splits, s);
+}
+
+// The same by the plan whose partial sums the fixed array of xrt_linear_static was made for: how many floats they are (0: not cut along k), and the product.
+long xrt_linear_split_fixed_floats(const void* a, const void* w, int M, int N, int K, int mode) {
+    if (M <= 16 || K % 64 != 0 || K < 128 || !xrt_linear_mfma_accepts(a, w, M, N, K, mode)) return 0;
+    const SplitPlan plan = split_plan(M, N, K, mode, false, true);
+    return plan.splits == 1 || plan.rows_w * (long)M >= (1L << 31) ? 0 : (long)plan.splits * M * plan.rows_w;
+}
+int xrt_linear_split_fixed(const void* a, const void* w, void* out, int out_dtype, int M, int N, int K, int mode, int activation, float* workspace, hipStream_t s) {
+    const Packing plain = {XRT_PACK_NONE, 0, 0, 0};
+    if (out_dtype == XRT_F32) return launch_split<float>((const bf16*)a, (const bf16*)w, (float*)out, M, N, K, mode, activation, plain, workspace, nullptr, nullptr, s, true);
+    return launch_split<bf16>((const bf16*)a, (const bf16*)w, (bf16*)out, M, N, K, mode, activation, plain, workspace, nullptr, nullptr, s, true);
 }
 
 // Whether a product runs through the tiles of this section (17 to 64 rows of x, or more rows and few

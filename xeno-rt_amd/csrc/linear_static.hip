@@ -17,6 +17,9 @@
 
 #define XRT_STATIC_MAX_DEVICES 64
 
+long xrt_linear_split_fixed_floats(const void* a, const void* w, int M, int N, int K, int mode);
+int xrt_linear_split_fixed(const void* a, const void* w, void* out, int out_dtype, int M, int N, int K, int mode, int activation, float* workspace, hipStream_t s);
+
 static __device__ __align__(256) float scratch[XRT_LINEAR_STATIC_FLOATS];
 
 // The address of `scratch` on each device. In host code the array's name is only a handle for
@@ -49,7 +52,18 @@ extern "C" int xrt_linear_static(const void* a, const void* w, int dtype, void* 
     XRT_REQUIRE(M >= 0 && N > 0 && K > 0, "linear (static): bad sizes M=%d N=%d K=%d", M, N, K);
     XRT_REQUIRE(mode >= 0 && mode <= 2, "linear (static): unknown mode %d", mode);
     XRT_REQUIRE(a && w && out, "linear (static): null operand");
-    const long need = xrt_linear_workspace(a, w, dtype, M, N, K, mode);
+    // Which products the array serves goes by a plan of its own, which cuts k into few parts; where xrt_linear would have more parts than
+    // fit, that plan is taken.
+    const long fixed = dtype == XRT_BF16 && M > 0 ? xrt_linear_split_fixed_floats(a, w, M, N, K, mode) : 0;
+    long need = xrt_linear_workspace(a, w, dtype, M, N, K, mode);
+    if (fixed > (long)XRT_LINEAR_STATIC_FLOATS) need = need > fixed ? need : fixed;
+    else if (need > (long)XRT_LINEAR_STATIC_FLOATS) {
+        if (fixed == 0) return xrt_linear(a, w, dtype, out, out_dtype, M, N, K, mode, nullptr, 0, stream);       // (not cut: without a workspace)
+        float* workspace = nullptr;
+        if (scratch_pointer(&workspace) != 0) return 1;
+        XRT_REQUIRE(out_dtype == XRT_F32 || (out_dtype == XRT_BF16 && mode != 1), "linear (static): output dtype %d in mode %d", out_dtype, mode);
+        return xrt_linear_split_fixed(a, w, out, out_dtype, M, N, K, mode, XRT_ACT_SILU, workspace, (hipStream_t)stream);
+    }
     XRT_REQUIRE(need <= (long)XRT_LINEAR_STATIC_FLOATS,
                 "linear (static): M=%d N=%d K=%d mode %d splits into %ld floats of partial sums, the fixed buffer holds %ld",
                 M, N, K, mode, need, (long)XRT_LINEAR_STATIC_FLOATS);
