@@ -469,7 +469,7 @@ __device__ __forceinline__ void gemm_tile(
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
                     for (int e = 0; e < 16; ++e) {
-                        const long m = min(m0 + wave_m * WAVE_M + i * 32 + (e / 4) * 8 + (lane / 32) * 4 + e % 4, (long)M - 1);
+                        const long m = min(m0 + wave_m * WAVE_M + i * 32 + (e / 4) * 8 + (lane / 32) * 4 + e % 4, M - 1);      // (of an int and a long: the double's min)
                         const long n = min(column[j], (long)N - 1);
                         before[j][e] = to_float(out[m * (long)N + n]);
                     }
