@@ -24,3 +24,12 @@ def test_products_have_no_double_precision(objects):
             doubles[kernel] += 1
     assert sum("gemm_mfma_kernel" in (name or "") for name in seen) > 10
     assert not doubles, doubles.most_common(5)
+
+
+# 512 registers a SIMD lane: up to 96 leave room for five wavefronts, up to 64 for eight.
+def test_the_kernel_that_adds_parts_of_q_k_v_leaves_room_for_other_wavefronts(objects):
+    of_parts = {name: fields for _, names in objects for name, fields in names.items() if "qkv_prepare_vector_kernel" in name and "Li0E" not in name}
+    assert len(of_parts) > 10
+    for name, fields in of_parts.items():
+        assert fields["vgpr_count"] <= (64 if "Li2EEE" in name else 96), name
+        assert fields["vgpr_spill_count"] == 0 and fields["private_segment_fixed_size"] == 0, name

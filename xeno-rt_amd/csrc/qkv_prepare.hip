@@ -14,7 +14,7 @@
 // step brings many tokens, the values go to their transposed cache blocks through workgroups of
 // their own, which turn tiles of 64 tokens in LDS so that writes to the cache are whole lines.
 // Where a key or a value lies inside its block: cache_layout.h.
-// A projection that was split along k comes as the float32 sums of its parts (PARTS): the vector kernel then adds
+// A projection that was split along k comes as the float32 sums of its parts (AT_ONCE > 0): the vector kernel then adds
 // them, in order, and rounds them to bfloat16 as the kernel that adds them alone does, before it goes on as ever.
 // The general kernel (one wavefront per (token, head), any even head size and rotation width)
 // takes the rest. A token with a negative slot is padding and is not cached. Per head, all
@@ -105,72 +105,65 @@ template <typename T, int N> struct alignas(sizeof(T) * N) Pack { T e[N]; };
 // The parts of a projection split along k: part p of element i at values[p * stride + i]. splits 0: there are none.
 struct QkvParts { const float* values; long stride; int splits; };
 
-// PIECES pieces of 16 bytes of a row of q/k/v, `apart` elements from one another; `at` counts elements from the first row's first. Asked for
-// with ask, which waits for nothing, and there with take: the parts' sums, four parts at a time (those beyond the last: that one again,
-// not added) for all pieces at once. (Piece by piece, with a branch around every part's addition, each waited for the one before it.)
-template <bool PARTS, int PIECES, typename T>
-struct QkvPieces {
-    static constexpr int VEC = 16 / (int)sizeof(T), AT_ONCE = 4, QUADS = VEC / 4;
-    Pack<T, VEC> pieces[PARTS ? 1 : PIECES];
-    float4 asked[PARTS ? AT_ONCE : 1][PIECES][QUADS];
-    const float* first;
-    long apart;
-    __device__ __forceinline__ void ask_parts(const QkvParts& parts, int p0) {
+// PIECES pieces of 16 bytes of a row of q/k/v, `apart` elements from one another; `at` counts elements from the first row's first. AT_ONCE 0: as they lie in
+// qkv. Else the parts' sums: AT_ONCE parts of all pieces are asked for at once (those beyond the last: that one again, not added), then added in order.
+// What is asked for stays within a turn: kept across turns (and across the angles, asked for ahead of them) it took a wavefront 154 registers
+// instead of 58, 74 or 90 (2, 3 or 4 at once), three wavefronts a SIMD instead of eight, six or five. Parts just written, microseconds, so / kept across / piece by
+// piece with a branch around every part: 333 tokens of 32 heads of 128 on 8 in three parts 8.2 / 9.1 / 8.2, in two 8.3 / 9.8 / 8.8; 100 tokens of 32 heads of 64 on 8 in
+// four 4.8 / 4.9 / 5.4. 17 to 160 tokens of four such shapes in 2 to 16 parts 0.87 / 0.93 / 1, 200 to 789 tokens 0.98 / 1.09 / 1.
+template <int AT_ONCE, int PIECES, typename T>
+__device__ __forceinline__ void read_qkv(const T* qkv, const QkvParts& parts, long at, long apart, Pack<T, 16 / (int)sizeof(T)> (&out)[PIECES]) {
+    constexpr int VEC = 16 / (int)sizeof(T);
+    if constexpr (AT_ONCE == 0) {
 #pragma unroll
-        for (int u = 0; u < AT_ONCE; ++u) {
-            const float* from = first + min(p0 + u, parts.splits - 1) * parts.stride;
+        for (int i = 0; i < PIECES; ++i) out[i] = *reinterpret_cast<const Pack<T, VEC>*>(qkv + at + i * apart);
+    } else {
+        static_assert(sizeof(T) == 2, "parts are rounded to bfloat16");
+        typedef float4 Asked[AT_ONCE][PIECES][2];
+        auto ask = [&](int p0, Asked& asked) {
 #pragma unroll
-            for (int i = 0; i < PIECES; ++i)
+            for (int u = 0; u < AT_ONCE; ++u) {
+                const float* from = parts.values + min(p0 + u, parts.splits - 1) * parts.stride + at;
 #pragma unroll
-                for (int q = 0; q < QUADS; ++q) asked[u][i][q] = *reinterpret_cast<const float4*>(from + i * apart + 4 * q);
-        }
-    }
-    __device__ __forceinline__ void ask(const T* qkv, const QkvParts& parts, long at, long pieces_apart) {
-        if constexpr (!PARTS) {
+                for (int i = 0; i < PIECES; ++i)
 #pragma unroll
-            for (int i = 0; i < PIECES; ++i) pieces[i] = *reinterpret_cast<const Pack<T, VEC>*>(qkv + at + i * pieces_apart);
-        } else {
-            static_assert(sizeof(T) == 2, "parts are rounded to bfloat16");
-            first = parts.values + at;
-            apart = pieces_apart;
-            ask_parts(parts, 0);
-        }
-    }
-    __device__ __forceinline__ void take(const QkvParts& parts, Pack<T, VEC> (&out)[PIECES]) {
-        if constexpr (!PARTS) {
-#pragma unroll
-            for (int i = 0; i < PIECES; ++i) out[i] = pieces[i];
-        } else {
-            float sum[PIECES][VEC] = {};
-            for (int p0 = 0;;) {
-#pragma unroll
-                for (int u = 0; u < AT_ONCE; ++u) {
-                    const bool there = p0 + u < parts.splits;
-#pragma unroll
-                    for (int i = 0; i < PIECES; ++i)
-#pragma unroll
-                        for (int q = 0; q < QUADS; ++q) {
-                            const float4 part = asked[u][i][q];
-                            float (&of)[VEC] = sum[i];
-                            of[4 * q] = there ? of[4 * q] + part.x : of[4 * q];
-                            of[4 * q + 1] = there ? of[4 * q + 1] + part.y : of[4 * q + 1];
-                            of[4 * q + 2] = there ? of[4 * q + 2] + part.z : of[4 * q + 2];
-                            of[4 * q + 3] = there ? of[4 * q + 3] + part.w : of[4 * q + 3];
-                        }
-                }
-                p0 += AT_ONCE;
-                if (p0 >= parts.splits) break;
-                __builtin_amdgcn_sched_barrier(0);             // (into the registers of the parts before)
-                ask_parts(parts, p0);
-                __builtin_amdgcn_sched_barrier(0);
+                    for (int q = 0; q < 2; ++q) asked[u][i][q] = *reinterpret_cast<const float4*>(from + i * apart + 4 * q);
             }
+        };
+        float sum[PIECES][VEC] = {};
+        auto add = [&](int p0, const Asked& asked) {
 #pragma unroll
-            for (int i = 0; i < PIECES; ++i)
+            for (int u = 0; u < AT_ONCE; ++u) {
+                const bool there = p0 + u < parts.splits;
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) out[i].e[e] = from_float<T>(sum[i][e]);
+                for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        const float4 part = asked[u][i][q];
+                        float* of = sum[i] + 4 * q;
+                        of[0] = there ? of[0] + part.x : of[0];
+                        of[1] = there ? of[1] + part.y : of[1];
+                        of[2] = there ? of[2] + part.z : of[2];
+                        of[3] = there ? of[3] + part.w : of[3];
+                    }
+            }
+        };
+        Asked first;                                           // (a turn of its own: nothing has been added up yet, 16 registers less)
+        ask(0, first);
+        add(0, first);
+        for (int p0 = AT_ONCE; p0 < parts.splits; p0 += AT_ONCE) {
+            __builtin_amdgcn_sched_barrier(0);
+            Asked more;
+            ask(p0, more);
+            __builtin_amdgcn_sched_barrier(0);
+            add(p0, more);
         }
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i)
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) out[i].e[e] = from_float<T>(sum[i][e]);
     }
-};
+}
 
 // 32 dims of the values of 64 consecutive tokens of a step and one key/value head: read row by row (a piece a thread), turned in
 // LDS, and written so that a store instruction of a wavefront takes 8 tokens of 8 dims: where the
@@ -185,7 +178,7 @@ template <typename T> struct ValueTile {
     long bases[XRT_WAVE];                                             // of the tile's tokens: their block (-1: none) ...
     int withins[XRT_WAVE];                                            // ... and their place in it
 };
-template <typename T, bool PARTS>
+template <typename T, int AT_ONCE>
 __device__ __forceinline__ void write_values(
     ValueTile<T>& shared, int first, int kv_head, int d0, T* __restrict__ qkv, const QkvParts& parts, int tokens, int n_heads, int n_kv_heads, int head_dim,
     const int* __restrict__ positions, const int* __restrict__ slots, T* __restrict__ v_cache,
@@ -212,11 +205,9 @@ __device__ __forceinline__ void write_values(
         const int r = i / pieces, d = (i % pieces) * VEC;
         const long from = min(first + r, tokens - 1);         // rows past the end repeat the last one; nobody writes them to the cache
         const long at = source + from * heads_total * head_dim + d0 + d;
-        QkvPieces<PARTS, 1, T> source_piece;
         Pack<T, VEC> piece[1];
-        source_piece.ask(qkv, parts, at, 0);
-        source_piece.take(parts, piece);
-        if constexpr (PARTS) if (first + r < tokens) *reinterpret_cast<Pack<T, VEC>*>(qkv + at) = piece[0];
+        read_qkv<AT_ONCE>(qkv, parts, at, 0, piece);
+        if constexpr (AT_ONCE > 0) if (first + r < tokens) *reinterpret_cast<Pack<T, VEC>*>(qkv + at) = piece[0];
         *reinterpret_cast<Pack<T, VEC>*>(&shared.tile[r][d]) = piece[0];
     }
     __syncthreads();
@@ -239,7 +230,7 @@ __device__ __forceinline__ void write_values(
 // the workgroup's heads.
 // One launch for both: as kernels of their own, values after heads, they took 11.5 + 6.1 us (2048 tokens, 32 heads of 128 on 8) and 3.3 + 4.1
 // (100 tokens, 32 heads of 64 on 8).
-template <typename T, typename TW, int LANES, bool PARTS>
+template <typename T, typename TW, int LANES, int AT_ONCE>
 __global__ void __launch_bounds__(WAVES * XRT_WAVE) qkv_prepare_vector_kernel(
     T* __restrict__ qkv, const QkvParts parts, int tokens, int n_heads, int n_kv_heads,
     const int* __restrict__ positions, const int* __restrict__ slots,
@@ -254,51 +245,43 @@ __global__ void __launch_bounds__(WAVES * XRT_WAVE) qkv_prepare_vector_kernel(
     constexpr int PIECES = (HEAD + TILE_DIMS - 1) / TILE_DIMS;
     const int value_blocks = value_tiles * n_kv_heads * PIECES;
     if ((int)blockIdx.x < value_blocks) {
-        write_values<T, PARTS>(shared.values, (int)blockIdx.x / PIECES % value_tiles * XRT_WAVE, (int)blockIdx.x / PIECES / value_tiles,
+        write_values<T, AT_ONCE>(shared.values, (int)blockIdx.x / PIECES % value_tiles * XRT_WAVE, (int)blockIdx.x / PIECES / value_tiles,
                                (int)blockIdx.x % PIECES * TILE_DIMS, qkv, parts, tokens, n_heads, n_kv_heads, HEAD, positions, slots, v_cache, block_table, table_stride, n_blocks);
         return;
     }
     float* cosines = shared.angles.cosines;
     float* sines = shared.angles.sines;
     const int wave = threadIdx.x / XRT_WAVE, lane = threadIdx.x % XRT_WAVE;
-    const int item = (int)blockIdx.x - value_blocks, chunks_here = PARTS ? chunks : 1;      // (a division less where it is known)
+    const int item = (int)blockIdx.x - value_blocks, chunks_here = AT_ONCE > 0 ? chunks : 1;      // (a division less where it is known)
     const int token = item / chunks_here, chunk = item % chunks_here;
     const int at = (lane % LANES) * VEC;           // this lane's elements: at.. in the lower half, HALF + at.. in the upper
     const int heads_total = n_heads + 2 * n_kv_heads;
     const int heads_here = value_blocks == 0 ? heads_total : n_heads + n_kv_heads;     // value heads come last
-    const int first_head = (chunk * WAVES + wave) * HEADS_PER_WAVE + lane / LANES;
-    // the parts of the first head are asked for before the angles are worked out, behind what those are made of
     const int pos = positions[token];
     const int slot = slots[token];
-    const float theta = rope_theta != nullptr ? rope_theta[min((int)threadIdx.x, HALF - 1)] : 1.f;
-    __builtin_amdgcn_sched_barrier(0);
-    QkvPieces<PARTS, 2, T> halves;
-    auto ask = [&](int head) { halves.ask(qkv, parts, ((long)token * heads_total + min(head, heads_total - 1)) * HEAD + at, HALF); };
-    if constexpr (PARTS) ask(first_head);
     if (rope_theta != nullptr) {
         for (int i = threadIdx.x; i < HALF; i += WAVES * XRT_WAVE) {
-            const float angle = (float)pos * rope_scale / (i < WAVES * XRT_WAVE ? theta : rope_theta[i]);
+            const float angle = (float)pos * rope_scale / rope_theta[i];
             sincosf(angle, &sines[i], &cosines[i]);
         }
     }
-    // (not __syncthreads, which would wait for the head that is on its way)
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    __syncthreads();
     const int within = pos % XRT_BLOCK_TOKENS;
-    const int step = chunks_here * WAVES * HEADS_PER_WAVE;
-    for (int head = first_head; head < heads_here; head = PARTS ? heads_here : head + step) {      // (with parts the chunks are as many as leave no workgroup a second round)
+    // (with parts the chunks are as many as leave no workgroup a second turn)
+    for (int head = (chunk * WAVES + wave) * HEADS_PER_WAVE + lane / LANES; head < heads_here; head = AT_ONCE > 0 ? heads_here : head + WAVES * HEADS_PER_WAVE) {
         // lanes of one head stay together: the exchanges below are within a head
         const bool is_q = head < n_heads, is_v = head >= n_heads + n_kv_heads, is_k = !is_q && !is_v;
-        T* row = qkv + ((long)token * heads_total + head) * HEAD;
-        if constexpr (!PARTS) ask(head);
+        const long row_at = ((long)token * heads_total + head) * HEAD;
+        T* row = qkv + row_at;
         Pack<T, VEC> both[2];
-        halves.take(parts, both);
+        read_qkv<AT_ONCE>(qkv, parts, row_at + at, HALF, both);
         const Pack<T, VEC> lower = both[0], upper = both[1];
         long cache_base = -1;
         if (!is_q && k_cache != nullptr)
             cache_base = cache_block_base(block_table, table_stride, n_blocks, slot, pos, n_kv_heads,
                                           head - n_heads - (is_v ? n_kv_heads : 0), HEAD);
         if (is_v) {
-            if constexpr (PARTS) {
+            if constexpr (AT_ONCE > 0) {
                 *reinterpret_cast<Pack<T, VEC>*>(row + at) = lower;
                 *reinterpret_cast<Pack<T, VEC>*>(row + HALF + at) = upper;
             }
@@ -416,29 +399,36 @@ static int prepare(void* qkv, const QkvParts& parts, int dtype, int tokens, int 
         const long blocks = (long)value_tiles * n_kv_heads * ((head_dim + TILE_DIMS - 1) / TILE_DIMS) + (long)tokens * chunks;
         XRT_REQUIRE(blocks < (1L << 31), "qkv_prepare: too many workgroups");
         const unsigned grid = (unsigned)blocks;
-#define XRT_VEC(T, TW, L, PARTS)                                                                           \
-    qkv_prepare_vector_kernel<T, TW, L, PARTS><<<grid, WAVES * XRT_WAVE, 0, s>>>(                          \
+#define XRT_VEC(T, TW, L, AT_ONCE)                                                                           \
+    qkv_prepare_vector_kernel<T, TW, L, AT_ONCE><<<grid, WAVES * XRT_WAVE, 0, s>>>(                          \
         (T*)qkv, parts, tokens, n_heads, n_kv_heads, positions, slots, (const TW*)q_norm, (const TW*)k_norm, \
         norm_eps, rope_theta, rope_scale, (T*)k_cache, (T*)v_cache, block_table, table_stride, n_blocks,   \
         value_tiles, chunks)
-#define XRT_VEC_LANES(T, TW, PARTS)                                                                        \
+#define XRT_VEC_LANES(T, TW, AT_ONCE)                                                                      \
     switch (lanes) {                                                                                       \
-        case 1: XRT_VEC(T, TW, 1, PARTS); break;                                                           \
-        case 2: XRT_VEC(T, TW, 2, PARTS); break;                                                           \
-        case 4: XRT_VEC(T, TW, 4, PARTS); break;                                                           \
-        case 8: XRT_VEC(T, TW, 8, PARTS); break;                                                           \
-        case 16: XRT_VEC(T, TW, 16, PARTS); break;                                                         \
-        case 32: XRT_VEC(T, TW, 32, PARTS); break;                                                         \
-        default: XRT_VEC(T, TW, 64, PARTS); break;                                                         \
+        case 1: XRT_VEC(T, TW, 1, AT_ONCE); break;                                                           \
+        case 2: XRT_VEC(T, TW, 2, AT_ONCE); break;                                                           \
+        case 4: XRT_VEC(T, TW, 4, AT_ONCE); break;                                                           \
+        case 8: XRT_VEC(T, TW, 8, AT_ONCE); break;                                                           \
+        case 16: XRT_VEC(T, TW, 16, AT_ONCE); break;                                                         \
+        case 32: XRT_VEC(T, TW, 32, AT_ONCE); break;                                                         \
+        default: XRT_VEC(T, TW, 64, AT_ONCE); break;                                                         \
     }
+// (a step's parts all in as few turns as four at once make, evenly)
+#define XRT_VEC_PARTS(TW)                                                                                  \
+    if (at_once <= 2) { XRT_VEC_LANES(bf16, TW, 2) }                                                       \
+    else if (at_once == 3) { XRT_VEC_LANES(bf16, TW, 3) }                                                  \
+    else { XRT_VEC_LANES(bf16, TW, 4) }
         if (parts.splits > 0) {
+            const int turns = (parts.splits + 3) / 4, at_once = (parts.splits + turns - 1) / turns;
             XRT_REQUIRE(dtype == XRT_BF16, "qkv_prepare: the parts of a projection become bfloat16");
-            if (norm_dtype == XRT_F32) { XRT_VEC_LANES(bf16, float, true) }
-            else { XRT_VEC_LANES(bf16, bf16, true) }
-        } else if (dtype == XRT_F32 && norm_dtype == XRT_F32) { XRT_VEC_LANES(float, float, false) }
-        else if (dtype == XRT_F32) { XRT_VEC_LANES(float, bf16, false) }
-        else if (norm_dtype == XRT_F32) { XRT_VEC_LANES(bf16, float, false) }
-        else { XRT_VEC_LANES(bf16, bf16, false) }
+            if (norm_dtype == XRT_F32) { XRT_VEC_PARTS(float) }
+            else { XRT_VEC_PARTS(bf16) }
+        } else if (dtype == XRT_F32 && norm_dtype == XRT_F32) { XRT_VEC_LANES(float, float, 0) }
+        else if (dtype == XRT_F32) { XRT_VEC_LANES(float, bf16, 0) }
+        else if (norm_dtype == XRT_F32) { XRT_VEC_LANES(bf16, float, 0) }
+        else { XRT_VEC_LANES(bf16, bf16, 0) }
+#undef XRT_VEC_PARTS
 #undef XRT_VEC_LANES
 #undef XRT_VEC
         XRT_LAUNCH_CHECK("qkv_prepare");
