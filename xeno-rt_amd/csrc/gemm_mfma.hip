@@ -1196,7 +1196,7 @@ constexpr int SPLIT_BM = 64, SPLIT_BN = 128;
 
 struct SplitPlan { int splits, k_per_split; long rows_w; int tile, columns; };      // tile: rows of x per tile (64, 128, 192 or 256), columns: rows of w
 
-// What a product of some hundred rows of x takes (nanoseconds) in parts along k, if it is gated (of others: what the fixed array of xrt_linear_static is asked for): tiles of 128 rows of x and `columns` rows of w, `places` of them to a compute
+// What a product of some hundred rows of x takes (nanoseconds) in parts along k, if it is gated (of others: the plan of few parts, and what the estimate below has to beat): tiles of 128 rows of x and `columns` rows of w, `places` of them to a compute
 // unit. A step of 64 along k takes `step`, `share` more for each tile that a compute unit has on average, and `beside` more where some have two; `once` is
 // start, end and the second kernel's start, `part` what a further part costs it, `sums` what a million partial sums cost to write and to read again. (Fitted to products of
 // every kind, 512 to 8192 rows of w, k from 512 to 14336, 65 to 1700 rows of x; of 2686 gated products drawn at random afterwards what it chooses is 0.9 % off the best of 27 on average.)
@@ -1324,7 +1324,7 @@ double few_rows_cut_time(int M, int N, int K, int steps, int parts) {
     return 5.287 + 0.051 * parts + sqrt(sqrt(loop2 * loop2 + memory2 * memory2)) + 2.444e-6 * parts * M * N;
 }
 
-// fixed: for xrt_linear_static, whose array holds the sums of so many parts and not of any number of them.
+// fixed: the plan of few parts, which xrt_linear_static takes where the sums of the product's own do not fit its array.
 SplitPlan plan_of(int M, int N, int K, int mode, bool whole_norm, bool fixed) {
     const long rows_w = mode == MODE_GATED ? 2L * N : N;
     const long tiles_n = (rows_w + SPLIT_BN - 1) / SPLIT_BN;
@@ -1817,7 +1817,7 @@ int xrt_linear_groups_mfma(const void* a, int lda, const void* w, long w_stride,
                                   activation, splits, s);
 }
 
-// The same by the plan whose partial sums the fixed array of xrt_linear_static was made for: how many floats they are (0: not cut along k), and the product.
+// The same by the plan of few parts (xrt_linear_static): how many floats its partial sums are (0: not cut along k), and the product.
 long xrt_linear_split_fixed_floats(const void* a, const void* w, int M, int N, int K, int mode) {
     if (M <= 16 || K % 64 != 0 || K < 128 || !xrt_linear_mfma_accepts(a, w, M, N, K, mode)) return 0;
     const SplitPlan plan = split_plan(M, N, K, mode, false, true);

@@ -52,22 +52,18 @@ extern "C" int xrt_linear_static(const void* a, const void* w, int dtype, void* 
     XRT_REQUIRE(M >= 0 && N > 0 && K > 0, "linear (static): bad sizes M=%d N=%d K=%d", M, N, K);
     XRT_REQUIRE(mode >= 0 && mode <= 2, "linear (static): unknown mode %d", mode);
     XRT_REQUIRE(a && w && out, "linear (static): null operand");
-    // Which products the array serves goes by a plan of its own, which cuts k into few parts; where xrt_linear would have more parts than
-    // fit, that plan is taken.
+    // xrt_linear's own plan where its sums fit. The plan of few parts (fixed: its sums) decides two things besides: a product that it does not cut runs uncut, so that
+    // calls which share no array stay free to overlap, and one whose own sums do not fit is cut by it.
     const long fixed = dtype == XRT_BF16 && M > 0 ? xrt_linear_split_fixed_floats(a, w, M, N, K, mode) : 0;
     long need = xrt_linear_workspace(a, w, dtype, M, N, K, mode);
-    if (fixed > (long)XRT_LINEAR_STATIC_FLOATS) need = need > fixed ? need : fixed;
-    else if (need > (long)XRT_LINEAR_STATIC_FLOATS) {
-        if (fixed == 0) return xrt_linear(a, w, dtype, out, out_dtype, M, N, K, mode, nullptr, 0, stream);       // (not cut: without a workspace)
-        float* workspace = nullptr;
-        if (scratch_pointer(&workspace) != 0) return 1;
-        XRT_REQUIRE(out_dtype == XRT_F32 || (out_dtype == XRT_BF16 && mode != 1), "linear (static): output dtype %d in mode %d", out_dtype, mode);
-        return xrt_linear_split_fixed(a, w, out, out_dtype, M, N, K, mode, XRT_ACT_SILU, workspace, (hipStream_t)stream);
-    }
-    XRT_REQUIRE(need <= (long)XRT_LINEAR_STATIC_FLOATS,
+    if (fixed == 0) need = 0;
+    const bool few_parts = need > (long)XRT_LINEAR_STATIC_FLOATS && fixed <= (long)XRT_LINEAR_STATIC_FLOATS;
+    XRT_REQUIRE(need <= (long)XRT_LINEAR_STATIC_FLOATS || few_parts,
                 "linear (static): M=%d N=%d K=%d mode %d splits into %ld floats of partial sums, the fixed buffer holds %ld",
                 M, N, K, mode, need, (long)XRT_LINEAR_STATIC_FLOATS);
+    XRT_REQUIRE(!few_parts || out_dtype == XRT_F32 || (out_dtype == XRT_BF16 && mode != 1), "linear (static): output dtype %d in mode %d", out_dtype, mode);
     float* workspace = nullptr;
     if (need > 0 && scratch_pointer(&workspace) != 0) return 1;
+    if (few_parts) return xrt_linear_split_fixed(a, w, out, out_dtype, M, N, K, mode, XRT_ACT_SILU, workspace, (hipStream_t)stream);
     return xrt_linear(a, w, dtype, out, out_dtype, M, N, K, mode, workspace, need, stream);
 }

@@ -98,9 +98,10 @@ int xrt_linear_with(const void* a, const void* w, const xrt_packing* packing, in
 // xrt_linear for callers that cannot allocate device memory: code under HIP graph capture, tight serving
 // loops, harnesses that forbid hipMalloc. It has no counterpart in the reference. The partial sums of a
 // product split along k go to a fixed array of XRT_LINEAR_STATIC_FLOATS floats (16 MiB) that the library
-// holds in device memory on every GPU it is used on; the call allocates nothing and refuses a product
-// whose partial sums do not fit (xrt_linear_workspace says how many floats a product needs). Calls on one
-// GPU share that array: calls that overlap there (different streams) race.
+// holds in device memory on every GPU it is used on; the call allocates nothing. It takes
+// every product whose partial sums fit (xrt_linear_workspace says how many floats a product needs), and of the others those
+// that fit when cut into fewer parts, or that run uncut; the rest it refuses. Calls on one GPU share that array: calls that overlap there (different
+// streams) race, those of products that xrt_linear does not cut (no floats) apart.
 #define XRT_LINEAR_STATIC_FLOATS (4L << 20)
 long xrt_linear_static_floats(void);       // XRT_LINEAR_STATIC_FLOATS, for callers that do not read this header
 int xrt_linear_static(const void* a, const void* w, int dtype, void* out, int out_dtype, int M, int N, int K,
