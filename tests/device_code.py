@@ -52,42 +52,6 @@ def kernels(path):
     return found
 
 
-def code_objects(library, folder):
-    """Paths of the library's gfx950 code objects, one a source file, written into `folder`."""
-    with open(library, "rb") as handle:
-        data = handle.read()
-    paths = []
-    at = data.find(MAGIC)
-    while at >= 0:
-        count, = struct.unpack_from("<Q", data, at + len(MAGIC))
-        entry = at + len(MAGIC) + 8
-        for _ in range(count):
-            offset, size, length = struct.unpack_from("<QQQ", data, entry)
-            target = data[entry + 24:entry + 24 + length]
-            entry += 24 + length
-            if b"gfx950" in target and size > 0:
-                paths.append(os.path.join(str(folder), f"{len(paths)}.co"))
-                with open(paths[-1], "wb") as out:
-                    out.write(data[at + offset:at + offset + size])
-        at = data.find(MAGIC, at + len(MAGIC))
-    return paths
-
-
-def kernels(path):
-    """{mangled name: {field: number}} of a code object's kernels: vgpr_count, vgpr_spill_count, private_segment_fixed_size and the like."""
-    notes = subprocess.run([_tool("llvm-readelf"), "--notes", path], capture_output=True, text=True, check=True).stdout
-    found, fields = {}, {}
-    for line in notes.splitlines():
-        field = re.match(r"\s*-?\s*\.(\w+):\s+(\S+)\s*$", line)
-        if field is None:
-            continue
-        if field[1] == "symbol":
-            fields = found.setdefault(field[2].strip("'").removesuffix(".kd"), {})
-        elif field[2].isdigit():
-            fields[field[1]] = int(field[2])
-    return found
-
-
 def instructions(path):
     """(kernel's mangled name, instruction) of every line of a code object's disassembly."""
     kernel = None
