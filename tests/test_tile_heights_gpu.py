@@ -89,7 +89,7 @@ def test_rows_dealt_evenly_to_tiles(ops, mode, size, packed):
 
 
 # The fixed array of xrt_linear_static holds the sums of few parts: where the product alone would have more of them, or parts where it had none, it is served as before.
-@pytest.mark.parametrize("m,n,k,mode", [(684, 696, 11456, "add"), (780, 1440, 7104, "store"), (842, 5152, 3072, "add"), (481, 4688, 1088, "add")])
+@pytest.mark.parametrize("m,n,k,mode", [(684, 696, 11456, "add"), (780, 1440, 7104, "store"), (842, 5152, 3072, "add"), (481, 4688, 1408, "add")])
 def test_products_of_the_fixed_array_whose_parts_would_not_fit(ops, m, n, k, mode):
     lib = ops.lib
     pointer = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731

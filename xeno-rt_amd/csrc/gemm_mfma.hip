@@ -1266,13 +1266,17 @@ Cut cut_by_parts_time(int M, long rows_w, int K, int mode, bool whole_norm = fal
 // from 2 to 16 of each timed, 150000 times in all: of 2400 others what it chooses is 1.5 % off the best of all on average, where the estimates above, which know the tiles of 128
 // and, for k from 4096 on and 512 rows, of 256 rows, and of 192 as a rule of thumb, were 4.5 % off: 520 rows of x, 4096 rows of w, k = 14336 84 -> 67 us, 2048 rows, k = 8192 45 -> 34, 200 rows, 5120 rows, k = 25600
 // 97 -> 72, 1100 rows, 4096 rows, k = 4096 63 -> 51.
+// Two shapes are fitted anew to 2500 products where cut and uncut are near each other (k up to 5000), timed with w from memory, as a model's layers find it: uncut in tiles of
+// 128 x 128 (the last of WHOLE; adding, it was taken for 25 % dearer than it is) and 128 x 64 of a short k, alone on its compute unit (14 % dearer). By the figures before, adding
+// products of a short k went in two parts where the workgroups then shared compute units (300 rows of x, 4096 rows of w, k = 256 13.2 us, uncut 9.4; 788 rows, 2048, k = 768 17.1, uncut 14.6).
+// Of 700 products drawn whose cut is another than before the estimate none takes more than 1.01 of what it took then (by the figures before 20 took over 1.05), and all of them 0.75.
 enum { KIND_STORE, KIND_NORMED, KIND_ADD };
 struct TileCost { double step, share, beside, part, bytes, again, sums, once[3], outs[3]; };
 struct CutShape { int rows, columns, places; TileCost cost; };
 constexpr CutShape CUT_128_BY_64 = {128, 64, 2, {0.295, 0.101, 0.149, 0.174, 0.203, 0.075, 1.385, {6.003, 6.308, 6.525}, {0.075, 1.864, 0.000}}},
                    // (at most one to a compute unit: four stages; of a short k eight wavefronts)
                    CUT_128_BY_64_ALONE = {128, 64, 2, {0.329, 0.000, 0.000, 0.219, 0.198, 0.185, 1.762, {5.174, 5.018, 5.524}, {0.169, 3.266, 0.312}}},
-                   CUT_128_BY_64_SHORT = {128, 64, 2, {0.242, 0.039, 0.000, 0.161, 0.165, 0.389, 1.681, {5.474, 5.756, 5.851}, {0.632, 2.781, 0.367}}},
+                   CUT_128_BY_64_SHORT = {128, 64, 2, {0.276, 0.012, 0.000, 0.233, 0.165, 0.389, 1.754, {4.364, 5.403, 4.433}, {1.168, 2.526, 1.469}}},
                    CUT_128_BY_128 = {128, 128, 2, {0.706, 0.122, 0.003, 0.147, 0.314, 0.105, 1.035, {6.869, 7.672, 6.806}, {0.169, 1.672, 0.754}}},
                    CUT_128_BY_128_THREE_STAGES = {128, 128, 1, {0.543, 0.000, 0.000, 0.204, 0.162, 0.161, 1.942, {5.855, 6.164, 5.901}, {0.694, 0.947, 0.788}}},
                    CUT_192 = {192, 256, 1, {0.759, 0.209, 0.000, 0.093, 0.165, 0.646, 0.850, {12.673, 13.490, 12.186}, {0.052, 1.386, 0.922}}},
@@ -1280,7 +1284,7 @@ constexpr CutShape CUT_128_BY_64 = {128, 64, 2, {0.295, 0.101, 0.149, 0.174, 0.2
                    WHOLE[] = {{256, 256, 1, {0.842, 0.410, 0.000, 0.000, 0.001, 0.196, 0.000, {7.279, 26.096, 21.168}, {0.429, 1.205, 0.632}}},
                               {192, 256, 1, {0.763, 0.224, 0.000, 0.000, 0.372, 0.000, 0.000, {5.708, 18.654, 14.700}, {0.527, 1.509, 0.977}}},
                               {128, 256, 1, {0.676, 0.106, 0.000, 0.000, 0.377, 0.000, 0.000, {4.336, 13.687, 9.568}, {0.572, 1.724, 1.275}}},
-                              {128, 128, 2, {0.712, 0.100, 0.039, 0.000, 0.434, 0.106, 0.000, {7.934, 9.724, 8.980}, {0.000, 1.506, 0.346}}}};
+                              {128, 128, 2, {0.592, 0.272, 0.000, 0.000, 0.457, 0.163, 0.000, {7.491, 8.395, 6.122}, {0.020, 2.493, 0.649}}}};
 double cut_time(const CutShape& shape, int M, int N, int K, int steps, int parts, int kind) {
     const TileCost& c = shape.cost;
     const long tiles = (long)((M + shape.rows - 1) / shape.rows) * ((N + shape.columns - 1) / shape.columns);
@@ -1353,8 +1357,12 @@ SplitPlan plan_of(int M, int N, int K, int mode, bool whole_norm, bool fixed) {
             const double time = few_rows_cut_time(M, N, K, per_part(parts), parts);
             if (time < best) { best = time; splits = parts; }
         }
-    } else if (mode == MODE_GATED || fixed) {
-        const Cut cut = cut_by_parts_time(M, rows_w, K, mode);
+    } else if (mode == MODE_GATED || fixed || M > (N < 1024 ? 2100 : 4608) || N > 16384) {
+        // Gated products, and others where the estimate below is not good for more rows or columns than it was fitted to. Drawn products whose cut it changes: of 185 with more
+        // than 16384 rows of w 24 took over 1.05 of the time by it (74 rows of x, 25600, k = 1024 22.5 -> 26.0 us), of 103 with more than 4608 rows of x 12 (5500 rows,
+        // 1024, k = 3072 46 -> 50), of 230 with more than 2100 and fewer than 1024 of w 17 (3763 rows, 256, k = 7168 27.6 -> 36.9). Within the line: 2100 to 4608 rows 3 of 359, and
+        // 0.91 on average (2600 rows, 2048, k = 8192 92 -> 84; 4300 rows, 1024, k = 3072 45 -> 43); k below 256 or above 25600 none of 223, 0.71; fewer than 256 rows of w 1 of 240, 0.55.
+        const Cut cut = cut_by_parts_time(M, rows_w, K, mode, whole_norm);
         splits = cut.splits;
         tile = cut.tile;
         columns = cut.columns;
