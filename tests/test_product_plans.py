@@ -49,7 +49,7 @@ def test_float32_products_of_a_short_k_take_the_tile_that_ends_soonest(lib, m, n
 # Products that are not gated, more than 64 rows: uncut where two parts take longer (the ends of an adding product's tiles are cheaper than a second kernel when k is short), and
 # by the rule for tiles of 128 and 256 rows where there are more rows of x or of w than the finer estimate was fitted to.
 @pytest.mark.parametrize("m,n,k,mode,parts", [
-    (300, 4096, 256, "add", 1), (597, 1536, 256, "add", 1), (863, 1344, 512, "add", 1), (96, 10240, 256, "add", 1), (788, 2048, 768, "add", 1), (152, 5248, 128, "add", 1), (188, 2288, 256, "add", 2),
+    (300, 4096, 256, "add", 1), (597, 1536, 256, "add", 1), (863, 1344, 512, "add", 1), (96, 10240, 256, "add", 1), (788, 2048, 768, "add", 1), (152, 5248, 128, "add", 1), (188, 2288, 256, "add", 2), (241, 1040, 24320, "store", 7),
     (74, 25600, 1024, "add", 1), (79, 28672, 768, "add", 1), (5300, 1024, 3072, "add", 1), (3763, 256, 7168, "add", 4), (3522, 256, 3072, "store", 2), (2932, 128, 2496, "store", 3),
     (2600, 2048, 8192, "add", 2), (4300, 1024, 3072, "add", 2), (4700, 1024, 2624, "add", 1), (100, 2048, 2048, "add", 4), (333, 4096, 14336, "add", 8)])
 def test_products_that_are_cut_along_k_and_those_that_are_not(lib, m, n, k, mode, parts):

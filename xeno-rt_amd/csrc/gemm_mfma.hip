@@ -1285,6 +1285,12 @@ constexpr CutShape CUT_128_BY_64 = {128, 64, 2, {0.295, 0.101, 0.149, 0.174, 0.2
                               {192, 256, 1, {0.763, 0.224, 0.000, 0.000, 0.372, 0.000, 0.000, {5.708, 18.654, 14.700}, {0.527, 1.509, 0.977}}},
                               {128, 256, 1, {0.676, 0.106, 0.000, 0.000, 0.377, 0.000, 0.000, {4.336, 13.687, 9.568}, {0.572, 1.724, 1.275}}},
                               {128, 128, 2, {0.592, 0.272, 0.000, 0.000, 0.457, 0.163, 0.000, {7.491, 8.395, 6.122}, {0.020, 2.493, 0.649}}}};
+// Whether the parts of tiles of 128 x 64 have a compute unit each, as they are dealt: four stages then (counted as dealt by columns, 39 tiles in six parts had none left: 150 x 2664, k = 5504
+// 19.5 -> 16.9 us, 98 x 5320, k = 6464 23.7 -> 22.2; 150 such products drawn 0.93 of their time, the worst 1.01).
+bool narrow_alone(int M, long rows_w, int K, int parts) {
+    const long tiles = (long)((M + 127) / 128) * ((rows_w + 63) / 64);
+    return part_ids(tiles, parts, deals_by_parts(64, tiles, K, parts)) <= XRT_COMPUTE_UNITS;
+}
 double cut_time(const CutShape& shape, int M, int N, int K, int steps, int parts, int kind) {
     const TileCost& c = shape.cost;
     const long tiles = (long)((M + shape.rows - 1) / shape.rows) * ((N + shape.columns - 1) / shape.columns);
@@ -1372,7 +1378,7 @@ SplitPlan plan_of(int M, int N, int K, int mode, bool whole_norm, bool fixed) {
         const int kind = mode == MODE_STORE ? KIND_STORE : whole_norm ? KIND_NORMED : KIND_ADD;
         auto time_of = [&](int rows, int wide, int parts) {
             const CutShape& shape = rows == 256 ? CUT_256 : rows == 192 ? CUT_192 : wide == 128 ? (M <= 256 ? CUT_128_BY_128_THREE_STAGES : CUT_128_BY_128)
-                : dealt((long)((M + 127) / 128) * ((N + 63) / 64)) * parts > XRT_COMPUTE_UNITS ? CUT_128_BY_64 : K < 4096 ? CUT_128_BY_64_SHORT : CUT_128_BY_64_ALONE;
+                : !narrow_alone(M, N, K, parts) ? CUT_128_BY_64 : K < 4096 ? CUT_128_BY_64_SHORT : CUT_128_BY_64_ALONE;
             return cut_time(shape, M, N, K, per_part(parts), parts, kind);
         };
         double whole = 1e30;
@@ -1698,8 +1704,7 @@ int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, b
     if (plan.columns == 64) {
         // a fourth stage where a compute unit has one workgroup anyway (2048 rows of w, k = 8192, 65 / 200 rows of x 16.0 / 22.5 -> 14.7 / 20.5 us with its
         // second kernel; k = 2048, 3072 rows, 100 rows of x 12.0 -> 11.5)
-        if (dealt((long)((M + 127) / 128) * ((rows_w + 63) / 64)) * plan.splits <= XRT_COMPUTE_UNITS)
-        {
+        if (narrow_alone(M, rows_w, K, plan.splits)) {
             // eight wavefronts where k is short (2048 rows of w, k = 2048, 72 / 160 rows of x 11.1 / 13.0 -> 10.6 / 12.7 us with its second kernel, 3072 rows 12.9 / 14.9 -> 12.4 / 14.4;
             // 4096 rows, k = 4096, 72 / 100 rows 16.6 / 17.6 in four, 17.3 / 18.6 in eight)
             if (K < 4096) return launch_kernel<128, 64, 4, 2, MODE_STORE, 64, 4, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
