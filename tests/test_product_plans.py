@@ -55,3 +55,23 @@ def test_float32_products_of_a_short_k_take_the_tile_that_ends_soonest(lib, m, n
 def test_products_that_are_cut_along_k_and_those_that_are_not(lib, m, n, k, mode, parts):
     rows, columns = ctypes.c_int(), ctypes.c_int()
     assert lib.xrt_linear_parts(m, n, k, MODES[mode], 0, ctypes.byref(rows), ctypes.byref(columns)) == parts
+
+
+# Every tile of every part is taken by one workgroup and no other, whichever way they are dealt to the eight dies (workgroup i runs on die i % 8); by parts, no die has more than
+# its share. By parts: tiles of 256 rows of w from k = 2112 on, narrower ones from k = 6208 on, and any that make a round less so.
+@pytest.mark.parametrize("m,n,k,mode,by_parts", [
+    (40, 4096, 4096, "add", 0), (61, 4096, 14336, "add", 1), (24, 2816, 2048, "store", 1), (64, 1000, 5248, "gated", 0), (100, 2048, 2048, "add", 0), (65, 3072, 1024, "store", 0),
+    (333, 4096, 14336, "add", 1), (333, 4096, 4096, "add", 0), (257, 2048, 14336, "store", 1), (778, 2048, 8192, "store", 1), (300, 12320, 2048, "add", 0), (150, 2664, 5504, "add", 1), (241, 1040, 24320, "store", 1), (520, 2048, 8192, "store", 1), (1100, 4096, 8192, "store", 1),
+    (199, 8200, 4096, "store", 1), (333, 6144, 4096, "store", 0), (700, 1000, 8192, "gated", 1), (2000, 1024, 3072, "add", 0)])
+def test_every_tile_of_every_part_has_one_workgroup(lib, m, n, k, mode, by_parts):
+    rows, columns, dealt = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    parts = lib.xrt_linear_parts(m, n, k, MODES[mode], 0, ctypes.byref(rows), ctypes.byref(columns))
+    groups = lib.xrt_linear_part_order(m, n, k, MODES[mode], 0, ctypes.byref(dealt), None, 0)
+    places = (ctypes.c_int * groups)()
+    assert lib.xrt_linear_part_order(m, n, k, MODES[mode], 0, ctypes.byref(dealt), places, groups) == groups
+    assert dealt.value == by_parts
+    tiles = -(-m // rows.value) * -(-(2 * n if mode == "gated" else n) // columns.value)
+    assert sorted(place for place in places if place >= 0) == list(range(parts * tiles))
+    if by_parts:
+        assert groups < parts * tiles + 8
+        assert max(sum(place >= 0 for place in places[die::8]) for die in range(8)) == -(-parts * tiles // 8)

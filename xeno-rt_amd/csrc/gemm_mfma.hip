@@ -41,7 +41,7 @@ enum { MODE_STORE = 0, MODE_ACCUMULATE = 1, MODE_GATED = 2 };
 // tiles, and a run is walked n-fastest inside panels of 8 n-tiles, so that the tiles that run at one time on an XCD share a
 // and w in its L2. An id beyond the tiles (grids are whole rounds over the XCDs) has none: m is negative.
 struct TilePlace { int m, n; };
-__device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, int tiles_n) {
+__host__ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, int tiles_n) {
     const int total = tiles_m * tiles_n;
     const int xcds = 8;
     id = (id % xcds) * ((total + xcds - 1) / xcds) + id / xcds;
@@ -54,11 +54,11 @@ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, int tiles_n
 }
 
 // The same of a product whose k is split into parts, in one of two orders. By columns: an XCD gets a run of tiles and all parts of them, a grid row each. By parts
-// (by_parts: their number): it gets a run of tiles and parts, part after part, so that it reads some slices of k of a, which its L2
+// (by_parts: their number; else 0, and `row` is the workgroup's grid row): it gets a run of tiles and parts, part after part, so that it reads some slices of k of a, which its L2
 // holds, instead of all of a, and no XCD has more to do for a number of tiles that does not divide.
 struct PartPlace { TilePlace tile; int part; };
-__device__ __forceinline__ PartPlace part_place(int id, int tiles_m, int tiles_n, int by_parts) {
-    if (by_parts == 0) return PartPlace{tile_place(id, tiles_m, tiles_n), (int)blockIdx.y};
+__host__ __device__ __forceinline__ PartPlace part_place(int id, int row, int tiles_m, int tiles_n, int by_parts) {
+    if (by_parts == 0) return PartPlace{tile_place(id, tiles_m, tiles_n), row};
     constexpr int XCDS = 8;
     const int tiles = tiles_m * tiles_n, total = tiles * by_parts;
     id = (id % XCDS) * ((total + XCDS - 1) / XCDS) + id / XCDS;
@@ -91,7 +91,7 @@ __device__ __forceinline__ void gemm_tile(
     bf16* lds_b = lds_a + 2 * BM * PITCH;                              // [2][BN][PITCH]
 
     // (a float32 store may be of a part; of the others none is, and their way to the first loads is shorter)
-    const PartPlace of_part = MODE == MODE_STORE && sizeof(TO) == 4 ? part_place(id, tiles_m, tiles_n, by_parts) : PartPlace{tile_place(id, tiles_m, tiles_n), 0};
+    const PartPlace of_part = MODE == MODE_STORE && sizeof(TO) == 4 ? part_place(id, blockIdx.y, tiles_m, tiles_n, by_parts) : PartPlace{tile_place(id, tiles_m, tiles_n), 0};
     const TilePlace place = of_part.tile;
     if (place.m < 0) return;
     // (rows, columns and byte offsets fit 32 bits: the launcher checks)
@@ -891,7 +891,7 @@ template <int BM, int MODE, typename TO, bool PARTS>
 __global__ void __launch_bounds__(8 * XRT_WAVE) gemm_large_kernel(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
     int tiles_m, int tiles_n, int by_parts, int k_per_split, const Packing packing, int activation, int height) {
-    const PartPlace place = PARTS ? part_place(blockIdx.x, tiles_m, tiles_n, by_parts) : PartPlace{tile_place(blockIdx.x, tiles_m, tiles_n), 0};
+    const PartPlace place = PARTS ? part_place(blockIdx.x, blockIdx.y, tiles_m, tiles_n, by_parts) : PartPlace{tile_place(blockIdx.x, tiles_m, tiles_n), 0};
     if (place.tile.m < 0) return;
     gemm_large_tile<BM, MODE, TO>(a, w, out, M, N, K, place.tile, 0, place.part, k_per_split, packing, activation, height);
 }
@@ -1913,6 +1913,22 @@ extern "C" int xrt_linear_parts(int M, int N, int K, int mode, int whole_norm, i
     *rows = plan.tile;
     *columns = plan.columns;
     return plan.splits;
+}
+
+// The order in which the workgroups of a product cut along k take its tiles and parts.
+extern "C" int xrt_linear_part_order(int M, int N, int K, int mode, int whole_norm, int* by_parts, int* places, int room) {
+    int rows = 0, columns = 0;
+    const int parts = xrt_linear_parts(M, N, K, mode, whole_norm, &rows, &columns);
+    if (parts < 2 || !by_parts || (room > 0 && !places)) return -1;
+    const long tiles_m = (M + rows - 1) / rows, tiles_n = ((mode == MODE_GATED ? 2L * N : N) + columns - 1) / columns;
+    *by_parts = deals_by_parts(columns, tiles_m * tiles_n, K, parts);
+    const long groups = part_ids(tiles_m * tiles_n, parts, *by_parts), in_a_row = *by_parts ? groups : groups / parts;
+    if (groups >= (1L << 31)) return -1;
+    for (long i = 0; i < min(groups, (long)room); ++i) {
+        const PartPlace place = part_place((int)(i % in_a_row), (int)(i / in_a_row), (int)tiles_m, (int)tiles_n, *by_parts ? parts : 0);
+        places[i] = place.tile.m < 0 ? -1 : (int)(place.part * tiles_m * tiles_n + place.tile.m * tiles_n + place.tile.n);
+    }
+    return (int)groups;
 }
 
 // Whether a product of 17 to 256 rows of x asks for w past the caches (k a multiple of 64).

@@ -130,6 +130,9 @@ long xrt_linear_whole_norm_workspace(const void* a, const void* w, int dtype, in
 // How a bfloat16 product of more than 16 rows and whole steps of 64 along k is cut along k: returns the number of parts (1: it is not; -1: not such a
 // product), and a tile's rows of x and of w. whole_norm: as one whose second kernel does the norm after it.
 int xrt_linear_parts(int M, int N, int K, int mode, int whole_norm, int* rows, int* columns);
+// The order of its workgroups: returns their number (-1: not cut), by_parts whether they take its tiles part after part, dealt to the dies in equal runs (otherwise a die takes a
+// run of tiles and all parts of them, a grid row each); places[i], for the first `room` of them: part * tiles + the tile's row of tiles * tiles in a row + its place there, or -1 (none).
+int xrt_linear_part_order(int M, int N, int K, int mode, int whole_norm, int* by_parts, int* places, int room);
 // The tiles of one that is not, more than 64 rows: 0, 1, 2: 256, 192 and 128 rows of x by 256 of w; 3: the first and the last of these in one launch; 4: 256 x 192; 5: 128 x 128;
 // 6: likewise in three stages; 7: 128 x 64 in four; 8, 9: 256 x 256 and 128 x 128 where k is no multiple of 64.
 int xrt_linear_tiles(int out_dtype, int M, int N, int K, int mode);
