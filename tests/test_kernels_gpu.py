@@ -591,8 +591,9 @@ def test_rmsnorm_done_by_the_second_kernel_of_a_product_of_many_rows(ops, m, hid
 
 @pytest.mark.parametrize("mode", ["gated", "store", "add"])
 def test_parts_along_k_make_one_round_on_every_die(ops, mode):
-    """Tiles are dealt to the eight dies in equal runs, the same in every part: what counts against a die's 32 compute units is its run times the parts. (With the
-    workgroups' number alone counted, 298 rows of x and 5328 of w went into six parts: 36 workgroups on seven dies, none on the eighth.)"""
+    """Parts of 192 rows are few enough for one round in either order of their workgroups. Dealt by columns, tiles come to the eight dies in equal runs, the same in every part, and a
+    die's run times the parts counts against its 32 compute units. (With the workgroups' number alone counted, 298 rows of x and 5328 of w went into six parts: 36 workgroups
+    on seven dies, none on the eighth.) Dealt by parts no die has more than that."""
     taken = 0
     for m in (150, 193, 224, 298, 333, 385, 409, 465, 500, 777):
         for rows_w in (1744, 2192, 4096, 5120, 5328, 6800, 7040, 9736, 10240, 10720):

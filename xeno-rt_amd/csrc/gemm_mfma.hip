@@ -53,9 +53,9 @@ __host__ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, in
     return TilePlace{in_panel / panel_width, panel * PANEL + in_panel % panel_width};
 }
 
-// The same of a product whose k is split into parts, in one of two orders. By columns: an XCD gets a run of tiles and all parts of them, a grid row each. By parts
-// (by_parts: their number; else 0, and `row` is the workgroup's grid row): it gets a run of tiles and parts, part after part, so that it reads some slices of k of a, which its L2
-// holds, instead of all of a, and no XCD has more to do for a number of tiles that does not divide.
+// The same of a product whose k is split into parts, in one of two orders. By columns: an XCD gets a run of tiles and all parts of them, a grid row each. By
+// parts (by_parts: their number; else 0, and `row` is the workgroup's grid row): it gets a run of tiles and parts, part after part, so that it reads some
+// slices of k of a, which its L2 holds, instead of all of a, and no XCD has more to do for a number of tiles that does not divide.
 struct PartPlace { TilePlace tile; int part; };
 __host__ __device__ __forceinline__ PartPlace part_place(int id, int row, int tiles_m, int tiles_n, int by_parts) {
     if (by_parts == 0) return PartPlace{tile_place(id, tiles_m, tiles_n), row};
@@ -570,8 +570,8 @@ constexpr int LARGE_BN = 256;
 //
 // height: the rows of a that a tile stands for, a multiple of 16 up to BM. The rows of a product are dealt to its tiles evenly (even_height), so that none has
 // more than it must: the first four wavefronts take half of the blocks of 16, or one more than the others, and a wavefront runs the loop that is made for its
-// number of blocks (all, one or two fewer). The chip's power bounds the loop, so that products left out are time: 333 rows in two tiles of 176 instead of 192 and 141, 28672 rows
-// of w in pairs, k = 4096 77.6 -> 73.9 us, 51200, k = 5120 194 -> 179; 400 rows (208 each) 221 -> 196.
+// number of blocks (all, one or two fewer). The chip's power bounds the loop, so that products left out are time: 333 rows in two tiles of 176 instead of 192
+// and 141, 28672 rows of w in pairs, k = 4096 77.6 -> 73.9 us, 51200, k = 5120 194 -> 179; 400 rows (208 each) 221 -> 196.
 template <int BM, int MODE, typename TO>
 __device__ __forceinline__ void gemm_large_tile(
     const bf16* __restrict__ a, const bf16* __restrict__ w, TO* __restrict__ out, int M, int N, int K,
@@ -1144,8 +1144,8 @@ int launch_mode(const bf16* a, const bf16* w, TO* out, int M, int N, int K, cons
             if constexpr (MODE == MODE_GATED) return launch_kernel<128, 64, 4, 1, MODE, 64, 4, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
             break;
         case TILES_128_BY_128_THREE_STAGES:
-            // (eight wavefronts: 66 such products drawn at random take 0.92 of what they take in four, the slowest 1.02; 14336 pairs, k = 4096, 100 rows 51.6 -> 50.1 us, 25600 pairs,
-            // k = 5120 121 -> 118)
+            // (eight wavefronts: 66 such products drawn at random take 0.92 of what they take in four, the slowest 1.02; 14336 pairs, k = 4096, 100 rows 51.6
+            // -> 50.1 us, 25600 pairs, k = 5120 121 -> 118)
             if constexpr (MODE == MODE_GATED) return launch_kernel<128, 128, 4, 2, MODE, 64, 3, TO>(a, w, out, M, N, K, packing, s, 1, 0, plain);
             break;
         case TILES_256: return launch_large<256, MODE, TO>(a, w, out, M, N, K, packing, activation, s);
@@ -1196,15 +1196,18 @@ constexpr int SPLIT_BM = 64, SPLIT_BN = 128;
 
 struct SplitPlan { int splits, k_per_split; long rows_w; int tile, columns; };      // tile: rows of x per tile (64, 128, 192 or 256), columns: rows of w
 
-// What a product of some hundred rows of x takes (nanoseconds) in parts along k, if it is gated (of others: the plan of few parts, and what the estimate below has to beat): tiles of 128 rows of x and `columns` rows of w, `places` of them to a compute
-// unit. A step of 64 along k takes `step`, `share` more for each tile that a compute unit has on average, and `beside` more where some have two; `once` is
-// start, end and the second kernel's start, `part` what a further part costs it, `sums` what a million partial sums cost to write and to read again. (Fitted to products of
-// every kind, 512 to 8192 rows of w, k from 512 to 14336, 65 to 1700 rows of x; of 2686 gated products drawn at random afterwards what it chooses is 0.9 % off the best of 27 on average.)
-// Workgroups are counted as the fullest die has them: counting their number alone put two rounds on seven of the eight dies where the tiles are no multiple of
-// eight (298 rows of x, 5328 rows of w in pairs, k = 9664: 77 us, 55 by the rule before this estimate).
+// What a product of some hundred rows of x takes (nanoseconds) in parts along k, if it is gated (of others: the plan of few parts, and what the estimate
+// below has to beat): tiles of 128 rows of x and `columns` rows of w, `places` of them to a compute unit. A step of 64 along k takes `step`, `share` more
+// for each tile that a compute unit has on average, and `beside` more where some have two; `once` is start, end and the second kernel's start, `part` what a
+// further part costs it, `sums` what a million partial sums cost to write and to read again. (Fitted to products of every kind, 512 to 8192 rows of w, k
+// from 512 to 14336, 65 to 1700 rows of x; of 2686 gated products drawn at random afterwards what it chooses is 0.9 % off the best of 27 on average.)
+// Workgroups are counted as the fullest die has them when they are dealt by columns, as all were when this was fitted: their number alone put two rounds on
+// seven of the eight dies where the tiles are no multiple of eight (298 rows of x, 5328 rows of w in pairs, k = 9664: 77 us, 55 by the rule before this
+// estimate). Dealt by parts they would make one now, and are still charged two. Charged as they are dealt, with the figures as they are, 300 gated products
+// whose cut that changes took 0.99 of their time, but 85 of them over 1.05 (up to 1.21: tiles of 128 where parts of 192 rows are better), so it stays.
 struct PartTime { int columns, places, once, step, share, beside, part, sums; };
 constexpr int DIES = 8;
-// Tiles are dealt to the dies in equal runs (tile_place): what the largest run comes to on all of them.
+// Tiles dealt to the dies by columns come in equal runs, the same in every part: what the largest run comes to on all of them.
 long dealt(long tiles) { return (tiles + DIES - 1) / DIES * DIES; }
 constexpr PartTime NARROW_PARTS = {64, 2, 5950, 256, 166, 95, 250, 1540}, WIDE_PARTS = {128, 1, 6630, 445, 200, 0, 251, 1720},
                    WIDE_PARTS_TWO = {128, 2, 7190, 592, 237, 0, 268, 1050};          // (two stages instead of three: two to a compute unit, beyond 256 rows)
@@ -1228,8 +1231,9 @@ long unsplit_time(int M, long rows_w, int K, int mode) {
     return 1000 + (mode == MODE_GATED ? least : least * 127 / 100);
 }
 struct Cut { int splits, tile, columns; };
-// Tiles of 128 x 64 or 128 x 128 and the number of parts by the estimates, against the product without a split, which saves a gated one the sums of both halves. (Narrow tiles read x
-// twice as often, which does not stay in a die's L2 when k is long: 4096 rows of w, k = 14336, 100 rows of x 34.7 us in wide tiles, 40.3 in narrow ones.)
+// Tiles of 128 x 64 or 128 x 128 and the number of parts by the estimates, against the product without a split, which saves a gated one the sums of both
+// halves. (Narrow tiles read x twice as often, which does not stay in a die's L2 when k is long: 4096 rows of w, k = 14336, 100 rows of x 34.7 us in wide
+// tiles, 40.3 in narrow ones.)
 Cut cut_by_parts_time(int M, long rows_w, int K, int mode, bool whole_norm = false) {
     const int units = K / 64;
     auto per_part = [&](int parts) { return (units + parts - 1) / parts; };
@@ -1247,7 +1251,7 @@ Cut cut_by_parts_time(int M, long rows_w, int K, int mode, bool whole_norm = fal
             if (time < best) { best = time; cut = Cut{parts, 128, shape.columns}; }
         }
     }
-    // Large tiles of 192 rows, in parts that make one round: fewer operands read a product, more at the ends (150 rows of x, 10240 rows of w, k = 5120
+    // Large tiles of 192 rows, in parts that make one round in either order: fewer operands read a product, more at the ends (150 rows of x, 10240 rows of w, k = 5120
     // 43 -> 34 us beside the best of the others).
     const long large = dealt((long)((M + 191) / 192) * ((rows_w + 255) / 256));
     for (int parts = 2; M > 128 && parts <= 16 && parts * large <= XRT_COMPUTE_UNITS; ++parts) {
@@ -1258,18 +1262,20 @@ Cut cut_by_parts_time(int M, long rows_w, int K, int mode, bool whole_norm = fal
     return cut;
 }
 
-// What every other product of more than 64 rows of x takes, in microseconds, cut or not. A step of 64 along k takes `step`, `share` more for each workgroup that a compute unit has
-// on average (up to `places` of them side by side), and `beside` where some have two; reading w, and `again` of what is read of x on all dies (on one, where
-// the parts are dealt so), takes `bytes` a megabyte; the larger of the two counts, smoothly. `part` and `sums` are what a part and a million partial sums cost the second kernel and the first;
-// once and outs (a million results) go by what the product does: store, add with the norm behind it (cut: in the second kernel; not cut: a kernel of its own), add.
-// Fitted to 8000 products (65 to 2100 rows of x, 256 to 16384 rows of w, k from 256 to 25600, half of them of widths that models have), every tile with every number of parts
-// from 2 to 16 of each timed, 150000 times in all: of 2400 others what it chooses is 1.5 % off the best of all on average, where the estimates above, which know the tiles of 128
-// and, for k from 4096 on and 512 rows, of 256 rows, and of 192 as a rule of thumb, were 4.5 % off: 520 rows of x, 4096 rows of w, k = 14336 84 -> 67 us, 2048 rows, k = 8192 45 -> 34, 200 rows, 5120 rows, k = 25600
-// 97 -> 72, 1100 rows, 4096 rows, k = 4096 63 -> 51.
-// Two shapes are fitted anew to 2500 products where cut and uncut are near each other (k up to 5000), timed with w from memory, as a model's layers find it: uncut in tiles of
-// 128 x 128 (the last of WHOLE; adding, it was taken for 25 % dearer than it is) and 128 x 64 of a short k, alone on its compute unit (14 % dearer). By the figures before, adding
-// products of a short k went in two parts where the workgroups then shared compute units (300 rows of x, 4096 rows of w, k = 256 13.2 us, uncut 9.4; 788 rows, 2048, k = 768 17.1, uncut 14.6).
-// Of 700 products drawn whose cut is another than before the estimate none takes more than 1.01 of what it took then (by the figures before 20 took over 1.05), and all of them 0.75.
+// What every other product of more than 64 rows of x takes, in microseconds, cut or not. A step of 64 along k takes `step`, `share` more for each workgroup
+// that a compute unit has on average (up to `places` of them side by side), and `beside` where some have two; reading w, and `again` of what is read of x on
+// all dies (on one, where the parts are dealt so), takes `bytes` a megabyte; the larger of the two counts, smoothly. `part` and `sums` are what a part and a
+// million partial sums cost the second kernel and the first; once and outs (a million results) go by what the product does: store, add with the norm behind
+// it (cut: in the second kernel; not cut: a kernel of its own), add.
+// Fitted to 8000 products (65 to 2100 rows of x, 256 to 16384 rows of w, k from 256 to 25600, half of them of widths that models have), every tile with
+// every number of parts from 2 to 16 of each timed, 150000 times in all: of 2400 others what it chooses is 1.5 % off the best of all on average, where the
+// estimates above, which know the tiles of 128 and, for k from 4096 on and 512 rows, of 256 rows, and of 192 as a rule of thumb, were 4.5 % off: 520 rows of
+// x, 4096 rows of w, k = 14336 84 -> 67 us, 2048 rows, k = 8192 45 -> 34, 200 rows, 5120 rows, k = 25600 97 -> 72, 1100 rows, 4096 rows, k = 4096 63 -> 51.
+// Two shapes are fitted anew to 2500 products where cut and uncut are near each other (k up to 5000), timed with w from memory, as a model's layers find it:
+// uncut in tiles of 128 x 128 (the last of WHOLE; adding, it was taken for 25 % dearer than it is) and 128 x 64 of a short k, alone on its compute unit (14
+// % dearer). By the figures before, adding products of a short k went in two parts where the workgroups then shared compute units (300 rows of x, 4096 rows
+// of w, k = 256 13.2 us, uncut 9.4; 788 rows, 2048, k = 768 17.1, uncut 14.6). Of 700 products drawn whose cut is another than before the estimate none
+// takes more than 1.01 of what it took then (by the figures before 20 took over 1.05), and all of them 0.75.
 enum { KIND_STORE, KIND_NORMED, KIND_ADD };
 struct TileCost { double step, share, beside, part, bytes, again, sums, once[3], outs[3]; };
 struct CutShape { int rows, columns, places; TileCost cost; };
@@ -1285,8 +1291,8 @@ constexpr CutShape CUT_128_BY_64 = {128, 64, 2, {0.295, 0.101, 0.149, 0.174, 0.2
                               {192, 256, 1, {0.763, 0.224, 0.000, 0.000, 0.372, 0.000, 0.000, {5.708, 18.654, 14.700}, {0.527, 1.509, 0.977}}},
                               {128, 256, 1, {0.676, 0.106, 0.000, 0.000, 0.377, 0.000, 0.000, {4.336, 13.687, 9.568}, {0.572, 1.724, 1.275}}},
                               {128, 128, 2, {0.592, 0.272, 0.000, 0.000, 0.457, 0.163, 0.000, {7.491, 8.395, 6.122}, {0.020, 2.493, 0.649}}}};
-// Whether the parts of tiles of 128 x 64 have a compute unit each, as they are dealt: four stages then (counted as dealt by columns, 39 tiles in six parts had none left: 150 x 2664, k = 5504
-// 19.5 -> 16.9 us, 98 x 5320, k = 6464 23.7 -> 22.2; 150 such products drawn 0.93 of their time, the worst 1.01).
+// Whether the parts of tiles of 128 x 64 have a compute unit each, as they are dealt: four stages then (counted as dealt by columns, 39 tiles in six parts had
+// none left: 150 x 2664, k = 5504 19.5 -> 16.9 us, 98 x 5320, k = 6464 23.7 -> 22.2; 150 such products drawn 0.93 of their time, the worst 1.01).
 bool narrow_alone(int M, long rows_w, int K, int parts) {
     const long tiles = (long)((M + 127) / 128) * ((rows_w + 63) / 64);
     return part_ids(tiles, parts, deals_by_parts(64, tiles, K, parts)) <= XRT_COMPUTE_UNITS;
@@ -1305,11 +1311,12 @@ double cut_time(const CutShape& shape, int M, int N, int K, int steps, int parts
     return c.once[kind] + c.part * parts + sqrt(sqrt(loop2 * loop2 + memory2 * memory2)) + (parts > 1 ? c.sums * parts * results : 0.) + c.outs[kind] * results;
 }
 
-// Gated products of 17 to 64 rows of x (nanoseconds): unsplit in one round of tiles of 64 x 64, every workgroup all of k, or in parts of 64 x 128 as many as the compute units
-// take, and a second kernel. A step of 64 along k takes its time however few the tiles, so a long k with few of them wants parts (64 rows of x, 1408 rows of w, k = 4096 20.4 us unsplit,
-// 13.2 in parts; 512 rows, k = 8192 36.4, 12.4; 10240 rows, k = 3072 21.2, 20.1) and a short one none (6144 rows of w, k = 1024, 24 rows of x 8.4 us, 10.1 in parts; 16384 rows, k = 2048, 64 rows
-// 17.7, 21.0). Fitted to 3841 products drawn at random (128 to 16384 rows of w, k of 128 to 16384, 17 to 64 rows of x, a third of them of widths that are multiples of 256): what the
-// estimates choose is 0.1 % off the better of the two on average and takes 0.91 of what parts alone do, 34 above 1.03, up to 1.17.
+// Gated products of 17 to 64 rows of x (nanoseconds): unsplit in one round of tiles of 64 x 64, every workgroup all of k, or in parts of 64 x 128 as many as
+// the compute units take, and a second kernel. A step of 64 along k takes its time however few the tiles, so a long k with few of them wants parts (64 rows of
+// x, 1408 rows of w, k = 4096 20.4 us unsplit, 13.2 in parts; 512 rows, k = 8192 36.4, 12.4; 10240 rows, k = 3072 21.2, 20.1) and a short one none (6144 rows
+// of w, k = 1024, 24 rows of x 8.4 us, 10.1 in parts; 16384 rows, k = 2048, 64 rows 17.7, 21.0). Fitted to 3841 products drawn at random (128 to 16384 rows of
+// w, k of 128 to 16384, 17 to 64 rows of x, a third of them of widths that are multiples of 256): what the estimates choose is 0.1 % off the better of the two
+// on average and takes 0.91 of what parts alone do, 34 above 1.03, up to 1.17.
 long narrow_gated_time(int M, long rows_w, int units) {
     const long share = dealt((rows_w + 63) / 64);              // (of the compute units; at most all of them)
     return 3970 + units * (243 + (77 * 64 + 33 * M) * share / (64 * XRT_COMPUTE_UNITS)) + 2510 * (M * rows_w / 1000) / 1000;
@@ -1319,9 +1326,9 @@ long few_rows_parts_time(int M, long rows_w, int per, int parts) {
     return 5330 + 94 * parts + per * (328 + 318 * groups / XRT_COMPUTE_UNITS + (groups > XRT_COMPUTE_UNITS ? 250 : 0)) + 2490 * parts * (M * rows_w / 1000) / 1000;
 }
 
-// Products of 17 to 64 rows of x that are not gated, in tiles of 64 x 128 and `parts` parts: microseconds, as above. Fitted to 6500 products (256 to 16384 rows of w, k from 256 to 20000); of 2700 others
-// the choice by it is 0.9 % off the best number of parts and takes 0.977 of as many parts as leave every compute unit one workgroup (61 rows, 4096 rows of w, k = 1024
-// 12.2 -> 10.4 us, 3072 rows, k = 2048 12.2 -> 11.9; 34 of them more than 1.04, up to 1.11).
+// Products of 17 to 64 rows of x that are not gated, in tiles of 64 x 128 and `parts` parts: microseconds, as above. Fitted to 6500 products (256 to 16384 rows
+// of w, k from 256 to 20000); of 2700 others the choice by it is 0.9 % off the best number of parts and takes 0.977 of as many parts as leave every compute
+// unit one workgroup (61 rows, 4096 rows of w, k = 1024 12.2 -> 10.4 us, 3072 rows, k = 2048 12.2 -> 11.9; 34 of them more than 1.04, up to 1.11).
 double few_rows_cut_time(int M, int N, int K, int steps, int parts) {
     const long tiles = (N + SPLIT_BN - 1) / SPLIT_BN;
     const long groups = part_ids(tiles, parts, deals_by_parts(SPLIT_BN, tiles, K, parts));
@@ -1364,10 +1371,11 @@ SplitPlan plan_of(int M, int N, int K, int mode, bool whole_norm, bool fixed) {
             if (time < best) { best = time; splits = parts; }
         }
     } else if (mode == MODE_GATED || fixed || M > (N < 1024 ? 2100 : 4608) || N > 16384) {
-        // Gated products, and others where the estimate below is not good for more rows or columns than it was fitted to. Drawn products whose cut it changes: of 185 with more
-        // than 16384 rows of w 24 took over 1.05 of the time by it (74 rows of x, 25600, k = 1024 22.5 -> 26.0 us), of 103 with more than 4608 rows of x 12 (5500 rows,
-        // 1024, k = 3072 46 -> 50), of 230 with more than 2100 and fewer than 1024 of w 17 (3763 rows, 256, k = 7168 27.6 -> 36.9). Within the line: 2100 to 4608 rows 3 of 359, and
-        // 0.91 on average (2600 rows, 2048, k = 8192 92 -> 84; 4300 rows, 1024, k = 3072 45 -> 43); k below 256 or above 25600 none of 223, 0.71; fewer than 256 rows of w 1 of 240, 0.55.
+        // Gated products, and others where the estimate below is not good for more rows or columns than it was fitted to. Drawn products whose cut it changes:
+        // of 185 with more than 16384 rows of w 24 took over 1.05 of the time by it (74 rows of x, 25600, k = 1024 22.5 -> 26.0 us), of 103 with more than 4608
+        // rows of x 12 (5500 rows, 1024, k = 3072 46 -> 50), of 230 with more than 2100 and fewer than 1024 of w 17 (3763 rows, 256, k = 7168 27.6 -> 36.9).
+        // Within the line: 2100 to 4608 rows 3 of 359, and 0.91 on average (2600 rows, 2048, k = 8192 92 -> 84; 4300 rows, 1024, k = 3072 45 -> 43); k below
+        // 256 or above 25600 none of 223, 0.71; fewer than 256 rows of w 1 of 240, 0.55.
         const Cut cut = cut_by_parts_time(M, rows_w, K, mode, whole_norm);
         splits = cut.splits;
         tile = cut.tile;
@@ -1681,10 +1689,10 @@ __global__ void __launch_bounds__(256) split_reduce_qkv_kernel(const float* __re
     }
 }
 
-// Parts of up to 64 rows of x: w past the caches where it cannot stay in them and k is long, which makes the runs of the parts long again. Ungated, so long a k is a feed-forward's
-// width, and the matrix back from it counts three times: the gated one of twice its size stands beside it. (700 products drawn at random, past the caches against through them:
-// such a w 0.97, 5120 rows, k = 25600, 32 rows of x 48.6 against 52.9 us; as large and k of 4096 to 16384 0.99, up to 1.08 with more than 48 rows of x; smaller and among
-// more than the caches hold 0.97 to 1.04, 60 MB of them in turn 1.03 to 1.25.)
+// Parts of up to 64 rows of x: w past the caches where it cannot stay in them and k is long, which makes the runs of the parts long again. Ungated, so long a k
+// is a feed-forward's width, and the matrix back from it counts three times: the gated one of twice its size stands beside it. (700 products drawn at random,
+// past the caches against through them: such a w 0.97, 5120 rows, k = 25600, 32 rows of x 48.6 against 52.9 us; as large and k of 4096 to 16384 0.99, up to
+// 1.08 with more than 48 rows of x; smaller and among more than the caches hold 0.97 to 1.04, 60 MB of them in turn 1.03 to 1.25.)
 bool parts_read_past_caches(long rows_w, int K, bool gated) { return K >= 16384 && cannot_stay(rows_w, K, gated ? 3 : 6); }
 
 // The product of all rows of w, ungated, into the workspace: [splits][M][rows_w]
@@ -1705,8 +1713,8 @@ int launch_parts(const bf16* a, const bf16* w, float* workspace, int M, int K, b
         // a fourth stage where a compute unit has one workgroup anyway (2048 rows of w, k = 8192, 65 / 200 rows of x 16.0 / 22.5 -> 14.7 / 20.5 us with its
         // second kernel; k = 2048, 3072 rows, 100 rows of x 12.0 -> 11.5)
         if (narrow_alone(M, rows_w, K, plan.splits)) {
-            // eight wavefronts where k is short (2048 rows of w, k = 2048, 72 / 160 rows of x 11.1 / 13.0 -> 10.6 / 12.7 us with its second kernel, 3072 rows 12.9 / 14.9 -> 12.4 / 14.4;
-            // 4096 rows, k = 4096, 72 / 100 rows 16.6 / 17.6 in four, 17.3 / 18.6 in eight)
+            // eight wavefronts where k is short (2048 rows of w, k = 2048, 72 / 160 rows of x 11.1 / 13.0 -> 10.6 / 12.7 us with its second kernel, 3072 rows
+            // 12.9 / 14.9 -> 12.4 / 14.4; 4096 rows, k = 4096, 72 / 100 rows 16.6 / 17.6 in four, 17.3 / 18.6 in eight)
             if (K < 4096) return launch_kernel<128, 64, 4, 2, MODE_STORE, 64, 4, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
             return launch_kernel<128, 64, 4, 1, MODE_STORE, 64, 4, float>(a, w, workspace, M, rows_w, K, packing, s, plan.splits, plan.k_per_split);
         }

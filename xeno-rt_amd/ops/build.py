@@ -21,8 +21,9 @@ CSRC = os.path.join(os.path.dirname(HERE), "csrc")
 LIBRARY_NAME = "libxrt_hip.so"
 ARCH = "gfx950"
 # packed float32 arithmetic is switched off for all device code of this library
-# The first 64 bytes of a kernel's arguments come in registers that are filled before it starts: a chain of short kernels otherwise begins each one with a wait for them.
-# (16 layers of the Llama-3.2-1B sizes over 100 tokens 1247 -> 1226 us, decode of one sequence at the Qwen3-0.6B sizes 845 -> 841, of eight at the 8B sizes 831 -> 828.)
+# The first of a kernel's arguments come in registers that are filled before it starts: a chain of short kernels otherwise begins each one with a wait for them. At most 14 words of
+# 32 bits (16 registers, two of which hold the address of the others), and only those ahead of the first structure passed by value: products get 8 to 14, a kernel whose second
+# argument is a structure gets one pointer. (16 layers of the Llama-3.2-1B sizes over 100 tokens 1247 -> 1226 us; decode steps of one and of eight sequences within what two runs differ by.)
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-mllvm", "-amdgpu-kernarg-preload-count=16", "-Wno-unused-command-line-argument"]
