@@ -58,11 +58,13 @@ def test_products_that_are_cut_along_k_and_those_that_are_not(lib, m, n, k, mode
 
 
 # Every tile of every part is taken by one workgroup and no other, whichever way they are dealt to the eight dies (workgroup i runs on die i % 8); by parts, no die has more than
-# its share. By parts: tiles of 256 rows of w from k = 2112 on, narrower ones from k = 6208 on, and any that make a round less so.
+# its share. By parts: tiles of 256 rows of w from k = 2112 on, narrower ones from k = 6208 on, and any that make a round less so; narrower ones not where the rows of tiles are many,
+# except in 8 parts.
 @pytest.mark.parametrize("m,n,k,mode,by_parts", [
     (40, 4096, 4096, "add", 0), (61, 4096, 14336, "add", 1), (24, 2816, 2048, "store", 1), (64, 1000, 5248, "gated", 0), (100, 2048, 2048, "add", 0), (65, 3072, 1024, "store", 0),
     (333, 4096, 14336, "add", 1), (333, 4096, 4096, "add", 0), (257, 2048, 14336, "store", 1), (778, 2048, 8192, "store", 1), (300, 12320, 2048, "add", 0), (150, 2664, 5504, "add", 1), (241, 1040, 24320, "store", 1), (520, 2048, 8192, "store", 1), (1100, 4096, 8192, "store", 1),
-    (199, 8200, 4096, "store", 1), (333, 6144, 4096, "store", 0), (700, 1000, 8192, "gated", 1), (2000, 1024, 3072, "add", 0)])
+    (199, 8200, 4096, "store", 1), (333, 6144, 4096, "store", 0), (700, 1000, 8192, "gated", 1), (2000, 1024, 3072, "add", 0),
+    (4998, 336, 11904, "gated", 0), (4548, 144, 14976, "gated", 0), (2300, 64, 9024, "gated", 0), (1838, 88, 7040, "store", 1), (2450, 96, 15168, "gated", 1)])
 def test_every_tile_of_every_part_has_one_workgroup(lib, m, n, k, mode, by_parts):
     rows, columns, dealt = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
     parts = lib.xrt_linear_parts(m, n, k, MODES[mode], 0, ctypes.byref(rows), ctypes.byref(columns))

@@ -994,10 +994,14 @@ bool reads_past_caches(int rows_of_tile, int M, int N, int K, int mode) {
 // Whether the tiles and parts of a product are dealt by parts (part_place): where k is so long that reading all of a on every XCD costs (tiles of 256 rows
 // of w read it less often, and gain from k = 3072 on: 0.95 of the time by columns beyond k = 6144, 0.97 to 0.98 below; narrower ones 0.97 beyond k = 6144, and 1.01
 // below, where an XCD's parts touch the pages of all of w for little), and where it makes a round less (0.79 to 0.94 up to 64 rows of x).
-bool deals_by_parts(int columns, long tiles, int K, int parts) {
-    if (parts < 2) return false;
+// Not in narrower tiles where the rows of tiles are many, unless each XCD gets a part of its own (8 parts): several XCDs' runs of a part then go down all of a, whose slice their
+// L2 does not hold, for few columns, and by columns they read an eighth of it each. 1300 products drawn, both ways timed: tiles of 64 rows of w up to 12 rows of tiles 0.93 (none above
+// 1.05), beyond that 1.14 (up to 1.7); of 128 up to 16 rows 0.95 (2 above 1.05), beyond that 1.05 (up to 1.2: 4548 rows of x, 144 pairs, k = 14976 67 -> 80 us); with 8 parts 0.95
+// there too; of 256 0.96 throughout.
+bool deals_by_parts(int columns, long tiles_m, long tiles_n, int K, int parts) {
+    if (parts < 2 || (columns < 256 && tiles_m > (columns == 64 ? 12 : 16) && parts % 8 != 0)) return false;
     auto rounds = [](long groups) { return (groups + XRT_COMPUTE_UNITS - 1) / XRT_COMPUTE_UNITS; };
-    return K > (columns >= 256 ? 2048 : 6144) || rounds(part_ids(tiles, parts, false)) > rounds(part_ids(tiles, parts, true));
+    return K > (columns >= 256 ? 2048 : 6144) || rounds(part_ids(tiles_m * tiles_n, parts, false)) > rounds(part_ids(tiles_m * tiles_n, parts, true));
 }
 
 template <int BM, int BN, int WM, int WN, int MODE, int DK, int STAGES, typename TO, bool PAST_CACHES = false>
@@ -1019,7 +1023,7 @@ int launch_kernel(const bf16* a, const bf16* w, TO* out, int M, int N, int K, co
         configured = true;
     }
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;
-    const bool by_parts = deals_by_parts(BN, (long)tiles_m * tiles_n, K, splits);
+    const bool by_parts = deals_by_parts(BN, tiles_m, tiles_n, K, splits);
     const long ids = part_ids((long)tiles_m * tiles_n, by_parts ? splits : 1, by_parts);         // a whole number of rounds over the XCDs
     XRT_REQUIRE(ids < (1L << 31), "linear (mfma): %ld tiles", ids);
     XRT_REQUIRE(splits == 1 || DK != 0, "linear (mfma): only whole tiles along k can be split");
@@ -1051,7 +1055,7 @@ int launch_large(const bf16* a, const bf16* w, TO* out, int M, int N, int K, con
     }
     XRT_REQUIRE(K % 64 == 0 && (splits == 1 || (PARTS && k_per_split % 64 == 0)), "linear (mfma): the large tiles take whole steps of 64 along k (K=%d)", K);
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN_OUT - 1) / BN_OUT;
-    const bool by_parts = deals_by_parts(LARGE_BN, (long)tiles_m * tiles_n, K, splits);
+    const bool by_parts = deals_by_parts(LARGE_BN, tiles_m, tiles_n, K, splits);
     const long ids = part_ids((long)tiles_m * tiles_n, by_parts ? splits : 1, by_parts);         // a whole number of rounds over the XCDs
     XRT_REQUIRE(ids < (1L << 31), "linear (mfma): %ld tiles", ids);
     kernel<<<dim3((unsigned)ids, by_parts ? 1 : splits), 8 * XRT_WAVE, lds, s>>>(a, w, out, M, N, K, tiles_m, tiles_n, by_parts ? splits : 0, splits == 1 ? K : k_per_split,
@@ -1294,14 +1298,14 @@ constexpr CutShape CUT_128_BY_64 = {128, 64, 2, {0.295, 0.101, 0.149, 0.174, 0.2
 // Whether the parts of tiles of 128 x 64 have a compute unit each, as they are dealt: four stages then (counted as dealt by columns, 39 tiles in six parts had
 // none left: 150 x 2664, k = 5504 19.5 -> 16.9 us, 98 x 5320, k = 6464 23.7 -> 22.2; 150 such products drawn 0.93 of their time, the worst 1.01).
 bool narrow_alone(int M, long rows_w, int K, int parts) {
-    const long tiles = (long)((M + 127) / 128) * ((rows_w + 63) / 64);
-    return part_ids(tiles, parts, deals_by_parts(64, tiles, K, parts)) <= XRT_COMPUTE_UNITS;
+    const long tiles_m = (M + 127) / 128, tiles_n = (rows_w + 63) / 64;
+    return part_ids(tiles_m * tiles_n, parts, deals_by_parts(64, tiles_m, tiles_n, K, parts)) <= XRT_COMPUTE_UNITS;
 }
 double cut_time(const CutShape& shape, int M, int N, int K, int steps, int parts, int kind) {
     const TileCost& c = shape.cost;
-    const long tiles = (long)((M + shape.rows - 1) / shape.rows) * ((N + shape.columns - 1) / shape.columns);
-    const bool by_parts = deals_by_parts(shape.columns, tiles, K, parts);
-    const long groups = part_ids(tiles, parts, by_parts), places = (long)shape.places * XRT_COMPUTE_UNITS;
+    const long tiles_m = (M + shape.rows - 1) / shape.rows, tiles_n = (N + shape.columns - 1) / shape.columns;
+    const bool by_parts = deals_by_parts(shape.columns, tiles_m, tiles_n, K, parts);
+    const long groups = part_ids(tiles_m * tiles_n, parts, by_parts), places = (long)shape.places * XRT_COMPUTE_UNITS;
     const long whole = groups / places, rest = groups % places;
     const double full = c.step + c.share * shape.places + c.beside;
     const double last = rest == 0 ? 0. : c.step + c.share * rest / XRT_COMPUTE_UNITS + (rest > XRT_COMPUTE_UNITS ? c.beside : 0.);
@@ -1331,7 +1335,7 @@ long few_rows_parts_time(int M, long rows_w, int per, int parts) {
 // unit one workgroup (61 rows, 4096 rows of w, k = 1024 12.2 -> 10.4 us, 3072 rows, k = 2048 12.2 -> 11.9; 34 of them more than 1.04, up to 1.11).
 double few_rows_cut_time(int M, int N, int K, int steps, int parts) {
     const long tiles = (N + SPLIT_BN - 1) / SPLIT_BN;
-    const long groups = part_ids(tiles, parts, deals_by_parts(SPLIT_BN, tiles, K, parts));
+    const long groups = part_ids(tiles, parts, deals_by_parts(SPLIT_BN, 1, tiles, K, parts));
     constexpr double STEP = 0.367, SHARE = 0.292, BESIDE = 0.313;
     const long whole = groups / XRT_COMPUTE_UNITS, rest = groups % XRT_COMPUTE_UNITS;
     const double share = SHARE * rest / XRT_COMPUTE_UNITS;
@@ -1929,7 +1933,7 @@ extern "C" int xrt_linear_part_order(int M, int N, int K, int mode, int whole_no
     const int parts = xrt_linear_parts(M, N, K, mode, whole_norm, &rows, &columns);
     if (parts < 2 || !by_parts || (room > 0 && !places)) return -1;
     const long tiles_m = (M + rows - 1) / rows, tiles_n = ((mode == MODE_GATED ? 2L * N : N) + columns - 1) / columns;
-    *by_parts = deals_by_parts(columns, tiles_m * tiles_n, K, parts);
+    *by_parts = deals_by_parts(columns, tiles_m, tiles_n, K, parts);
     const long groups = part_ids(tiles_m * tiles_n, parts, *by_parts), in_a_row = *by_parts ? groups : groups / parts;
     if (groups >= (1L << 31)) return -1;
     for (long i = 0; i < min(groups, (long)room); ++i) {
