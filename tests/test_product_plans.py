@@ -77,3 +77,16 @@ def test_every_tile_of_every_part_has_one_workgroup(lib, m, n, k, mode, by_parts
     if by_parts:
         assert groups < parts * tiles + 8
         assert max(sum(place >= 0 for place in places[die::8]) for die in range(8)) == -(-parts * tiles // 8)
+
+
+# The same of products that are not cut. Side by side on a die (workgroups i, i + 8, ..): tiles of one column where there are up to four rows of them, of one row in panels of
+# eight otherwise, and wherever k is no multiple of 64.
+@pytest.mark.parametrize("tiles_m,tiles_n,k,down", [(3, 96, 4096, True), (3, 96, 4128, False), (4, 50, 64, True), (4, 50, 72, False), (5, 40, 4096, False), (1, 300, 4100, True),
+                                                    (2, 7, 320, True), (40, 6, 2048, False), (9, 13, 100, False)])
+def test_every_tile_has_one_workgroup(lib, tiles_m, tiles_n, k, down):
+    groups = lib.xrt_linear_tile_order(tiles_m, tiles_n, k, None, 0)
+    places = (ctypes.c_int * groups)()
+    assert lib.xrt_linear_tile_order(tiles_m, tiles_n, k, places, groups) == groups
+    assert groups < tiles_m * tiles_n + 8 and sorted(place for place in places if place >= 0) == list(range(tiles_m * tiles_n))
+    first, second = places[0], places[8]
+    assert second - first == (1 if tiles_m == 1 or not down else tiles_n)

@@ -39,14 +39,16 @@ enum { MODE_STORE = 0, MODE_ACCUMULATE = 1, MODE_GATED = 2 };
 
 // Which tile of tiles_m x tiles_n a workgroup takes. Ids are dealt to the XCDs round-robin: each XCD gets a contiguous run of
 // tiles, and a run is walked n-fastest inside panels of 8 n-tiles, so that the tiles that run at one time on an XCD share a
-// and w in its L2. An id beyond the tiles (grids are whole rounds over the XCDs) has none: m is negative.
+// and w in its L2; m-fastest where there are up to four rows of tiles (a panel's tiles of one n would often lie on two XCDs, which then both read their w), but not where k
+// is no multiple of 64 (panels): operands then go through the registers, and tiles of one n that run side by side took up to 1.12 times as long as those of one m (331 rows of
+// x, 12696 of w, k = 8480 160 -> 180 us; 150 such products otherwise the same). An id beyond the tiles (grids are whole rounds over the XCDs) has none: m is negative.
 struct TilePlace { int m, n; };
-__host__ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, int tiles_n) {
+__host__ __device__ __forceinline__ TilePlace tile_place(int id, int tiles_m, int tiles_n, bool panels = false) {
     const int total = tiles_m * tiles_n;
     const int xcds = 8;
     id = (id % xcds) * ((total + xcds - 1) / xcds) + id / xcds;
     if (id >= total) return TilePlace{-1, 0};
-    if (tiles_m <= 4) return TilePlace{id % tiles_m, id / tiles_m};     // (a panel's tiles of one n would often lie on two XCDs, which then both read their w)
+    if (tiles_m <= 4 && !panels) return TilePlace{id % tiles_m, id / tiles_m};
     constexpr int PANEL = 8;
     const int panel = id / (PANEL * tiles_m), in_panel = id % (PANEL * tiles_m);
     const int panel_width = min(PANEL, tiles_n - panel * PANEL);
@@ -91,7 +93,8 @@ __device__ __forceinline__ void gemm_tile(
     bf16* lds_b = lds_a + 2 * BM * PITCH;                              // [2][BN][PITCH]
 
     // (a float32 store may be of a part; of the others none is, and their way to the first loads is shorter)
-    const PartPlace of_part = MODE == MODE_STORE && sizeof(TO) == 4 ? part_place(id, blockIdx.y, tiles_m, tiles_n, by_parts) : PartPlace{tile_place(id, tiles_m, tiles_n), 0};
+    const PartPlace of_part = MODE == MODE_STORE && sizeof(TO) == 4 && DK != 0 ? part_place(id, blockIdx.y, tiles_m, tiles_n, by_parts)
+                                                                               : PartPlace{tile_place(id, tiles_m, tiles_n, DK == 0), 0};
     const TilePlace place = of_part.tile;
     if (place.m < 0) return;
     // (rows, columns and byte offsets fit 32 bits: the launcher checks)
@@ -1925,6 +1928,17 @@ extern "C" int xrt_linear_parts(int M, int N, int K, int mode, int whole_norm, i
     *rows = plan.tile;
     *columns = plan.columns;
     return plan.splits;
+}
+
+// The order in which the workgroups of one that is not cut take its tiles.
+extern "C" int xrt_linear_tile_order(int tiles_m, int tiles_n, int K, int* places, int room) {
+    if (tiles_m <= 0 || tiles_n <= 0 || (long)tiles_m * tiles_n >= (1L << 30) || K <= 0 || (room > 0 && !places)) return -1;
+    const int groups = (tiles_m * tiles_n + 7) / 8 * 8;
+    for (int i = 0; i < min(groups, room); ++i) {
+        const TilePlace place = tile_place(i, tiles_m, tiles_n, K % 64 != 0);
+        places[i] = place.m < 0 ? -1 : place.m * tiles_n + place.n;
+    }
+    return groups;
 }
 
 // The order in which the workgroups of a product cut along k take its tiles and parts.

@@ -136,6 +136,8 @@ int xrt_linear_part_order(int M, int N, int K, int mode, int whole_norm, int* by
 // The tiles of one that is not, more than 64 rows: 0, 1, 2: 256, 192 and 128 rows of x by 256 of w; 3: the first and the last of these in one launch; 4: 256 x 192; 5: 128 x 128;
 // 6: likewise in three stages; 7: 128 x 64 in four; 8, 9: 256 x 256 and 128 x 128 where k is no multiple of 64.
 int xrt_linear_tiles(int out_dtype, int M, int N, int K, int mode);
+// The order in which its workgroups take them, tiles_m rows of tiles_n: places[i] for the first `room` workgroups, row * tiles_n + column or -1 (none). Returns the workgroups.
+int xrt_linear_tile_order(int tiles_m, int tiles_n, int K, int* places, int room);
 // Whether a bfloat16 product of 17 to 256 rows of x (k a multiple of 64) asks for w past the caches: 1 where it cannot stay there until the next step. -1: no such product.
 int xrt_linear_past_caches(int M, int N, int K, int mode);
 // The tile that a float32 product of more than 16 rows of a takes (k a multiple of 4): its rows of a, and whether its wavefronts share
