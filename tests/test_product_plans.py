@@ -90,3 +90,12 @@ def test_every_tile_has_one_workgroup(lib, tiles_m, tiles_n, k, down):
     assert groups < tiles_m * tiles_n + 8 and sorted(place for place in places if place >= 0) == list(range(tiles_m * tiles_n))
     first, second = places[0], places[8]
     assert second - first == (1 if tiles_m == 1 or not down else tiles_n)
+
+
+# 17 to 64 rows, not gated: at most one workgroup to a compute unit, and fewer parts than that leaves room for where their sums cost more than they save.
+@pytest.mark.parametrize("m,n,k,parts", [(20, 12288, 8192, 2), (28, 9104, 16448, 3), (20, 12496, 7680, 2), (32, 12288, 14336, 2), (61, 4096, 1024, 4), (64, 3072, 2048, 4), (64, 3008, 1024, 4),
+                                         (61, 4096, 14336, 8), (40, 16384, 2048, 2), (40, 16512, 2048, 1)])
+def test_few_rows_take_no_more_than_a_workgroup_a_compute_unit(lib, m, n, k, parts):
+    rows, columns = ctypes.c_int(), ctypes.c_int()
+    assert lib.xrt_linear_parts(m, n, k, MODES["add"], 0, ctypes.byref(rows), ctypes.byref(columns)) == parts
+    assert parts * -(-n // columns.value) <= 256

@@ -1334,8 +1334,8 @@ long few_rows_parts_time(int M, long rows_w, int per, int parts) {
 }
 
 // Products of 17 to 64 rows of x that are not gated, in tiles of 64 x 128 and `parts` parts: microseconds, as above. Fitted to 6500 products (256 to 16384 rows
-// of w, k from 256 to 20000); of 2700 others the choice by it is 0.9 % off the best number of parts and takes 0.977 of as many parts as leave every compute
-// unit one workgroup (61 rows, 4096 rows of w, k = 1024 12.2 -> 10.4 us, 3072 rows, k = 2048 12.2 -> 11.9; 34 of them more than 1.04, up to 1.11).
+// of w, k from 256 to 20000); of 2700 others the choice by it is 0.9 % off the best number of parts (61 rows, 4096 rows of w, k = 1024 12.2 -> 10.4 us, 3072
+// rows, k = 2048 12.2 -> 11.9). 454 whose number of parts it changes take 0.87 of as many as leave every compute unit one workgroup, the worst 1.01.
 double few_rows_cut_time(int M, int N, int K, int steps, int parts) {
     const long tiles = (N + SPLIT_BN - 1) / SPLIT_BN;
     const long groups = part_ids(tiles, parts, deals_by_parts(SPLIT_BN, 1, tiles, K, parts));
@@ -1365,15 +1365,16 @@ SplitPlan plan_of(int M, int N, int K, int mode, bool whole_norm, bool fixed) {
             if (parts == 1 || narrow_gated_time(M, rows_w, units) < few_rows_parts_time(M, rows_w, per, (units + per - 1) / per)) { splits = 1; columns = 64; }
         }
     } else if (M <= SPLIT_BM) {
-        // As many parts as leave every compute unit one workgroup, or a number that is a twentieth better by the estimate. A product whose tiles leave no room for
-        // two parts is not cut, and what the parts sum up fits the fixed array of xrt_linear_static.
+        // As many parts as leave every compute unit one workgroup, or fewer that are a twentieth better by the estimate. (More, for a w so wide that they leave units idle: with w
+        // from memory, which bounds such a product, 346 drawn took 1.01 of the time, 124 of them over 1.03 and up to 1.12: 20 rows, 12288 rows of w, k = 8192 39.0 us in two
+        // parts, 42.0 in five.) A product whose tiles leave no room for two parts is not cut, and what the parts sum up fits the fixed array of xrt_linear_static.
         splits = min((int)(XRT_COMPUTE_UNITS / tiles_n), min(16, units));
         if (splits > 1) {
             splits = (units + per_part(splits) - 1) / per_part(splits);
             best = 0.95 * few_rows_cut_time(M, N, K, per_part(splits), splits);
         }
         for (int parts = 2; splits > 1 && parts <= 16; ++parts) {
-            if (!some(parts) || parts * tiles_n > 2 * XRT_COMPUTE_UNITS || (long)parts * M * N > XRT_LINEAR_STATIC_FLOATS) continue;
+            if (!some(parts) || parts * tiles_n > XRT_COMPUTE_UNITS || (long)parts * M * N > XRT_LINEAR_STATIC_FLOATS) continue;
             const double time = few_rows_cut_time(M, N, K, per_part(parts), parts);
             if (time < best) { best = time; splits = parts; }
         }
